@@ -60,10 +60,9 @@ int pcvl_perm_plan_create(const int32_t *h_n, const int64_t *h_offsets, int64_t 
                           int max_chunk_log2, pcvl_perm_plan *out);
 
 /* As pcvl_perm_plan_create, with the kernel variant of single-order batches:
- * 0 picks by order, 1 keeps Gray-code row 1 in VGPRs, 2 reads it from LDS
- * (fewer VGPRs, more resident waves); 3 and 4 are 1 and 2 with each row flip
- * fused into the preceding term.  Mixed-order batches ignore it.  Used by the
- * autotuner. */
+ * 0, 1 and 3 take the low rows of a block by order (two up to order 24, one
+ * above), 2 and 4 always one (fewer VGPRs, more resident waves).  Mixed-order
+ * batches ignore it.  Used by the autotuner. */
 int pcvl_perm_plan_create_ex(const int32_t *h_n, const int64_t *h_offsets, int64_t count,
                              int max_chunk_log2, int variant, pcvl_perm_plan *out);
 

@@ -1,8 +1,7 @@
 """Autotuner for the batched permanent kernel.
 
-For a batch shape (order n, batch size) it times every kernel variant (row 1
-of the Gray code in VGPRs or in LDS; row flips as a separate phase or fused
-into the product) and lane-chunk length that the plan API accepts, on the
+For a batch shape (order n, batch size) it times both kernel variants (low
+rows by order, or one low row) and every lane-chunk length that the plan API accepts, on the
 current GPU, and keeps the fastest; for a mixed-order batch it tunes the
 chunk length; for a SLOS plan it times every applicable layer kernel.
 Results are cached in a JSON file keyed by device name and shape, so tuning
@@ -19,7 +18,7 @@ from .permanent import PermanentPlan
 
 _CACHE_PATH = os.environ.get("PCVL_AUTOTUNE_CACHE",
                              os.path.join(os.path.expanduser("~"), ".cache", "perceval_amd", "autotune.json"))
-VARIANTS = (1, 2, 3, 4)
+VARIANTS = (1, 2)
 CHUNKS = (8, 10, 11, 12, 13, 14)
 
 

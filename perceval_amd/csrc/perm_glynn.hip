@@ -6,18 +6,19 @@
 // Step t of the binary-reflected Gray code flips row 1 + ctz(t); the sign of
 // term t is (-1)^t.
 //
-// Work decomposition (orders 9..28): the 2^{n-1} steps of a matrix are cut
-// into lane chunks of 2^c steps; one wavefront takes 64 consecutive chunks.
-// Because a chunk starts at a multiple of 2^c, every lane flips the same row
-// at the same step, so the flipped row is wave-uniform and is read from LDS
-// with a broadcast address; only the flip direction of rows >= 2 differs
-// between lanes and is applied as a per-lane +-1 FMA.  Row 1 (flipped every
-// other step) stays in VGPRs with compile-time flip directions.  Column sums
-// are rebuilt from scratch at each chunk start, which bounds the drift of the
-// running sums to 2^c updates.  One persistent launch drains a cost-sorted
-// queue of wave items of mixed order (largest first), then a second kernel
-// sums each matrix's wave partials in a fixed order (bit-reproducible).
-// Orders 0..8 take one matrix per thread.
+// Work decomposition (orders 9..28): the 2^{n-1} terms of a matrix are cut
+// into lane chunks of 2^c terms; one wavefront takes 64 consecutive chunks.
+// The lowest one or two rows after row 0 are the low rows: a block of 2 or 4
+// terms takes every low sign pattern, and the Gray code runs over the high
+// rows, one flip per block.  Because a chunk starts at a multiple of 2^c,
+// every lane flips the same high row at the same block, so the constants of a
+// flip are wave-uniform; only its direction differs between lanes and is
+// applied as a per-lane +-1 FMA.  The running sums are rebuilt from scratch at
+// each chunk start, which bounds their drift to 2^(c-2) or 2^(c-1) updates.
+// One persistent launch drains a cost-sorted queue of wave items of mixed
+// order (largest first), then a second kernel sums each matrix's wave partials
+// in a fixed order (bit-reproducible).  Orders 0..8 take one matrix per
+// thread.
 #include "common.h"
 #include "../../include/pcvl_hip.h"
 
@@ -45,214 +46,210 @@ struct PermItem {
     int32_t c;         // log2 of Gray-code steps per lane
 };
 
-// ---------------------------------------------------------------- products
+// --------------------------------------------------------------- wave path
 
-// Orders one Gray-code step after the previous term: the column sums are
-// passed through an empty asm that also reads the accumulator, so no update
-// of cs can be hoisted above the product that reads the old cs.  Without it
-// the optimiser computes all column-sum generations of an unrolled block
-// first and keeps them live together (4x the VGPRs, then spills).
-template <int N>
-__device__ __forceinline__ void pin_after(cd *cs, const cd &acc)
-{
-#pragma unroll
-    for (int j = 0; j < N; j++)
-        asm volatile("" : "+v"(cs[j].r), "+v"(cs[j].i) : "v"(acc.r), "v"(acc.i));
-}
-
-// prod_{j < N-1} cs[j] as four independent chains (ILP for FP64 latency).
-template <int N>
-__device__ __forceinline__ cd prod_head(const cd *cs)
-{
-    static_assert(N >= 5, "wave path needs N >= 5");
-    cd p0 = cs[0], p1 = cs[1], p2 = cs[2], p3 = cs[3];
-#pragma unroll
-    for (int j = 4; j < N - 1; j++) {
-        if ((j & 3) == 0) p0 = cmul(p0, cs[j]);
-        else if ((j & 3) == 1) p1 = cmul(p1, cs[j]);
-        else if ((j & 3) == 2) p2 = cmul(p2, cs[j]);
-        else p3 = cmul(p3, cs[j]);
-    }
-    return cmul(cmul(p0, p1), cmul(p2, p3));
-}
-
-template <int N>
-__device__ __forceinline__ void term_add(cd &acc, const cd *cs)
-{
-    cfma_acc(acc, prod_head<N>(cs), cs[N - 1]);
-}
-
-template <int N>
-__device__ __forceinline__ void term_sub(cd &acc, const cd *cs)
-{
-    cfms_acc(acc, prod_head<N>(cs), cs[N - 1]);
-}
-
-// cs += s * row, row read from LDS at a wave-uniform address.
-template <int N>
-__device__ __forceinline__ void flip_lds(cd *cs, const cd *__restrict__ row, double s)
-{
-#pragma unroll
-    for (int j = 0; j < N; j++) {
-        cd a = row[j];
-        cs[j].r = fma(s, a.r, cs[j].r);
-        cs[j].i = fma(s, a.i, cs[j].i);
-    }
-}
-
-// c += s * a, placed after dep: the empty asm makes the update wait for the
-// product that consumed the old c, so both generations are never live.
-__device__ __forceinline__ void flip_one(cd &c, const cd &a, double s, const cd &dep)
-{
-    // Not volatile: a volatile asm has unmodelled side effects, which would
-    // also stop the scheduler from issuing LDS reads of the row above it.
-    asm("" : "+v"(c.r), "+v"(c.i) : "v"(dep.r), "v"(dep.i));
-    c.r = fma(s, a.r, c.r);
-    c.i = fma(s, a.i, c.i);
-}
-
-// Returns v, made to look dependent on dep: keeps loads at an offset of v
+// Returns v, made to look dependent on dep: keeps LDS reads at an offset of v
 // inside the loop that dep counts (they would otherwise be hoisted as loop
-// invariant, holding whole rows in VGPRs).
-__device__ __forceinline__ int loop_variant(int v, uint32_t dep)
+// invariant, holding them in VGPRs).
+__device__ __forceinline__ int perm_loop_variant(int v, uint32_t dep)
 {
     asm("" : "+s"(v) : "s"(dep));
     return v;
 }
 
-// One Gray-code term (added, or subtracted when SUB) fused with the flip to the
-// next step: column j is flipped as soon as its product chain has consumed it,
-// so row reads from LDS spread over the product's arithmetic instead of
-// forming a separate latency-bound phase.
-template <int N, bool SUB>
-__device__ __forceinline__ void term_flip(cd &acc, cd *cs, const cd *row, double s)
-{
-    static_assert(N >= 9, "every chain needs a second factor");
-    cd p0 = cs[0], p1 = cs[1], p2 = cs[2], p3 = cs[3];
-#pragma unroll
-    for (int j = 4; j < N - 1; j++) {
-        cd &pk = ((j & 3) == 0) ? p0 : ((j & 3) == 1) ? p1 : ((j & 3) == 2) ? p2 : p3;
-        pk = cmul(pk, cs[j]);
-        if (j < 8) flip_one(cs[j - 4], row[j - 4], s, pk);
-        flip_one(cs[j], row[j], s, pk);
-    }
-    const cd h = cmul(cmul(p0, p1), cmul(p2, p3));
-    if (SUB) cfms_acc(acc, h, cs[N - 1]);
-    else cfma_acc(acc, h, cs[N - 1]);
-    flip_one(cs[N - 1], row[N - 1], s, acc);
-}
+// Entries of a row, read through the scalar data path (wave-uniform address).
+typedef const __attribute__((address_space(4))) double *scalar_row;
 
-// --------------------------------------------------------------- wave path
+// Low rows of an order: two up to order 24, one above.  The state of a pair is
+// 16 VGPRs with two (T, T', E_1, E_2) and 12 with one, and two waves per SIMD
+// leave 256: at order 25 two low rows would spill inside the loop.
+constexpr int PERM_LOW2_MAX = 24;
+constexpr int perm_low_rows(int n, bool one) { return (n <= PERM_LOW2_MAX && !one) ? 2 : 1; }
 
-// One wave item: 64 lanes x 2^c steps of one order-N matrix.  sA is this
-// wave's LDS slice holding 2*A (row-major).
-template <int N, int R1 = 0>
+// One wave item: 64 lanes x 2^c terms of one order-N matrix.
+//
+// The term's product over columns is taken in column pairs.  With T the column
+// sums at low-row signs +1, a pair's product is V = T T', and flipping low
+// row r takes V to V - E_r with E_r = 2 (s a'_r + s' a_r) (s: the sums without
+// row r).  E_r is linear in the sums, so a flip of high row q with new sign x
+// adds x H_r[q] to it, H_r[q] = 4 (a_q a'_r + a'_q a_r) a constant of the
+// matrix; likewise E_2 with low row 1 flipped is E_2 - G, G = H_2[1].  Per
+// pair and 2^LOW terms that is 4 operations for T T', 4 to flip T and T', 2
+// per E_r and 2 per further term (8 with the E_2 - G of two low rows): 20 for
+// 4 terms (LOW = 2), 12 for 2 (LOW = 1), where updating and multiplying the
+// two column sums of each term takes 8.  An order-N term costs 2.5 N (3 N)
+// + 4 (N/2 - 1) operations instead of 6 N - 4.
+//
+// sA is this wave's LDS slice (N x N).  High rows of the pair columns are
+// overwritten with H_1 | H_2 (H_1 | unused); the rows of A that a flip adds to
+// T come through the scalar cache, so the two constant streams (2 x 16 bytes
+// per column and flip) use different paths: LDS alone would need 93% of its
+// 128 B/clk at order 20.
+template <int N, int LOW>
 __device__ __forceinline__ cd glynn_wave_item(const double *__restrict__ mats, const PermItem &it, cd *sA)
 {
+    static_assert(N >= 9 && (LOW == 1 || LOW == 2), "unsupported order or low rows");
+    constexpr int P = N / 2;
+    constexpr bool ODD = (N & 1) != 0;
     const int lane = threadIdx.x & 63;
     const cd *A = reinterpret_cast<const cd *>(mats) + it.mat_off;
-    for (int e = lane; e < N * N; e += 64) {
-        cd v = A[e];
-        sA[e] = {2.0 * v.r, 2.0 * v.i};
-    }
+    for (int e = lane; e < N * N; e += 64) sA[e] = A[e];
     __syncthreads();
 
     const int c = it.c;
-    const uint64_t steps = 1ull << c;
-    const uint64_t base = (uint64_t)(it.chunk0 + (uint32_t)lane) << c;
+    const uint32_t blocks = 1u << (c - LOW);
+    const uint64_t base = (uint64_t)(it.chunk0 + (uint32_t)lane) << (c - LOW);   // in blocks of 2^LOW terms
     const uint64_t g0 = base ^ (base >> 1);
 
-    // Column sums for delta = Gray(base): cs_j = (1/2) sum_i delta_i (2 a_ij).
-    cd cs[N];
+    // Column sums at low signs +1 and the high signs of Gray(base).
+    cd T[N];
 #pragma unroll
-    for (int j = 0; j < N; j++) cs[j] = sA[j];
+    for (int j = 0; j < N; j++) {
+        T[j] = cadd(sA[j], sA[N + j]);
+        if constexpr (LOW == 2) T[j] = cadd(T[j], sA[2 * N + j]);
+        if (j & 1) asm volatile("" ::: "memory");   // a few reads in flight, not all rows in VGPRs
+    }
 #pragma unroll 1
-    for (int i = 1; i < N; i++) {
-        const double d = ((g0 >> (i - 1)) & 1) ? -1.0 : 1.0;
+    for (int i = LOW + 1; i < N; i++) {
+        const double d = ((g0 >> (i - LOW - 1)) & 1) ? -1.0 : 1.0;
         const cd *row = sA + i * N;
 #pragma unroll
         for (int j = 0; j < N; j++) {
-            cd a = row[j];
-            cs[j].r = fma(d, a.r, cs[j].r);
-            cs[j].i = fma(d, a.i, cs[j].i);
+            T[j].r = fma(d, row[j].r, T[j].r);
+            T[j].i = fma(d, row[j].i, T[j].i);
         }
     }
+    // 2 (s a'_r + s' a_r), s = T - a_r
+    auto deriv = [&](int p, int r) {
+        const cd a = sA[r * N + 2 * p], b = sA[r * N + 2 * p + 1];
+        const cd s = {T[2 * p].r - a.r, T[2 * p].i - a.i}, t = {T[2 * p + 1].r - b.r, T[2 * p + 1].i - b.i};
+        cd e = cmul(s, b);
+        cfma_acc(e, t, a);
+        return cd{2.0 * e.r, 2.0 * e.i};
+    };
+    cd E1[P], E2[LOW == 2 ? P : 1];
 #pragma unroll
-    for (int j = 0; j < N; j++) cs[j] = {0.5 * cs[j].r, 0.5 * cs[j].i};
+    for (int p = 0; p < P; p++) {
+        E1[p] = deriv(p, 1);
+        if constexpr (LOW == 2) E2[p] = deriv(p, 2);
+        asm volatile("" ::: "memory");
+    }
+    __syncthreads();
+    // In place: H_1, H_2 over the pair columns of the high rows; with two low
+    // rows G goes over row 0, and rows 1, 2 stay (2 a of an odd last column).
+    auto pair_const = [&](int q, int r, int p) {
+        const cd aq = sA[q * N + 2 * p], bq = sA[q * N + 2 * p + 1];
+        const cd ar = sA[r * N + 2 * p], br = sA[r * N + 2 * p + 1];
+        cd h = cmul(aq, br);
+        cfma_acc(h, bq, ar);
+        return cd{4.0 * h.r, 4.0 * h.i};
+    };
+    for (int e = lane; e < (N - 1 - LOW) * P; e += 64) {
+        const int q = LOW + 1 + e / P, p = e % P;
+        const cd h1 = pair_const(q, 1, p);
+        cd h2 = h1;
+        if constexpr (LOW == 2) h2 = pair_const(q, 2, p);
+        sA[q * N + 2 * p] = h1;
+        sA[q * N + 2 * p + 1] = h2;
+    }
+    if constexpr (LOW == 2) {
+        if (lane < P) sA[lane] = pair_const(2, 1, lane);
+    }
+    __syncthreads();
+    cd o1 = {0.0, 0.0}, o2 = {0.0, 0.0};   // 2 a_1, 2 a_2 of an odd last column
+    if constexpr (ODD) {
+        o1 = {2.0 * sA[N + N - 1].r, 2.0 * sA[N + N - 1].i};
+        if constexpr (LOW == 2) o2 = {2.0 * sA[2 * N + N - 1].r, 2.0 * sA[2 * N + N - 1].i};
+    }
 
-    // Row 1 flips every other step: keep it in VGPRs (R1 = 1, 3), read it
-    // from LDS like the other rows (R1 = 2, 4: fewer VGPRs and more waves), or
-    // pick by order (R1 = 0: in VGPRs up to order 26, the largest that fits
-    // without spilling; at orders 23-24 that is 5% faster than three waves
-    // per SIMD reading it from LDS).  R1 = 3, 4 fuse each flip into the
-    // preceding term.
-    constexpr bool kRow1InRegs = (R1 == 1) || (R1 == 3) || (R1 == 0 && N <= 26);
-    constexpr bool kFused = (R1 >= 3);
-    cd r1[kRow1InRegs ? N : 1];
-    if constexpr (kRow1InRegs) {
+    // Blocks alternate in sign (the parity of the high Gray bits): instead of
+    // a sign, each block starts its sums from the negated sums so far.
+    cd accp = {0.0, 0.0}, accm = {0.0, 0.0};   // terms of even / odd low parity
+    for (uint32_t v = 0; v < blocks; v++) {
+        // the flip that follows: high row LOW + 1 + b.  On the last block this
+        // is the first flip of the next chunk (row c + 1 <= N - 6, in bounds);
+        // its result is discarded.
+        const int b = __builtin_ctz(v + 1);
+        const uint64_t t = base + v + 1;
+        const double s1 = (((t >> b) ^ (t >> (b + 1))) & 1) ? -1.0 : 1.0;
+        const double s2 = s1 + s1;
+        const cd *hrow = sA + (b + LOW + 1) * N;
+        const scalar_row arow = (scalar_row)(uintptr_t)(A + (size_t)(b + LOW + 1) * N);
+        const cd *grow = sA + perm_loop_variant(0, v);
+        cd q[1 << LOW];
 #pragma unroll
-        for (int j = 0; j < N; j++) r1[j] = sA[N + j];
-    }
-
-    cd acc = {0.0, 0.0};
-    if constexpr (kFused) {
-        for (uint64_t u = 0; u < steps; u += 4) {
-            const cd *row1 = kRow1InRegs ? r1 : sA + loop_variant(N, (uint32_t)u);
-            term_flip<N, false>(acc, cs, row1, -1.0);          // t = base+u, then row 1 -> delta -1
-            uint64_t t2 = base + u + 2;
-            const double s2 = (((t2 >> 1) ^ (t2 >> 2)) & 1) ? -1.0 : 1.0;
-            term_flip<N, true>(acc, cs, sA + loop_variant(2 * N, (uint32_t)u), s2);   // t+1, then row 2
-            term_flip<N, false>(acc, cs, row1, 1.0);           // t+2, then row 1 -> delta +1
-            // t+3, then row 1 + ctz(u+4) >= 3 (on the last block: first step of
-            // the next chunk, row c+1 <= N-6, result discarded)
-            const int b = __builtin_ctzll(u + 4);
-            uint64_t t4 = base + u + 4;
-            const double s4 = (((t4 >> b) ^ (t4 >> (b + 1))) & 1) ? -1.0 : 1.0;
-            term_flip<N, true>(acc, cs, sA + (b + 1) * N, s4);
-        }
-        __syncthreads();
-        return acc;
-    }
-    // Steps are taken four at a time; c >= 2 so base has two zero low bits.
-    for (uint64_t u = 0; u < steps; u += 4) {
-        term_add<N>(acc, cs);                 // t = base+u, even
-        pin_after<N>(cs, acc);
-        if constexpr (kRow1InRegs) {          // t = base+u+1: row 1 -> delta -1
+        for (int p = 0; p < P; p++) {
+            cd &x = T[2 * p], &y = T[2 * p + 1];
+            cd V[1 << LOW];   // signs of the low rows: ++, -+, (+-, --)
+            V[0] = cmul(x, y);
+            V[1] = {V[0].r - E1[p].r, V[0].i - E1[p].i};
+            if constexpr (LOW == 2) {
+                const cd g = grow[p];
+                const cd e = {E2[p].r - g.r, E2[p].i - g.i};
+                V[2] = {V[0].r - E2[p].r, V[0].i - E2[p].i};
+                V[3] = {V[1].r - e.r, V[1].i - e.i};
+            }
+            // T and E of the pair are free once its values are formed: the
+            // empty asm keeps the flips behind them, or both generations of
+            // many pairs would be live together
+            constexpr int last = (1 << LOW) - 1;
+            asm("" : "+v"(x.r), "+v"(x.i), "+v"(y.r), "+v"(y.i), "+v"(E1[p].r), "+v"(E1[p].i)
+                : "v"(V[1].r), "v"(V[last].i), "v"(V[last].r), "v"(V[1].i));
+            if constexpr (LOW == 2) asm("" : "+v"(E2[p].r), "+v"(E2[p].i) : "v"(V[2].r), "v"(V[2].i), "v"(V[3].r));
+            x.r = fma(s2, arow[4 * p], x.r);
+            x.i = fma(s2, arow[4 * p + 1], x.i);
+            y.r = fma(s2, arow[4 * p + 2], y.r);
+            y.i = fma(s2, arow[4 * p + 3], y.i);
+            const cd h1 = hrow[2 * p];
+            E1[p].r = fma(s1, h1.r, E1[p].r);
+            E1[p].i = fma(s1, h1.i, E1[p].i);
+            if constexpr (LOW == 2) {
+                const cd h2 = hrow[2 * p + 1];
+                E2[p].r = fma(s1, h2.r, E2[p].r);
+                E2[p].i = fma(s1, h2.i, E2[p].i);
+            }
+            if (p == 0) {
 #pragma unroll
-            for (int j = 0; j < N; j++) { cs[j].r -= r1[j].r; cs[j].i -= r1[j].i; }
-        } else {
-            flip_lds<N>(cs, sA + N, -1.0);
-        }
-        term_sub<N>(acc, cs);
-        pin_after<N>(cs, acc);
-        {                                     // t = base+u+2: row 2
-            uint64_t t = base + u + 2;
-            double s = (((t >> 1) ^ (t >> 2)) & 1) ? -1.0 : 1.0;
-            flip_lds<N>(cs, sA + 2 * N, s);
-        }
-        term_add<N>(acc, cs);
-        pin_after<N>(cs, acc);
-        if constexpr (kRow1InRegs) {          // t = base+u+3: row 1 -> delta +1
+                for (int k = 0; k < (1 << LOW); k++) q[k] = V[k];
+            } else if (p < P - 1 || ODD) {
 #pragma unroll
-            for (int j = 0; j < N; j++) { cs[j].r += r1[j].r; cs[j].i += r1[j].i; }
-        } else {
-            flip_lds<N>(cs, sA + N, 1.0);
+                for (int k = 0; k < (1 << LOW); k++) q[k] = cmul(q[k], V[k]);
+            } else {
+                accp = {-accp.r, -accp.i};
+                accm = {-accm.r, -accm.i};
+                cfma_acc(accp, q[0], V[0]);
+                cfma_acc(accm, q[1], V[1]);
+                if constexpr (LOW == 2) {
+                    cfma_acc(accm, q[2], V[2]);
+                    cfma_acc(accp, q[3], V[3]);
+                }
+            }
+            // keeps the next pair's products behind this one's, so that one
+            // pair's values are live at a time
+            if (p + 1 < P) {
+                cd &nx = T[2 * p + 2];
+                asm("" : "+v"(nx.r), "+v"(nx.i) : "v"(q[0].r), "v"(q[(1 << LOW) - 1].i));
+            }
         }
-        term_sub<N>(acc, cs);
-        pin_after<N>(cs, acc);
-        {
-            // t = base+u+4: row 1 + ctz(u+4) >= 3.  On the last block this is
-            // the first step of the next chunk (row c+1 <= N-6, in bounds); its
-            // result is discarded, and taking it unconditionally keeps the
-            // loop body a single basic block.
-            const int b = __builtin_ctzll(u + 4);
-            uint64_t t = base + u + 4;
-            double s = (((t >> b) ^ (t >> (b + 1))) & 1) ? -1.0 : 1.0;
-            flip_lds<N>(cs, sA + (b + 1) * N, s);
+        if constexpr (ODD) {
+            cd &x = T[N - 1];
+            const cd m1 = {x.r - o1.r, x.i - o1.i};
+            accp = {-accp.r, -accp.i};
+            accm = {-accm.r, -accm.i};
+            cfma_acc(accp, q[0], x);
+            cfma_acc(accm, q[1], m1);
+            if constexpr (LOW == 2) {
+                cfma_acc(accm, q[2], cd{x.r - o2.r, x.i - o2.i});
+                cfma_acc(accp, q[3], cd{m1.r - o2.r, m1.i - o2.i});
+            }
+            x.r = fma(s2, arow[2 * (N - 1)], x.r);
+            x.i = fma(s2, arow[2 * (N - 1) + 1], x.i);
         }
     }
     __syncthreads();   // sA is reused by the next item of this wave
-    return acc;
+    const double sg = (blocks & 1) ? 1.0 : -1.0;   // the last block's sign (base is even unless it is the only one)
+    const double sb = (blocks == 1 && (base & 1)) ? -sg : sg;
+    return {sb * (accp.r - accm.r), sb * (accp.i - accm.i)};
 }
 
 __device__ __forceinline__ cd wave_sum(cd v)
@@ -265,21 +262,21 @@ __device__ __forceinline__ cd wave_sum(cd v)
     return v;
 }
 
-template <int NLO, int NHI, int R1>
+template <int NLO, int NHI, bool ONE>
 __device__ __forceinline__ cd dispatch_item(const double *__restrict__ mats, const PermItem &it, cd *sA)
 {
     if constexpr (NLO > NHI) {
         return {0.0, 0.0};
     } else {
-        if (it.n == NLO) return glynn_wave_item<NLO, R1>(mats, it, sA);
-        return dispatch_item<NLO + 1, NHI, R1>(mats, it, sA);
+        if (it.n == NLO) return glynn_wave_item<NLO, perm_low_rows(NLO, ONE)>(mats, it, sA);
+        return dispatch_item<NLO + 1, NHI, ONE>(mats, it, sA);
     }
 }
 
 // Persistent wave kernel: one wavefront per workgroup, items pulled from a
 // cost-sorted queue with an atomic cursor.  The cursor is returned to zero by
 // perm_finalize so the same plan can be replayed (also inside a HIP graph).
-template <int NLO, int NHI, int R1 = 0>
+template <int NLO, int NHI, bool ONE = false>
 __global__ void __launch_bounds__(64, 2) perm_wave_kernel(const double *__restrict__ mats,
                                                        const PermItem *__restrict__ items, int64_t nitems,
                                                        unsigned long long *cursor, cd *__restrict__ partials)
@@ -309,7 +306,7 @@ __global__ void __launch_bounds__(64, 2) perm_wave_kernel(const double *__restri
             it.c = __builtin_amdgcn_readfirstlane(raw.c);
         }
         if (it.n < NLO || it.n > NHI || it.c < 2 || it.c > it.n - 7) continue;
-        cd v = dispatch_item<NLO, NHI, R1>(mats, it, sA);
+        cd v = dispatch_item<NLO, NHI, ONE>(mats, it, sA);
         v = wave_sum(v);
         if (threadIdx.x == 0) partials[it.slot] = v;
     }
@@ -400,7 +397,7 @@ struct PermPlanImpl {
     int64_t nbig = 0;          // items of orders 29..32, after the nitems others in the queue
     int grid_big = 0;
     int single_n = 0;          // order shared by every wave item, or 0 if mixed
-    int variant = 0;           // 0 auto, 1..4 (single-order plans): row 1 in VGPRs / LDS, separate / fused flips
+    int variant = 0;           // 0, 1, 3: low rows by order; 2, 4 (single-order plans): one low row
     int grid = 0;
     PermItem *d_items = nullptr;
     unsigned long long *d_cursor = nullptr;   // [0]: the queue of orders <= 28, [1]: orders 29..32
@@ -422,21 +419,23 @@ static int pick_chunk_log2(int n, int max_c)
     return c;
 }
 
-template <int NLO, int NHI, int R1>
+template <int NLO, int NHI, bool ONE>
 static int launch_wave(const PermPlanImpl *p, const double *mats, hipStream_t st, const PermItem *items,
                        int64_t nitems, unsigned long long *cursor, int grid)
 {
-    hipLaunchKernelGGL((perm_wave_kernel<NLO, NHI, R1>), dim3(grid), dim3(64), 0, st, mats, items, nitems, cursor,
+    hipLaunchKernelGGL((perm_wave_kernel<NLO, NHI, ONE>), dim3(grid), dim3(64), 0, st, mats, items, nitems, cursor,
                        p->d_partials);
     PCVL_HIP_CHECK(hipGetLastError());
     return OK;
 }
 
-template <int NLO, int NHI, int R1>
+template <int NLO, int NHI, bool ONE>
 static int launch_wave(const PermPlanImpl *p, const double *mats, hipStream_t st)
 {
-    return launch_wave<NLO, NHI, R1>(p, mats, st, p->d_items, p->nitems, p->d_cursor, p->grid);
+    return launch_wave<NLO, NHI, ONE>(p, mats, st, p->d_items, p->nitems, p->d_cursor, p->grid);
 }
+
+static bool perm_one_low_row(int variant) { return variant == 2 || variant == 4; }
 
 template <int N>
 static int launch_single(PermPlanImpl *p, const double *mats, hipStream_t st)
@@ -446,11 +445,10 @@ static int launch_single(PermPlanImpl *p, const double *mats, hipStream_t st)
         return ERR_ARG;
     } else {
         if (p->single_n == N) {
-            if (p->variant == 1) return launch_wave<N, N, 1>(p, mats, st);
-            if (p->variant == 2) return launch_wave<N, N, 2>(p, mats, st);
-            if (p->variant == 3) return launch_wave<N, N, 3>(p, mats, st);
-            if (p->variant == 4) return launch_wave<N, N, 4>(p, mats, st);
-            return launch_wave<N, N, 0>(p, mats, st);
+            if constexpr (N <= PERM_LOW2_MAX) {
+                if (perm_one_low_row(p->variant)) return launch_wave<N, N, true>(p, mats, st);
+            }
+            return launch_wave<N, N, false>(p, mats, st);
         }
         return launch_single<N + 1>(p, mats, st);
     }
@@ -463,11 +461,10 @@ static const void *single_kernel_ptr(int n, int variant)
         return nullptr;
     } else {
         if (n == N) {
-            if (variant == 1) return reinterpret_cast<const void *>(&perm_wave_kernel<N, N, 1>);
-            if (variant == 2) return reinterpret_cast<const void *>(&perm_wave_kernel<N, N, 2>);
-            if (variant == 3) return reinterpret_cast<const void *>(&perm_wave_kernel<N, N, 3>);
-            if (variant == 4) return reinterpret_cast<const void *>(&perm_wave_kernel<N, N, 4>);
-            return reinterpret_cast<const void *>(&perm_wave_kernel<N, N, 0>);
+            if constexpr (N <= PERM_LOW2_MAX) {
+                if (perm_one_low_row(variant)) return reinterpret_cast<const void *>(&perm_wave_kernel<N, N, true>);
+            }
+            return reinterpret_cast<const void *>(&perm_wave_kernel<N, N, false>);
         }
         return single_kernel_ptr<N + 1>(n, variant);
     }
@@ -547,12 +544,12 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
     int rw = 0, rwb = 0;
     if (nmax >= 0) {
         const void *kp = single_n ? single_kernel_ptr<PERM_WAVE_MIN>(single_n, kvariant)
-                                  : reinterpret_cast<const void *>(&perm_wave_kernel<PERM_WAVE_MIN, PERM_WAVE_MAX, 0>);
+                                  : reinterpret_cast<const void *>(&perm_wave_kernel<PERM_WAVE_MIN, PERM_WAVE_MAX, false>);
         int rc = resident_waves(kp, &rw);
         if (rc != OK) return rc;
     }
     if (any_big) {
-        int rc = resident_waves(reinterpret_cast<const void *>(&perm_wave_kernel<PERM_BIG_MIN, PERM_BIG_MAX, 0>), &rwb);
+        int rc = resident_waves(reinterpret_cast<const void *>(&perm_wave_kernel<PERM_BIG_MIN, PERM_BIG_MAX, false>), &rwb);
         if (rc != OK) return rc;
     }
     // Tail refinement, per launch: the matrices whose items form the last
@@ -724,11 +721,11 @@ extern "C" int pcvl_perm_plan_execute(pcvl_perm_plan plan, const double *d_mats,
     if (p.nwave_mats > 0) {
         int rc = OK;
         if (p.nbig > 0)   // orders 29..32 first: the longest items
-            rc = launch_wave<PERM_BIG_MIN, PERM_BIG_MAX, 0>(&p, d_mats, stream, p.d_items + p.nitems, p.nbig,
+            rc = launch_wave<PERM_BIG_MIN, PERM_BIG_MAX, false>(&p, d_mats, stream, p.d_items + p.nitems, p.nbig,
                                                             p.d_cursor + 1, p.grid_big);
         if (rc == OK && p.nitems > 0)
             rc = p.single_n ? launch_single<PERM_WAVE_MIN>(&p, d_mats, stream)
-                            : launch_wave<PERM_WAVE_MIN, PERM_WAVE_MAX, 0>(&p, d_mats, stream);
+                            : launch_wave<PERM_WAVE_MIN, PERM_WAVE_MAX, false>(&p, d_mats, stream);
         if (rc != OK) return rc;
         int blocks = (int)((p.nwave_mats + 255) / 256);
         hipLaunchKernelGGL(perm_finalize_kernel, dim3(blocks), dim3(256), 0, stream, p.d_wave_idx,

@@ -77,6 +77,26 @@ def test_kernel_variants_vs_oracle(gpu, n, variant):
             assert _rel(g, r) < REL_TOL, (n, variant, chunk, g, r)
 
 
+@pytest.mark.parametrize("n", [9, 10, 19, 24, 25, 26])
+def test_block_edges_vs_oracle(gpu, n):
+    """Orders at the edges of the two kernels of the wave path (odd and even
+    columns, two low rows up to order 24, one above), with one block per lane
+    (its sign is the lane's), two, and many; Gaussian entries of uneven column
+    scale, so that a pair's products and their updates differ by 10^6."""
+    import torch
+    from perceval_amd.permanent import PermanentPlan, pack
+    rng = np.random.RandomState(900 + n)
+    mats = [(rng.randn(n, n) + 1j * rng.randn(n, n)) * 10.0 ** rng.uniform(-3, 3, size=n) for _ in range(2)]
+    orders, flat = pack(mats)
+    ref = _oracle(mats)
+    for chunk in (2, 3, 11):
+        plan = PermanentPlan(orders, max_chunk_log2=chunk)
+        got = plan(torch.from_numpy(flat).cuda()).cpu().numpy()
+        plan.close()
+        for g, r in zip(got, ref):
+            assert _rel(g, r) < REL_TOL, (n, chunk, g, r)
+
+
 def test_mixed_batch_config_shape(gpu):
     # Same generator as the batched-permanent workload (n uniform in 12..24 from
     # one 64x64 Haar unitary), 4096 matrices; every matrix of order <= 16 and a
