@@ -131,8 +131,12 @@ __device__ __forceinline__ cd glynn_wave_item(const double *__restrict__ mats, c
 #pragma unroll
     for (int p = 0; p < P; p++) {
         E1[p] = deriv(p, 1);
-        if constexpr (LOW == 2) E2[p] = deriv(p, 2);
-        asm volatile("" ::: "memory");
+        // formed here, not sunk past the barriers with every row it reads live
+        asm volatile("" : "+v"(E1[p].r), "+v"(E1[p].i) : : "memory");
+        if constexpr (LOW == 2) {
+            E2[p] = deriv(p, 2);
+            asm volatile("" : "+v"(E2[p].r), "+v"(E2[p].i) : : "memory");
+        }
     }
     __syncthreads();
     // In place: H_1, H_2 over the pair columns of the high rows; with two low
@@ -162,51 +166,94 @@ __device__ __forceinline__ cd glynn_wave_item(const double *__restrict__ mats, c
         if constexpr (LOW == 2) o2 = {2.0 * sA[2 * N + N - 1].r, 2.0 * sA[2 * N + N - 1].i};
     }
 
+    // The constants of a pair's flip: H_1, H_2 and G from LDS, the rows of A
+    // through the scalar cache.
+    constexpr bool AHEAD = N <= 22;   // above, H_2 and G are read in their own turn: 8 VGPRs less
+    struct PairConst {
+        cd h1, h2, g;
+        double a[4];
+    };
+    auto load_pair = [&](PairConst &k, int b, int p, uint32_t v) {
+        const cd *hrow = sA + (b + LOW + 1) * N;
+        const scalar_row arow = (scalar_row)(uintptr_t)(A + (size_t)(b + LOW + 1) * N);
+        k.h1 = hrow[2 * p];
+        if constexpr (LOW == 2) {
+            if constexpr (AHEAD) {
+                k.h2 = hrow[2 * p + 1];
+                k.g = (sA + perm_loop_variant(0, v))[p];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) k.a[i] = arow[4 * p + i];
+    };
     // Blocks alternate in sign (the parity of the high Gray bits): instead of
     // a sign, each block starts its sums from the negated sums so far.
     cd accp = {0.0, 0.0}, accm = {0.0, 0.0};   // terms of even / odd low parity
+    PairConst kc, kn;
+    load_pair(kn, 0, 0, 0);
     for (uint32_t v = 0; v < blocks; v++) {
         // the flip that follows: high row LOW + 1 + b.  On the last block this
         // is the first flip of the next chunk (row c + 1 <= N - 6, in bounds);
         // its result is discarded.
-        const int b = __builtin_ctz(v + 1);
+        const int b = __builtin_ctz(v + 1), bnext = __builtin_ctz(v + 2);
         const uint64_t t = base + v + 1;
         const double s1 = (((t >> b) ^ (t >> (b + 1))) & 1) ? -1.0 : 1.0;
         const double s2 = s1 + s1;
-        const cd *hrow = sA + (b + LOW + 1) * N;
-        const scalar_row arow = (scalar_row)(uintptr_t)(A + (size_t)(b + LOW + 1) * N);
-        const cd *grow = sA + perm_loop_variant(0, v);
         cd q[1 << LOW];
 #pragma unroll
         for (int p = 0; p < P; p++) {
+            // A pair's constants are read while the pair before it is worked
+            // on: wait for this pair's, start the next one's, then compute.
+            // The scheduling barriers keep that order (and the values of one
+            // pair at a time in VGPRs); without them a read sits 2-4
+            // instructions before its use, 30 times per block.
+            kc = kn;
+            asm volatile("" : "+v"(kc.h1.r), "+v"(kc.h1.i), "+s"(kc.a[0]), "+s"(kc.a[1]), "+s"(kc.a[2]), "+s"(kc.a[3]));
+            if constexpr (LOW == 2) {
+                if constexpr (AHEAD) {
+                    asm volatile("" : "+v"(kc.h2.r), "+v"(kc.h2.i), "+v"(kc.g.r), "+v"(kc.g.i));
+                } else {
+                    kc.g = (sA + perm_loop_variant(0, v))[p];
+                    kc.h2 = (sA + (b + LOW + 1) * N)[2 * p + 1];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (p + 1 < P) load_pair(kn, b, p + 1, v);
+            else load_pair(kn, bnext, 0, v);
+            double oa[2];
+            if constexpr (ODD) {
+                if (p == P - 1) {
+                    const scalar_row arow = (scalar_row)(uintptr_t)(A + (size_t)(b + LOW + 1) * N);
+                    oa[0] = arow[2 * (N - 1)];
+                    oa[1] = arow[2 * (N - 1) + 1];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
             cd &x = T[2 * p], &y = T[2 * p + 1];
             cd V[1 << LOW];   // signs of the low rows: ++, -+, (+-, --)
             V[0] = cmul(x, y);
             V[1] = {V[0].r - E1[p].r, V[0].i - E1[p].i};
             if constexpr (LOW == 2) {
-                const cd g = grow[p];
-                const cd e = {E2[p].r - g.r, E2[p].i - g.i};
+                const cd e = {E2[p].r - kc.g.r, E2[p].i - kc.g.i};
                 V[2] = {V[0].r - E2[p].r, V[0].i - E2[p].i};
                 V[3] = {V[1].r - e.r, V[1].i - e.i};
             }
-            // T and E of the pair are free once its values are formed: the
-            // empty asm keeps the flips behind them, or both generations of
-            // many pairs would be live together
+            // T and E of the pair are free once its values are formed: flip
+            // them to the next block (the empty asm keeps the flips behind
+            // the values, so that they happen in place)
             constexpr int last = (1 << LOW) - 1;
             asm("" : "+v"(x.r), "+v"(x.i), "+v"(y.r), "+v"(y.i), "+v"(E1[p].r), "+v"(E1[p].i)
-                : "v"(V[1].r), "v"(V[last].i), "v"(V[last].r), "v"(V[1].i));
-            if constexpr (LOW == 2) asm("" : "+v"(E2[p].r), "+v"(E2[p].i) : "v"(V[2].r), "v"(V[2].i), "v"(V[3].r));
-            x.r = fma(s2, arow[4 * p], x.r);
-            x.i = fma(s2, arow[4 * p + 1], x.i);
-            y.r = fma(s2, arow[4 * p + 2], y.r);
-            y.i = fma(s2, arow[4 * p + 3], y.i);
-            const cd h1 = hrow[2 * p];
-            E1[p].r = fma(s1, h1.r, E1[p].r);
-            E1[p].i = fma(s1, h1.i, E1[p].i);
+                : "v"(V[1].r), "v"(V[1].i), "v"(V[last].r), "v"(V[last].i));
+            if constexpr (LOW == 2) asm("" : "+v"(E2[p].r), "+v"(E2[p].i) : "v"(V[2].r), "v"(V[2].i), "v"(V[3].r), "v"(V[3].i));
+            x.r = fma(s2, kc.a[0], x.r);
+            x.i = fma(s2, kc.a[1], x.i);
+            y.r = fma(s2, kc.a[2], y.r);
+            y.i = fma(s2, kc.a[3], y.i);
+            E1[p].r = fma(s1, kc.h1.r, E1[p].r);
+            E1[p].i = fma(s1, kc.h1.i, E1[p].i);
             if constexpr (LOW == 2) {
-                const cd h2 = hrow[2 * p + 1];
-                E2[p].r = fma(s1, h2.r, E2[p].r);
-                E2[p].i = fma(s1, h2.i, E2[p].i);
+                E2[p].r = fma(s1, kc.h2.r, E2[p].r);
+                E2[p].i = fma(s1, kc.h2.i, E2[p].i);
             }
             if (p == 0) {
 #pragma unroll
@@ -224,26 +271,24 @@ __device__ __forceinline__ cd glynn_wave_item(const double *__restrict__ mats, c
                     cfma_acc(accp, q[3], V[3]);
                 }
             }
-            // keeps the next pair's products behind this one's, so that one
-            // pair's values are live at a time
-            if (p + 1 < P) {
-                cd &nx = T[2 * p + 2];
-                asm("" : "+v"(nx.r), "+v"(nx.i) : "v"(q[0].r), "v"(q[(1 << LOW) - 1].i));
+            if constexpr (ODD) {
+                if (p == P - 1) {
+                    cd &z = T[N - 1];
+                    const cd m1 = {z.r - o1.r, z.i - o1.i};
+                    accp = {-accp.r, -accp.i};
+                    accm = {-accm.r, -accm.i};
+                    cfma_acc(accp, q[0], z);
+                    cfma_acc(accm, q[1], m1);
+                    if constexpr (LOW == 2) {
+                        cfma_acc(accm, q[2], cd{z.r - o2.r, z.i - o2.i});
+                        cfma_acc(accp, q[3], cd{m1.r - o2.r, m1.i - o2.i});
+                    }
+                    asm("" : "+v"(z.r), "+v"(z.i) : "v"(accp.r), "v"(accp.i), "v"(accm.r), "v"(accm.i));
+                    z.r = fma(s2, oa[0], z.r);
+                    z.i = fma(s2, oa[1], z.i);
+                }
             }
-        }
-        if constexpr (ODD) {
-            cd &x = T[N - 1];
-            const cd m1 = {x.r - o1.r, x.i - o1.i};
-            accp = {-accp.r, -accp.i};
-            accm = {-accm.r, -accm.i};
-            cfma_acc(accp, q[0], x);
-            cfma_acc(accm, q[1], m1);
-            if constexpr (LOW == 2) {
-                cfma_acc(accm, q[2], cd{x.r - o2.r, x.i - o2.i});
-                cfma_acc(accp, q[3], cd{m1.r - o2.r, m1.i - o2.i});
-            }
-            x.r = fma(s2, arow[2 * (N - 1)], x.r);
-            x.i = fma(s2, arow[2 * (N - 1) + 1], x.i);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     __syncthreads();   // sA is reused by the next item of this wave
