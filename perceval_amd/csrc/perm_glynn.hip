@@ -60,9 +60,10 @@ __device__ __forceinline__ int perm_loop_variant(int v, uint32_t dep)
 // Entries of a row, read through the scalar data path (wave-uniform address).
 typedef const __attribute__((address_space(4))) double *scalar_row;
 
-// Low rows of an order: two up to order 24, one above.  The state of a pair is
-// 16 VGPRs with two (T, T', E_1, E_2) and 12 with one, and two waves per SIMD
-// leave 256: at order 25 two low rows would spill inside the loop.
+// Low rows of an order: two up to order 24, one above.  A pair's state is 16
+// VGPRs with two (T, T', E_1, E_2) and 12 with one, and two waves per SIMD
+// leave 256: 256 order-24 matrices take 6.80 ms with two (8.83 before), orders
+// 25 and up would spill inside the block loop.
 constexpr int PERM_LOW2_MAX = 24;
 constexpr int perm_low_rows(int n, bool one) { return (n <= PERM_LOW2_MAX && !one) ? 2 : 1; }
 
@@ -78,7 +79,12 @@ constexpr int perm_low_rows(int n, bool one) { return (n <= PERM_LOW2_MAX && !on
 // per E_r and 2 per further term (8 with the E_2 - G of two low rows): 20 for
 // 4 terms (LOW = 2), 12 for 2 (LOW = 1), where updating and multiplying the
 // two column sums of each term takes 8.  An order-N term costs 2.5 N (3 N)
-// + 4 (N/2 - 1) operations instead of 6 N - 4.
+// + 4 (N/2 - 1) operations instead of 6 N - 4: 86 instead of 116 at order 20.
+// Bound by FP64 issue: 4,096 order-20 matrices take 5.82 ms (8.00 ms with one
+// update and product per column and term), 1,000 of orders 12..24 3.99 ms
+// (5.22 ms); 6.50 and 4.01 ms with each constant read just before its use.
+// The sums are updated once per block, so they drift less: error against
+// direct float64 sums 3.3e-14 (9.9e-14) at order 20.
 //
 // sA is this wave's LDS slice (N x N).  High rows of the pair columns are
 // overwritten with H_1 | H_2 (H_1 | unused); the rows of A that a flip adds to
