@@ -11,6 +11,7 @@
 // min(1, p(y) q(x) / (p(x) q(y))); with exact p and q its stationary law is
 // exactly p.
 #include "common.h"
+#include "glynn_blocks.h"
 #include "../../include/pcvl_hip.h"
 
 #include <algorithm>
@@ -250,12 +251,20 @@ __global__ void mis_gather_kernel(const int32_t *__restrict__ prop, const int64_
 // One wavefront per proposal; lanes take (o, inner chunk) units.
 constexpr int MISP_MAX_N = 28;
 
+// Low rows of the block loop (glynn_blocks.h): two up to order 24, one above,
+// as in the permanent kernel; below order 6 there is no block loop.
+constexpr int MISP_PAIR_MIN = 6;
+constexpr int misp_low_rows(int n) { return n <= 24 ? 2 : 1; }
+
+template <int N>
 struct MispShared {
-    cd A[MISP_MAX_N * MISP_MAX_N];   // rows of the fixed / unique / group modes
-    int kg[MISP_MAX_N];              // multiplicity of each group
-    int rmode[MISP_MAX_N];           // mode of each stored row
-    int gmode[MISP_MAX_N], gcnt[MISP_MAX_N];   // distinct modes of the sequence and their counts
-    int nu, ng;                      // unique rows (besides the fixed one), groups
+    static constexpr int LOW = misp_low_rows(N), P = N / 2;
+    cd A[N * N];                                          // rows of the fixed / unique / group modes
+    cd H[N >= MISP_PAIR_MIN ? (N - LOW) * P * LOW : 1];   // pair constants of the unique rows after the low ones
+    cd G[P > 0 ? P : 1];
+    int kg[MISP_MAX_N];                                   // multiplicity of each group
+    int w0[MISP_MAX_N];                                   // first weight of each group
+    double w[2 * MISP_MAX_N];                             // (-1)^t C(k_g, t), t = 0..k_g
 };
 
 // prod_c h[c]; four independent chains from N >= 8 (ILP for FP64 latency).
@@ -287,14 +296,6 @@ __device__ __forceinline__ void misp_prod_acc(cd &acc, const cd *h, bool neg)
     if (neg) { acc.r -= p.r; acc.i -= p.i; } else { acc.r += p.r; acc.i += p.i; }
 }
 
-// Returns v, made to look dependent on dep, so LDS reads at offset v stay
-// inside the loop that dep counts instead of being hoisted into VGPRs.
-__device__ __forceinline__ int misp_loop_variant(int v, uint32_t dep)
-{
-    asm("" : "+s"(v) : "s"(dep));
-    return v;
-}
-
 // Keeps the next update of h behind the term that read it (no hoisting of
 // column-sum generations, which would multiply the live VGPRs).
 template <int N>
@@ -323,11 +324,17 @@ constexpr int MISP_MAX_C = 10;
 
 // record: [0] nu [1] ng [2] c [3] slices [4..5] units (int64) [6] nrow
 //         [8 ..] row modes (fixed, unique, groups)  [8 + MAX_N ..] group sizes
-__global__ void mis_plan_kernel(const int32_t *__restrict__ seq, int64_t B, int n, int m, int32_t *__restrict__ rec,
-                                int32_t *__restrict__ nslices, unsigned long long *__restrict__ cursor)
+// Also packs the input columns of U (Uc: m x n), whose rows the slice kernel
+// then reads contiguously.
+__global__ void mis_plan_kernel(const cd *__restrict__ U, const int32_t *__restrict__ cols,
+                                const int32_t *__restrict__ seq, int64_t B, int n, int m, cd *__restrict__ Uc,
+                                int32_t *__restrict__ rec, int32_t *__restrict__ nslices,
+                                unsigned long long *__restrict__ cursor)
 {
     const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b == 0) *cursor = 0ull;
+    for (int64_t e = b; e < (int64_t)m * n; e += (int64_t)gridDim.x * blockDim.x)
+        Uc[e] = U[(e / n) * m + cols[e % n]];
     if (b >= B) return;
     int32_t *R = rec + b * MISP_REC;
     const int32_t *sq = seq + b * n;
@@ -390,20 +397,23 @@ __global__ void mis_plan_kernel(const int32_t *__restrict__ seq, int64_t B, int 
     // count that is not a multiple of 64 idles lanes in the last pass, while
     // short units repeat the column-sum set-up more often.  Take the c with
     // the least estimated wave time, in per-lane FP64 operations: passes x
-    // (2^c Gray steps of 6n+2 operations + the set-up) + about 1000 per slice
+    // (2^c Gray steps + the set-up) + about 1000 per slice
     // (record and rows into LDS, search, reduction).
     const int cmax = nu < MISP_MAX_C ? nu : MISP_MAX_C;
-    const double step_ops = 6.0 * n + 2.0;
-    const double setup_ops = 2.0 * n * (2 + nu + ng) + 30.0 * ng;
+    const int low = misp_low_rows(n);
+    const double setup_ops = 2.0 * n * (2 + nu + ng) + 20.0 * ng;
     int c = cmax;
     double best = -1.0;
     for (int cc = cmax; cc >= 0 && cc >= cmax - 5; cc--) {
         const uint32_t un = O << (nu - cc);
+        const bool pairs = n >= MISP_PAIR_MIN && cc >= low;   // block loop: a term's operations, the pairs' set-up
+        const double step_ops = pairs ? (low == 2 ? 4.5 : 5.0) * n : 6.0 * n + 2.0;
+        const double pair_ops = pairs ? 6.0 * n * low : 0.0;
         const uint32_t sl_c = (un + 63) / 64 < (uint32_t)MISP_MAX_SLICES ? (un + 63) / 64 : (uint32_t)MISP_MAX_SLICES;
         const uint32_t per = (un + sl_c - 1) / sl_c;
         const uint32_t full = un / per, rest = un - full * per;
         const uint32_t passes = full * ((per + 63) / 64) + (rest + 63) / 64;
-        const double est = (double)passes * ((double)(1u << cc) * step_ops + setup_ops) + 1000.0 * (double)sl_c;
+        const double est = (double)passes * ((double)(1u << cc) * step_ops + setup_ops + pair_ops) + 1000.0 * (double)sl_c;
         if (best < 0.0 || est < best) { best = est; c = cc; }
     }
     const uint32_t units = O << (nu - c);
@@ -467,13 +477,19 @@ __global__ void mis_owner_kernel(const int64_t *__restrict__ slice0, int64_t B, 
     for (int64_t g = g0; g < g1; g++) owner[g] = ((uint64_t)b << 6) | (uint64_t)(g - g0);
 }
 
+// Bound by FP64 issue (VALU busy 89% at 2.15 GHz).  A unit's terms run in the
+// column-pair blocks of glynn_blocks.h (86 operations per order-20 term), the
+// rest is the set-up of each unit's column sums and lanes without a unit in a
+// proposal's last pass.  100,000 chain samples at m = 60, n = 20 take 49.7 ms
+// (63.9 ms with one update and product per column and term).
 template <int N>
-__global__ void __launch_bounds__(64) mis_slice_kernel(const cd *__restrict__ U, int m, const int32_t *__restrict__ cols,
+__global__ void __launch_bounds__(64, 2) mis_slice_kernel(const cd *__restrict__ Uc,
                                                        const int32_t *__restrict__ rec, const int64_t *__restrict__ slice0,
                                                        const uint64_t *__restrict__ owner, int64_t B,
                                                        unsigned long long *__restrict__ cursor, cd *__restrict__ partial)
 {
-    __shared__ MispShared sh;
+    __shared__ MispShared<N> sh;
+    constexpr int LOW = MispShared<N>::LOW, P = MispShared<N>::P;
     __shared__ int32_t srec[MISP_REC];
     const int lane = threadIdx.x;
     const int64_t total = slice0[B];
@@ -486,33 +502,72 @@ __global__ void __launch_bounds__(64) mis_slice_kernel(const cd *__restrict__ U,
         if (g >= total) break;
         // proposal p and slice s of global slice g, packed as p * 64 + s
         const uint64_t own = owner[g];
-        const int64_t pidx = (int64_t)(own >> 6);
+        const int64_t pidx = (int64_t)(((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(own >> 38)) << 32) |
+                                       __builtin_amdgcn_readfirstlane((uint32_t)(own >> 6)));
         const int s = (int)(own & 63u);
         for (int e = lane; e < MISP_REC; e += 64) srec[e] = rec[pidx * MISP_REC + e];
         __syncthreads();
-        const int nu = srec[0], ng = srec[1], c = srec[2], slices = srec[3], nrow = srec[6];
+        // wave-uniform: loop bounds and row addresses in SGPRs
+        const int nu = __builtin_amdgcn_readfirstlane(srec[0]), ng = __builtin_amdgcn_readfirstlane(srec[1]);
+        const int c = __builtin_amdgcn_readfirstlane(srec[2]), slices = __builtin_amdgcn_readfirstlane(srec[3]);
+        const int nrow = __builtin_amdgcn_readfirstlane(srec[6]);
         const uint64_t units = (uint64_t)(uint32_t)srec[4] | ((uint64_t)(uint32_t)srec[5] << 32);
         for (int e = lane; e < nrow * N; e += 64) {
             const int r = e / N, cc = e % N;
-            sh.A[e] = U[(size_t)srec[8 + r] * m + cols[cc]];
+            sh.A[e] = Uc[(size_t)srec[8 + r] * N + cc];
         }
-        if (lane < ng) sh.kg[lane] = srec[8 + MISP_MAX_N + lane];
+        if (lane < ng) {
+            const int k = srec[8 + MISP_MAX_N + lane];
+            int w0 = 0;
+            for (int gg = 0; gg < lane; gg++) w0 += srec[8 + MISP_MAX_N + gg] + 1;
+            sh.kg[lane] = k;
+            sh.w0[lane] = w0;
+            double w = 1.0;   // every quotient is a whole number
+            for (int t = 0; t <= k; t++) {
+                sh.w[w0 + t] = w;
+                w = -w * (double)(k - t) / (double)(t + 1);
+            }
+        }
         __syncthreads();
+        // proposals with at least LOW Gray-coded rows per unit run in blocks
+        const bool pairs = N >= MISP_PAIR_MIN && c >= LOW;
+        if constexpr (N >= MISP_PAIR_MIN) {
+            if (pairs) {
+                auto pair_const = [&](int q, int r, int p) {
+                    cd h = cmul(sh.A[q * N + 2 * p], sh.A[r * N + 2 * p + 1]);
+                    cfma_acc(h, sh.A[q * N + 2 * p + 1], sh.A[r * N + 2 * p]);
+                    return h;
+                };
+                for (int e = lane; e < (nu - LOW) * P * LOW; e += 64) {
+                    const int q = e / (P * LOW), pr = e % (P * LOW);
+                    sh.H[e] = pair_const(LOW + 1 + q, 1 + pr % LOW, pr / LOW);
+                }
+                if constexpr (LOW == 2) {
+                    if (lane < P) sh.G[lane] = pair_const(2, 1, lane);
+                }
+                __syncthreads();
+            }
+        }
         const uint64_t nchunks = 1ull << (nu - c);
         const uint64_t per = (units + (uint64_t)slices - 1) / (uint64_t)slices;
         const uint64_t u0 = (uint64_t)s * per;
         const uint64_t u1 = (u0 + per < units) ? u0 + per : units;
         cd acc = {0.0, 0.0};
         for (uint64_t unit = u0 + (uint64_t)lane; unit < u1; unit += 64) {
-            uint64_t o = unit / nchunks;
-            const uint64_t chunk = unit % nchunks;
+            uint32_t o = (uint32_t)(unit >> (nu - c));   // below 2^28
+            const uint64_t chunk = unit & (nchunks - 1);
             const uint64_t base = chunk << c;
-            const uint64_t g0 = base ^ (base >> 1);
+            const uint64_t g0 = base ^ (base >> 1);   // low bits zero: the low rows of a block start at +1
             cd h[N];
 #pragma unroll
             for (int cc = 0; cc < N; cc++) h[cc] = {0.5 * sh.A[cc].r, 0.5 * sh.A[cc].i};
+            // Gray signs of the unique rows.  With blocks, the high rows follow
+            // the Gray code of the block index and the low rows stay at +1.
+            const uint64_t hb = base >> LOW;
+            const uint64_t signs = pairs ? (hb ^ (hb >> 1)) << LOW : g0;
+#pragma unroll 1
             for (int i = 1; i <= nu; i++) {
-                const double d = ((g0 >> (i - 1)) & 1) ? -0.5 : 0.5;
+                const double d = ((signs >> (i - 1)) & 1) ? -0.5 : 0.5;
 #pragma unroll
                 for (int cc = 0; cc < N; cc++) {
                     h[cc].r = fma(d, sh.A[i * N + cc].r, h[cc].r);
@@ -521,13 +576,13 @@ __global__ void __launch_bounds__(64) mis_slice_kernel(const cd *__restrict__ U,
             }
             // group digits of o (mixed radix k_g + 1) and the weight W_o
             double W = 1.0;
+#pragma unroll 1
             for (int gg = 0; gg < ng; gg++) {
                 const int k = sh.kg[gg];
-                const int t = (int)(o % (uint64_t)(k + 1));
-                o /= (uint64_t)(k + 1);
-                double binom = 1.0;
-                for (int i = 1; i <= t; i++) binom = binom * (double)(k - t + i) / (double)i;
-                W *= (t & 1) ? -binom : binom;
+                const uint32_t quot = o / (uint32_t)(k + 1);
+                const int t = (int)(o - quot * (uint32_t)(k + 1));
+                o = quot;
+                W *= sh.w[sh.w0[gg] + t];
                 const double f = 0.5 * (double)(k - 2 * t);
 #pragma unroll
                 for (int cc = 0; cc < N; cc++) {
@@ -536,55 +591,43 @@ __global__ void __launch_bounds__(64) mis_slice_kernel(const cd *__restrict__ U,
                 }
             }
             cd part = {0.0, 0.0};
-            const uint64_t steps = 1ull << c;
-            if (c >= 2) {
-                // Four steps per iteration; base is a multiple of 4, so row 1
-                // (first unique row) flips to delta -1 after the first term
-                // and back after the third.  Row 1 sits in VGPRs up to order
-                // 22 and is read from LDS above (VGPR budget of two waves).
-                constexpr bool kR1Regs = N <= 22;
-                cd r1[kR1Regs ? N : 1];
-                if constexpr (kR1Regs) {
+            if (pairs) {
+                if constexpr (N >= MISP_PAIR_MIN) {
+                    cd E1[P], E2[LOW == 2 ? P : 1];
+                    auto deriv = [&](int p, int r) {   // s a' + s' a, s = h - a / 2
+                        const cd a = sh.A[r * N + 2 * p], b = sh.A[r * N + 2 * p + 1];
+                        const cd x = {fma(-0.5, a.r, h[2 * p].r), fma(-0.5, a.i, h[2 * p].i)};
+                        const cd y = {fma(-0.5, b.r, h[2 * p + 1].r), fma(-0.5, b.i, h[2 * p + 1].i)};
+                        cd e = cmul(x, b);
+                        cfma_acc(e, y, a);
+                        return e;
+                    };
 #pragma unroll
-                    for (int cc = 0; cc < N; cc++) r1[cc] = sh.A[N + cc];
-                }
-                for (uint64_t u = 0; u < steps; u += 4) {
-                    const cd *row1 = kR1Regs ? r1 : sh.A + misp_loop_variant(N, (uint32_t)u);
-                    const cd *row2 = sh.A + misp_loop_variant(2 * N, (uint32_t)u);
-                    misp_prod_acc<N>(part, h, false);             // t = base+u
-                    misp_pin<N>(h, part);
-#pragma unroll
-                    for (int cc = 0; cc < N; cc++) { h[cc].r -= row1[cc].r; h[cc].i -= row1[cc].i; }
-                    misp_prod_acc<N>(part, h, true);              // t+1
-                    misp_pin<N>(h, part);
-                    {
-                        const uint64_t t = base + u + 2;          // row 2
-                        const double sg = (((t >> 1) ^ (t >> 2)) & 1) ? -1.0 : 1.0;
-#pragma unroll
-                        for (int cc = 0; cc < N; cc++) {
-                            h[cc].r = fma(sg, row2[cc].r, h[cc].r);
-                            h[cc].i = fma(sg, row2[cc].i, h[cc].i);
+                    for (int p = 0; p < P; p++) {
+                        E1[p] = deriv(p, 1);
+                        asm volatile("" : "+v"(E1[p].r), "+v"(E1[p].i) : : "memory");
+                        if constexpr (LOW == 2) {
+                            E2[p] = deriv(p, 2);
+                            asm volatile("" : "+v"(E2[p].r), "+v"(E2[p].i) : : "memory");
                         }
                     }
-                    misp_prod_acc<N>(part, h, false);             // t+2
-                    misp_pin<N>(h, part);
-#pragma unroll
-                    for (int cc = 0; cc < N; cc++) { h[cc].r += row1[cc].r; h[cc].i += row1[cc].i; }
-                    misp_prod_acc<N>(part, h, true);              // t+3
-                    misp_pin<N>(h, part);
-                    if (u + 4 < steps) {                          // row 1 + ctz(u+4) <= c <= nu
-                        const uint64_t t = base + u + 4;
-                        const int bb = __builtin_ctzll(u + 4);
-                        const double sg = (((t >> bb) ^ (t >> (bb + 1))) & 1) ? -1.0 : 1.0;
-                        const cd *row = sh.A + (bb + 1) * N;
-#pragma unroll
-                        for (int cc = 0; cc < N; cc++) {
-                            h[cc].r = fma(sg, row[cc].r, h[cc].r);
-                            h[cc].i = fma(sg, row[cc].i, h[cc].i);
-                        }
+                    cd o1 = {0.0, 0.0}, o2 = {0.0, 0.0};
+                    if constexpr ((N & 1) != 0) {
+                        o1 = sh.A[N + N - 1];
+                        if constexpr (LOW == 2) o2 = sh.A[2 * N + N - 1];
                     }
+                    // rows past the last one (read for a flip that is
+                    // discarded) are taken as row 0, within the record and Uc
+                    typedef const __attribute__((address_space(4))) int32_t *scalar_int;
+                    const scalar_int modes = (scalar_int)(uintptr_t)(rec + pidx * MISP_REC + 8);
+                    part = glynn_blocks<N, LOW, P * LOW, LOW, true>(
+                        h, E1, E2, o1, o2, sh.H, sh.G, 1u << (c - LOW), hb, [&](int b) {
+                            const int q = LOW + 1 + b;
+                            return (scalar_row)(uintptr_t)(Uc + (size_t)modes[q < nrow ? q : 0] * N);
+                        });
                 }
             } else {
+                const uint64_t steps = 1ull << c;
                 for (uint64_t u = 0; u < steps; u++) {
                     const uint64_t t = base + u;
                     if (u) {
@@ -626,21 +669,21 @@ __global__ void mis_finalize_kernel(const cd *__restrict__ partial, const int64_
 }
 
 template <int N>
-static int launch_mis_slices(int n, const cd *U, int m, const int32_t *cols, const int32_t *rec, const int64_t *slice0,
+static int launch_mis_slices(int n, const cd *Uc, const int32_t *rec, const int64_t *slice0,
                              const uint64_t *owner, int64_t B, unsigned long long *cursor, cd *partial, hipStream_t st)
 {
     if constexpr (N > MISP_MAX_N) {
         set_error("photon number above 28");
         return ERR_ARG;
     } else {
-        if (n != N) return launch_mis_slices<N + 1>(n, U, m, cols, rec, slice0, owner, B, cursor, partial, st);
+        if (n != N) return launch_mis_slices<N + 1>(n, Uc, rec, slice0, owner, B, cursor, partial, st);
         int dev = 0, cus = 0, per_cu = 0;
         PCVL_HIP_CHECK(hipGetDevice(&dev));
         PCVL_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(&mis_slice_kernel<N>), 64, 0));
         if (per_cu < 1) per_cu = 1;
         const int grid = (int)std::min<int64_t>(B * MISP_MAX_SLICES, (int64_t)cus * per_cu);
-        hipLaunchKernelGGL((mis_slice_kernel<N>), dim3(grid), dim3(64), 0, st, U, m, cols, rec, slice0, owner, B,
+        hipLaunchKernelGGL((mis_slice_kernel<N>), dim3(grid), dim3(64), 0, st, Uc, rec, slice0, owner, B,
                            cursor, partial);
         PCVL_HIP_CHECK(hipGetLastError());
         return OK;
@@ -657,7 +700,7 @@ extern "C" int pcvl_mis_permanents(const double *d_U, int m, const int32_t *d_co
     PCVL_ARG_CHECK(m >= 1 && n >= 1 && n <= MISP_MAX_N && B >= 0, "bad sizes (1 <= n <= 28)");
     if (B == 0) return OK;
     PCVL_ARG_CHECK(d_U && d_cols && d_seq && d_out, "null device buffer");
-    // stream-ordered workspace: records | slice counts | slice offsets | cursor | partials | slice owners
+    // stream-ordered workspace: records | slice counts | slice offsets | cursor | partials | slice owners | columns of U
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     const size_t b_rec = al(sizeof(int32_t) * (size_t)B * MISP_REC);
     const size_t b_ns = al(sizeof(int32_t) * (size_t)B);
@@ -665,17 +708,19 @@ extern "C" int pcvl_mis_permanents(const double *d_U, int m, const int32_t *d_co
     const size_t b_cur = al(sizeof(unsigned long long));
     const size_t b_part = al(sizeof(cd) * (size_t)B * MISP_MAX_SLICES);
     const size_t b_own = al(sizeof(uint64_t) * (size_t)B * MISP_MAX_SLICES);
+    const size_t b_uc = al(sizeof(cd) * (size_t)m * (size_t)n);
     char *blk = nullptr;
-    PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk), b_rec + b_ns + b_s0 + b_cur + b_part + b_own, stream));
+    PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk), b_rec + b_ns + b_s0 + b_cur + b_part + b_own + b_uc, stream));
     int32_t *rec = reinterpret_cast<int32_t *>(blk);
     int32_t *ns = reinterpret_cast<int32_t *>(blk + b_rec);
     int64_t *s0 = reinterpret_cast<int64_t *>(blk + b_rec + b_ns);
     unsigned long long *cur = reinterpret_cast<unsigned long long *>(blk + b_rec + b_ns + b_s0);
     cd *part = reinterpret_cast<cd *>(blk + b_rec + b_ns + b_s0 + b_cur);
     uint64_t *own = reinterpret_cast<uint64_t *>(blk + b_rec + b_ns + b_s0 + b_cur + b_part);
+    cd *uc = reinterpret_cast<cd *>(blk + b_rec + b_ns + b_s0 + b_cur + b_part + b_own);
     int rc = OK;
-    hipLaunchKernelGGL(mis_plan_kernel, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, stream, d_seq, B, n, m, rec, ns,
-                       cur);
+    hipLaunchKernelGGL(mis_plan_kernel, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, stream,
+                       reinterpret_cast<const cd *>(d_U), d_cols, d_seq, B, n, m, uc, rec, ns, cur);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) {
         hipLaunchKernelGGL(mis_scan_kernel, dim3(1), dim3(1024), 0, stream, ns, B, s0);
@@ -689,7 +734,7 @@ extern "C" int pcvl_mis_permanents(const double *d_U, int m, const int32_t *d_co
         set_error(std::string("mis plan: ") + hipGetErrorString(e));
         rc = ERR_HIP;
     } else {
-        rc = launch_mis_slices<1>(n, reinterpret_cast<const cd *>(d_U), m, d_cols, rec, s0, own, B, cur, part, stream);
+        rc = launch_mis_slices<1>(n, uc, rec, s0, own, B, cur, part, stream);
     }
     if (rc == OK) {
         hipLaunchKernelGGL(mis_finalize_kernel, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, stream, part, s0, B,

@@ -20,6 +20,7 @@
 // in a fixed order (bit-reproducible).  Orders 0..8 take one matrix per
 // thread.
 #include "common.h"
+#include "glynn_blocks.h"
 #include "../../include/pcvl_hip.h"
 
 #include <algorithm>
@@ -48,18 +49,6 @@ struct PermItem {
 
 // --------------------------------------------------------------- wave path
 
-// Returns v, made to look dependent on dep: keeps LDS reads at an offset of v
-// inside the loop that dep counts (they would otherwise be hoisted as loop
-// invariant, holding them in VGPRs).
-__device__ __forceinline__ int perm_loop_variant(int v, uint32_t dep)
-{
-    asm("" : "+s"(v) : "s"(dep));
-    return v;
-}
-
-// Entries of a row, read through the scalar data path (wave-uniform address).
-typedef const __attribute__((address_space(4))) double *scalar_row;
-
 // Low rows of an order: two up to order 24, one above.  A pair's state is 16
 // VGPRs with two (T, T', E_1, E_2) and 12 with one, and two waves per SIMD
 // leave 256: 256 order-24 matrices take 6.80 ms with two (8.83 before), orders
@@ -67,24 +56,12 @@ typedef const __attribute__((address_space(4))) double *scalar_row;
 constexpr int PERM_LOW2_MAX = 24;
 constexpr int perm_low_rows(int n, bool one) { return (n <= PERM_LOW2_MAX && !one) ? 2 : 1; }
 
-// One wave item: 64 lanes x 2^c terms of one order-N matrix.
-//
-// The term's product over columns is taken in column pairs.  With T the column
-// sums at low-row signs +1, a pair's product is V = T T', and flipping low
-// row r takes V to V - E_r with E_r = 2 (s a'_r + s' a_r) (s: the sums without
-// row r).  E_r is linear in the sums, so a flip of high row q with new sign x
-// adds x H_r[q] to it, H_r[q] = 4 (a_q a'_r + a'_q a_r) a constant of the
-// matrix; likewise E_2 with low row 1 flipped is E_2 - G, G = H_2[1].  Per
-// pair and 2^LOW terms that is 4 operations for T T', 4 to flip T and T', 2
-// per E_r and 2 per further term (8 with the E_2 - G of two low rows): 20 for
-// 4 terms (LOW = 2), 12 for 2 (LOW = 1), where updating and multiplying the
-// two column sums of each term takes 8.  An order-N term costs 2.5 N (3 N)
-// + 4 (N/2 - 1) operations instead of 6 N - 4: 86 instead of 116 at order 20.
-// Bound by FP64 issue: 4,096 order-20 matrices take 5.82 ms (8.00 ms with one
-// update and product per column and term), 1,000 of orders 12..24 3.99 ms
-// (5.22 ms); 6.50 and 4.01 ms with each constant read just before its use.
-// The sums are updated once per block, so they drift less: error against
-// direct float64 sums 3.3e-14 (9.9e-14) at order 20.
+// One wave item: 64 lanes x 2^c terms of one order-N matrix, in the column
+// pairs of glynn_blocks.h.  Bound by FP64 issue: 4,096 order-20 matrices take
+// 5.82 ms (8.00 ms with one update and product per column and term), 1,000 of
+// orders 12..24 3.99 ms (5.22 ms).  The sums are updated once per block, so
+// they drift less: error against direct float64 sums 3.3e-14 (9.9e-14) at
+// order 20.
 //
 // sA is this wave's LDS slice (N x N).  High rows of the pair columns are
 // overwritten with H_1 | H_2 (H_1 | unused); the rows of A that a flip adds to
@@ -172,135 +149,11 @@ __device__ __forceinline__ cd glynn_wave_item(const double *__restrict__ mats, c
         if constexpr (LOW == 2) o2 = {2.0 * sA[2 * N + N - 1].r, 2.0 * sA[2 * N + N - 1].i};
     }
 
-    // The constants of a pair's flip: H_1, H_2 and G from LDS, the rows of A
-    // through the scalar cache.
-    constexpr bool AHEAD = N <= 22;   // above, H_2 and G are read in their own turn: 8 VGPRs less
-    struct PairConst {
-        cd h1, h2, g;
-        double a[4];
-    };
-    auto load_pair = [&](PairConst &k, int b, int p, uint32_t v) {
-        const cd *hrow = sA + (b + LOW + 1) * N;
-        const scalar_row arow = (scalar_row)(uintptr_t)(A + (size_t)(b + LOW + 1) * N);
-        k.h1 = hrow[2 * p];
-        if constexpr (LOW == 2) {
-            if constexpr (AHEAD) {
-                k.h2 = hrow[2 * p + 1];
-                k.g = (sA + perm_loop_variant(0, v))[p];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) k.a[i] = arow[4 * p + i];
-    };
-    // Blocks alternate in sign (the parity of the high Gray bits): instead of
-    // a sign, each block starts its sums from the negated sums so far.
-    cd accp = {0.0, 0.0}, accm = {0.0, 0.0};   // terms of even / odd low parity
-    PairConst kc, kn;
-    load_pair(kn, 0, 0, 0);
-    for (uint32_t v = 0; v < blocks; v++) {
-        // the flip that follows: high row LOW + 1 + b.  On the last block this
-        // is the first flip of the next chunk (row c + 1 <= N - 6, in bounds);
-        // its result is discarded.
-        const int b = __builtin_ctz(v + 1), bnext = __builtin_ctz(v + 2);
-        const uint64_t t = base + v + 1;
-        const double s1 = (((t >> b) ^ (t >> (b + 1))) & 1) ? -1.0 : 1.0;
-        const double s2 = s1 + s1;
-        cd q[1 << LOW];
-#pragma unroll
-        for (int p = 0; p < P; p++) {
-            // A pair's constants are read while the pair before it is worked
-            // on: wait for this pair's, start the next one's, then compute.
-            // The scheduling barriers keep that order (and the values of one
-            // pair at a time in VGPRs); without them a read sits 2-4
-            // instructions before its use, 30 times per block.
-            kc = kn;
-            asm volatile("" : "+v"(kc.h1.r), "+v"(kc.h1.i), "+s"(kc.a[0]), "+s"(kc.a[1]), "+s"(kc.a[2]), "+s"(kc.a[3]));
-            if constexpr (LOW == 2) {
-                if constexpr (AHEAD) {
-                    asm volatile("" : "+v"(kc.h2.r), "+v"(kc.h2.i), "+v"(kc.g.r), "+v"(kc.g.i));
-                } else {
-                    kc.g = (sA + perm_loop_variant(0, v))[p];
-                    kc.h2 = (sA + (b + LOW + 1) * N)[2 * p + 1];
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if (p + 1 < P) load_pair(kn, b, p + 1, v);
-            else load_pair(kn, bnext, 0, v);
-            double oa[2];
-            if constexpr (ODD) {
-                if (p == P - 1) {
-                    const scalar_row arow = (scalar_row)(uintptr_t)(A + (size_t)(b + LOW + 1) * N);
-                    oa[0] = arow[2 * (N - 1)];
-                    oa[1] = arow[2 * (N - 1) + 1];
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            cd &x = T[2 * p], &y = T[2 * p + 1];
-            cd V[1 << LOW];   // signs of the low rows: ++, -+, (+-, --)
-            V[0] = cmul(x, y);
-            V[1] = {V[0].r - E1[p].r, V[0].i - E1[p].i};
-            if constexpr (LOW == 2) {
-                const cd e = {E2[p].r - kc.g.r, E2[p].i - kc.g.i};
-                V[2] = {V[0].r - E2[p].r, V[0].i - E2[p].i};
-                V[3] = {V[1].r - e.r, V[1].i - e.i};
-            }
-            // T and E of the pair are free once its values are formed: flip
-            // them to the next block (the empty asm keeps the flips behind
-            // the values, so that they happen in place)
-            constexpr int last = (1 << LOW) - 1;
-            asm("" : "+v"(x.r), "+v"(x.i), "+v"(y.r), "+v"(y.i), "+v"(E1[p].r), "+v"(E1[p].i)
-                : "v"(V[1].r), "v"(V[1].i), "v"(V[last].r), "v"(V[last].i));
-            if constexpr (LOW == 2) asm("" : "+v"(E2[p].r), "+v"(E2[p].i) : "v"(V[2].r), "v"(V[2].i), "v"(V[3].r), "v"(V[3].i));
-            x.r = fma(s2, kc.a[0], x.r);
-            x.i = fma(s2, kc.a[1], x.i);
-            y.r = fma(s2, kc.a[2], y.r);
-            y.i = fma(s2, kc.a[3], y.i);
-            E1[p].r = fma(s1, kc.h1.r, E1[p].r);
-            E1[p].i = fma(s1, kc.h1.i, E1[p].i);
-            if constexpr (LOW == 2) {
-                E2[p].r = fma(s1, kc.h2.r, E2[p].r);
-                E2[p].i = fma(s1, kc.h2.i, E2[p].i);
-            }
-            if (p == 0) {
-#pragma unroll
-                for (int k = 0; k < (1 << LOW); k++) q[k] = V[k];
-            } else if (p < P - 1 || ODD) {
-#pragma unroll
-                for (int k = 0; k < (1 << LOW); k++) q[k] = cmul(q[k], V[k]);
-            } else {
-                accp = {-accp.r, -accp.i};
-                accm = {-accm.r, -accm.i};
-                cfma_acc(accp, q[0], V[0]);
-                cfma_acc(accm, q[1], V[1]);
-                if constexpr (LOW == 2) {
-                    cfma_acc(accm, q[2], V[2]);
-                    cfma_acc(accp, q[3], V[3]);
-                }
-            }
-            if constexpr (ODD) {
-                if (p == P - 1) {
-                    cd &z = T[N - 1];
-                    const cd m1 = {z.r - o1.r, z.i - o1.i};
-                    accp = {-accp.r, -accp.i};
-                    accm = {-accm.r, -accm.i};
-                    cfma_acc(accp, q[0], z);
-                    cfma_acc(accm, q[1], m1);
-                    if constexpr (LOW == 2) {
-                        cfma_acc(accm, q[2], cd{z.r - o2.r, z.i - o2.i});
-                        cfma_acc(accp, q[3], cd{m1.r - o2.r, m1.i - o2.i});
-                    }
-                    asm("" : "+v"(z.r), "+v"(z.i) : "v"(accp.r), "v"(accp.i), "v"(accm.r), "v"(accm.i));
-                    z.r = fma(s2, oa[0], z.r);
-                    z.i = fma(s2, oa[1], z.i);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
+    const cd sum = glynn_blocks<N, LOW, N, 2, false>(T, E1, E2, o1, o2, sA + (LOW + 1) * N, sA, blocks, base, [&](int b) {
+        return (scalar_row)(uintptr_t)(A + (size_t)(b + LOW + 1) * N);
+    });
     __syncthreads();   // sA is reused by the next item of this wave
-    const double sg = (blocks & 1) ? 1.0 : -1.0;   // the last block's sign (base is even unless it is the only one)
-    const double sb = (blocks == 1 && (base & 1)) ? -sg : sg;
-    return {sb * (accp.r - accm.r), sb * (accp.i - accm.i)};
+    return sum;
 }
 
 __device__ __forceinline__ cd wave_sum(cd v)

@@ -201,6 +201,33 @@ def test_multiset_permanents_vs_oracle(gpu, m, n):
     mis.close()
 
 
+@pytest.mark.parametrize("n", [5, 6, 7, 24, 25])
+def test_multiset_permanents_block_edges(gpu, n):
+    """Orders around the block loop's limits (none below 6, two low rows up to
+    24, one above), with 0..4 unique rows besides the fixed one: fewer than
+    the low rows, exactly them (one block, no flip), and one flip more."""
+    import torch
+    from perceval_amd.mis import LearnedMIS, ProposalNet
+    m = 30
+    U = haar_unitary(m, seed=50 + n)
+    inp = [1] * n + [0] * (m - n)
+    seqs = []
+    for unique in range(0, min(n, 6)):
+        left = n - unique
+        if left == 1:
+            continue
+        pair = left - 2 if left > 3 else left     # groups of left - 2 and 2, or one of left
+        s = list(range(10, 10 + unique)) + [3] * pair + [7] * (left - pair)
+        seqs.append(sorted(s))
+    seqs = np.array(seqs, dtype=np.int32)
+    mis = LearnedMIS(U, inp, ProposalNet(m, n, hidden=8), chunk=64)
+    got = mis.permanents(torch.from_numpy(seqs).cuda()).cpu().numpy()
+    for s, g in zip(seqs, got):
+        ref = oracle.perm_large(oracle.submatrix(U, inp, np.bincount(s, minlength=m)), threads=8)
+        assert abs(g - ref) <= 1e-10 * abs(ref) + 1e-14, (s, g, ref)
+    mis.close()
+
+
 def test_multiset_permanents_mixed_costs_deterministic(gpu):
     """A batch mixing collision-free, bunched and single-mode proposals (costs
     from 1 to 2^15 terms), against the oracle, and bit-identical when run twice."""
