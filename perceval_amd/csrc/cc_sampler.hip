@@ -13,15 +13,17 @@
 //
 // Mapping: one launch per photon step k, specialised on k so that each step
 // gets its own register allocation; within a launch one wavefront owns one
-// sample (persistent over samples).  The 2^{k-2} Gray-code terms are split
-// over the 32 lane pairs; partial sums of the k sub-permanents are reduced
-// across the wave, then lane i computes the weight of candidate row i and a
-// wave prefix sum draws r_k.  Per-sample state (permuted columns, drawn modes)
+// sample (persistent over samples), or one slice of a sample's terms from step
+// 14 on.  The terms (2^{k-2}; from step 10 on fewer, repeated rows being summed
+// by multiplicity) are split over the 32 lane pairs; partial sums of the k
+// sub-permanents are reduced across the wave, then lane i computes the weight
+// of candidate row i and a wave prefix sum draws r_k.  Per-sample state (permuted columns, drawn modes)
 // lives in a caller-provided workspace.  Random numbers
 // are the counter-based uniforms of common.h: stream = sample index, counters
 // 0..n-2 for the column permutation (Fisher-Yates, i = n-1 down to 1) and
 // n-1+k-1 for the k-th photon, so a run is fixed by its seed.
 #include "common.h"
+#include "slices.h"
 #include "../../include/pcvl_hip.h"
 
 #include <algorithm>
@@ -41,6 +43,9 @@ struct CCShared {
     cd sub[K];
     int pc[K];                           // cols[perm[l]]: input mode of permuted column l
     int r[K];
+    // multiset steps: distinct output modes in the order fixed, unique, groups
+    int mode[K], kg[K], w0[K];           // kg, w0: copies and first weight of each group
+    double w[2 * K];                     // (-1)^t C(k_g, t), t = 0..k_g
 };
 
 // Partial sums of the k sub-permanents over this lane pair's chunk of
@@ -50,17 +55,14 @@ struct CCShared {
 // column has column sum 1 and never flips).  Per term each lane forms the
 // prefix products of its half and the half total T; the partners swap T, and
 // prod_{l' != l} c_l' = prefix(l) * suffix(l) * T_partner comes out of one
-// backward pass.  acc[j] is this lane's partial for column c0 + j.  With
-// PLOG2 > 0 the 2^{rows-1} terms are cut into 2^PLOG2 parts and the wave
-// takes part `part` only (terms part * 2^{rows-1-PLOG2} onwards).
-template <int K, int PLOG2 = 0>
-__device__ __forceinline__ void subperm_pair(const cd *__restrict__ B, int lane, cd *acc, uint32_t part = 0)
+// backward pass.  acc[j] is this lane's partial for column c0 + j. 
+template <int K>
+__device__ __forceinline__ void subperm_pair(const cd *__restrict__ B, int lane, cd *acc)
 {
     constexpr int rows = K - 1;
     constexpr int h = K / 2;
     constexpr int hmax = K - h;
-    constexpr int total_log2 = rows - 1 - PLOG2;          // 2^{rows-1-PLOG2} terms in the part
-    static_assert(total_log2 >= 0, "more parts than Gray-code terms");
+    constexpr int total_log2 = rows - 1;                   // 2^{rows-1} terms
     constexpr int c = total_log2 > 5 ? total_log2 - 5 : 0; // 32 pairs
     constexpr int active_pairs = total_log2 > 5 ? 32 : (1 << total_log2);
     const int half = lane & 1;
@@ -71,7 +73,7 @@ __device__ __forceinline__ void subperm_pair(const cd *__restrict__ B, int lane,
     for (int j = 0; j < hmax; j++) acc[j] = {0.0, 0.0};
     if (pair >= active_pairs) return;
     const uint32_t steps = 1u << c;
-    const uint32_t base = (part << total_log2) + ((uint32_t)pair << c);
+    const uint32_t base = (uint32_t)pair << c;
     const uint32_t g0 = base ^ (base >> 1);
 
     // For odd K the even lane's last column is padding: it reads a valid
@@ -135,6 +137,223 @@ __device__ __forceinline__ void subperm_pair(const cd *__restrict__ B, int lane,
     }
 }
 
+// ---- multiset terms ---------------------------------------------------------
+//
+// From step CC_MULTI on, rows of B that repeat (photons already drawn in one
+// mode) are summed by multiplicity: k copies of a row enter the column sums
+// only through their sign total k - 2t, with weight (-1)^t C(k, t), so a group
+// of k copies takes k + 1 terms instead of 2^k.  At m = 60 the 19 rows of step
+// 20 leave 0.27 of the 2^18 terms on average, and fewer the smaller m is.
+// One row of weight 1 is the fixed row (delta = +1), the other unique rows are
+// walked in Gray-code order, and the group digits t_g form an outer
+// mixed-radix index o with weight W_o.  With half column sums h (a flip adds
+// the row)
+//     sub_l = 2 sum_o W_o sum_{t < 2^nu} (-1)^t prod_{l' != l} h_l'.
+// The O 2^nu terms are cut into units of 2^c Gray steps, one unit per lane
+// pair at a time.
+constexpr int CC_MULTI = 10;     // below, the terms are one or two passes of the 32 pairs
+// From step 14 on, a sample's units are cut into slices (20,000 samples at
+// m = 60: step 15 takes 0.86 ms against 0.98 with one wave per sample, step 13
+// would lose the four extra launches).
+constexpr int CC_SLICED = 14;
+constexpr int CC_MAX_C = 8;
+
+// Most slices of a sample at step k: at most 2^13 terms each up to step 27
+// (0.2 ms of one wave: the tail when the last slices drain), 4,096 slices
+// above (their partial sums are added one after another by the draw).
+constexpr int cc_slice_cap(int k) { return k < CC_SLICED ? 1 : k < 16 ? 2 : k <= 27 ? 1 << (k - 15) : 4096; }
+
+struct CCPlan {
+    int nu, ng, c, slices;
+    uint32_t units;
+};
+
+// Plans the rows sh.r[0..K-2] of a sample, one wave: fills sh.mode, sh.kg,
+// sh.w0, sh.w.  Every field of the result is wave-uniform.
+template <int K>
+__device__ __forceinline__ CCPlan cc_plan(CCShared<K> &sh, int lane)
+{
+    constexpr int rows = K - 1;
+    const int r = lane < rows ? sh.r[lane] : -1 - lane;
+    int cnt = 0, first = 64;
+#pragma unroll
+    for (int i = 0; i < rows; i++) {
+        const bool same = __builtin_amdgcn_readlane(r, i) == r;
+        cnt += same ? 1 : 0;
+        if (same && first == 64) first = i;
+    }
+    const bool lead = lane < rows && first == lane;   // first photon of its mode
+    const uint64_t um = __ballot(lead && cnt == 1), gm = __ballot(lead && cnt > 1);
+    const uint64_t below = (1ull << lane) - 1;
+    CCPlan p;
+    p.ng = __builtin_popcountll(gm);
+    p.nu = um ? __builtin_popcountll(um) - 1 : 0;
+    // the fixed row: the first unique row, else one copy of the first group
+    const int fixed = __builtin_ctzll(um ? um : gm);
+    if (lane == fixed) sh.mode[0] = r;
+    if (lead && cnt == 1 && lane != fixed) sh.mode[__builtin_popcountll(um & below)] = r;
+    int k = 0;
+    if (lead && cnt > 1) {
+        k = cnt - (lane == fixed ? 1 : 0);
+        const int g = __builtin_popcountll(gm & below);
+        sh.mode[1 + p.nu + g] = r;
+        sh.kg[g] = k;
+    }
+    uint32_t O = (uint32_t)k + 1;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) O *= (uint32_t)__shfl_xor((int)O, off, 64);
+    O = __builtin_amdgcn_readfirstlane(O);
+    __syncthreads();
+    if (lane < p.ng) {
+        int w0 = 0;
+        for (int g = 0; g < lane; g++) w0 += sh.kg[g] + 1;
+        sh.w0[lane] = w0;
+        const int kk = sh.kg[lane];
+        double w = 1.0;   // every quotient is a whole number
+        for (int t = 0; t <= kk; t++) {
+            sh.w[w0 + t] = w;
+            w = -w * (double)(kk - t) / (double)(t + 1);
+        }
+    }
+    // Unit length 2^c: short units fill the lane pairs of the last pass, long
+    // ones repeat the column-sum set-up less often.  The c of least estimated
+    // time, in operations per lane: passes x (2^c terms + set-up) + the slice's
+    // own cost (rows into LDS, reduction of K sums).
+    const int cmax = p.nu < CC_MAX_C ? p.nu : CC_MAX_C;
+    const uint32_t setup = (uint32_t)((K + 1) * (2 + p.nu + p.ng) + 24 * p.ng + 40);
+    uint32_t best = 0xffffffffu;
+    p.c = cmax;
+    p.slices = 1;
+    p.units = O << (p.nu - cmax);
+    for (int c = cmax; c >= 0 && c >= cmax - 4; c--) {
+        const uint32_t units = O << (p.nu - c);
+        const uint32_t want = (units + 31) / 32;
+        const uint32_t sl = want < (uint32_t)cc_slice_cap(K) ? want : (uint32_t)cc_slice_cap(K);
+        const uint32_t per = (units + sl - 1) / sl;
+        const uint32_t full = units / per, rest = units - full * per;
+        const uint32_t passes = full * ((per + 31) / 32) + (rest + 31) / 32;
+        const float est = (float)passes * (float)((7 * K + 24) * (1 << c) + (int)setup) + 4000.0f * (float)sl;
+        const uint32_t e = __float_as_uint(est);   // positive floats order as their bits
+        if (e < best) {
+            best = e;
+            p.c = c;
+            p.slices = (int)sl;
+            p.units = units;
+        }
+    }
+    __syncthreads();
+    return p;
+}
+
+// The value of the other lane of the pair, as a DPP move (no LDS round trip).
+__device__ __forceinline__ double pair_swap(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);   // quad_perm [1, 0, 3, 2]
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Bound by FP64 issue (14 K + 16 operations per term over the pair).  20,000
+// samples at m = 60, n = 20 take 34.3 ms; 106.7 ms with all 2^{k-2} terms, one
+// wave per sample, the row of a flip read at its use and the pair's exchange
+// through LDS (38.1 ms with multiplicities and slices alone).
+//
+// Partial sums of the K sub-permanents (before the factor 2) over units
+// [u0, u1) of a planned sample; columns over the lane pair as in subperm_pair.
+// A holds the 1 + nu + ng distinct rows.
+template <int K>
+__device__ __forceinline__ void subperm_units(const CCShared<K> &sh, const CCPlan &pl, uint32_t u0, uint32_t u1,
+                                              int lane, cd *acc)
+{
+    constexpr int h = K / 2;
+    constexpr int hmax = K - h;
+    const cd *A = sh.B;
+    const int half = lane & 1;
+    const int c0 = half ? h : 0;
+    const int ncol = half ? hmax : h;
+    const double pad = (hmax - 1 < ncol) ? 1.0 : 0.0;
+#pragma unroll
+    for (int j = 0; j < hmax; j++) acc[j] = {0.0, 0.0};
+    for (uint32_t unit = u0 + (uint32_t)(lane >> 1); unit < u1; unit += 32) {
+        uint32_t o = unit >> (pl.nu - pl.c);
+        const uint32_t base = (unit & ((1u << (pl.nu - pl.c)) - 1)) << pl.c;
+        const uint32_t g0 = base ^ (base >> 1);
+        cd cs[hmax];
+#pragma unroll
+        for (int j = 0; j < hmax; j++) {
+            const double f = (j == hmax - 1) ? pad : 1.0;
+            const cd a = A[c0 + j];
+            cs[j] = {fma(0.5 * f, a.r, 1.0 - f), 0.5 * f * a.i};
+        }
+        auto add_row = [&](int i, double d) {
+            const double dl = d * pad;
+#pragma unroll
+            for (int j = 0; j < hmax; j++) {
+                const double dj = (j == hmax - 1) ? dl : d;
+                const cd a = A[i * K + c0 + j];
+                cs[j].r = fma(dj, a.r, cs[j].r);
+                cs[j].i = fma(dj, a.i, cs[j].i);
+            }
+        };
+#pragma unroll 1
+        for (int i = 1; i <= pl.nu; i++) add_row(i, ((g0 >> (i - 1)) & 1) ? -0.5 : 0.5);
+        double W = 1.0;
+#pragma unroll 1
+        for (int g = 0; g < pl.ng; g++) {
+            const int k = sh.kg[g];
+            const uint32_t quot = o / (uint32_t)(k + 1);
+            const int t = (int)(o - quot * (uint32_t)(k + 1));
+            o = quot;
+            W *= sh.w[sh.w0[g] + t];
+            add_row(1 + pl.nu + g, 0.5 * (double)(k - 2 * t));
+        }
+        if (base & 1u) W = -W;   // units of one term (c = 0): the term's Gray sign
+        const uint32_t steps = 1u << pl.c;
+        for (uint32_t u = 0; u < steps; u++) {
+            // the flip to the next term; after the last one (of row 0, say)
+            // its result is discarded
+            const uint32_t t = base + u + 1;
+            const int b = __builtin_ctz(u + 1);   // base is a multiple of 2^c
+            const double s = (((t >> b) ^ (t >> (b + 1))) & 1) ? -1.0 : 1.0;
+            const cd *row = A + (b < pl.nu ? b + 1 : 0) * K + c0;
+            cd P[hmax];
+            P[0] = {1.0, 0.0};
+            if constexpr (hmax > 1) P[1] = cs[0];
+#pragma unroll
+            for (int j = 2; j < hmax; j++) P[j] = cmul(P[j - 1], cs[j - 1]);
+            // The backward pass flips each column once it is through with it;
+            // the row's entries are read AHEAD columns before.
+            constexpr int AHEAD = 3;
+            cd nv[hmax];
+#pragma unroll
+            for (int j = hmax - 1; j >= 0 && j > hmax - 1 - AHEAD; j--) nv[j] = row[j];
+            __builtin_amdgcn_sched_barrier(0);
+            const cd T = (hmax == 1) ? cs[0] : cmul(P[hmax - 1], cs[hmax - 1]);
+            cd S;
+            S.r = W * pair_swap(T.r);
+            S.i = W * pair_swap(T.i);
+            W = -W;
+#pragma unroll
+            for (int j = hmax - 1; j >= 0; j--) {
+                if (j >= AHEAD) nv[j - AHEAD] = row[j - AHEAD];
+                if (j >= 1) {
+                    cfma_acc(acc[j], P[j], S);
+                    S = cmul(S, cs[j]);
+                } else {
+                    acc[0].r += S.r;
+                    acc[0].i += S.i;
+                }
+                const double sj = (j == hmax - 1) ? s * pad : s;
+                // in place: behind the product that read the old sum
+                asm("" : "+v"(cs[j].r), "+v"(cs[j].i) : "v"(S.r), "v"(S.i));
+                cs[j].r = fma(sj, nv[j].r, cs[j].r);
+                cs[j].i = fma(sj, nv[j].i, cs[j].i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+}
+
 __device__ __forceinline__ double wave_sum_d(double v)
 {
 #pragma unroll
@@ -165,6 +384,32 @@ __device__ __forceinline__ void subperms(CCShared<K> &sh, int lane)
         if (lane == 0 && j < h) sh.sub[j] = {re * scale, im * scale};
         if (lane == 1) sh.sub[h + j] = {re * scale, im * scale};
     }
+}
+
+// The partial sums of units [u0, u1) to dst[0..K-1].
+template <int K>
+__device__ __forceinline__ void subperms_units(const CCShared<K> &sh, const CCPlan &pl, uint32_t u0, uint32_t u1,
+                                               int lane, cd *dst)
+{
+    constexpr int h = K / 2;
+    constexpr int hmax = K - h;
+    cd acc[hmax];
+    subperm_units<K>(sh, pl, u0, u1, lane, acc);
+#pragma unroll
+    for (int j = 0; j < hmax; j++) {
+        const double re = pair_sum_d(acc[j].r), im = pair_sum_d(acc[j].i);
+        if (lane == 0 && j < h) dst[j] = {2.0 * re, 2.0 * im};
+        if (lane == 1) dst[h + j] = {2.0 * re, 2.0 * im};
+    }
+}
+
+// Distinct rows of a planned sample into sh.B: A[mode, perm[0..K-1]].
+template <int K>
+__device__ __forceinline__ void load_rows(CCShared<K> &sh, const CCPlan &pl, const cd *__restrict__ U, int m, int lane)
+{
+    for (int e = lane; e < (1 + pl.nu + pl.ng) * K; e += 64)
+        sh.B[e] = U[(size_t)sh.mode[e / K] * m + sh.pc[e % K]];
+    __syncthreads();
 }
 
 // Column permutation of each sample (Fisher-Yates, counters 0..n-2):
@@ -288,14 +533,20 @@ __global__ void __launch_bounds__(64) cc_step_kernel(const cd *__restrict__ U, i
         if constexpr (K == 1) {
             if (lane == 0) sh.sub[0] = {1.0, 0.0};
         } else {
-            // B = 2 * A[r_1..r_{k-1}, perm[0..k-1]] with A = U[:, cols]
-            for (int e = lane; e < (K - 1) * K; e += 64) {
-                const int i = e / K, l = e % K;
-                const cd a = U[(size_t)sh.r[i] * m + sh.pc[l]];
-                sh.B[e] = {2.0 * a.r, 2.0 * a.i};
+            if constexpr (K >= CC_MULTI) {
+                const CCPlan pl = cc_plan<K>(sh, lane);
+                load_rows<K>(sh, pl, U, m, lane);
+                subperms_units<K>(sh, pl, 0, pl.units, lane, sh.sub);
+            } else {
+                // B = 2 * A[r_1..r_{k-1}, perm[0..k-1]] with A = U[:, cols]
+                for (int e = lane; e < (K - 1) * K; e += 64) {
+                    const int i = e / K, l = e % K;
+                    const cd a = U[(size_t)sh.r[i] * m + sh.pc[l]];
+                    sh.B[e] = {2.0 * a.r, 2.0 * a.i};
+                }
+                __syncthreads();
+                subperms<K>(sh, lane);
             }
-            __syncthreads();
-            subperms<K>(sh, lane);
         }
         __syncthreads();
         cc_draw<K>(sh, U, m, n, s, seed, stream, lane, r_all);
@@ -303,80 +554,92 @@ __global__ void __launch_bounds__(64) cc_step_kernel(const cd *__restrict__ U, i
     }
 }
 
-// Steps above CC_SPLIT: the 2^{K-2} Gray-code terms of a sample are cut into
-// 2^{K - CC_SPLIT} parts of 2^{CC_SPLIT - 2} terms, one wave per (sample,
-// part), so that even one sample fills the device.  cc_part_kernel writes
-// each part's pair-summed partial sub-permanents; cc_split_draw_kernel sums a
-// sample's parts in part order, scales, and draws.  The cut depends on K
-// only, so a sample's draws do not depend on how many samples a call holds.
-constexpr int CC_SPLIT = 20;
-constexpr size_t CC_PART_BYTES = size_t(256) << 20;   // partial sums of one chunk of samples
+// Steps from CC_SLICED on: a sample's units are cut into slices (at most
+// cc_slice_cap(K), by its own rows only, so that its draws do not depend on how
+// many samples a call holds).  cc_count_kernel plans the slices of every
+// sample, launch_slice_owners lists them, cc_slice_kernel runs them from one
+// cursor (so that samples of very different cost, and a single one, balance
+// over the device) and writes each slice's partial sub-permanents, and
+// cc_slice_draw_kernel sums a sample's slices in order and draws.
+constexpr size_t CC_PART_BYTES = size_t(256) << 20;   // slices of one chunk of samples
 
-constexpr int cc_parts_log2(int k) { return k > CC_SPLIT ? k - CC_SPLIT : 0; }
-
-// Samples of one chunk [s0, s0 + nchunk): item t = (sample s0 + t / P, part t % P).
+// Samples of one chunk [s0, s0 + nchunk).
 template <int K>
-__global__ void __launch_bounds__(64) cc_part_kernel(const cd *__restrict__ U, int m, int n, int64_t s0,
-                                                     int64_t nchunk, const int32_t *__restrict__ pc_all,
-                                                     const int32_t *__restrict__ r_all, cd *__restrict__ partials)
+__global__ void __launch_bounds__(64) cc_count_kernel(int n, int64_t s0, int64_t nchunk,
+                                                      const int32_t *__restrict__ r_all, int32_t *__restrict__ nslices,
+                                                      unsigned long long *__restrict__ cursor)
 {
-    constexpr int PLOG2 = cc_parts_log2(K);
-    constexpr int64_t P = int64_t(1) << PLOG2;
-    constexpr int h = K / 2;
-    constexpr int hmax = K - h;
     __shared__ CCShared<K> sh;
     const int lane = threadIdx.x;
-    for (int64_t t = blockIdx.x; t < nchunk * P; t += gridDim.x) {
-        const int64_t sl = t >> PLOG2;
-        const uint32_t part = (uint32_t)(t & (P - 1));
-        const int64_t s = s0 + sl;
-        if (lane < K) sh.pc[lane] = pc_all[s * n + lane];
-        if (lane < K - 1) sh.r[lane] = r_all[s * n + lane];
+    if (blockIdx.x == 0 && lane == 0) *cursor = 0ull;
+    for (int64_t t = blockIdx.x; t < nchunk; t += gridDim.x) {
+        if (lane < K - 1) sh.r[lane] = r_all[(s0 + t) * n + lane];
         __syncthreads();
-        for (int e = lane; e < (K - 1) * K; e += 64) {
-            const int i = e / K, l = e % K;
-            const cd a = U[(size_t)sh.r[i] * m + sh.pc[l]];
-            sh.B[e] = {2.0 * a.r, 2.0 * a.i};
-        }
-        __syncthreads();
-        cd acc[hmax];
-        subperm_pair<K, PLOG2>(sh.B, lane, acc, part);
-        cd *dst = partials + t * K;
-#pragma unroll
-        for (int j = 0; j < hmax; j++) {
-            const double re = pair_sum_d(acc[j].r), im = pair_sum_d(acc[j].i);
-            if (lane == 0 && j < h) dst[j] = {re, im};
-            if (lane == 1) dst[h + j] = {re, im};
-        }
+        const CCPlan pl = cc_plan<K>(sh, lane);
+        if (lane == 0) nslices[t] = pl.slices;
         __syncthreads();
     }
 }
 
 template <int K>
-__global__ void __launch_bounds__(64) cc_split_draw_kernel(const cd *__restrict__ U, int m, int n, int64_t s0,
+__global__ void __launch_bounds__(64, K <= 20 ? 3 : 2) cc_slice_kernel(const cd *__restrict__ U, int m, int n, int64_t s0,
+                                                      int64_t nchunk, const int32_t *__restrict__ pc_all,
+                                                      const int32_t *__restrict__ r_all,
+                                                      const int64_t *__restrict__ slice0,
+                                                      const uint64_t *__restrict__ owner,
+                                                      unsigned long long *__restrict__ cursor, cd *__restrict__ partials)
+{
+    __shared__ CCShared<K> sh;
+    const int lane = threadIdx.x;
+    const int64_t total = slice0[nchunk];
+    // a wave takes at most `total` slices, so the loop is bounded whatever the cursor holds
+    for (int64_t iter = 0; iter < total; iter++) {
+        unsigned long long gk = 0;
+        if (lane == 0) gk = atomicAdd(cursor, 1ull);
+        gk = __shfl(gk, 0, 64);
+        const int64_t g = (int64_t)gk;
+        if (g >= total) break;
+        int64_t t;
+        int slice;
+        slice_owner(owner[g], t, slice);
+        const int64_t s = s0 + t;
+        if (lane < K) sh.pc[lane] = pc_all[s * n + lane];
+        if (lane < K - 1) sh.r[lane] = r_all[s * n + lane];
+        __syncthreads();
+        const CCPlan pl = cc_plan<K>(sh, lane);
+        load_rows<K>(sh, pl, U, m, lane);
+        const uint32_t per = (pl.units + (uint32_t)pl.slices - 1) / (uint32_t)pl.slices;
+        const uint32_t u0 = (uint32_t)slice * per;
+        const uint32_t u1 = u0 + per < pl.units ? u0 + per : pl.units;
+        subperms_units<K>(sh, pl, u0, u1, lane, partials + g * K);
+        __syncthreads();
+    }
+}
+
+template <int K>
+__global__ void __launch_bounds__(64) cc_slice_draw_kernel(const cd *__restrict__ U, int m, int n, int64_t s0,
                                                            int64_t nchunk, uint64_t seed, uint64_t first,
                                                            const int32_t *__restrict__ pc_all,
                                                            int32_t *__restrict__ r_all,
                                                            const int64_t *__restrict__ gidx,
+                                                           const int64_t *__restrict__ slice0,
                                                            const cd *__restrict__ partials)
 {
-    constexpr int64_t P = int64_t(1) << cc_parts_log2(K);
     __shared__ CCShared<K> sh;
     const int lane = threadIdx.x;
-    const double scale = ldexp(1.0, -(K - 2));
-    for (int64_t sl = blockIdx.x; sl < nchunk; sl += gridDim.x) {
-        const int64_t s = s0 + sl;
+    for (int64_t t = blockIdx.x; t < nchunk; t += gridDim.x) {
+        const int64_t s = s0 + t;
         const uint64_t stream = first + (uint64_t)(gidx ? gidx[s] : s);
         if (lane < K) {
             sh.pc[lane] = pc_all[s * n + lane];
             cd v = {0.0, 0.0};
-            const cd *src = partials + sl * P * K + lane;
-            for (int64_t p = 0; p < P; p++) {   // in part order
-                const cd x = src[p * K];
+            const int64_t g1 = slice0[t + 1];
+            for (int64_t g = slice0[t]; g < g1; g++) {   // in slice order
+                const cd x = partials[g * K + lane];
                 v.r += x.r;
                 v.i += x.i;
             }
-            sh.sub[lane] = {v.r * scale, v.i * scale};
+            sh.sub[lane] = v;
         }
         __syncthreads();
         cc_draw<K>(sh, U, m, n, s, seed, stream, lane, r_all);
@@ -397,30 +660,41 @@ __global__ void cc_finish_kernel(const int32_t *__restrict__ r_all, int m, int n
     out[e] = v;
 }
 
-// Samples per chunk of the split steps, and the partial sums a chunk needs.
-static int64_t cc_chunk(int n)
-{
-    const int64_t per_sample = (int64_t(1) << cc_parts_log2(n)) * n * (int64_t)sizeof(cd);
-    return std::max<int64_t>(1, (int64_t)CC_PART_BYTES / per_sample);
-}
+// Workspace of the sliced steps, for chunks of samples sized by the largest
+// step of the call: slice counts | slice offsets | cursor | owners | partial sums.
+struct CCSliceWork {
+    int64_t chunk = 0;
+    size_t o_s0 = 0, o_cur = 0, o_own = 0, o_part = 0, total = 0;
+};
 
-static size_t cc_partial_bytes(int n, int64_t count)
+static CCSliceWork cc_slice_work(int n, int64_t count)
 {
-    if (n <= CC_SPLIT) return 0;
-    return (size_t)std::min(count, cc_chunk(n)) * ((size_t)1 << cc_parts_log2(n)) * (size_t)n * sizeof(cd);
+    CCSliceWork w;
+    if (n < CC_SLICED || count <= 0) return w;
+    const size_t cap = (size_t)cc_slice_cap(n);
+    const size_t per_sample = cap * ((size_t)n * sizeof(cd) + sizeof(uint64_t));
+    w.chunk = std::min(count, std::max<int64_t>(1, (int64_t)(CC_PART_BYTES / per_sample)));
+    auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
+    const size_t c = (size_t)w.chunk;
+    w.o_s0 = al(sizeof(int32_t) * c);
+    w.o_cur = w.o_s0 + al(sizeof(int64_t) * (c + 1));
+    w.o_own = w.o_cur + 256;
+    w.o_part = w.o_own + al(sizeof(uint64_t) * c * cap);
+    w.total = w.o_part + al(sizeof(cd) * c * cap * (size_t)n);
+    return w;
 }
 
 template <int K>
 static int launch_step(int k, const cd *U, int m, int n, int64_t count, uint64_t seed, uint64_t first,
-                       const int32_t *pc, int32_t *r, cd *partials, int cus, hipStream_t st,
+                       const int32_t *pc, int32_t *r, char *work, int cus, hipStream_t st,
                        const int64_t *gidx = nullptr)
 {
     if constexpr (K > CC_MAX_N) {
         set_error("internal: photon step out of range");
         return ERR_ARG;
     } else {
-        if (k != K) return launch_step<K + 1>(k, U, m, n, count, seed, first, pc, r, partials, cus, st, gidx);
-        if constexpr (K <= CC_SPLIT) {
+        if (k != K) return launch_step<K + 1>(k, U, m, n, count, seed, first, pc, r, work, cus, st, gidx);
+        if constexpr (K < CC_SLICED) {
             int per_cu = 0;
             PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
                 &per_cu, reinterpret_cast<const void *>(&cc_step_kernel<K>), 64, 0));
@@ -430,26 +704,33 @@ static int launch_step(int k, const cd *U, int m, int n, int64_t count, uint64_t
                                gidx);
             PCVL_HIP_CHECK(hipGetLastError());
         } else {
-            constexpr int64_t P = int64_t(1) << cc_parts_log2(K);
-            int per_cu_p = 0, per_cu_d = 0;
+            int per_cu_s = 0, per_cu_d = 0;
             PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu_p, reinterpret_cast<const void *>(&cc_part_kernel<K>), 64, 0));
+                &per_cu_s, reinterpret_cast<const void *>(&cc_slice_kernel<K>), 64, 0));
             PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu_d, reinterpret_cast<const void *>(&cc_split_draw_kernel<K>), 64, 0));
-            per_cu_p = std::max(per_cu_p, 1);
+                &per_cu_d, reinterpret_cast<const void *>(&cc_slice_draw_kernel<K>), 64, 0));
+            per_cu_s = std::max(per_cu_s, 1);
             per_cu_d = std::max(per_cu_d, 1);
-            // chunks sized for the photon count n of the call (the largest
-            // partial buffer of its steps), so the workspace holds any step's
-            const int64_t chunk = cc_chunk(n);
-            for (int64_t s0 = 0; s0 < count; s0 += chunk) {
-                const int64_t nchunk = std::min(chunk, count - s0);
-                const int gp = (int)std::min<int64_t>(nchunk * P, (int64_t)cus * per_cu_p);
-                hipLaunchKernelGGL((cc_part_kernel<K>), dim3(gp), dim3(64), 0, st, U, m, n, s0, nchunk, pc, r,
-                                   partials);
-                PCVL_HIP_CHECK(hipGetLastError());
+            const CCSliceWork w = cc_slice_work(n, count);
+            int32_t *ns = reinterpret_cast<int32_t *>(work);
+            int64_t *slice0 = reinterpret_cast<int64_t *>(work + w.o_s0);
+            unsigned long long *cursor = reinterpret_cast<unsigned long long *>(work + w.o_cur);
+            uint64_t *owner = reinterpret_cast<uint64_t *>(work + w.o_own);
+            cd *partials = reinterpret_cast<cd *>(work + w.o_part);
+            for (int64_t s0 = 0; s0 < count; s0 += w.chunk) {
+                const int64_t nchunk = std::min(w.chunk, count - s0);
                 const int gd = (int)std::min<int64_t>(nchunk, (int64_t)cus * per_cu_d);
-                hipLaunchKernelGGL((cc_split_draw_kernel<K>), dim3(gd), dim3(64), 0, st, U, m, n, s0, nchunk, seed,
-                                   first, pc, r, gidx, partials);
+                hipLaunchKernelGGL((cc_count_kernel<K>), dim3((unsigned)std::min<int64_t>(nchunk, (int64_t)cus * 16)),
+                                   dim3(64), 0, st, n, s0, nchunk, r, ns, cursor);
+                PCVL_HIP_CHECK(hipGetLastError());
+                int rc = launch_slice_owners(ns, nchunk, slice0, owner, st);
+                if (rc != OK) return rc;
+                const int gs = (int)std::min<int64_t>(nchunk * cc_slice_cap(K), (int64_t)cus * per_cu_s);
+                hipLaunchKernelGGL((cc_slice_kernel<K>), dim3(gs), dim3(64), 0, st, U, m, n, s0, nchunk, pc, r, slice0,
+                                   owner, cursor, partials);
+                PCVL_HIP_CHECK(hipGetLastError());
+                hipLaunchKernelGGL((cc_slice_draw_kernel<K>), dim3(gd), dim3(64), 0, st, U, m, n, s0, nchunk, seed,
+                                   first, pc, r, gidx, slice0, partials);
                 PCVL_HIP_CHECK(hipGetLastError());
             }
         }
@@ -466,9 +747,9 @@ extern "C" int pcvl_cc_workspace_bytes(int n, int64_t count, size_t *bytes)
     PCVL_ARG_CHECK(bytes != nullptr, "bytes is null");
     PCVL_ARG_CHECK(n >= 0 && n <= CC_MAX_N && count >= 0, "n outside [0, 30] or count < 0");
     // pc (count*n) | r (count*n) | cols (CC_MAX_N), then from a 256-byte
-    // boundary the partial sums of the split steps (more than 20 photons)
+    // boundary the slices of the sliced steps (16 photons and more)
     const size_t head = sizeof(int32_t) * ((size_t)2 * (size_t)count * (size_t)std::max(n, 1) + (size_t)CC_MAX_N);
-    const size_t part = cc_partial_bytes(n, count);
+    const size_t part = cc_slice_work(n, count).total;
     *bytes = part ? ((head + 255) & ~size_t(255)) + part : head;
     return OK;
 }
@@ -499,12 +780,12 @@ extern "C" int pcvl_cc_samples(const double *d_U, int m, const int32_t *h_in_occ
         PCVL_HIP_CHECK(hipGetLastError());
         return OK;
     }
-    // workspace: pc (count*n) | r (count*n) | cols (CC_MAX_N) | partial sums
+    // workspace: pc (count*n) | r (count*n) | cols (CC_MAX_N) | slices
     int32_t *pc = static_cast<int32_t *>(d_work);
     int32_t *r = pc + (size_t)count * n;
     int32_t *d_cols = r + (size_t)count * n;
     const size_t head = sizeof(int32_t) * ((size_t)2 * (size_t)count * (size_t)n + (size_t)CC_MAX_N);
-    cd *partials = reinterpret_cast<cd *>(static_cast<char *>(d_work) + ((head + 255) & ~size_t(255)));
+    char *slices = static_cast<char *>(d_work) + ((head + 255) & ~size_t(255));
     PCVL_HIP_CHECK(hipMemcpyAsync(d_cols, cols.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, stream));
     const cd *U = reinterpret_cast<const cd *>(d_U);
     int dev = 0, cus = 0;
@@ -514,7 +795,7 @@ extern "C" int pcvl_cc_samples(const double *d_U, int m, const int32_t *h_in_occ
                        seed, first_sample, pc);
     PCVL_HIP_CHECK(hipGetLastError());
     for (int k = 1; k <= n; k++) {
-        int rc = launch_step<1>(k, U, m, n, count, seed, first_sample, pc, r, partials, cus, stream);
+        int rc = launch_step<1>(k, U, m, n, count, seed, first_sample, pc, r, slices, cus, stream);
         if (rc != OK) return rc;
     }
     const int64_t tot = count * m;
@@ -561,13 +842,13 @@ extern "C" int pcvl_cc_samples_multi(const double *d_U, int m, const int32_t *h_
     }
     int nmax = 1;
     for (int n : ns) nmax = std::max(nmax, n);
-    // device block: pc | r (gmax * nmax each) | inp | gidx (gmax) | cols (ninputs * nmax) | partial sums
+    // device block: pc | r (gmax * nmax each) | inp | gidx (gmax) | cols (ninputs * nmax) | slices
     const size_t b_pr = sizeof(int32_t) * (size_t)gmax * nmax;
     const size_t b_inp = sizeof(int32_t) * (size_t)gmax;
     const size_t b_gidx = sizeof(int64_t) * (size_t)gmax;
     const size_t b_cols = sizeof(int32_t) * (size_t)ninputs * nmax;
     size_t b_part = 0;
-    for (int n : ns) b_part = std::max(b_part, cc_partial_bytes(n, gmax));
+    for (int n : ns) b_part = std::max(b_part, cc_slice_work(n, gmax).total);
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     char *blk = nullptr;
     PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk),
@@ -577,7 +858,7 @@ extern "C" int pcvl_cc_samples_multi(const double *d_U, int m, const int32_t *h_
     int32_t *d_inp = reinterpret_cast<int32_t *>(blk + 2 * al(b_pr));
     int64_t *d_gidx = reinterpret_cast<int64_t *>(blk + 2 * al(b_pr) + al(b_inp));
     int32_t *d_cols = reinterpret_cast<int32_t *>(blk + 2 * al(b_pr) + al(b_inp) + al(b_gidx));
-    cd *partials = reinterpret_cast<cd *>(blk + 2 * al(b_pr) + al(b_inp) + al(b_gidx) + al(b_cols));
+    char *slices = blk + 2 * al(b_pr) + al(b_inp) + al(b_gidx) + al(b_cols);
     const cd *U = reinterpret_cast<const cd *>(d_U);
     int dev = 0, cus = 0;
     int rc = OK;
@@ -605,7 +886,7 @@ extern "C" int pcvl_cc_samples_multi(const double *d_U, int m, const int32_t *h_
             e = hipGetLastError();
             if (e != hipSuccess) { set_error(std::string("cc_init_multi: ") + hipGetErrorString(e)); rc = ERR_HIP; break; }
             for (int k = 1; k <= n && rc == OK; k++)
-                rc = launch_step<1>(k, U, m, n, count, seed, first_sample, pc, r, partials, cus, stream, d_gidx);
+                rc = launch_step<1>(k, U, m, n, count, seed, first_sample, pc, r, slices, cus, stream, d_gidx);
             if (rc != OK) break;
         }
         const int64_t tot = count * m;

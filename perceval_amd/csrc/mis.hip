@@ -12,6 +12,7 @@
 // exactly p.
 #include "common.h"
 #include "glynn_blocks.h"
+#include "slices.h"
 #include "../../include/pcvl_hip.h"
 
 #include <algorithm>
@@ -424,59 +425,6 @@ __global__ void mis_plan_kernel(const cd *__restrict__ U, const int32_t *__restr
     nslices[b] = slices;
 }
 
-// Exclusive prefix of the slice counts, one block: slice0[b], total at
-// slice0[B].  4096 counts per pass, four consecutive ones per thread (their
-// loads in flight together); a shuffle scan of the thread sums per wave and
-// the 16 wave totals through LDS.
-__global__ void __launch_bounds__(1024) mis_scan_kernel(const int32_t *__restrict__ nslices, int64_t B,
-                                                        int64_t *__restrict__ slice0)
-{
-    __shared__ int wsum[16];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    int64_t carry = 0;
-    for (int64_t base = 0; base < B; base += 4096) {
-        const int64_t i0 = base + 4 * (int64_t)t;
-        int v[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = i0 + q < B ? nslices[i0 + q] : 0;   // at most 64 each
-        const int own = v[0] + v[1] + v[2] + v[3];
-        int x = own;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int y = __shfl_up(x, off, 64);
-            if (lane >= off) x += y;
-        }
-        if (lane == 63) wsum[wv] = x;
-        __syncthreads();
-        int before = 0, total = 0;
-#pragma unroll
-        for (int k = 0; k < 16; k++) {
-            const int w = wsum[k];
-            if (k < wv) before += w;
-            total += w;
-        }
-        int64_t run = carry + before + x - own;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            if (i0 + q < B) slice0[i0 + q] = run;
-            run += v[q];
-        }
-        carry += total;
-        __syncthreads();   // wsum is rewritten by the next pass
-    }
-    if (t == 0) slice0[B] = carry;
-}
-
-// Owner of every slice, packed as proposal * 64 + slice (slices per
-// proposal <= 64), so a wave finds its slice's proposal with one load.
-__global__ void mis_owner_kernel(const int64_t *__restrict__ slice0, int64_t B, uint64_t *__restrict__ owner)
-{
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const int64_t g0 = slice0[b], g1 = slice0[b + 1];
-    for (int64_t g = g0; g < g1; g++) owner[g] = ((uint64_t)b << 6) | (uint64_t)(g - g0);
-}
-
 // Bound by FP64 issue (VALU busy 89% at 2.15 GHz).  A unit's terms run in the
 // column-pair blocks of glynn_blocks.h (86 operations per order-20 term), the
 // rest is the set-up of each unit's column sums and lanes without a unit in a
@@ -500,11 +448,10 @@ __global__ void __launch_bounds__(64, 2) mis_slice_kernel(const cd *__restrict__
         gk = __shfl(gk, 0, 64);
         const int64_t g = (int64_t)gk;
         if (g >= total) break;
-        // proposal p and slice s of global slice g, packed as p * 64 + s
-        const uint64_t own = owner[g];
-        const int64_t pidx = (int64_t)(((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(own >> 38)) << 32) |
-                                       __builtin_amdgcn_readfirstlane((uint32_t)(own >> 6)));
-        const int s = (int)(own & 63u);
+        // proposal and slice of global slice g
+        int64_t pidx;
+        int s;
+        slice_owner(owner[g], pidx, s);
         for (int e = lane; e < MISP_REC; e += 64) srec[e] = rec[pidx * MISP_REC + e];
         __syncthreads();
         // wave-uniform: loop bounds and row addresses in SGPRs
@@ -722,18 +669,12 @@ extern "C" int pcvl_mis_permanents(const double *d_U, int m, const int32_t *d_co
     hipLaunchKernelGGL(mis_plan_kernel, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, stream,
                        reinterpret_cast<const cd *>(d_U), d_cols, d_seq, B, n, m, uc, rec, ns, cur);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(mis_scan_kernel, dim3(1), dim3(1024), 0, stream, ns, B, s0);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(mis_owner_kernel, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, stream, s0, B, own);
-        e = hipGetLastError();
-    }
     if (e != hipSuccess) {
         set_error(std::string("mis plan: ") + hipGetErrorString(e));
         rc = ERR_HIP;
-    } else {
+    }
+    if (rc == OK) rc = launch_slice_owners(ns, B, s0, own, stream);
+    if (rc == OK) {
         rc = launch_mis_slices<1>(n, uc, rec, s0, own, B, cur, part, stream);
     }
     if (rc == OK) {

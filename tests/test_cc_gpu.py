@@ -32,6 +32,20 @@ def test_same_seed_same_samples(gpu, m, inp):
     assert same >= 0.999, same
 
 
+@pytest.mark.parametrize("m,n,count", [(1, 12, 4), (2, 16, 400), (3, 11, 2000), (4, 17, 400), (9, 10, 2000),
+                                       (12, 15, 800), (12, 16, 400), (40, 17, 200), (6, 22, 60)])
+def test_same_seed_same_samples_repeated_rows(gpu, m, n, count):
+    """Photons that share modes are summed by multiplicity from step 10 on
+    (slices from step 16): from all photons in one mode (no unique row, units
+    of one term) to mostly distinct ones, the oracle's samples seed for seed."""
+    from perceval_amd.sampling import cc_samples
+    U = haar_unitary(m, seed=10 * m + n)
+    inp = [n // m + (1 if i < n % m else 0) for i in range(m)]
+    g = cc_samples(U, inp, count, seed=17)
+    c = oracle.cc_samples(U, inp, count, seed=17)
+    assert np.array_equal(g, c), np.nonzero(np.any(g != c, axis=1))[0][:10]
+
+
 def test_same_seed_same_samples_m60_n20(gpu):
     from perceval_amd.sampling import cc_samples
     U = haar_unitary(60, seed=60)
