@@ -747,7 +747,7 @@ extern "C" int pcvl_cc_workspace_bytes(int n, int64_t count, size_t *bytes)
     PCVL_ARG_CHECK(bytes != nullptr, "bytes is null");
     PCVL_ARG_CHECK(n >= 0 && n <= CC_MAX_N && count >= 0, "n outside [0, 30] or count < 0");
     // pc (count*n) | r (count*n) | cols (CC_MAX_N), then from a 256-byte
-    // boundary the slices of the sliced steps (16 photons and more)
+    // boundary the slices of the sliced steps (14 photons and more)
     const size_t head = sizeof(int32_t) * ((size_t)2 * (size_t)count * (size_t)std::max(n, 1) + (size_t)CC_MAX_N);
     const size_t part = cc_slice_work(n, count).total;
     *bytes = part ? ((head + 255) & ~size_t(255)) + part : head;

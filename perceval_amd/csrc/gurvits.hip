@@ -35,6 +35,9 @@ struct GurvitsItem {
     int32_t pad;
 };
 
+// Scale of a matrix that keeps the FP64 products (see gurvits_int8_kernel).
+constexpr int32_t GURVITS_FP64 = INT32_MIN;
+
 template <int NP>
 __device__ __forceinline__ cd gurvits_prod(const cd *y)
 {
@@ -136,7 +139,8 @@ template <int NP>
 __global__ void __launch_bounds__(64 * GURVITS_WAVES, NP <= 32 ? 3 : 1) gurvits_mfma_kernel(const cd *__restrict__ mats,
                                                           const GurvitsItem *__restrict__ items, int64_t count,
                                                           int parts, int64_t iters, int64_t per, uint64_t seed,
-                                                          uint64_t stream0, double *__restrict__ partial)
+                                                          uint64_t stream0, double *__restrict__ partial,
+                                                          const int32_t *__restrict__ scale)
 {
     constexpr int RB = NP / 16, KB = NP / 4;
     // A is read from LDS at each product: the registers it would take cost a
@@ -150,6 +154,7 @@ __global__ void __launch_bounds__(64 * GURVITS_WAVES, NP <= 32 ? 3 : 1) gurvits_
     for (int64_t wi = blockIdx.x; wi < nwork; wi += gridDim.x) {
         const int64_t b = wi / parts;
         const int64_t q = wi % parts;
+        if (scale && scale[b] != GURVITS_FP64) continue;   // taken by gurvits_int8_kernel
         const int n = __builtin_amdgcn_readfirstlane(items[b].n);
         const int64_t off = items[b].off;
         for (int e = threadIdx.x; e < NP * NP; e += 64 * GURVITS_WAVES) {
@@ -246,28 +251,266 @@ __global__ void __launch_bounds__(64 * GURVITS_WAVES, NP <= 32 ? 3 : 1) gurvits_
     }
 }
 
-__global__ void gurvits_finalize_kernel(const double *__restrict__ partial, int64_t count, int parts, int64_t iters,
-                                        cd *__restrict__ est, double *__restrict__ err)
+// ---- y = A x in integers -----------------------------------------------------
+//
+// The signs are whole numbers, so y = A x can be formed exactly from the digits
+// of a fixed-point A on the int8 matrix cores, 64 times the rate of the FP64
+// ones.  Row i is scaled by a power of two to components below 1 and rounded to
+// 63 bits, a 2^63 = sum_s d_s 2^(13 s) with five balanced digits d_s, and
+// d_s = lo + 64 hi splits a digit into two int8: one v_mfma_i32_16x16x64_i8
+// per digit takes the lo parts against x = +-1 in its first 32 products and the
+// hi parts against +-64 in the other 32.  |sum d_s x| <= 2^17, so two digits
+// share an int32 and three conversions and FMAs make a component of y.  The
+// rounding of a row is 2^-64 of its largest component, a thousandth of what
+// the FP64 sum of the row rounds; components down to 2^-10 of it are exact.
+// Error of the means against long double sums over the same draws (16 Haar
+// submatrices, 10^5 draws): 4.2e-16, 4.8e-16, 9.2e-16 at orders 30, 21, 12,
+// where the FP64 products give 1.4e-15, 9.1e-16, 1.6e-15.
+// Matrices where it would show (a component below 2^-40 of its row's largest,
+// or one that is not finite) keep the FP64 products.
+//
+// Operand slots: lane l and byte j of its 16 hold row (A) or sample (B) l % 16
+// and slot 16 (l / 16) + j; A and B pair equal slots, whatever k the
+// instruction gives them.  Slot t is column t % 32, lo part for t < 32, hi
+// above.  The result's register v of lane l is row 4 (l / 16) + v of the row
+// block and sample l % 16.  A padding row (i >= n) is 1 in column n, whose sign
+// is always +1, so that it multiplies by y = 1.
+typedef int gv_i4 __attribute__((ext_vector_type(4)));
+constexpr int GURVITS_DIGITS = 5;
+// Rounds of waves that a call is cut into: each part is dispatched as its own
+// workgroup (64 matrices of order 30, 10^6 samples: 2.03 ms; 2.21 ms with four
+// rounds on resident waves, whose compute units do not run at one speed).
+constexpr int GURVITS_ROUNDS = 8;
+// Samples of a call from which the integer products pay for their two more
+// launches (about 20 us): at orders 17..32 2.1M samples take 276 against 344
+// us, at orders 9..16 4.2M samples save 35 us.
+constexpr int64_t gurvits_int8_min(int nmax) { return nmax <= 16 ? int64_t(1) << 22 : int64_t(1) << 21; }
+
+// Fragments of one matrix: [row block][component][digit][lane].
+constexpr int gurvits_frags(int np) { return np / 16 * 2 * GURVITS_DIGITS * 64; }
+
+template <int NP>
+__global__ void __launch_bounds__(256) gurvits_digits_kernel(const cd *__restrict__ mats,
+                                                             const GurvitsItem *__restrict__ items, int64_t count,
+                                                             gv_i4 *__restrict__ frags, int32_t *__restrict__ scale)
 {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ cd sA[NP * NP];
+    __shared__ int sexp[NP];
+    __shared__ int sbad;
+    const int tid = threadIdx.x;
+    // one block per (matrix, row block, component)
+    constexpr int RC = NP / 16 * 2, PER = gurvits_frags(NP) / RC;
+    for (int64_t w = blockIdx.x; w < count * RC; w += gridDim.x) {
+        const int64_t b = w / RC;
+        const int rc = (int)(w % RC);
+        const int n = items[b].n;
+        const int64_t off = items[b].off;
+        if (tid == 0) sbad = 0;
+        for (int e = tid; e < NP * NP; e += 256) {
+            const int i = e / NP, j = e % NP;
+            cd v = {0.0, 0.0};
+            if (i < n && j < n) v = mats[off + (int64_t)i * n + j];
+            else if (i >= n && j == n) v.r = 1.0;   // n < NP here
+            sA[e] = v;
+        }
+        __syncthreads();
+        for (int i = tid >> 3; i < NP; i += 32) {   // eight lanes per row
+            double mx = 0.0, mn = INFINITY;        // largest and smallest nonzero component
+            bool bad = false;
+            for (int j = tid & 7; j < NP; j += 8) {
+                const cd v = sA[i * NP + j];
+                const double x = fabs(v.r), y = fabs(v.i);
+                bad |= !(x < INFINITY) || !(y < INFINITY);
+                mx = fmax(mx, fmax(x, y));
+                mn = fmin(mn, fmin(x > 0.0 ? x : INFINITY, y > 0.0 ? y : INFINITY));
+            }
+#pragma unroll
+            for (int o = 4; o >= 1; o >>= 1) {
+                mx = fmax(mx, __shfl_xor(mx, o, 64));
+                mn = fmin(mn, __shfl_xor(mn, o, 64));
+                bad |= __shfl_xor((int)bad, o, 64) != 0;
+            }
+            bad |= mn < ldexp(mx, -40);
+            if ((tid & 7) == 0) {
+                sexp[i] = bad || mx == 0.0 ? 0 : ilogb(mx) + 1;   // |components| 2^-e < 1
+                if (bad) sbad = 1;
+            }
+        }
+        __syncthreads();
+        if (tid == 0 && rc == 0) {
+            int E = 0;
+            for (int i = 0; i < n; i++) E += sexp[i];
+            for (int i = n; i < NP; i++) E += sexp[i];   // padding rows: 2^-1 each against an exponent of 1
+            scale[b] = sbad ? GURVITS_FP64 : E;
+        }
+        if (!sbad) {
+            for (int f = tid; f < PER; f += 256) {
+                const int lane = f & 63, ds = f >> 6;
+                const int comp = rc & 1, row = 16 * (rc >> 1) + (lane & 15), g = lane >> 4;
+                const int e = sexp[row];
+                union { gv_i4 v; int8_t b[16]; } u;
+                for (int j = 0; j < 16; j++) {
+                    const int col = (16 * g + j) & 31;
+                    int d = 0;
+                    if (col < NP) {
+                        const cd a = sA[row * NP + col];
+                        // below 2^63 in magnitude, as the component is below 1
+                        int64_t v = __double2ll_rn(ldexp(comp ? a.i : a.r, 63 - e));
+                        for (int k = 0; k <= ds; k++) {   // balanced digits from the low end
+                            d = k < GURVITS_DIGITS - 1 ? (int)(((v & 8191) ^ 4096) - 4096) : (int)v;
+                            v = (v - d) >> 13;
+                        }
+                    }
+                    const int hi = (d + 32) >> 6;
+                    u.b[j] = (int8_t)(g >= 2 ? hi : d - 64 * hi);
+                }
+                frags[w * PER + f] = u.v;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// One wave per (matrix, part), 64 samples' signs at a time, 16 samples per
+// product.  A's fragments stay in VGPRs.  Bound by the vector ALU (busy 88%;
+// the matrix cores 30%): the conversions and FMAs of each y component and the
+// product over rows.  64 matrices of order 30, 10^6 samples each, take 2.03 ms
+// (4.79 ms on the FP64 matrix cores).
+template <int NP>
+__global__ void __launch_bounds__(64, NP <= 16 ? 4 : 3) gurvits_int8_kernel(const gv_i4 *__restrict__ frags,
+                                                                             const GurvitsItem *__restrict__ items,
+                                                                             int64_t count, int parts, int64_t iters,
+                                                                             int64_t per, uint64_t seed,
+                                                                             uint64_t stream0,
+                                                                             double *__restrict__ partial,
+                                                                             const int32_t *__restrict__ scale)
+{
+    constexpr int RB = NP / 16, ND = GURVITS_DIGITS;
+    const int lane = threadIdx.x;
+    const int col = lane & 15, quad = lane >> 4;
+    const int64_t nwork = count * parts;
+    // signs to bytes: x = base ^ (byte mask & flip): +-1 in the lo slots, +-64 in the hi ones
+    const uint32_t xbase = quad < 2 ? 0x01010101u : 0x40404040u;
+    const uint32_t xflip = quad < 2 ? 0xFEFEFEFEu : 0x80808080u;
+    for (int64_t wi = blockIdx.x; wi < nwork; wi += gridDim.x) {
+        const int64_t b = wi / parts;
+        const int64_t q = wi % parts;
+        if (scale[b] == GURVITS_FP64) continue;
+        const int n = __builtin_amdgcn_readfirstlane(items[b].n);
+        gv_i4 a[RB][2][ND];
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int s = 0; s < ND; s++)
+                    a[rb][c][s] = frags[b * gurvits_frags(NP) + ((rb * 2 + c) * ND + s) * 64 + lane];
+        const uint32_t mask = n >= 32 ? ~0u : ((1u << n) - 1);
+        const int64_t s_lo = q * per;
+        const int64_t s_hi = (s_lo + per < iters) ? s_lo + per : iters;
+        cd sum = {0.0, 0.0};
+        double sq = 0.0;
+        for (int64_t s0 = s_lo; s0 < s_hi; s0 += 64) {
+            // signs of sample s0 + lane; the columns from n on keep +1
+            const uint32_t mine = (uint32_t)rand64(seed, stream0 + (uint64_t)b, (uint64_t)(s0 + lane)) & mask;
+#pragma unroll 1
+            for (int sub = 0; sub < 4; sub++) {
+                if (s0 + 16 * sub >= s_hi) break;
+                const uint32_t bits = (uint32_t)__shfl((int)mine, 16 * sub + col, 64);
+                const uint32_t half = bits >> (16 * (quad & 1));
+                gv_i4 x;
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    const uint32_t nib = (half >> (4 * w)) & 15u;
+                    const uint32_t one = __umul24(nib, 0x204081u) & 0x01010101u;   // bit k to byte k
+                    uint32_t up = one << 8;
+                    asm("" : "+v"(up));   // or the byte mask becomes a quarter-rate multiplication by 255
+                    x[w] = (int)(((up - one) & xflip) ^ xbase);
+                }
+                // y comes out as 2^11 times the scaled row's sum; the sign is
+                // prod_j x_j, in one of the sample's four lanes
+                const double start = RB == 2 ? 0x1p-88 : 0x1p-44;
+                cd p = {quad == 0 && (__builtin_popcount(bits) & 1) ? -start : start, 0.0};
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++) {
+                    double y[2][4];
+#pragma unroll
+                    for (int c = 0; c < 2; c++) {
+                        gv_i4 d[ND];
+#pragma unroll
+                        for (int s = 0; s < ND; s++)
+                            d[s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[rb][c][s], x, gv_i4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                        for (int v = 0; v < 4; v++) {
+                            const int lo = (d[1][v] << 13) + d[0][v], mid = (d[3][v] << 13) + d[2][v];
+                            y[c][v] = fma((double)lo, 0x1p-52, fma((double)mid, 0x1p-26, (double)d[4][v]));
+                        }
+                    }
+#pragma unroll
+                    for (int v = 0; v < 4; v++) p = cmul(p, cd{y[0][v], y[1][v]});
+                }
+                // this lane's rows, then the sample's four lanes
+                cd o = {__shfl_xor(p.r, 16, 64), __shfl_xor(p.i, 16, 64)};
+                p = cmul(p, o);
+                o = {__shfl_xor(p.r, 32, 64), __shfl_xor(p.i, 32, 64)};
+                p = cmul(p, o);
+                // all four lanes hold the product: each adds one group of 16 in four
+                if (quad == sub && s0 + 16 * sub + col < s_hi) {
+                    sum.r += p.r;
+                    sum.i += p.i;
+                    sq = fma(p.r, p.r, fma(p.i, p.i, sq));
+                }
+            }
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            sum.r += __shfl_xor(sum.r, o, 64);
+            sum.i += __shfl_xor(sum.i, o, 64);
+            sq += __shfl_xor(sq, o, 64);
+        }
+        if (lane == 0) {
+            partial[3 * wi] = sum.r;
+            partial[3 * wi + 1] = sum.i;
+            partial[3 * wi + 2] = sq;
+        }
+    }
+}
+
+// scale: powers of two of the matrices' rows that the sums leave out (NULL or
+// GURVITS_FP64: none).
+__global__ void gurvits_finalize_kernel(const double *__restrict__ partial, int64_t count, int parts, int64_t iters,
+                                        const int32_t *__restrict__ scale, cd *__restrict__ est,
+                                        double *__restrict__ err)
+{
+    const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // one wave per matrix
+    const int lane = threadIdx.x & 63;
     if (b >= count) return;
     double sr = 0.0, si = 0.0, sq = 0.0;
-    for (int q = 0; q < parts; q++) {
+    for (int q = lane; q < parts; q += 64) {
         const double *pp = partial + 3 * (b * parts + q);
         sr += pp[0];
         si += pp[1];
         sq += pp[2];
     }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        sr += __shfl_xor(sr, o, 64);
+        si += __shfl_xor(si, o, 64);
+        sq += __shfl_xor(sq, o, 64);
+    }
+    if (lane != 0) return;
     const double inv = 1.0 / (double)iters;
     const cd mean = {sr * inv, si * inv};
     const double var = sq * inv - (mean.r * mean.r + mean.i * mean.i);
-    est[b] = mean;
-    err[b] = 2.5758293035489004 * sqrt((var > 0.0 ? var : 0.0) * inv);
+    const int E = scale && scale[b] != GURVITS_FP64 ? scale[b] : 0;
+    est[b] = {ldexp(mean.r, E), ldexp(mean.i, E)};
+    err[b] = ldexp(2.5758293035489004 * sqrt((var > 0.0 ? var : 0.0) * inv), E);
 }
 
 template <int NP>
 static int launch_gurvits(const cd *mats, const GurvitsItem *items, int64_t count, int parts, int64_t iters,
-                          int64_t per, uint64_t seed, uint64_t stream0, double *partial, hipStream_t st)
+                          int64_t per, uint64_t seed, uint64_t stream0, double *partial, const int32_t *scale,
+                          hipStream_t st)
 {
     int dev = 0, cus = 0, per_cu = 0;
     PCVL_HIP_CHECK(hipGetDevice(&dev));
@@ -282,11 +525,40 @@ static int launch_gurvits(const cd *mats, const GurvitsItem *items, int64_t coun
     const int grid = (int)std::min<int64_t>(count * parts, (int64_t)cus * per_cu);
     if constexpr (MF)
         hipLaunchKernelGGL((gurvits_mfma_kernel<NP>), dim3(grid), dim3(threads), 0, st, mats, items, count, parts,
-                           iters, per, seed, stream0, partial);
+                           iters, per, seed, stream0, partial, scale);
     else
         hipLaunchKernelGGL((gurvits_kernel<NP>), dim3(grid), dim3(64), 0, st, mats, items, count, parts, iters, per,
                            seed, stream0, partial);
     PCVL_HIP_CHECK(hipGetLastError());
+    return OK;
+}
+
+// Integer products: digits of every matrix, the int8 kernel, and the FP64
+// kernel for the matrices that keep it (usually none: its waves leave at once).
+template <int NP>
+static int launch_gurvits_int8(const cd *mats, const GurvitsItem *items, int64_t count, int parts, int64_t iters,
+                               int64_t per, uint64_t seed, uint64_t stream0, double *partial, gv_i4 *frags,
+                               int32_t *scale, int cus, hipStream_t st)
+{
+    hipLaunchKernelGGL((gurvits_digits_kernel<NP>), dim3((unsigned)std::min<int64_t>(count * (NP / 8), (int64_t)cus * 8)),
+                       dim3(256), 0, st, mats, items, count, frags, scale);
+    PCVL_HIP_CHECK(hipGetLastError());
+    const unsigned grid = (unsigned)std::min<int64_t>(count * parts, int64_t(1) << 30);
+    hipLaunchKernelGGL((gurvits_int8_kernel<NP>), dim3(grid), dim3(64), 0, st, frags, items, count, parts, iters, per,
+                       seed, stream0, partial, scale);
+    PCVL_HIP_CHECK(hipGetLastError());
+    return launch_gurvits<NP>(mats, items, count, parts, iters, per, seed, stream0, partial, scale, st);
+}
+
+// Parts of a matrix for the integer kernel: equal rounds of the resident
+// waves, each part at least 1,024 samples.
+template <int NP>
+static int gurvits_int8_parts(int64_t count, int64_t iters, int cus, int *parts)
+{
+    int per_cu = 0;
+    PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per_cu, reinterpret_cast<const void *>(&gurvits_int8_kernel<NP>), 64, 0));
+    *parts = (int)std::max<int64_t>(1, std::min<int64_t>(GURVITS_ROUNDS * (int64_t)cus * std::max(per_cu, 1) / count, iters / 1024));
     return OK;
 }
 
@@ -309,18 +581,34 @@ extern "C" int pcvl_gurvits_batch(const double *d_mats, const int32_t *h_n, cons
         items[(size_t)b] = GurvitsItem{h_offsets[b], h_n[b], 0};
         nmax = std::max(nmax, (int)h_n[b]);
     }
+    int dev = 0, cus = 0;
+    PCVL_HIP_CHECK(hipGetDevice(&dev));
+    PCVL_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    // Integer products for orders 9..32 (orders up to 8 take the vector kernel,
+    // above 32 a digit's two halves do not fit the 64 products of an instruction)
+    const bool int8 = nmax > 8 && nmax <= 32 && count <= INT32_MAX &&
+                      (double)count * (double)iters >= (double)gurvits_int8_min(nmax);
     // samples of a matrix are split into parts of at least 64 * 16 samples so
     // that the batch fills the device (4 waves per SIMD of 256 CUs)
     int parts = (int)std::max<int64_t>(1, std::min<int64_t>((4096 + count - 1) / count, iters / 1024));
+    if (int8) {
+        int rc = nmax <= 16 ? gurvits_int8_parts<16>(count, iters, cus, &parts)
+                            : gurvits_int8_parts<32>(count, iters, cus, &parts);
+        if (rc != OK) return rc;
+    }
     const int64_t per = (iters + parts - 1) / parts;
     parts = (int)((iters + per - 1) / per);
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     const size_t b_items = al(sizeof(GurvitsItem) * items.size());
     const size_t b_part = al(sizeof(double) * 3 * (size_t)count * parts);
+    const size_t b_scale = int8 ? al(sizeof(int32_t) * (size_t)count) : 0;
+    const size_t b_frag = int8 ? sizeof(gv_i4) * (size_t)gurvits_frags(nmax <= 16 ? 16 : 32) * (size_t)count : 0;
     char *blk = nullptr;
-    PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk), b_items + b_part, stream));
+    PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk), b_items + b_part + b_scale + b_frag, stream));
     GurvitsItem *d_items = reinterpret_cast<GurvitsItem *>(blk);
     double *d_part = reinterpret_cast<double *>(blk + b_items);
+    int32_t *d_scale = int8 ? reinterpret_cast<int32_t *>(blk + b_items + b_part) : nullptr;
+    gv_i4 *d_frag = reinterpret_cast<gv_i4 *>(blk + b_items + b_part + b_scale);
     hipError_t e = hipMemcpyAsync(d_items, items.data(), sizeof(GurvitsItem) * items.size(), hipMemcpyHostToDevice,
                                   stream);
     int rc = OK;
@@ -329,13 +617,21 @@ extern "C" int pcvl_gurvits_batch(const double *d_mats, const int32_t *h_n, cons
         rc = ERR_HIP;
     } else {
         const cd *mats = reinterpret_cast<const cd *>(d_mats);
-        if (nmax <= 8) rc = launch_gurvits<8>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, stream);
-        else if (nmax <= 16) rc = launch_gurvits<16>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, stream);
-        else if (nmax <= 32) rc = launch_gurvits<32>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, stream);
-        else rc = launch_gurvits<48>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, stream);
+        if (int8 && nmax <= 16)
+            rc = launch_gurvits_int8<16>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, d_frag, d_scale, cus, stream);
+        else if (int8)
+            rc = launch_gurvits_int8<32>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, d_frag, d_scale, cus, stream);
+        else if (nmax <= 8)
+            rc = launch_gurvits<8>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, nullptr, stream);
+        else if (nmax <= 16)
+            rc = launch_gurvits<16>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, nullptr, stream);
+        else if (nmax <= 32)
+            rc = launch_gurvits<32>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, nullptr, stream);
+        else
+            rc = launch_gurvits<48>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, nullptr, stream);
         if (rc == OK) {
-            hipLaunchKernelGGL(gurvits_finalize_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream,
-                               d_part, count, parts, iters, reinterpret_cast<cd *>(d_est), d_err);
+            hipLaunchKernelGGL(gurvits_finalize_kernel, dim3((unsigned)((count + 3) / 4)), dim3(256), 0, stream,
+                               d_part, count, parts, iters, d_scale, reinterpret_cast<cd *>(d_est), d_err);
             e = hipGetLastError();
             if (e != hipSuccess) { set_error(std::string("gurvits finalize: ") + hipGetErrorString(e)); rc = ERR_HIP; }
         }

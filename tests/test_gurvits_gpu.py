@@ -32,6 +32,40 @@ def test_gurvits_batch_vs_oracle(gpu, orders):
         assert abs(err[b] - ref_err) <= 1e-6 * ref_err + 1e-6 * scale / np.sqrt(iters), (orders[b], err[b], ref_err)
 
 
+@pytest.mark.parametrize("orders", [[9, 15, 16], [3, 17, 31, 32], [30, 30]])
+def test_gurvits_integer_products_vs_oracle(gpu, orders):
+    """Calls long enough for the integer products: padding rows and none, an
+    order below the kernel's, entries at the ends of the fixed point (rows of
+    scale 2^-300 and 2^200, zero rows and components, powers of two), and
+    matrices whose entries keep the FP64 products (a component of 2^-50 of its
+    row's largest; one that is not finite) beside ones that do not.  Sums are
+    compared as in test_gurvits_batch_vs_oracle."""
+    from perceval_amd.permanent import gurvits
+    rng = np.random.RandomState(sum(orders))
+    mats = [(rng.randn(n, n) + 1j * rng.randn(n, n)) / np.sqrt(n) for n in orders]
+    n = orders[-1]
+    scaled = (rng.randn(n, n) + 1j * rng.randn(n, n)) / np.sqrt(n)
+    scaled[0] *= 2.0 ** -300
+    scaled[1] *= 2.0 ** 200
+    structured = rng.randint(-1, 2, size=(n, n)) * 2.0 ** rng.randint(-9, 1, size=(n, n)) + 0j
+    structured[:, 1] = 1j
+    tiny = mats[-1].copy()
+    tiny[2, 3] = 2.0 ** -50
+    zero_row = mats[-1].copy()
+    zero_row[n - 1] = 0.0
+    nan = mats[-1].copy()
+    nan[0, 0] = np.nan
+    mats += [scaled, structured, tiny, zero_row, nan]
+    iters, seed = (1 << 22) // len(mats) + 77, 7
+    est, err = gurvits(mats, iters, seed=seed)
+    assert np.isnan(est[-1]) and est[-2] == 0.0 and err[-2] == 0.0
+    for b, M in enumerate(mats[:-2]):
+        ref_est, ref_err = oracle.gurvits(M, iters, seed=seed, stream=b)
+        scale = max(ref_err * np.sqrt(iters) / 2.5758293035489004, abs(ref_est), 1e-300)
+        assert abs(est[b] - ref_est) <= 1e-11 * scale, (b, est[b], ref_est)
+        assert abs(err[b] - ref_err) <= 1e-6 * ref_err, (b, err[b], ref_err)
+
+
 def test_gurvits_exact_cases(gpu):
     from perceval_amd.permanent import gurvits
     est, err = gurvits([np.eye(7), np.array([[3 - 2j]]), np.zeros((0, 0))], 100, seed=3)
