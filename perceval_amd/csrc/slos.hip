@@ -1107,9 +1107,13 @@ extern "C" int pcvl_slos_plan_destroy(pcvl_slos_plan plan)
 // still to add are summed over the node's targets, the mode with the largest
 // sum (lowest on ties) becomes a child taking every target that still has a
 // photon there, and the rest is decomposed again; a target with no photon
-// left is mapped to the node.  Shared prefixes are computed once.  Execution
-// is depth first: node layers live in one buffer per depth, so a node's
-// parent layer is still in place when the node is computed.
+// left is mapped to the node.  Shared prefixes are computed once.  Where every
+// node's layer fits TREE_LEVEL_BYTES of workspace together, the nodes of one
+// depth run in one launch (20 modes, 37 inputs of 6..8 photons: 101 launches
+// and 875 us one node at a time, see the batch kernel).  Larger trees, whose
+// layers fill the device by themselves, and those without a block layout run
+// depth first: node layers live in one buffer per depth, so a node's parent
+// layer is still in place when the node is computed.
 
 struct TreeOp {
     int k;              // layer of the node (photons)
@@ -1119,6 +1123,16 @@ struct TreeOp {
     double inv_prod_in; // 1 / prod t! of that input
 };
 
+// A node that has children or outputs (k >= 1), for the launches by depth.
+struct TreeNode {
+    int k, mk;
+    int parent;                // node index, -1: the vacuum
+    bool has_children;
+    std::vector<int> inputs;   // inputs that end here
+};
+
+constexpr size_t TREE_LEVEL_BYTES = size_t(1) << 30;
+
 struct SlosTreeImpl {
     int m = 0, nmax = 0, w = 0, ninputs = 0;
     std::vector<uint64_t> counts;       // N_0..N_nmax
@@ -1127,13 +1141,16 @@ struct SlosTreeImpl {
     std::vector<size_t> level_off;      // byte offset of depth buffer k in the workspace
     size_t work_bytes = 0;
     std::vector<TreeOp> ops;            // depth-first launch list
+    std::vector<TreeNode> nodes;
+    std::vector<int> level_ops;         // by depth: first entry of depth k in d_ops (nmax + 2 entries); empty: depth first
+    BlkBatchOp *d_ops = nullptr;
     uint64_t *d_T = nullptr, *d_E = nullptr;
     int grid_cap = 0;
     BlkLayout blk;                      // block layout of the layers, when they allow it
 };
 
 static void tree_decompose(SlosTreeImpl &t, int k, int mk, std::vector<std::vector<int32_t>> targets,
-                           std::vector<int> ids, const std::vector<double> &inv_pin)
+                           std::vector<int> ids, const std::vector<double> &inv_pin, int parent = -1)
 {
     std::vector<int> here;
     std::vector<std::vector<int32_t>> tg;
@@ -1146,6 +1163,11 @@ static void tree_decompose(SlosTreeImpl &t, int k, int mk, std::vector<std::vect
     }
     // the node itself: its layer feeds children (to_level) and/or outputs
     const bool has_children = !tg.empty();
+    int self = -1;
+    if (k > 0) {
+        self = (int)t.nodes.size();
+        t.nodes.push_back(TreeNode{k, mk, parent, has_children, here});
+    }
     if (k > 0) {
         if (has_children) t.ops.push_back(TreeOp{k, mk, 1, -1, 1.0});
         for (int id : here) t.ops.push_back(TreeOp{k, mk, 0, id, inv_pin[(size_t)id]});
@@ -1169,10 +1191,62 @@ static void tree_decompose(SlosTreeImpl &t, int k, int mk, std::vector<std::vect
                 rid.push_back(tid[i]);
             }
         }
-        tree_decompose(t, k + 1, best, std::move(child), std::move(cid), inv_pin);
+        tree_decompose(t, k + 1, best, std::move(child), std::move(cid), inv_pin, self);
         tg = std::move(rest);
         tid = std::move(rid);
     }
+}
+
+// Workspace and launch table of the tree by depth, when its layers fit.
+static int tree_levels(SlosTreeImpl &t, const std::vector<double> &inv_pin)
+{
+    auto layer_bytes = [&](int k) { return ((sizeof(cd) * (size_t)t.counts[(size_t)k]) + 255) & ~size_t(255); };
+    size_t total = layer_bytes(0);
+    for (const TreeNode &nd : t.nodes) {
+        if (!nd.has_children) continue;
+        total += layer_bytes(nd.k);
+        if (total > TREE_LEVEL_BYTES) return OK;
+    }
+    size_t off = layer_bytes(0);   // the vacuum first
+    std::vector<int64_t> at(t.nodes.size(), -1);
+    for (size_t i = 0; i < t.nodes.size(); i++) {
+        if (!t.nodes[i].has_children) continue;
+        at[i] = (int64_t)off;
+        off += layer_bytes(t.nodes[i].k);
+    }
+    std::vector<BlkBatchOp> ops;
+    std::vector<int> first;
+    for (int k = 0; k <= t.nmax; k++) {
+        first.push_back((int)ops.size());
+        for (size_t i = 0; i < t.nodes.size(); i++) {
+            const TreeNode &nd = t.nodes[i];
+            if (nd.k != k) continue;
+            BlkBatchOp op;
+            op.par_off = nd.parent < 0 ? 0 : at[(size_t)nd.parent];
+            op.mk = nd.mk;
+            op.pad = 0;
+            for (size_t q = 0; q < std::max<size_t>(1, nd.inputs.size()); q++) {
+                op.lvl_off = q == 0 ? at[i] : -1;
+                op.out_off = nd.inputs.empty() ? -1 : t.out_off[(size_t)nd.inputs[q]];
+                op.inv_prod_in = nd.inputs.empty() ? 1.0 : inv_pin[(size_t)nd.inputs[q]];
+                ops.push_back(op);
+            }
+        }
+    }
+    first.push_back((int)ops.size());
+    if (ops.empty()) return OK;
+    hipError_t e = hipMalloc(&t.d_ops, sizeof(BlkBatchOp) * ops.size());
+    if (e != hipSuccess) { t.d_ops = nullptr; set_error(std::string("hipMalloc(slos tree ops): ") + hipGetErrorString(e)); return ERR_ALLOC; }
+    e = hipMemcpy(t.d_ops, ops.data(), sizeof(BlkBatchOp) * ops.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(t.d_ops);
+        t.d_ops = nullptr;
+        set_error(std::string("hipMemcpy(slos tree ops): ") + hipGetErrorString(e));
+        return ERR_HIP;
+    }
+    t.level_ops = std::move(first);
+    t.work_bytes = off;
+    return OK;
 }
 
 struct pcvl_slos_tree_s {
@@ -1256,6 +1330,7 @@ extern "C" int pcvl_slos_tree_create(int m, const int32_t *h_inputs, int count, 
         set_error("SLOS tree: modes and photons too many for the per-state kernel's tables");
         rc = ERR_RANGE;
     }
+    if (rc == OK && t.blk.d_mem) rc = tree_levels(t, inv_pin);
     if (rc != OK) { blk_layout_destroy(&t.blk); (void)hipFree(t.d_T); delete plan; return rc; }
     *out = plan;
     return OK;
@@ -1294,6 +1369,7 @@ extern "C" int pcvl_slos_tree_execute(pcvl_slos_tree plan, const double *d_U, in
         PCVL_HIP_CHECK(hipGetLastError());
     }
     for (const TreeOp &op : t.ops) {
+        if (op.k != 0 && !t.level_ops.empty()) continue;   // run by depth below
         if (op.k == 0) {   // input with no photon: vacuum output
             hipLaunchKernelGGL(slos_vacuum_kernel, dim3(1), dim3(64), 0, stream,
                                reinterpret_cast<double *>(static_cast<char *>(d_out) + esz * (size_t)t.out_off[(size_t)op.input]),
@@ -1329,6 +1405,14 @@ extern "C" int pcvl_slos_tree_execute(pcvl_slos_tree plan, const double *d_U, in
                                op.inv_prod_in);
         PCVL_HIP_CHECK(hipGetLastError());
     }
+    if (!t.level_ops.empty())
+        for (int k = 1; k <= t.nmax; k++) {
+            const int a = t.level_ops[(size_t)k], n = t.level_ops[(size_t)k + 1] - a;
+            if (n == 0) continue;
+            const int rc = blk_batch_launch(t.blk, t.d_ops + a, n, work, static_cast<char *>(d_out),
+                                            mode == PCVL_SLOS_PROBS, U, t.m, k, stream);
+            if (rc != OK) return rc;
+        }
     return OK;
 }
 
@@ -1337,6 +1421,7 @@ extern "C" int pcvl_slos_tree_destroy(pcvl_slos_tree plan)
     if (!plan) return OK;
     hipError_t e = hipSuccess;
     if (plan->impl.d_T) e = hipFree(plan->impl.d_T);
+    if (plan->impl.d_ops) (void)hipFree(plan->impl.d_ops);
     blk_layout_destroy(&plan->impl.blk);
     delete plan;
     if (e != hipSuccess) { set_error(std::string("hipFree(slos tree): ") + hipGetErrorString(e)); return ERR_HIP; }

@@ -160,4 +160,18 @@ bool blk_layout_ok(int m, int nmax);
 int blk_layer_launch(const BlkLayout &lay, const cd *parent, void *out, const cd *U, int m, int mk, int k, bool probs,
                      double inv_prod_in, bool sentinel, hipStream_t stream);
 
+// One node of an input tree at layer k: parent layer at byte par_off of the
+// workspace, coefficients to byte lvl_off of it (< 0: none), output to element
+// out_off of the output buffer (< 0: none).
+struct BlkBatchOp {
+    int64_t par_off, lvl_off, out_off;
+    double inv_prod_in;
+    int32_t mk, pad;
+};
+
+// Enqueues layer k of nops nodes (d_ops: device), probabilities or
+// coefficients to `out`, in one launch.  Unmasked layouts.
+int blk_batch_launch(const BlkLayout &lay, const BlkBatchOp *d_ops, int nops, char *work, char *out, bool probs,
+                     const cd *U, int m, int k, hipStream_t stream);
+
 } // namespace pcvl

@@ -107,6 +107,37 @@ __device__ __forceinline__ void blk_store(cd *p, cd v)
     __builtin_nontemporal_store(v.i, &p->i);
 }
 
+// Where a layer's children go.  MODE 0: coefficients to out; 1: probabilities
+// to out; 2 (batches): coefficients to lvl if there is one, and probabilities
+// (probs) or coefficients to out if there is one.
+struct BlkDest {
+    void *out;
+    cd *lvl;
+    bool probs;
+};
+
+template <int MODE>
+__device__ __forceinline__ bool blk_wants_prob(const BlkDest &d)
+{
+    return MODE == 1 || (MODE == 2 && d.out && d.probs);
+}
+
+template <int MODE>
+__device__ __forceinline__ void blk_emit(const BlkDest &d, size_t o, cd acc, double pf, double inv_prod_in)
+{
+    if (MODE == 0) {
+        blk_store(reinterpret_cast<cd *>(d.out) + o, acc);
+    } else if (MODE == 1) {
+        blk_store(reinterpret_cast<double *>(d.out) + o, prob_from_coef(acc, pf, inv_prod_in));
+    } else {
+        if (d.lvl) blk_store(d.lvl + o, acc);
+        if (d.out) {
+            if (d.probs) blk_store(reinterpret_cast<double *>(d.out) + o, prob_from_coef(acc, pf, inv_prod_in));
+            else blk_store(reinterpret_cast<cd *>(d.out) + o, acc);
+        }
+    }
+}
+
 __device__ __forceinline__ void blk_heralds(cd &acc, const cd *__restrict__ parent, const uint2 *__restrict__ her,
                                             uint32_t nher, const cd *su, int mfree, uint32_t loc)
 {
@@ -169,7 +200,7 @@ __device__ __forceinline__ void blk_suffix(cd &acc, const char *ps, const uint32
 // herald modes, prefix modes, suffix modes, each increasing.
 template <int MODE>
 __device__ __forceinline__ void blk_item_a(
-    const BlkGroup &g, uint32_t item, uint32_t lane, const cd *__restrict__ parent, void *__restrict__ out,
+    const BlkGroup &g, uint32_t item, uint32_t lane, const cd *__restrict__ parent, const BlkDest &out,
     const cd *su, int h, int wsfx, int mfree, const uint2 *__restrict__ her, const double *__restrict__ spf,
     const uint32_t *__restrict__ sslot, const BlkRec *__restrict__ recs, double inv_prod_in)
 {
@@ -186,7 +217,8 @@ __device__ __forceinline__ void blk_item_a(
     uint32_t sw[8];
 #pragma unroll
     for (int d = 0; d < 8; d++) sw[d] = d < smax ? ts[(size_t)d * S] : 0xffffffffu;
-    const double pfs = MODE == 1 ? spf[g.tpf + beta] : 0.0;
+    const bool want = blk_wants_prob<MODE>(out);
+    const double pfs = want ? spf[g.tpf + beta] : 0.0;
     const uint32_t Bk = rw[0], PEh = rw[1];
     const int cnt = (int)rw[2];
     cd acc = {0.0, 0.0};
@@ -234,13 +266,13 @@ __device__ __forceinline__ void blk_item_a(
             if (sw[t] != 0xffffffffu) cfma_acc(acc, qv[t], su[h + (int)(sw[t] & 31u)]);
     }
     const size_t o = (size_t)g.out_base + Bk + beta;
-    if (MODE == 0) {
-        blk_store(reinterpret_cast<cd *>(out) + o, acc);
-    } else {
+    double pf = 0.0;
+    if (want) {
         double pfa;
         __builtin_memcpy(&pfa, &rw[8], sizeof(double));
-        blk_store(reinterpret_cast<double *>(out) + o, prob_from_coef(acc, pfa * pfs * blk_hfact(g), inv_prod_in));
+        pf = pfa * pfs * blk_hfact(g);
     }
+    blk_emit<MODE>(out, o, acc, pf, inv_prod_in);
 }
 
 // One wave item of a group whose blocks are smaller than a wave: 64
@@ -248,7 +280,7 @@ __device__ __forceinline__ void blk_item_a(
 // occupied prefix modes in LDS, per thread).
 template <int MODE, bool PFI>
 __device__ __forceinline__ void blk_item_b(
-    const BlkGroup &g, uint32_t item, uint32_t lane, int tid, const cd *__restrict__ parent, void *__restrict__ out,
+    const BlkGroup &g, uint32_t item, uint32_t lane, int tid, const cd *__restrict__ parent, const BlkDest &out,
     const cd *su, uint32_t *lpe, uint8_t *lmd, int h, int wsfx, int mfree, const uint2 *__restrict__ her,
     const uint32_t *__restrict__ Th, const uint64_t *__restrict__ TE, const uint64_t *__restrict__ CTE, int wt,
     const uint32_t *__restrict__ f32, const double *__restrict__ fd, const double *__restrict__ spf,
@@ -314,12 +346,8 @@ __device__ __forceinline__ void blk_item_b(
         blk_suffix(acc, reinterpret_cast<const char *>(parent + g.par_base + (Bk - PEh)), sslot + g.tslot + beta, S,
                    smax, su, h);
     const size_t o = (size_t)g.out_base + Bk + beta;
-    if (MODE == 0) {
-        blk_store(reinterpret_cast<cd *>(out) + o, acc);
-    } else {
-        const double pf = (double)pfp * spf[g.tpf + beta] * blk_hfact(g);
-        blk_store(reinterpret_cast<double *>(out) + o, prob_from_coef(acc, pf, inv_prod_in));
-    }
+    const double pf = blk_wants_prob<MODE>(out) ? (double)pfp * spf[g.tpf + beta] * blk_hfact(g) : 0.0;
+    blk_emit<MODE>(out, o, acc, pf, inv_prod_in);
 }
 
 // Persistent layer kernel: the workgroups of XCD x (blockIdx % 8, dispatch
@@ -328,8 +356,8 @@ __device__ __forceinline__ void blk_item_b(
 // same group at a time and each on a contiguous part of it (each XCD has its
 // own L2).  Waves take items at a stride of the XCD's waves.
 template <int MODE, bool PFI>
-__global__ void __launch_bounds__(BLK_THREADS) slos_block_kernel(
-    const cd *__restrict__ parent, void *__restrict__ out, const cd *__restrict__ U, int m, int mk, int k,
+__device__ __forceinline__ void blk_layer(
+    const cd *__restrict__ parent, const BlkDest &out, const cd *__restrict__ U, int m, int mk, int k,
     uint32_t nchild, int h, int wsfx, int mfree, int mloc, const int32_t *__restrict__ rowmap,
     const BlkGroup *__restrict__ groups, int ngroups, const uint2 *__restrict__ her,
     const char *__restrict__ tabs, BlkTabOffsets to, int wt, const double *__restrict__ spf,
@@ -361,7 +389,7 @@ __global__ void __launch_bounds__(BLK_THREADS) slos_block_kernel(
         uint4 *gdst = reinterpret_cast<uint4 *>(sg);
         for (int e = tid; e < ngroups * (int)(sizeof(BlkGroup) / sizeof(uint4)); e += BLK_THREADS) gdst[e] = gsrc[e];
     }
-    if (sentinel && blockIdx.x == 0 && tid == 0) reinterpret_cast<cd *>(out)[nchild] = cd{0.0, 0.0};
+    if (sentinel && blockIdx.x == 0 && tid == 0) reinterpret_cast<cd *>(out.out)[nchild] = cd{0.0, 0.0};
     __syncthreads();
 
     const uint32_t lane = tid & 63u;
@@ -396,6 +424,40 @@ __global__ void __launch_bounds__(BLK_THREADS) slos_block_kernel(
                                       wt, f32, fd, spf, sslot, inv_prod_in);
         }
     }
+}
+
+template <int MODE, bool PFI>
+__global__ void __launch_bounds__(BLK_THREADS) slos_block_kernel(
+    const cd *__restrict__ parent, void *__restrict__ out, const cd *__restrict__ U, int m, int mk, int k,
+    uint32_t nchild, int h, int wsfx, int mfree, int mloc, const int32_t *__restrict__ rowmap,
+    const BlkGroup *__restrict__ groups, int ngroups, const uint2 *__restrict__ her,
+    const char *__restrict__ tabs, BlkTabOffsets to, int wt, const double *__restrict__ spf,
+    const uint32_t *__restrict__ sslot, const BlkRec *__restrict__ recs, double inv_prod_in, int sentinel)
+{
+    blk_layer<MODE, PFI>(parent, BlkDest{out, nullptr, MODE == 1}, U, m, mk, k, nchild, h, wsfx, mfree, mloc, rowmap,
+                         groups, ngroups, her, tabs, to, wt, spf, sslot, recs, inv_prod_in, sentinel);
+}
+
+// Layer k of several nodes of an input tree: blockIdx.y is the node, the
+// workgroups of one node as in slos_block_kernel (gridDim.x is a multiple of
+// 8, so the XCD of a workgroup is still blockIdx.x % 8).  A tree's small
+// layers are bound by launch and first-load latency: 37 inputs of 6..8 photons
+// in 20 modes took 878 us in 100 launches of 8-11 us one node at a time, and
+// take 209 us in one launch per depth (each node's layer computed once, where
+// a node with children and outputs took two).
+template <bool PFI>
+__global__ void __launch_bounds__(BLK_THREADS) slos_block_batch_kernel(
+    char *work, char *outb, int probs, const BlkBatchOp *__restrict__ ops, const cd *__restrict__ U, int m, int k,
+    uint32_t nchild, int h, int wsfx, int mfree, int mloc, const BlkGroup *__restrict__ groups, int ngroups,
+    const uint2 *__restrict__ her, const char *__restrict__ tabs, BlkTabOffsets to, int wt,
+    const double *__restrict__ spf, const uint32_t *__restrict__ sslot, const BlkRec *__restrict__ recs)
+{
+    const BlkBatchOp op = ops[blockIdx.y];
+    const size_t esz = probs ? sizeof(double) : sizeof(cd);
+    const BlkDest dst = {op.out_off >= 0 ? outb + (size_t)op.out_off * esz : nullptr,
+                         op.lvl_off >= 0 ? reinterpret_cast<cd *>(work + op.lvl_off) : nullptr, probs != 0};
+    blk_layer<2, PFI>(reinterpret_cast<const cd *>(work + op.par_off), dst, U, m, op.mk, k, nchild, h, wsfx, mfree,
+                      mloc, nullptr, groups, ngroups, her, tabs, to, wt, spf, sslot, recs, op.inv_prod_in, 0);
 }
 
 // ------------------------------------------------------------------ host
@@ -1004,6 +1066,39 @@ int blk_layer_launch(const BlkLayout &lay, const cd *parent, void *out, const cd
                        reinterpret_cast<const uint32_t *>(base + lay.off_slot),
                        reinterpret_cast<const BlkRec *>(base + lay.off_rec), inv_prod_in, sentinel ? 1 : 0);
     PCVL_HIP_CHECK(hipGetLastError());
+    return OK;
+}
+
+int blk_batch_launch(const BlkLayout &lay, const BlkBatchOp *d_ops, int nops, char *work, char *out, bool probs,
+                     const cd *U, int m, int k, hipStream_t stream)
+{
+    if (k < 1 || k > lay.nlayers || !lay.d_mem || !lay.row_identity) {
+        set_error("block SLOS: batch outside the layout");
+        return ERR_ARG;
+    }
+    if (lay.items[(size_t)k] == 0) return OK;
+    const uint64_t want = (lay.items[(size_t)k] + (BLK_THREADS / 64) - 1) / (BLK_THREADS / 64);
+    const char *base = lay.d_mem;
+    const BlkGroup *groups = reinterpret_cast<const BlkGroup *>(base + lay.group_off[(size_t)k]);
+    const size_t lds = blk_lds_bytes(lay, k);
+    const BlkTabOffsets to = {(uint32_t)(lay.off_te - lay.off_th), (uint32_t)(lay.off_cte - lay.off_th),
+                              (uint32_t)(lay.off_f32 - lay.off_th), (uint32_t)(lay.off_fd - lay.off_th),
+                              (uint32_t)(lay.off_row - lay.off_th)};
+    auto kp = lay.nmax <= 12 ? slos_block_batch_kernel<true> : slos_block_batch_kernel<false>;
+    for (int o = 0; o < nops; o += 32768) {
+        const int ny = std::min(nops - o, 32768);
+        // about one resident round of workgroups over all nodes, each node at
+        // least 16 (a workgroup's tables cost it a few microseconds of loads)
+        const uint64_t cap = std::max<uint64_t>(16, ((uint64_t)lay.grid_cap / (uint64_t)ny + 7) / 8 * 8);
+        const uint32_t grid = (uint32_t)((std::min<uint64_t>(want, cap) + 7) / 8 * 8);
+        hipLaunchKernelGGL(kp, dim3(grid, (unsigned)ny), dim3(BLK_THREADS), lds, stream, work, out, probs ? 1 : 0,
+                           d_ops + o, U, m, k, (uint32_t)lay.counts[(size_t)k], lay.h, lay.w, lay.m, lay.mloc, groups,
+                           (int)lay.groups[(size_t)k].size(), reinterpret_cast<const uint2 *>(base + lay.off_her),
+                           base + lay.off_th, to, lay.wt, reinterpret_cast<const double *>(base + lay.off_pf),
+                           reinterpret_cast<const uint32_t *>(base + lay.off_slot),
+                           reinterpret_cast<const BlkRec *>(base + lay.off_rec));
+        PCVL_HIP_CHECK(hipGetLastError());
+    }
     return OK;
 }
 

@@ -384,6 +384,31 @@ def test_slos_tree_vs_oracle_and_single_plans(gpu, m, inputs):
     tree.close()
 
 
+def test_slos_tree_depth_first_vs_single_plans(gpu):
+    """A tree whose layers take more than 1 GiB runs depth first, one layer
+    buffer per depth; compared with the same inputs' single plans at the bar of
+    the test above (a tree may add the photons in another order).  A repeated
+    input and one that ends inside another's path are part of it."""
+    from perceval_amd.slos import PROBS, SlosPlan, SlosTree
+    m = 24
+    inputs = [[1] * 9 + [0] * 15, [0] * 15 + [1] * 9, [2] * 4 + [1] + [0] * 19, [1] * 7 + [0] * 17, [1] * 9 + [0] * 15]
+    U = haar_unitary(m, seed=11)
+    tree = SlosTree(inputs)
+    assert tree.work_bytes < 2 ** 30   # depth first: one buffer per depth
+    for s, got in zip(inputs, tree.run(U, PROBS)):
+        plan = SlosPlan(s)
+        assert (got - plan.run(U, PROBS)).abs().max().item() < 1e-13, s
+        plan.close()
+    tree.close()
+    small = SlosTree([r[-12:] for r in ([0] * 12 + [1] * 5 + [0] * 7, [0] * 12 + [1] * 4 + [0] * 8, [0] * 24,
+                                       [0] * 12 + [1] * 5 + [0] * 7)])
+    for s, got in zip(small.inputs, small.run(haar_unitary(12, seed=3), PROBS)):
+        plan = SlosPlan(s)
+        assert (got - plan.run(haar_unitary(12, seed=3), PROBS)).abs().max().item() < 1e-13, s
+        plan.close()
+    small.close()
+
+
 def test_slos_backend_preprocess_shares_a_tree(gpu):
     from perceval_amd.backends import SLOSBackend
     from perceval_amd.components import Unitary
