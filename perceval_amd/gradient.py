@@ -170,7 +170,11 @@ def mesh_adjoint(program: MeshProgram, phases, in_occ, targets, want_probs: bool
     state, targets)."""
     import torch
     in_occ = tuple(int(v) for v in in_occ)
-    targets = np.ascontiguousarray(np.asarray([list(t) for t in targets], dtype=np.int32))
+    # an array is taken as it is: a list per target costs more than the kernel
+    # (462 targets: 0.25 ms of a 0.08 ms call)
+    if not (isinstance(targets, np.ndarray) and targets.ndim == 2):
+        targets = [list(t) for t in targets]
+    targets = np.ascontiguousarray(np.asarray(targets, dtype=np.int32))
     w = None if weights is None else np.asarray(weights, dtype=np.float64).reshape(-1)
     if w is not None and w.size != len(targets):
         raise ValueError(f"expected {len(targets)} target weights, got {w.size}")

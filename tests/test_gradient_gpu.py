@@ -231,3 +231,79 @@ def test_weighted_observable_over_every_output(gpu):
     x = torch.from_numpy(phases).cuda().requires_grad_(True)
     target_probability(x, prog, inp, targets, lam).sum().backward()
     assert np.max(np.abs(x.grad.cpu().numpy() - grad)) < 1e-12
+
+
+def _torch_reference(prog, phases, inp, targets, weights):
+    """Loss and gradient of sum_s w_s P(s) by torch autograd on the CPU: the
+    program op by op, permanents by Glynn's formula over all sign vectors."""
+    import torch
+    ph = torch.tensor(phases, dtype=torch.float64, requires_grad=True)
+    cols = [i for i, v in enumerate(inp) for _ in range(v)]
+    n = len(cols)
+    rows = torch.tensor([[q for q, v in enumerate(t) for _ in range(v)] for t in targets])
+    norm = torch.tensor([oracle.prodnfact(t) * oracle.prodnfact(inp) for t in targets], dtype=torch.float64)
+    w = torch.tensor(weights, dtype=torch.float64)
+    losses = []
+    for b in range(ph.shape[0]):
+        U = list(torch.eye(prog.m, dtype=torch.complex128))
+        for k, q, p, c in zip(prog.kind, prog.mode, prog.param, prog.const.reshape(-1, 8)):
+            if k == 0:
+                phi = ph[b, int(p)] if p >= 0 else torch.tensor(c[0], dtype=torch.float64)
+                U[q] = U[q] * torch.polar(torch.ones_like(phi), phi)
+            else:
+                M = torch.tensor(c[0::2] + 1j * c[1::2])
+                U[q], U[q + 1] = M[0] * U[q] + M[1] * U[q + 1], M[2] * U[q] + M[3] * U[q + 1]
+        sub = torch.stack(U)[rows][:, :, cols]            # (T, n, n)
+        amp = 0
+        for t in range(2 ** (n - 1)):
+            s = torch.tensor([1.0] + [1.0 - 2.0 * ((t >> i) & 1) for i in range(n - 1)], dtype=torch.complex128)
+            amp = amp + s.real.prod() * (s[:, None] * sub).sum(dim=1).prod(dim=1)
+        amp = amp / 2.0 ** (n - 1)
+        losses.append(((amp.real ** 2 + amp.imag ** 2) / norm * w).sum())
+    (grad,) = torch.autograd.grad(torch.stack(losses).sum(), ph)
+    return torch.stack(losses).detach().numpy(), grad.numpy()
+
+
+@pytest.mark.parametrize("kind,m,n,T", [("phases", 1, 3, 1), ("mixed", 5, 2, 15), ("mixed", 5, 3, 33),
+                                        ("mesh", 4, 4, 17), ("mesh", 6, 5, 130), ("mesh", 8, 7, 300),
+                                        ("mesh", 5, 8, 257), ("mesh", 9, 1, 9), ("bricks", 3, 2, 6)])
+def test_cells_passes_and_blocks_vs_torch(gpu, kind, m, n, T):
+    """One mode alone, phases on modes no splitter touches, fixed phases, cells
+    of several ops, a program of so many cells that they are formed in the sweep
+    ("bricks"), sub-blocks of targets that are not full, one thread per row and
+    per target (7 and 8 photons: two per target), and two passes of targets.
+    Rounding over the ops and 2^(n-1) terms stays below 10^4 ulp."""
+    from perceval_amd.components import BS, PS, Circuit
+    from perceval_amd.gradient import MeshProgram, mesh_adjoint
+    rng = np.random.RandomState(m * 100 + T)
+    if kind == "mesh":
+        circuit = clements_mesh(m)
+    else:
+        circuit = Circuit(m)
+        k = 0
+        if kind == "phases":
+            for k in range(3):
+                circuit.add(0, PS(f"p{k}"))
+            circuit.add(0, PS(0.3))
+        elif kind == "mixed":
+            circuit.add(m - 1, PS("last0")).add(0, PS("first")).add(1, PS(0.7))
+            for q in (0, 2, 1, 1, 0):   # mode m - 1 stays without a splitter
+                circuit.add(q, BS(theta=float(rng.uniform(0.3, 2.5)), phi_tr=0.4)).add(q + 1, PS(f"q{k}"))
+                k += 1
+            circuit.add(m - 1, PS("last1")).add(0, PS("end"))
+        else:
+            for k in range(1500):
+                circuit.add(k % 2, BS(theta=float(rng.uniform(0.3, 2.5))))
+                circuit.add((k // 2) % 3, PS(f"b{k}") if k % 97 == 0 else PS(0.1 * (k % 7)))
+                circuit.add((k + 1) % 2, BS(theta=float(rng.uniform(0.3, 2.5))))
+    prog = MeshProgram(circuit)
+    inp = [n // m + (1 if i < n % m else 0) for i in range(m)]
+    states = oracle.fock_enumerate(m, n)
+    targets = np.array(states)[np.sort(rng.choice(len(states), T, replace=False))]
+    weights = rng.uniform(-2, 2, size=T)
+    phases = rng.uniform(0, 2 * math.pi, size=(2, prog.nparams))
+    loss, grad = mesh_adjoint(prog, phases, inp, targets, weights=weights)
+    ref_l, ref_g = _torch_reference(prog, phases, inp, targets, weights)
+    tol = 1e4 * 2.0 ** -53 * max(1.0, np.abs(weights).sum())
+    assert np.max(np.abs(loss.cpu().numpy() - ref_l)) < tol
+    assert np.max(np.abs(grad.cpu().numpy() - ref_g)) < tol * max(1.0, np.abs(ref_g).max())
