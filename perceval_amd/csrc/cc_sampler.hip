@@ -11,8 +11,9 @@
 // pass over the rows of B: per Gray-code term, the k column sums c_l are
 // shared and prod_{l' != l} c_l' is the product of a prefix and a suffix.
 //
-// Mapping: one launch per photon step k, specialised on k so that each step
-// gets its own register allocation; within a launch one wavefront owns one
+// Mapping: one launch for steps 1..9 of up to 64 modes (16 lanes a sample), then
+// one launch per photon step k, specialised on k so that each step
+// gets its own register allocation; within such a launch one wavefront owns one
 // sample (persistent over samples), or one slice of a sample's terms from step
 // 14 on.  The terms (2^{k-2}; from step 10 on fewer, repeated rows being summed
 // by multiplicity) are split over the 32 lane pairs; partial sums of the k
@@ -431,20 +432,30 @@ __global__ void cc_init_kernel(const int32_t *__restrict__ cols, int n, int64_t 
     for (int l = 0; l < n; l++) pc[s * n + l] = cols[perm[l]];
 }
 
-// Several input states with the same photon number: sample s of the batch
-// is global sample gidx[s] (its counter stream) of input inp[s], whose
-// photon columns are cols[inp[s] * n ...].
-__global__ void cc_init_multi_kernel(const int32_t *__restrict__ cols, const int32_t *__restrict__ inp,
-                                     const int64_t *__restrict__ gidx, int n, int64_t count, uint64_t seed,
-                                     uint64_t first, int32_t *__restrict__ pc)
+// Several input states with the same photon number: the batch holds
+// start[g + 1] - start[g] samples of its g-th input, whose photon columns are
+// cols[g * n ...] and whose first output row is row0[g].  Sample s of the batch
+// is global sample gidx[s] (its output row and counter stream).
+__global__ void cc_init_multi_kernel(const int32_t *__restrict__ cols, const int64_t *__restrict__ start,
+                                     const int64_t *__restrict__ row0, int ninputs, int n, int64_t count,
+                                     uint64_t seed, uint64_t first, int64_t *__restrict__ gidx,
+                                     int32_t *__restrict__ pc)
 {
     const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= count) return;
-    const int32_t *c = cols + (size_t)inp[s] * n;
+    int g = 0, hi = ninputs - 1;   // the last input that starts at or before s
+    while (g < hi) {
+        const int mid = (g + hi + 1) >> 1;
+        if (start[mid] <= s) g = mid;
+        else hi = mid - 1;
+    }
+    const int64_t row = row0[g] + (s - start[g]);
+    gidx[s] = row;
+    const int32_t *c = cols + (size_t)g * n;
     int perm[CC_MAX_N];
     for (int l = 0; l < n; l++) perm[l] = l;
     uint64_t ctr = 0;
-    const uint64_t stream = first + (uint64_t)gidx[s];
+    const uint64_t stream = first + (uint64_t)row;
     for (int i = n - 1; i >= 1; i--) {
         const double u = uniform01(seed, stream, ctr++);
         int j = (int)(u * (i + 1));
@@ -551,6 +562,235 @@ __global__ void __launch_bounds__(64) cc_step_kernel(const cd *__restrict__ U, i
         __syncthreads();
         cc_draw<K>(sh, U, m, n, s, seed, stream, lane, r_all);
         __syncthreads();
+    }
+}
+
+// ---- the first steps in one launch --------------------------------------------
+//
+// Steps 1..CC_FIRST of a sample are a few dozen terms each; with a launch and a
+// wave per step their time goes to gathers, barriers and launches.  Here 16
+// lanes take a sample through all of them: U sits in LDS, the sample's modes and
+// columns in registers, sums and scans go through DPP moves within the 16
+// lanes, and no barrier is needed.  With CC_FIRST photons or fewer the kernel
+// writes the output rows, else the drawn modes for the steps that follow.
+// What bounds it now: the chain of LDS reads and FP64 sums of a sample, with
+// one or two waves per SIMD from 7 photons on (256 registers hold the columns).
+// Measured, a launch per step -> one launch: 20 modes, 37 inputs of 6..8
+// photons x 2,000 samples, 991 -> 180 us (26 launches of 21..49 us -> 3 of 14,
+// 26 and 58 us); 9 photons x 50,000, 20 modes 875 -> 227 us, 64 modes 892 ->
+// 310 us; 9 photons x 16, 64 modes 93 -> 56 us; 2 photons x 16, 39 -> 32 us.
+// CC_FIRST: the steps below CC_MULTI, which sum without multiplicities.
+// CC_FIRST_MODES: U and its padding take 65 KiB of LDS there, two workgroups a
+// CU; above, one launch per step from step 1.
+constexpr int CC_FIRST = CC_MULTI - 1;
+constexpr int CC_FIRST_MODES = 64;
+
+template <int CTRL>
+__device__ __forceinline__ double row_dpp(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
+// Sum over the 16 lanes of a row, every lane receiving it.
+__device__ __forceinline__ double row_sum(double v)
+{
+    v += row_dpp<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+    v += row_dpp<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+    v += row_dpp<0x141>(v);   // row_half_mirror
+    v += row_dpp<0x140>(v);   // row_mirror
+    return v;
+}
+
+// Inclusive sums over the 16 lanes of a row (row_shr 1, 2, 4, 8; zeros enter).
+__device__ __forceinline__ double row_scan(double v)
+{
+    v += row_dpp<0x111>(v);
+    v += row_dpp<0x112>(v);
+    v += row_dpp<0x114>(v);
+    v += row_dpp<0x118>(v);
+    return v;
+}
+
+// Photon K of a sample: row = output modes so far (16-byte offsets of their
+// rows of U in LDS), pc = 16-byte offsets of its columns.  Returns the mode.
+template <int K, int CH>
+__device__ __forceinline__ int cc_first_step(const char *sU, int m, int ldu, const int (&row)[CC_FIRST],
+                                             const int (&pc)[CC_FIRST], int lane, int shift, double u)
+{
+    auto at = [&](int r, int c) { return *reinterpret_cast<const cd *>(sU + r + c); };
+    cd sub[K];
+    if constexpr (K == 1) {
+        sub[0] = {1.0, 0.0};
+    } else {
+        // 2^(K-2) terms, 2^CL per lane, Gray-code order; half column sums
+        constexpr int TL = K - 2, CL = TL > 4 ? TL - 4 : 0;
+        constexpr int active = TL > 4 ? 16 : 1 << TL;
+        const uint32_t base = (uint32_t)lane << CL;
+        const uint32_t g0 = base ^ (base >> 1);
+        cd cs[K];
+#pragma unroll
+        for (int l = 0; l < K; l++) {
+            const cd a = at(row[0], pc[l]);
+            cs[l] = {0.5 * a.r, 0.5 * a.i};
+        }
+#pragma unroll
+        for (int i = 1; i < K - 1; i++) {
+            const double d = ((g0 >> (i - 1)) & 1) ? -0.5 : 0.5;
+#pragma unroll
+            for (int l = 0; l < K; l++) {
+                const cd a = at(row[i], pc[l]);
+                cs[l].r = fma(d, a.r, cs[l].r);
+                cs[l].i = fma(d, a.i, cs[l].i);
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < K; l++) sub[l] = {0.0, 0.0};
+        double sign = CL == 0 && (base & 1) ? -1.0 : 1.0;
+        if (active < 16 && lane >= active) sign = 0.0;
+#pragma unroll
+        for (int q = 0; q < (1 << CL); q++) {
+            if (q) {
+                const int b = __builtin_ctz(q);
+                const uint32_t t = base + q;
+                const double s = (((t >> b) ^ (t >> (b + 1))) & 1) ? -1.0 : 1.0;
+#pragma unroll
+                for (int l = 0; l < K; l++) {
+                    const cd a = at(row[b + 1], pc[l]);
+                    cs[l].r = fma(s, a.r, cs[l].r);
+                    cs[l].i = fma(s, a.i, cs[l].i);
+                }
+            }
+            cd P[K];
+            P[0] = {1.0, 0.0};
+            P[1] = cs[0];
+#pragma unroll
+            for (int l = 2; l < K; l++) P[l] = cmul(P[l - 1], cs[l - 1]);
+            const double sg = (q & 1) ? -sign : sign;
+            cd S = {sg, 0.0};
+#pragma unroll
+            for (int l = K - 1; l >= 1; l--) {
+                if (l == K - 1) {
+                    sub[l].r = fma(sg, P[l].r, sub[l].r);
+                    sub[l].i = fma(sg, P[l].i, sub[l].i);
+                    S = {sg * cs[l].r, sg * cs[l].i};
+                } else {
+                    cfma_acc(sub[l], P[l], S);
+                    S = cmul(S, cs[l]);
+                }
+            }
+            sub[0].r += S.r;
+            sub[0].i += S.i;
+        }
+#pragma unroll
+        for (int l = 0; l < K; l++) sub[l] = {row_sum(sub[l].r), row_sum(sub[l].i)};
+    }
+    // weights of candidate rows c * 16 + lane, then the draw as in cc_draw
+    double wv[CH], total = 0.0;
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        const int i = c * 16 + lane;
+        wv[c] = 0.0;
+        if (i < m) {
+            cd a = {0.0, 0.0};
+#pragma unroll
+            for (int l = 0; l < K; l++) cfma_acc(a, at(i * ldu * 16, pc[l]), sub[l]);
+            wv[c] = a.r * a.r + a.i * a.i;
+        }
+        total += row_sum(wv[c]);
+    }
+    const double target = u * total;
+    int pick = m - 1;
+    double below = 0.0;
+    bool found = false;
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        const double incl = row_scan(wv[c]);
+        const bool hit = c * 16 + lane < m && target < below + incl;
+        const uint32_t mask = (uint32_t)(__ballot(hit) >> shift) & 0xFFFFu;
+        if (!found && mask) {
+            pick = c * 16 + (int)__builtin_ctz(mask);
+            found = true;
+        }
+        below += row_sum(wv[c]);
+    }
+    return pick;
+}
+
+template <int K, int KMAX, int CH>
+__device__ __forceinline__ void cc_first_steps(const char *sU, int m, int ldu, int (&row)[CC_FIRST],
+                                               const int (&pc)[CC_FIRST], int (&r)[CC_FIRST], int lane, int shift,
+                                               double my_u)
+{
+    if constexpr (K <= KMAX) {
+        const double u = __shfl(my_u, K - 1, 16);
+        r[K - 1] = cc_first_step<K, CH>(sU, m, ldu, row, pc, lane, shift, u);
+        row[K - 1] = r[K - 1] * ldu * 16;
+        cc_first_steps<K + 1, KMAX, CH>(sU, m, ldu, row, pc, r, lane, shift, my_u);
+    }
+}
+
+// Photons 1..KMAX of every sample (KMAX = min(n, CC_FIRST)); rows of U up to
+// 16 CH.  out: the occupation rows when n == KMAX, else unused.
+template <int KMAX, int CH>
+__global__ void __launch_bounds__(256) cc_first_kernel(const cd *__restrict__ U, int m, int n, int64_t count,
+                                                       uint64_t seed, uint64_t first,
+                                                       const int32_t *__restrict__ pc_all, int32_t *__restrict__ r_all,
+                                                       const int64_t *__restrict__ gidx, int32_t *__restrict__ out)
+{
+    extern __shared__ cd s_u[];
+    const int ldu = m | 1;   // no bank conflicts down a column
+    for (int e = threadIdx.x; e < m * m; e += 256) s_u[(e / m) * ldu + e % m] = U[e];
+    __syncthreads();
+    const int lane = threadIdx.x & 15, shift = threadIdx.x & 48;
+    // the 16 lanes of a sample run together; a wave's samples past the end repeat the last one
+    for (int64_t s0 = (int64_t)blockIdx.x * 16; s0 < count; s0 += (int64_t)gridDim.x * 16) {
+        const int64_t mine = s0 + (threadIdx.x >> 4);
+        const int64_t s = mine < count ? mine : count - 1;
+        const int64_t global = gidx ? gidx[s] : s;
+        int pc[CC_FIRST], row[CC_FIRST], r[CC_FIRST];
+#pragma unroll
+        for (int l = 0; l < KMAX; l++) pc[l] = pc_all[s * n + l] * 16;
+        const double my_u = uniform01(seed, first + (uint64_t)global, (uint64_t)(n - 1 + lane));   // photon lane + 1
+        cc_first_steps<1, KMAX, CH>(reinterpret_cast<const char *>(s_u), m, ldu, row, pc, r, lane, shift, my_u);
+        if (mine < count) {
+            if (n == KMAX) {
+                int32_t *o = out + global * m;
+#pragma unroll
+                for (int c = 0; c < CH; c++) {
+                    const int i = c * 16 + lane;
+                    int v = 0;
+#pragma unroll
+                    for (int k = 0; k < KMAX; k++) v += r[k] == i ? 1 : 0;
+                    if (i < m) o[i] = v;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < KMAX; k++)
+                    if (lane == k) r_all[s * n + k] = r[k];
+            }
+        }
+    }
+}
+
+template <int KMAX>
+static int launch_first(int kmax, const cd *U, int m, int n, int64_t count, uint64_t seed, uint64_t first,
+                        const int32_t *pc, int32_t *r, const int64_t *gidx, int32_t *out, int cus, hipStream_t st)
+{
+    if constexpr (KMAX > CC_FIRST) {
+        set_error("internal: first steps out of range");
+        return ERR_ARG;
+    } else {
+        if (kmax != KMAX) return launch_first<KMAX + 1>(kmax, U, m, n, count, seed, first, pc, r, gidx, out, cus, st);
+        auto kp = m <= 32 ? cc_first_kernel<KMAX, 2> : cc_first_kernel<KMAX, 4>;
+        const size_t lds = sizeof(cd) * (size_t)m * (m | 1);
+        int per_cu = 0;
+        PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kp), 256, lds));
+        const int grid = (int)std::min<int64_t>((count + 15) / 16, (int64_t)cus * std::max(per_cu, 1));
+        hipLaunchKernelGGL(kp, dim3(grid), dim3(256), lds, st, U, m, n, count, seed, first, pc, r, gidx, out);
+        PCVL_HIP_CHECK(hipGetLastError());
+        return OK;
     }
 }
 
@@ -738,6 +978,32 @@ static int launch_step(int k, const cd *U, int m, int n, int64_t count, uint64_t
     }
 }
 
+// Every photon of `count` samples whose columns are in pc, and their output
+// rows (row gidx[s], or s): the first steps, the steps after them, the rows.
+static int cc_run(const cd *U, int m, int n, int64_t count, uint64_t seed, uint64_t first, const int32_t *pc,
+                  int32_t *r, char *work, const int64_t *gidx, int32_t *out, int cus, hipStream_t st)
+{
+    int k = 1;
+    if (m <= CC_FIRST_MODES) {
+        const int kmax = std::min(n, CC_FIRST);
+        const int rc = launch_first<1>(kmax, U, m, n, count, seed, first, pc, r, gidx, out, cus, st);
+        if (rc != OK || n == kmax) return rc;
+        k = kmax + 1;
+    }
+    for (; k <= n; k++) {
+        const int rc = launch_step<1>(k, U, m, n, count, seed, first, pc, r, work, cus, st, gidx);
+        if (rc != OK) return rc;
+    }
+    const int64_t tot = count * m;
+    if (gidx)
+        hipLaunchKernelGGL(cc_finish_multi_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, r, gidx, m, n,
+                           count, out);
+    else
+        hipLaunchKernelGGL(cc_finish_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, r, m, n, count, out);
+    PCVL_HIP_CHECK(hipGetLastError());
+    return OK;
+}
+
 } // namespace pcvl
 
 using namespace pcvl;
@@ -794,14 +1060,8 @@ extern "C" int pcvl_cc_samples(const double *d_U, int m, const int32_t *h_in_occ
     hipLaunchKernelGGL(cc_init_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, d_cols, n, count,
                        seed, first_sample, pc);
     PCVL_HIP_CHECK(hipGetLastError());
-    for (int k = 1; k <= n; k++) {
-        int rc = launch_step<1>(k, U, m, n, count, seed, first_sample, pc, r, slices, cus, stream);
-        if (rc != OK) return rc;
-    }
-    const int64_t tot = count * m;
-    hipLaunchKernelGGL(cc_finish_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, stream, r, m, n, count,
-                       d_out);
-    PCVL_HIP_CHECK(hipGetLastError());
+    const int rc = cc_run(U, m, n, count, seed, first_sample, pc, r, slices, nullptr, d_out, cus, stream);
+    if (rc != OK) return rc;
     // the host column list copied above must outlive the copy
     PCVL_HIP_CHECK(hipStreamSynchronize(stream));
     return OK;
@@ -829,75 +1089,81 @@ extern "C" int pcvl_cc_samples_multi(const double *d_U, int m, const int32_t *h_
     const int64_t total = row0[(size_t)ninputs];
     if (total == 0) return OK;
     PCVL_ARG_CHECK(d_U && d_out, "null device buffer");
-    // group the samples by photon number; each group runs one launch sequence
-    std::vector<int> ns;
-    for (int i = 0; i < ninputs; i++)
-        if (h_counts[i] > 0 && std::find(ns.begin(), ns.end(), (int)cols[(size_t)i].size()) == ns.end())
-            ns.push_back((int)cols[(size_t)i].size());
-    int64_t gmax = 0;
-    for (int n : ns) {
-        int64_t c = 0;
-        for (int i = 0; i < ninputs; i++) if ((int)cols[(size_t)i].size() == n) c += h_counts[i];
-        gmax = std::max(gmax, c);
+    // group the inputs by photon number; each group runs one launch sequence.
+    // The tables of all groups (first sample and output row of each input, its
+    // photon columns) go to the device in one copy.
+    struct Group { int n; int64_t count = 0; std::vector<int> inputs; size_t o_start = 0, o_row = 0, o_cols = 0; };
+    std::vector<Group> groups;
+    for (int i = 0; i < ninputs; i++) {
+        if (h_counts[i] == 0) continue;
+        const int n = (int)cols[(size_t)i].size();
+        size_t g = 0;
+        while (g < groups.size() && groups[g].n != n) g++;
+        if (g == groups.size()) { groups.emplace_back(); groups[g].n = n; }
+        groups[g].inputs.push_back(i);
+        groups[g].count += h_counts[i];
     }
-    int nmax = 1;
-    for (int n : ns) nmax = std::max(nmax, n);
-    // device block: pc | r (gmax * nmax each) | inp | gidx (gmax) | cols (ninputs * nmax) | slices
-    const size_t b_pr = sizeof(int32_t) * (size_t)gmax * nmax;
-    const size_t b_inp = sizeof(int32_t) * (size_t)gmax;
-    const size_t b_gidx = sizeof(int64_t) * (size_t)gmax;
-    const size_t b_cols = sizeof(int32_t) * (size_t)ninputs * nmax;
-    size_t b_part = 0;
-    for (int n : ns) b_part = std::max(b_part, cc_slice_work(n, gmax).total);
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
+    std::vector<char> tab;
+    int64_t gmax = 0;
+    int nmax = 1;
+    size_t b_part = 0;
+    for (Group &g : groups) {
+        const size_t ni = g.inputs.size();
+        g.o_start = al(tab.size());
+        g.o_row = g.o_start + al(sizeof(int64_t) * ni);
+        g.o_cols = g.o_row + al(sizeof(int64_t) * ni);
+        tab.resize(g.o_cols + al(sizeof(int32_t) * ni * (size_t)std::max(g.n, 1)), 0);
+        int64_t at = 0;
+        for (size_t q = 0; q < ni; q++) {
+            const int i = g.inputs[q];
+            reinterpret_cast<int64_t *>(tab.data() + g.o_start)[q] = at;
+            reinterpret_cast<int64_t *>(tab.data() + g.o_row)[q] = row0[(size_t)i];
+            for (int l = 0; l < g.n; l++)
+                reinterpret_cast<int32_t *>(tab.data() + g.o_cols)[q * (size_t)g.n + l] = cols[(size_t)i][(size_t)l];
+            at += h_counts[i];
+        }
+        gmax = std::max(gmax, g.count);
+        nmax = std::max(nmax, g.n);
+    }
+    for (const Group &g : groups) b_part = std::max(b_part, cc_slice_work(g.n, gmax).total);
+    // device block: pc | r (gmax * nmax each) | gidx (gmax) | tables | slices
+    const size_t b_pr = al(sizeof(int32_t) * (size_t)gmax * nmax);
+    const size_t b_gidx = al(sizeof(int64_t) * (size_t)gmax);
     char *blk = nullptr;
-    PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk),
-                                  2 * al(b_pr) + al(b_inp) + al(b_gidx) + al(b_cols) + al(b_part), stream));
+    PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk), 2 * b_pr + b_gidx + al(tab.size()) + al(b_part), stream));
     int32_t *pc = reinterpret_cast<int32_t *>(blk);
-    int32_t *r = reinterpret_cast<int32_t *>(blk + al(b_pr));
-    int32_t *d_inp = reinterpret_cast<int32_t *>(blk + 2 * al(b_pr));
-    int64_t *d_gidx = reinterpret_cast<int64_t *>(blk + 2 * al(b_pr) + al(b_inp));
-    int32_t *d_cols = reinterpret_cast<int32_t *>(blk + 2 * al(b_pr) + al(b_inp) + al(b_gidx));
-    char *slices = blk + 2 * al(b_pr) + al(b_inp) + al(b_gidx) + al(b_cols);
+    int32_t *r = reinterpret_cast<int32_t *>(blk + b_pr);
+    int64_t *d_gidx = reinterpret_cast<int64_t *>(blk + 2 * b_pr);
+    char *d_tab = blk + 2 * b_pr + b_gidx;
+    char *slices = d_tab + al(tab.size());
     const cd *U = reinterpret_cast<const cd *>(d_U);
     int dev = 0, cus = 0;
     int rc = OK;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) { set_error(std::string("device query: ") + hipGetErrorString(e)); rc = ERR_HIP; }
-    for (int n : ns) {
+    if (e == hipSuccess) e = hipMemcpyAsync(d_tab, tab.data(), tab.size(), hipMemcpyHostToDevice, stream);
+    if (e != hipSuccess) { set_error(std::string("cc multi tables: ") + hipGetErrorString(e)); rc = ERR_HIP; }
+    for (const Group &g : groups) {
         if (rc != OK) break;
-        std::vector<int32_t> inp, ctab((size_t)ninputs * nmax, 0);
-        std::vector<int64_t> gidx;
-        for (int i = 0; i < ninputs; i++) {
-            if ((int)cols[(size_t)i].size() != n) continue;
-            for (int l = 0; l < n; l++) ctab[(size_t)i * n + l] = cols[(size_t)i][(size_t)l];
-            for (int64_t s = 0; s < h_counts[i]; s++) { inp.push_back(i); gidx.push_back(row0[(size_t)i] + s); }
-        }
-        const int64_t count = (int64_t)gidx.size();
-        if (count == 0) continue;
-        e = hipMemcpyAsync(d_inp, inp.data(), sizeof(int32_t) * inp.size(), hipMemcpyHostToDevice, stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(d_gidx, gidx.data(), sizeof(int64_t) * gidx.size(), hipMemcpyHostToDevice, stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(d_cols, ctab.data(), sizeof(int32_t) * ctab.size(), hipMemcpyHostToDevice, stream);
-        if (e != hipSuccess) { set_error(std::string("hipMemcpyAsync(cc multi): ") + hipGetErrorString(e)); rc = ERR_HIP; break; }
-        if (n > 0) {
-            hipLaunchKernelGGL(cc_init_multi_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, d_cols,
-                               d_inp, d_gidx, n, count, seed, first_sample, pc);
-            e = hipGetLastError();
-            if (e != hipSuccess) { set_error(std::string("cc_init_multi: ") + hipGetErrorString(e)); rc = ERR_HIP; break; }
-            for (int k = 1; k <= n && rc == OK; k++)
-                rc = launch_step<1>(k, U, m, n, count, seed, first_sample, pc, r, slices, cus, stream, d_gidx);
-            if (rc != OK) break;
-        }
-        const int64_t tot = count * m;
-        hipLaunchKernelGGL(cc_finish_multi_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, stream, r, d_gidx,
-                           m, n, count, d_out);
+        const unsigned blocks = (unsigned)((g.count + 255) / 256);
+        hipLaunchKernelGGL(cc_init_multi_kernel, dim3(blocks), dim3(256), 0, stream,
+                           reinterpret_cast<const int32_t *>(d_tab + g.o_cols),
+                           reinterpret_cast<const int64_t *>(d_tab + g.o_start),
+                           reinterpret_cast<const int64_t *>(d_tab + g.o_row), (int)g.inputs.size(), g.n, g.count, seed,
+                           first_sample, d_gidx, pc);
         e = hipGetLastError();
-        if (e != hipSuccess) { set_error(std::string("cc_finish_multi: ") + hipGetErrorString(e)); rc = ERR_HIP; break; }
-        // the host tables of this group must outlive their copies
-        e = hipStreamSynchronize(stream);
-        if (e != hipSuccess) { set_error(std::string("cc multi: ") + hipGetErrorString(e)); rc = ERR_HIP; break; }
+        if (e != hipSuccess) { set_error(std::string("cc_init_multi: ") + hipGetErrorString(e)); rc = ERR_HIP; break; }
+        if (g.n > 0) {
+            rc = cc_run(U, m, g.n, g.count, seed, first_sample, pc, r, slices, d_gidx, d_out, cus, stream);
+        } else {
+            hipLaunchKernelGGL(cc_finish_multi_kernel, dim3((unsigned)((g.count * m + 255) / 256)), dim3(256), 0,
+                               stream, r, d_gidx, m, 0, g.count, d_out);
+            e = hipGetLastError();
+            if (e != hipSuccess) { set_error(std::string("cc_finish_multi: ") + hipGetErrorString(e)); rc = ERR_HIP; }
+        }
     }
+    // the host tables must outlive their copy, and results are ready on return
     hipError_t se = hipStreamSynchronize(stream);
     hipError_t fe = hipFreeAsync(blk, stream);
     if (rc == OK && se != hipSuccess) { set_error(std::string("cc multi: ") + hipGetErrorString(se)); rc = ERR_HIP; }

@@ -46,6 +46,22 @@ def test_same_seed_same_samples_repeated_rows(gpu, m, n, count):
     assert np.array_equal(g, c), np.nonzero(np.any(g != c, axis=1))[0][:10]
 
 
+@pytest.mark.parametrize("m", [1, 5, 15, 16, 17, 32, 33, 64, 65])
+def test_same_seed_same_samples_first_steps(gpu, m):
+    """Steps 1..9 run in one launch up to 64 modes, 16 lanes a sample: photon
+    numbers 1..10, modes around multiples of 16 and both sides of 32 and 64,
+    repeated rows, and a count that is no multiple of the samples per block."""
+    from perceval_amd.sampling import cc_samples, cc_samples_multi_device
+    U = haar_unitary(m, seed=7 * m)
+    inputs = [[n // m + (1 if i < n % m else 0) for i in range(m)] for n in range(1, 11)]
+    multi = cc_samples_multi_device(U, inputs, [37] * 10, seed=21, first_sample=5).cpu().numpy()
+    for n, inp in enumerate(inputs, 1):
+        g = cc_samples(U, inp, 37, seed=21, first_sample=5 + 37 * (n - 1))
+        c = oracle.cc_samples(U, inp, 37, seed=21, first_sample=5 + 37 * (n - 1))
+        assert np.array_equal(g, c), (n, np.nonzero(np.any(g != c, axis=1))[0][:10])
+        assert np.array_equal(multi[37 * (n - 1):37 * n], c), n
+
+
 def test_same_seed_same_samples_m60_n20(gpu):
     from perceval_amd.sampling import cc_samples
     U = haar_unitary(60, seed=60)
