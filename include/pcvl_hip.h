@@ -354,6 +354,24 @@ int pcvl_mlp_adam(float *d_w, const float *d_g, float *d_m1, float *d_m2, uint16
                   int64_t count, float lr, float beta1, float beta2, float eps, int step,
                   hipStream_t stream);
 
+/* The same step on up to four tensors at once (tables of device pointers on
+ * the host; d_wbf16[k] may be NULL). */
+int pcvl_mlp_adam_multi(int tensors, float *const *d_w, const float *const *d_g, float *const *d_m1,
+                        float *const *d_m2, uint16_t *const *d_wbf16, const int64_t *counts, float lr,
+                        float beta1, float beta2, float eps, int step, hipStream_t stream);
+
+/* Loss per row and gradients of scale * sum(loss) of the proposal network of n
+ * photons over m modes with H hidden units, for R rows x (R x (m + n)) with
+ * targets and mask bounds, in one pass (deterministic).  Networks up to 64
+ * modes, 96 inputs (m + n) and 256 hidden units; the workspace call returns 0
+ * floats for larger ones, which the products above compute.  d_work is aligned
+ * to 16 bytes. */
+int pcvl_mis_grads_workspace(int R, int m, int n, int H, int64_t *floats);
+int pcvl_mis_grads(const float *d_x, int R, int m, int n, int H, const uint16_t *d_W1, const float *d_b1,
+                   const uint16_t *d_W2, const float *d_b2, const int32_t *d_target, const int32_t *d_lo,
+                   float scale, float *d_loss, float *d_dW1, float *d_db1, float *d_dW2, float *d_db2,
+                   float *d_work, int64_t work_floats, hipStream_t stream);
+
 /* bf16 (round to nearest even) copy of fp32 weights. */
 int pcvl_mlp_to_bf16(const float *d_w, uint16_t *d_wbf16, int64_t count, hipStream_t stream);
 

@@ -77,6 +77,12 @@ SIGNATURES = {
                             c_void_p]),
     "pcvl_mlp_adam": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_i64, ctypes.c_float,
                               ctypes.c_float, ctypes.c_float, ctypes.c_float, c_int, c_void_p]),
+    "pcvl_mlp_adam_multi": (c_int, [c_int, P(c_void_p), P(c_void_p), P(c_void_p), P(c_void_p), P(c_void_p), P(c_i64),
+                                    ctypes.c_float, ctypes.c_float, ctypes.c_float, ctypes.c_float, c_int, c_void_p]),
+    "pcvl_mis_grads_workspace": (c_int, [c_int, c_int, c_int, c_int, P(c_i64)]),
+    "pcvl_mis_grads": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                               c_void_p, ctypes.c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                               c_i64, c_void_p]),
     "pcvl_mlp_to_bf16": (c_int, [c_void_p, c_void_p, c_i64, c_void_p]),
     "pcvl_mis_features": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "pcvl_mis_features_all": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),

@@ -79,6 +79,16 @@ class ProposalNet:
         import torch
         lib = _lib()
         R = x.shape[0]
+        need = ctypes.c_int64()
+        _native.check(lib.pcvl_mis_grads_workspace(R, self.m, self.n, self.H, ctypes.byref(need)), "grads_workspace")
+        if need.value:   # the whole pass in one launch
+            loss = torch.empty(R, dtype=torch.float32, device=x.device)
+            grads = [torch.empty_like(p) for p in self.params]
+            work = self._workspace(need.value, x.device)
+            _native.check(lib.pcvl_mis_grads(_p(x), R, self.m, self.n, self.H, _p(self.W1b), _p(self.b1),
+                                             _p(self.W2b), _p(self.b2), _p(target), _p(lo), float(scale), _p(loss),
+                                             *(_p(g) for g in grads), _p(work), work.numel(), _s()), "grads")
+            return loss, grads
         h, z = self.forward(x)
         loss = torch.empty(R, dtype=torch.float32, device=x.device)
         dz = torch.empty_like(z)
@@ -108,18 +118,26 @@ class ProposalNet:
             f = ctypes.c_int64()
             _native.check(lib.pcvl_mlp_wgrad_workspace(R, mo, no, ctypes.byref(f)), "wgrad_workspace")
             need = max(need, f.value)
+        return self._workspace(need, device)
+
+    def _workspace(self, need: int, device):
+        import torch
         if getattr(self, "_wwork", None) is None or self._wwork.numel() < need or self._wwork.device != device:
             self._wwork = torch.empty(max(1, need), dtype=torch.float32, device=device)
         return self._wwork
 
     def adam_step(self, grads, lr: float = 1e-3, beta1: float = 0.9, beta2: float = 0.999, eps: float = 1e-8):
-        lib = _lib()
         self._step += 1
-        bf = {0: self.W1b, 2: self.W2b}
-        for k, (p, g) in enumerate(zip(self.params, grads)):
-            _native.check(lib.pcvl_mlp_adam(_p(p), _p(g), _p(self._m1[k]), _p(self._m2[k]),
-                                            _p(bf[k]) if k in bf else None, p.numel(), lr, beta1, beta2, eps,
-                                            self._step, _s()), "adam")
+        pairs = list(zip(self.params, grads))
+        n = len(pairs)
+
+        def table(tensors):
+            return (ctypes.c_void_p * n)(*(None if t is None else _p(t) for t in tensors))
+        counts = (ctypes.c_int64 * n)(*(p.numel() for p, _ in pairs))
+        _native.check(_lib().pcvl_mlp_adam_multi(n, table(p for p, _ in pairs), table(g for _, g in pairs),
+                                                 table(self._m1[:n]), table(self._m2[:n]),
+                                                 table((self.W1b, None, self.W2b, None)[:n]), counts, lr, beta1,
+                                                 beta2, eps, self._step, _s()), "adam")
 
     # ------------------------------------------------------------------ data
     def teacher_forcing(self, seqs):

@@ -50,6 +50,48 @@ def test_network_gradients_vs_oracle(gpu):
         assert np.max(np.abs(gg - rg)) <= 1e-5 * max(1.0, np.max(np.abs(rg))), np.max(np.abs(gg - rg))
 
 
+@pytest.mark.parametrize("m,n,H,B", [(1, 1, 1, 1), (3, 2, 40, 17), (17, 15, 33, 70), (33, 16, 64, 3),
+                                     (60, 20, 256, 700), (64, 32, 256, 300), (64, 33, 256, 20), (65, 3, 16, 50),
+                                     (10, 4, 257, 50)])
+def test_training_step_shapes_vs_oracle(gpu, m, n, H, B):
+    """Loss, gradients and the Adam step on both sides of the one-launch pass
+    (64 modes, 96 inputs, 256 hidden units): one row to several tiles of 32 per
+    workgroup, widths around multiples of 16, rows without an allowed target.
+    The bars are those of the gradient and Adam tests above and below."""
+    import torch
+    from perceval_amd.mis import ProposalNet
+    rng = np.random.RandomState(m + n)
+    seqs = np.sort(rng.randint(0, m, size=(B, n)), axis=1).astype(np.int32)
+    net = ProposalNet(m, n, hidden=H, seed=3)
+    for p, sd in zip(net.params, (0.3, 0.1, 0.3, 0.1)):
+        p.copy_(torch.from_numpy((sd * rng.randn(*p.shape)).astype(np.float32)).cuda())
+    net.refresh_bf16()
+    x, lo, tgt = net.teacher_forcing(torch.from_numpy(seqs).cuda())
+    X, LO, TG = mlp_oracle.features(seqs, m)
+    assert np.array_equal(x.cpu().numpy(), X) and np.array_equal(lo.cpu().numpy(), LO)
+    assert np.array_equal(tgt.cpu().numpy(), TG)
+    bad = np.arange(0, B * n, 7) if B * n > 7 else np.arange(0)
+    tgt[torch.from_numpy(bad).cuda()] = torch.from_numpy(np.where(bad % 2, m, -1).astype(np.int32)).cuda()
+    w0 = [p.double().cpu().numpy() for p in net.params]
+    loss, grads = net.loss_and_grads(x, lo, tgt, 1.0 / B)
+    loss2, grads2 = net.loss_and_grads(x, lo, tgt, 1.0 / B)
+    assert torch.equal(loss, loss2) and all(torch.equal(a, b) for a, b in zip(grads, grads2))
+    keep = np.setdiff1d(np.arange(B * n), bad)
+    ref_loss, ref_grads = mlp_oracle.loss_and_grads(*w0, X[keep], LO[keep], TG[keep], 1.0 / B)
+    got = loss.cpu().numpy()
+    assert np.isposinf(got[bad]).all()
+    assert np.allclose(got[keep], ref_loss, rtol=1e-5, atol=1e-5)
+    for gg, rg in zip(grads, ref_grads):
+        gg = gg.double().cpu().numpy()
+        assert np.max(np.abs(gg - rg)) <= 1e-5 * max(1.0, np.max(np.abs(rg))), np.max(np.abs(gg - rg))
+    net.adam_step(grads, lr=1e-2)
+    for p, w, gg in zip(net.params, w0, grads):
+        ref, _, _ = mlp_oracle.adam(w, gg.double().cpu().numpy(), np.zeros(w.shape), np.zeros(w.shape), 1e-2, 0.9,
+                                    0.999, 1e-8, 1)
+        assert np.allclose(p.cpu().numpy(), ref, rtol=1e-5, atol=1e-6)
+    assert torch.equal(net.W1b, net.W1.bfloat16()) and torch.equal(net.W2b, net.W2.bfloat16())
+
+
 def test_adam_step_vs_oracle(gpu):
     import torch
     from perceval_amd import _native
