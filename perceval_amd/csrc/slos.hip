@@ -978,21 +978,25 @@ extern "C" int pcvl_slos_plan_execute(pcvl_slos_plan plan, const double *d_U, in
         set_error("SLOS kernel not applicable to this plan's layer sizes");
         return ERR_ARG;
     }
-    // Layer 0 is the vacuum coefficient 1; layer 1 reads it from bufA[0].
-    hipLaunchKernelGGL(slos_vacuum_kernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<double *>(bufA), 2);
-    PCVL_HIP_CHECK(hipGetLastError());
+    const int front = kernel == 8 ? p.blk.front : 0;   // layers of the first launch
+    if (front == 0) {
+        // Layer 0 is the vacuum coefficient 1; layer 1 reads it from bufA[0].
+        hipLaunchKernelGGL(slos_vacuum_kernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<double *>(bufA), 2);
+        PCVL_HIP_CHECK(hipGetLastError());
+    }
     const cd *prev = bufA;
     // masks with several final sub-layers: the last layer goes to the end of
     // the workspace in sub-layer order, then to d_out in FSArray order
     void *last_dst = p.d_perm ? static_cast<void *>(bufA + slos_work_main(p)) : static_cast<void *>(d_out);
-    for (int k = 1; k <= p.n; k++) {
+    for (int k = std::max(front, 1); k <= p.n; k++) {
         const uint64_t nc = p.counts[k];
         const bool last = (k == p.n);
         void *dst = last ? last_dst : static_cast<void *>(prev == bufA ? bufB : bufA);
         const bool probs = last && mode == PCVL_SLOS_PROBS;
         if (kernel == 8) {
-            const int rc = blk_layer_launch(p.blk, prev, dst, U, p.m, p.mk[k - 1], k, probs, p.inv_prod_in, !last,
-                                            stream);
+            const int rc = k == front ? blk_front_launch(p.blk, dst, U, p.m, p.mk, probs, p.inv_prod_in, !last, stream)
+                                      : blk_layer_launch(p.blk, prev, dst, U, p.m, p.mk[k - 1], k, probs, p.inv_prod_in,
+                                                         !last, stream);
             if (rc != OK) return rc;
         } else if (kernel == 6) {
             const uint64_t tile = 3ull * SLOS7_THREADS;

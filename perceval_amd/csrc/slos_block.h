@@ -91,6 +91,14 @@ struct BlkLayout {
     std::vector<size_t> group_off;               // byte offset of layer k's groups in d_mem
     size_t off_th = 0, off_te = 0, off_cte = 0, off_f32 = 0, off_fd = 0, off_pf = 0, off_slot = 0, off_row = 0,
            off_her = 0, off_rec = 0;
+    // First layers in one launch (blk_front_launch): layers 1..front (0: none)
+    int front = 0;
+    std::vector<int> front_slots;                // parents of a child of layer k, at most
+    std::vector<uint32_t> front_off;             // first word of layer k's parent words, from off_front
+    uint32_t front_staged = 0;                   // words that the workgroups copy into LDS (leading layers)
+    int front_staged_layers = 0;
+    uint32_t front_cap[2] = {0, 0};              // LDS entries for the layers k % 2 == 0, 1 below the last one
+    size_t off_front = 0, off_front_pf = 0;      // parent words; factorial products of layer `front` if it is the last
     int cmax = 1;             // most occupied prefix modes of a block: min(h, nmax)
     uint64_t nrec = 0;        // block records
     char *d_mem = nullptr;
@@ -158,6 +166,12 @@ bool blk_layout_ok(int m, int nmax);
 // inv_prod_in).  sentinel: write one zero coefficient after the last child
 // (read by the successor kernels of the next layer).
 int blk_layer_launch(const BlkLayout &lay, const cd *parent, void *out, const cd *U, int m, int mk, int k, bool probs,
+                     double inv_prod_in, bool sentinel, hipStream_t stream);
+
+// Layers 1..lay.front from the vacuum in one launch, mk[k - 1] the input mode
+// of layer k; layer lay.front goes to out (probabilities where it is the last
+// layer and probs is set).
+int blk_front_launch(const BlkLayout &lay, void *out, const cd *U, int m, const std::vector<int32_t> &mk, bool probs,
                      double inv_prod_in, bool sentinel, hipStream_t stream);
 
 // One node of an input tree at layer k: parent layer at byte par_off of the

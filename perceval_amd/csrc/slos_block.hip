@@ -460,6 +460,98 @@ __global__ void __launch_bounds__(BLK_THREADS) slos_block_batch_kernel(
                       mloc, nullptr, groups, ngroups, her, tabs, to, wt, spf, sslot, recs, op.inv_prod_in, 0);
 }
 
+// ---- the first layers in one launch ---------------------------------------------
+//
+// A layer of a few thousand children is a launch, a table fetch and a gather,
+// one after the other, 4.7 us whatever its size.  Here every workgroup computes
+// layers 1..front - 1 for itself, in LDS, and then its share of layer `front`:
+// the parents of these few children come from a table of (rank << 8) | mode
+// words, slot d of child c at word d * count + c, in the order of summation of
+// the layer kernels (herald, prefix, suffix modes, each increasing), so the
+// amplitudes are the same bits.  Bound by the latency of a layer (table words,
+// LDS gather, barrier: about 1 us at 1,000 states), the launch itself 10 us
+// from the caller.  12 modes, 6 photons (12,376 outputs): 33 -> 12.4 us, seven
+// launches -> one; 24 modes, 6 photons 53 -> 29 us; 2 modes, 30 photons 326 ->
+// 16 us.  Repeating a layer against a launch for it: with layers to 4,608
+// states 16 photons in 5 modes take 29 us, to 2,304 48 us, 13 photons in 6
+// modes 34 and 41 us; larger ones outgrow the LDS (8,192: the same times).
+constexpr int FRONT_THREADS = 1024;
+constexpr uint32_t FRONT_STATES = 4608;     // largest layer that every workgroup computes
+constexpr uint32_t FRONT_LAST = 32768;      // largest layer that they share (its words: 4 per parent)
+constexpr uint32_t FRONT_STAGED = 8192;     // parent words copied into LDS, all layers fetched together
+constexpr size_t FRONT_LDS = 150 * 1024;
+constexpr int FRONT_MAX = 30;
+
+struct FrontLayers {
+    uint32_t count[FRONT_MAX + 1], off[FRONT_MAX + 1];
+    int32_t slots[FRONT_MAX + 1], mk[FRONT_MAX + 1];
+};
+
+// Sum over the parents of child c of a layer of `count`.
+__device__ __forceinline__ cd front_child(const uint32_t *words, uint32_t count, uint32_t c, int slots,
+                                          const cd *parent, const cd *su)
+{
+    cd acc = {0.0, 0.0};
+    for (int d0 = 0; d0 < slots; d0 += 4) {
+        uint32_t w[4];
+        cd pv[4], uv[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) w[t] = d0 + t < slots ? words[(size_t)(d0 + t) * count + c] : 0xffffffffu;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            pv[t] = cd{0.0, 0.0};
+            uv[t] = cd{0.0, 0.0};
+            if (w[t] != 0xffffffffu) {
+                pv[t] = parent[w[t] >> 8];
+                uv[t] = su[w[t] & 255u];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) cfma_acc(acc, pv[t], uv[t]);   // zero past the list: adds an exact 0
+    }
+    return acc;
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(FRONT_THREADS) slos_front_kernel(
+    const cd *__restrict__ U, int m, int mloc, const int32_t *__restrict__ rowmap, const uint32_t *__restrict__ words,
+    const double *__restrict__ pf, FrontLayers f, int front, int staged_layers, uint32_t staged, uint32_t cap0,
+    uint32_t cap1, uint32_t share, void *__restrict__ out, double inv_prod_in, int sentinel)
+{
+    extern __shared__ cd s_front[];
+    cd *even = s_front, *odd = even + cap0, *su = odd + cap1;            // layers by parity; U column of each layer
+    uint32_t *sw = reinterpret_cast<uint32_t *>(su + (size_t)front * mloc);
+    const int tid = threadIdx.x;
+    for (uint32_t e = tid; e < staged; e += FRONT_THREADS) sw[e] = words[e];
+    for (int e = tid; e < front * mloc; e += FRONT_THREADS) {
+        const int k = e / mloc, i = e - k * mloc;
+        su[e] = U[(size_t)(rowmap ? rowmap[i] : i) * m + f.mk[k + 1]];
+    }
+    if (tid == 0) even[0] = cd{1.0, 0.0};
+    if (sentinel && blockIdx.x == 0 && tid == 0) reinterpret_cast<cd *>(out)[f.count[front]] = cd{0.0, 0.0};
+    __syncthreads();
+    for (int k = 1; k < front; k++) {
+        const uint32_t count = f.count[k];
+        const cd *parent = (k & 1) ? even : odd;
+        cd *child = (k & 1) ? odd : even;
+        const cd *u = su + (k - 1) * mloc;
+        if (k <= staged_layers) {
+            for (uint32_t c = tid; c < count; c += FRONT_THREADS)
+                child[c] = front_child(sw + f.off[k], count, c, f.slots[k], parent, u);
+        } else {
+            for (uint32_t c = tid; c < count; c += FRONT_THREADS)
+                child[c] = front_child(words + f.off[k], count, c, f.slots[k], parent, u);
+        }
+        __syncthreads();
+    }
+    const uint32_t count = f.count[front], lo = blockIdx.x * share, hi = min(lo + share, count);
+    for (uint32_t c = lo + tid; c < hi; c += FRONT_THREADS) {
+        const cd acc = front_child(words + f.off[front], count, c, f.slots[front], (front & 1) ? even : odd,
+                                   su + (front - 1) * mloc);
+        blk_emit<MODE>(BlkDest{out, nullptr, MODE == 1}, c, acc, MODE == 1 ? pf[c] : 0.0, inv_prod_in);
+    }
+}
+
 // ------------------------------------------------------------------ host
 
 bool blk_layout_ok(int m, int nmax)
@@ -501,6 +593,39 @@ static uint64_t local_rank(const std::vector<int> &beta)
 }
 
 static size_t blk_lds_bytes(const BlkLayout &lay, int k);
+
+// LDS of the launch of layers 1..front.
+static size_t front_lds(const BlkLayout &lay, int front, uint32_t staged)
+{
+    return sizeof(cd) * ((size_t)lay.front_cap[0] + lay.front_cap[1] + (size_t)front * lay.mloc) +
+           sizeof(uint32_t) * staged;
+}
+
+// As many first layers as keep the repeated ones within FRONT_STATES, the
+// shared one within FRONT_LAST and the LDS; one layer alone gains nothing but
+// the vacuum's launch, which still counts.  Words hold modes below 256 (the
+// most a plan takes) and ranks below 2^24.
+static void front_choose(BlkLayout *lay)
+{
+    lay->front_slots.assign((size_t)lay->nlayers + 1, 0);
+    lay->front_off.assign((size_t)lay->nlayers + 1, 0);
+    uint32_t cap[2] = {1, 0};
+    for (int k = 1; k <= std::min(lay->nlayers, FRONT_MAX); k++) {
+        if (lay->counts[(size_t)k] > FRONT_LAST) break;
+        const uint32_t keep[2] = {lay->front_cap[0], lay->front_cap[1]};
+        lay->front_cap[0] = cap[0];
+        lay->front_cap[1] = cap[1];
+        if (front_lds(*lay, k, FRONT_STAGED) > FRONT_LDS) {
+            lay->front_cap[0] = keep[0];
+            lay->front_cap[1] = keep[1];
+            break;
+        }
+        lay->front = k;
+        lay->front_slots[(size_t)k] = std::min(k, lay->mloc);
+        if (lay->counts[(size_t)k] > FRONT_STATES) break;
+        cap[k & 1] = std::max(cap[k & 1], (uint32_t)lay->counts[(size_t)k]);
+    }
+}
 
 int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vector<BlkSub>> &subs,
                              const std::vector<uint64_t> &counts, const std::vector<int32_t> &rowmap,
@@ -592,33 +717,28 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     // of whole-wave groups get their walk precomputed (records)
     lay.cmax = std::max(1, std::min(h, nmax));
     std::vector<BlkRec> recs;
-    auto add_records = [&](int K, int r) {
+    // every block (K, r) in order: f(B_k, PE_h, (mode, PE_j) of its occupied prefix modes, prod alpha!)
+    auto for_blocks = [&](int K, int r, auto &&f) {
         std::vector<int> alpha((size_t)h, 0);
         alpha[0] = K;
         const uint64_t nb = nstates(h, K);
         std::vector<int> after((size_t)h + 1, 0);
+        std::vector<std::pair<uint32_t, uint32_t>> occ;
         for (uint64_t i = 0; i < nb; i++) {
-            BlkRec rec{};
             uint64_t Bk = 0, PE = 0;
             double pf = 1.0;
             for (int q = h - 1; q >= 0; q--) after[(size_t)q] = after[(size_t)q + 1] + alpha[(size_t)q];
-            int cnt = 0;
+            occ.clear();
             for (int q = 0; q < h; q++) {
                 const uint64_t tev = te[(size_t)q * wt + r + after[(size_t)q + 1]];
                 Bk += tev & 0xffffffffull;
                 if (alpha[(size_t)q] > 0) {
-                    rec.w[4 + cnt / 4] |= (uint32_t)q << (8 * (cnt % 4));
-                    rec.w[10 + cnt] = (uint32_t)PE;
-                    cnt++;
+                    occ.push_back({(uint32_t)q, (uint32_t)PE});
                     for (int v = 2; v <= alpha[(size_t)q]; v++) pf *= v;
                 }
                 PE += tev >> 32;
             }
-            rec.w[0] = (uint32_t)Bk;
-            rec.w[1] = (uint32_t)PE;
-            rec.w[2] = (uint32_t)cnt;
-            std::memcpy(&rec.w[8], &pf, sizeof(double));
-            recs.push_back(rec);
+            f((uint32_t)Bk, (uint32_t)PE, occ, pf);
             if (i + 1 < nb) {   // next alpha in descending lexicographic order
                 const int tail = alpha[(size_t)h - 1];
                 alpha[(size_t)h - 1] = 0;
@@ -628,6 +748,21 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
                 alpha[(size_t)t + 1] = tail + 1;
             }
         }
+    };
+    using BlkOcc = std::vector<std::pair<uint32_t, uint32_t>>;
+    auto add_records = [&](int K, int r) {
+        for_blocks(K, r, [&](uint32_t Bk, uint32_t PEh, const BlkOcc &occ, double pf) {
+            BlkRec rec{};
+            rec.w[0] = Bk;
+            rec.w[1] = PEh;
+            rec.w[2] = (uint32_t)occ.size();
+            for (size_t c = 0; c < occ.size(); c++) {
+                rec.w[4 + c / 4] |= occ[c].first << (8 * (c % 4));
+                rec.w[10 + c] = occ[c].second;
+            }
+            std::memcpy(&rec.w[8], &pf, sizeof(double));
+            recs.push_back(rec);
+        });
     };
     // records hold at most 16 occupied prefix modes and mode indices below 256
     const bool use_records = lay.cmax <= BLK_REC_MAX && h <= 256;
@@ -690,6 +825,41 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
         }
         lay.items[(size_t)k] = items;
     }
+    // the first layers in one launch: how many, and their parent words
+    std::vector<uint32_t> fwords;
+    std::vector<double> fpf;
+    front_choose(&lay);
+    for (int k = 1; k <= lay.front; k++) {
+        const uint32_t cnt = (uint32_t)lay.counts[(size_t)k];
+        const bool last = k == lay.nlayers;
+        const size_t off0 = fwords.size();
+        lay.front_off[(size_t)k] = (uint32_t)off0;
+        fwords.resize(off0 + (size_t)lay.front_slots[(size_t)k] * cnt, 0xffffffffu);
+        if (last) fpf.assign(cnt, 1.0);
+        for (const BlkSub &sub : subs[(size_t)k])
+            for (int r = 0; r <= sub.kf; r++) {
+                const uint32_t S = (uint32_t)nstates(w, r);
+                const int ns = std::min(r, w);
+                for_blocks(sub.kf - r, r, [&](uint32_t Bk, uint32_t PEh, const BlkOcc &occ, double pf) {
+                    for (uint32_t b = 0; b < S; b++) {
+                        const uint32_t loc = Bk + b, c = sub.out_base + loc;
+                        size_t at = off0 + c;
+                        auto put = [&](uint32_t rank, uint32_t mode) { fwords[at] = (rank << 8) | mode; at += cnt; };
+                        for (const auto &e : sub.her) put(e.second + loc, (uint32_t)m + e.first);
+                        for (const auto &e : occ) put(sub.par_base + loc - e.second, e.first);
+                        for (int d = 0; d < ns; d++) {
+                            const uint32_t word = sslot[(size_t)tslot[(size_t)r] + (size_t)d * S + b];
+                            if (word != 0xffffffffu) put(sub.par_base + Bk - PEh + (word >> 5), (uint32_t)h + (word & 31u));
+                        }
+                        if (last) fpf[c] = pf * spf[(size_t)tpf[(size_t)r] + b] * sub.hfact;
+                    }
+                });
+            }
+        if (k < lay.front && k == lay.front_staged_layers + 1 && fwords.size() <= FRONT_STAGED) {
+            lay.front_staged_layers = k;
+            lay.front_staged = (uint32_t)fwords.size();
+        }
+    }
     // one device allocation
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     size_t off = 0;
@@ -709,6 +879,8 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     lay.off_slot = off; off += al(sizeof(uint32_t) * std::max<size_t>(sslot.size(), 1));
     lay.nrec = recs.size();
     lay.off_rec = off; off += al(sizeof(BlkRec) * std::max<size_t>(recs.size(), 1));
+    lay.off_front = off; off += al(sizeof(uint32_t) * std::max<size_t>(fwords.size(), 1));
+    lay.off_front_pf = off; off += al(sizeof(double) * std::max<size_t>(fpf.size(), 1));
     lay.bytes = off;
     if (blk_lds_bytes(lay, lay.nlayers) > 160 * 1024) {
         set_error("block SLOS layout: the walk tables and lists outgrow the LDS (too many modes and photons)");
@@ -729,6 +901,8 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     std::memcpy(host.data() + lay.off_pf, spf.data(), sizeof(double) * spf.size());
     if (!sslot.empty()) std::memcpy(host.data() + lay.off_slot, sslot.data(), sizeof(uint32_t) * sslot.size());
     if (!recs.empty()) std::memcpy(host.data() + lay.off_rec, recs.data(), sizeof(BlkRec) * recs.size());
+    if (!fwords.empty()) std::memcpy(host.data() + lay.off_front, fwords.data(), sizeof(uint32_t) * fwords.size());
+    if (!fpf.empty()) std::memcpy(host.data() + lay.off_front_pf, fpf.data(), sizeof(double) * fpf.size());
     *out = std::move(lay);
     return OK;
 }
@@ -1065,6 +1239,39 @@ int blk_layer_launch(const BlkLayout &lay, const cd *parent, void *out, const cd
                        reinterpret_cast<const double *>(base + lay.off_pf),
                        reinterpret_cast<const uint32_t *>(base + lay.off_slot),
                        reinterpret_cast<const BlkRec *>(base + lay.off_rec), inv_prod_in, sentinel ? 1 : 0);
+    PCVL_HIP_CHECK(hipGetLastError());
+    return OK;
+}
+
+int blk_front_launch(const BlkLayout &lay, void *out, const cd *U, int m, const std::vector<int32_t> &mk, bool probs,
+                     double inv_prod_in, bool sentinel, hipStream_t stream)
+{
+    const int front = lay.front;
+    if (front < 1 || (int)mk.size() < front || !lay.d_mem || (probs && front != lay.nlayers)) {
+        set_error("block SLOS: first layers outside the layout");
+        return ERR_ARG;
+    }
+    const uint32_t count = (uint32_t)lay.counts[(size_t)front];
+    if (count == 0) return OK;
+    FrontLayers f = {};
+    for (int k = 0; k <= front; k++) {
+        f.count[k] = (uint32_t)lay.counts[(size_t)k];
+        if (k == 0) continue;
+        f.off[k] = lay.front_off[(size_t)k];
+        f.slots[k] = lay.front_slots[(size_t)k];
+        f.mk[k] = mk[(size_t)k - 1];
+    }
+    // 256 children a workgroup; at most one workgroup per CU (256)
+    const uint32_t groups = std::min<uint32_t>(256, (count + 255) / 256);
+    const uint32_t share = (count + groups - 1) / groups;
+    const char *base = lay.d_mem;
+    auto kp = probs ? slos_front_kernel<1> : slos_front_kernel<0>;
+    hipLaunchKernelGGL(kp, dim3((count + share - 1) / share), dim3(FRONT_THREADS),
+                       front_lds(lay, front, lay.front_staged), stream, U, m, lay.mloc,
+                       lay.row_identity ? nullptr : reinterpret_cast<const int32_t *>(base + lay.off_row),
+                       reinterpret_cast<const uint32_t *>(base + lay.off_front),
+                       reinterpret_cast<const double *>(base + lay.off_front_pf), f, front, lay.front_staged_layers,
+                       lay.front_staged, lay.front_cap[0], lay.front_cap[1], share, out, inv_prod_in, sentinel ? 1 : 0);
     PCVL_HIP_CHECK(hipGetLastError());
     return OK;
 }

@@ -30,6 +30,21 @@ def test_fock_rank_unrank_exact(gpu, m, n):
     assert np.array_equal(back, states)
 
 
+@pytest.mark.parametrize("m,n", [(2, 1), (2, 30), (3, 29), (4, 25), (5, 15), (5, 16), (6, 13), (12, 6), (24, 5),
+                                 (40, 4), (200, 2), (256, 2)])
+def test_slos_first_layers_bits(gpu, m, n):
+    """The first layers run in one launch, up to 4,608 states repeated by every
+    workgroup and 32,768 shared: all layers in it, one layer after it, several
+    after it.  The amplitudes are the per-state kernel's bits."""
+    from perceval_amd.slos import COEFS, PROBS, SlosPlan
+    U = haar_unitary(m, seed=m + n)
+    inp = [n // m + (1 if i < n % m else 0) for i in range(m)]
+    plan, ref = SlosPlan(inp), SlosPlan(inp)
+    ref.set_kernel(1)
+    assert np.array_equal(plan.run(U, COEFS).cpu().numpy(), ref.run(U, COEFS).cpu().numpy())
+    assert np.max(np.abs(plan.run(U, PROBS).cpu().numpy() - ref.run(U, PROBS).cpu().numpy())) <= ABS_TOL
+
+
 def test_fock_rank_unrank_m24_n10_sampled(gpu):
     from perceval_amd.slos import fock_rank, fock_unrank
     total = oracle.fock_count(24, 10)
