@@ -585,24 +585,6 @@ __global__ void __launch_bounds__(64) cc_step_kernel(const cd *__restrict__ U, i
 constexpr int CC_FIRST = CC_MULTI - 1;
 constexpr int CC_FIRST_MODES = 64;
 
-template <int CTRL>
-__device__ __forceinline__ double row_dpp(double v)
-{
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-
-// Sum over the 16 lanes of a row, every lane receiving it.
-__device__ __forceinline__ double row_sum(double v)
-{
-    v += row_dpp<0xB1>(v);    // quad_perm [1, 0, 3, 2]
-    v += row_dpp<0x4E>(v);    // quad_perm [2, 3, 0, 1]
-    v += row_dpp<0x141>(v);   // row_half_mirror
-    v += row_dpp<0x140>(v);   // row_mirror
-    return v;
-}
-
 // Inclusive sums over the 16 lanes of a row (row_shr 1, 2, 4, 8; zeros enter).
 __device__ __forceinline__ double row_scan(double v)
 {

@@ -72,6 +72,25 @@ __device__ __forceinline__ void cfma_acc(cd &acc, cd a, cd b)
     acc.i = fma(a.i, b.r, acc.i);
 }
 
+// A DPP move of a double within rows of 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ double row_dpp(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
+// Sum over the 16 lanes of a row, every lane receiving it.
+__device__ __forceinline__ double row_sum(double v)
+{
+    v += row_dpp<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+    v += row_dpp<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+    v += row_dpp<0x141>(v);   // row_half_mirror
+    v += row_dpp<0x140>(v);   // row_mirror
+    return v;
+}
+
 // acc -= a * b.
 __device__ __forceinline__ void cfms_acc(cd &acc, cd a, cd b)
 {

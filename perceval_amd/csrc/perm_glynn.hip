@@ -17,8 +17,8 @@
 // each chunk start, which bounds their drift to 2^(c-2) or 2^(c-1) updates.
 // One persistent launch drains a cost-sorted queue of wave items of mixed
 // order (largest first), then a second kernel sums each matrix's wave partials
-// in a fixed order (bit-reproducible).  Orders 0..8 take one matrix per
-// thread.
+// in a fixed order (bit-reproducible).  Orders 0..8 take 16 lanes per
+// matrix.
 #include "common.h"
 #include "glynn_blocks.h"
 #include "../../include/pcvl_hip.h"
@@ -31,13 +31,14 @@
 
 namespace pcvl {
 
-constexpr int PERM_WAVE_MIN = 9;
+constexpr int PERM_WAVE_MIN = 11;
 constexpr int PERM_WAVE_MAX = 28;   // the mixed-order launch
 // Orders 29..32 run in a launch of their own (their registers would lower the
 // occupancy of the mixed launch), from their own part of the queue.
 constexpr int PERM_BIG_MIN = PERM_WAVE_MAX + 1;
 constexpr int PERM_BIG_MAX = 32;
-constexpr int PERM_SMALL_MAX = 8;
+constexpr int PERM_THREAD_MAX = 5;  // a thread per matrix
+constexpr int PERM_SMALL_MAX = 10;  // 16 lanes per matrix
 
 struct PermItem {
     int64_t mat_off;   // complex offset of the matrix in the packed array
@@ -182,44 +183,50 @@ __device__ __forceinline__ cd dispatch_item(const double *__restrict__ mats, con
 // perm_finalize so the same plan can be replayed (also inside a HIP graph).
 template <int NLO, int NHI, bool ONE = false>
 __global__ void __launch_bounds__(64, 2) perm_wave_kernel(const double *__restrict__ mats,
-                                                       const PermItem *__restrict__ items, int64_t nitems,
+                                                       const PermItem *__restrict__ items,
+                                                       const uint32_t *__restrict__ groups, int64_t ngroups,
                                                        unsigned long long *cursor, cd *__restrict__ partials)
 {
     __shared__ cd sA[NHI * NHI];
-    // A wave can take at most nitems items, so the loop is bounded whatever
+    // A wave can take at most ngroups groups, so the loop is bounded whatever
     // the cursor holds; items whose order or chunk size lies outside what
     // this instantiation handles are skipped (their slot is left untouched).
-    for (int64_t iter = 0; iter < nitems; iter++) {
+    // The first group of a wave is its own, the others come from the cursor.
+    uint64_t g = blockIdx.x;
+    for (int64_t iter = 0; iter < ngroups && g < (uint64_t)ngroups; iter++) {
+        const uint32_t lo = __builtin_amdgcn_readfirstlane(groups[g]), hi = __builtin_amdgcn_readfirstlane(groups[g + 1]);
+        for (uint32_t ku = lo; ku < hi; ku++) {
+            PermItem it;
+            {
+                const PermItem raw = items[ku];
+                it.mat_off = (int64_t)(((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)raw.mat_off >> 32)) << 32) |
+                                       __builtin_amdgcn_readfirstlane((uint32_t)raw.mat_off));
+                it.chunk0 = __builtin_amdgcn_readfirstlane(raw.chunk0);
+                it.slot = __builtin_amdgcn_readfirstlane(raw.slot);
+                it.n = __builtin_amdgcn_readfirstlane(raw.n);
+                it.c = __builtin_amdgcn_readfirstlane(raw.c);
+            }
+            if (it.n < NLO || it.n > NHI || it.c < 2 || it.c > it.n - 7) continue;
+            cd v = dispatch_item<NLO, NHI, ONE>(mats, it, sA);
+            v = wave_sum(v);
+            if (threadIdx.x == 0) partials[it.slot] = v;
+        }
         unsigned long long k = 0;
         if (threadIdx.x == 0) k = atomicAdd(cursor, 1ull);
         k = __shfl(k, 0, 64);
-        // The item index and every field of the item are wave-uniform; say so,
+        // The group index and every field of an item are wave-uniform; say so,
         // so that loop control and LDS row addresses live in SGPRs.
         const uint32_t k_lo = __builtin_amdgcn_readfirstlane((uint32_t)k);
         const uint32_t k_hi = __builtin_amdgcn_readfirstlane((uint32_t)(k >> 32));
-        const uint64_t ku = ((uint64_t)k_hi << 32) | k_lo;
-        if (ku >= (uint64_t)nitems) break;
-        PermItem it;
-        {
-            const PermItem raw = items[ku];
-            it.mat_off = (int64_t)(((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)raw.mat_off >> 32)) << 32) |
-                                   __builtin_amdgcn_readfirstlane((uint32_t)raw.mat_off));
-            it.chunk0 = __builtin_amdgcn_readfirstlane(raw.chunk0);
-            it.slot = __builtin_amdgcn_readfirstlane(raw.slot);
-            it.n = __builtin_amdgcn_readfirstlane(raw.n);
-            it.c = __builtin_amdgcn_readfirstlane(raw.c);
-        }
-        if (it.n < NLO || it.n > NHI || it.c < 2 || it.c > it.n - 7) continue;
-        cd v = dispatch_item<NLO, NHI, ONE>(mats, it, sA);
-        v = wave_sum(v);
-        if (threadIdx.x == 0) partials[it.slot] = v;
+        g = gridDim.x + (((uint64_t)k_hi << 32) | k_lo);
     }
 }
 
 // --------------------------------------------------------------- small path
 
+// Orders up to PERM_THREAD_MAX, one thread per matrix.
 template <int N>
-__device__ cd glynn_small(const cd *__restrict__ A)
+__device__ __forceinline__ cd glynn_thread(const cd *__restrict__ A)
 {
     if constexpr (N == 0) {
         return {1.0, 0.0};
@@ -227,22 +234,21 @@ __device__ cd glynn_small(const cd *__restrict__ A)
         cd cs[N];
 #pragma unroll
         for (int j = 0; j < N; j++) {
-            cd s = {0.0, 0.0};
-            for (int i = 0; i < N; i++) s = cadd(s, A[i * N + j]);
-            cs[j] = s;
+            cs[j] = A[j];
+#pragma unroll
+            for (int i = 1; i < N; i++) cs[j] = cadd(cs[j], A[i * N + j]);
         }
         cd acc = {0.0, 0.0};
-        uint32_t g = 0;
+#pragma unroll
         for (uint32_t t = 0; t < (1u << (N - 1)); t++) {
             if (t) {
-                int b = __builtin_ctz(t);
-                g ^= 1u << b;
-                double s = ((g >> b) & 1) ? -2.0 : 2.0;
-                const cd *row = A + (b + 1) * N;
+                const int b = __builtin_ctz(t);
+                const double d = ((t >> (b + 1)) & 1) ? 2.0 : -2.0;   // Gray bit b goes back, or on
 #pragma unroll
                 for (int j = 0; j < N; j++) {
-                    cs[j].r = fma(s, row[j].r, cs[j].r);
-                    cs[j].i = fma(s, row[j].i, cs[j].i);
+                    const cd a = A[(b + 1) * N + j];
+                    cs[j].r = fma(d, a.r, cs[j].r);
+                    cs[j].i = fma(d, a.i, cs[j].i);
                 }
             }
             cd p = cs[0];
@@ -250,31 +256,113 @@ __device__ cd glynn_small(const cd *__restrict__ A)
             for (int j = 1; j < N; j++) p = cmul(p, cs[j]);
             if (t & 1) { acc.r -= p.r; acc.i -= p.i; } else { acc.r += p.r; acc.i += p.i; }
         }
-        double sc = ldexp(1.0, -(N - 1));
+        constexpr double sc = 1.0 / (1 << (N - 1));
         return {acc.r * sc, acc.i * sc};
     }
 }
 
 template <int N>
-__device__ __forceinline__ cd dispatch_small(int n, const cd *A)
+__device__ __forceinline__ cd dispatch_thread(int n, const cd *A)
+{
+    if constexpr (N > PERM_THREAD_MAX) {
+        return {0.0, 0.0};
+    } else {
+        if (n == N) return glynn_thread<N>(A);
+        return dispatch_thread<N + 1>(n, A);
+    }
+}
+
+// Orders above, to PERM_SMALL_MAX, 16 lanes per matrix, A in LDS: lane bits sign rows 1..4, the
+// remaining rows run through their Gray code with the column sums in registers.
+template <int N>
+__device__ __forceinline__ cd glynn_row(const cd *A, int lane)
+{
+    static_assert(N >= 5, "all 16 lanes take terms");
+    constexpr int LB = 4;
+    // unrolled, orders 9 and 10 keep rows in registers ahead of their use and spill
+    constexpr int R = N <= 8 ? N : 3, S = N <= 8 ? 8 : 2;
+    cd cs[N];
+#pragma unroll
+    for (int j = 0; j < N; j++) cs[j] = A[j];
+#pragma unroll R
+    for (int i = 1; i < N; i++) {
+        const double d = i <= LB && ((lane >> (i - 1)) & 1) ? -1.0 : 1.0;
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            const cd a = A[i * N + j];
+            cs[j].r = fma(d, a.r, cs[j].r);
+            cs[j].i = fma(d, a.i, cs[j].i);
+        }
+    }
+    cd acc = {0.0, 0.0};
+#pragma unroll S
+    for (uint32_t t = 0; t < (1u << (N - 1 - LB)); t++) {
+        if (t) {
+            const int b = __builtin_ctz(t);
+            const double d = ((t >> (b + 1)) & 1) ? 2.0 : -2.0;   // Gray bit b goes back, or on
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                const cd a = A[(LB + 1 + b) * N + j];
+                cs[j].r = fma(d, a.r, cs[j].r);
+                cs[j].i = fma(d, a.i, cs[j].i);
+            }
+        }
+        cd p = cs[0];
+#pragma unroll
+        for (int j = 1; j < N; j++) p = cmul(p, cs[j]);
+        if (t & 1) { acc.r -= p.r; acc.i -= p.i; } else { acc.r += p.r; acc.i += p.i; }
+    }
+    if (__popc(lane) & 1) acc = {-acc.r, -acc.i};
+    constexpr double sc = 1.0 / (1 << (N - 1));
+    return {row_sum(acc.r) * sc, row_sum(acc.i) * sc};
+}
+
+template <int N>
+__device__ __forceinline__ cd dispatch_row(int n, const cd *A, int lane)
 {
     if constexpr (N > PERM_SMALL_MAX) {
         return {0.0, 0.0};
     } else {
-        if (n == N) return glynn_small<N>(A);
-        return dispatch_small<N + 1>(n, A);
+        if (n == N) return glynn_row<N>(A, lane);
+        return dispatch_row<N + 1>(n, A, lane);
     }
 }
 
-__global__ void perm_small_kernel(const double *__restrict__ mats, const int64_t *__restrict__ idx,
-                                  const int64_t *__restrict__ offs, const int32_t *__restrict__ ns,
-                                  int64_t count, cd *__restrict__ out)
+// The plan lists its small matrices by order; nthread of them go a thread each
+// (workgroups below `first`), the others 16 lanes each.  Bound by launch and
+// load latency at everyday counts (7 us from the caller).  Measured, a thread
+// per matrix -> 16 lanes: 12,376 of order 6 18.4 -> 6.9 us, of order 8 118 ->
+// 7.5 (column sums and rows of one thread spilled to scratch, 194 waves for 256
+// CUs).  Orders 9 and 10 took a wave and an item of the queue each: 12,376 of
+// order 9 202 -> 13.8, of order 10 252 -> 24.7, one of order 10 10.2 -> 9.3.
+// PERM_THREAD_MAX: 100,000 of order 5 take 14 us a thread each and 54 in 16
+// lanes, of order 6 65 and 23.  PERM_SMALL_MAX: 20,000 of order 11 are 112 us in
+// the queue, and 16 lanes would do 64 terms each, ten times order 8's work.
+constexpr int PERM_ROWS = 16;
+constexpr int PERM_ROW_LD = PERM_SMALL_MAX * PERM_SMALL_MAX + 1;   // the four matrices of a wave on different banks
+
+__global__ void __launch_bounds__(16 * PERM_ROWS, 4) perm_small_kernel(
+    const double *__restrict__ mats, const int64_t *__restrict__ idx, const int64_t *__restrict__ offs,
+    const int32_t *__restrict__ ns, int64_t count, int64_t nthread, unsigned first, cd *__restrict__ out)
 {
-    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= count) return;
-    int64_t b = idx[k];
-    const cd *A = reinterpret_cast<const cd *>(mats) + offs[k];
-    out[b] = dispatch_small<0>(ns[k], A);
+    __shared__ cd s_mat[PERM_ROWS * PERM_ROW_LD];
+    if (blockIdx.x < first) {
+        const int64_t k = (int64_t)blockIdx.x * (16 * PERM_ROWS) + threadIdx.x;
+        if (k < nthread) out[idx[k]] = dispatch_thread<0>(ns[k], reinterpret_cast<const cd *>(mats) + offs[k]);
+        return;
+    }
+    const int lane = threadIdx.x & 15, row = threadIdx.x >> 4;
+    const int64_t k = nthread + (int64_t)(blockIdx.x - first) * PERM_ROWS + row;
+    const bool in = k < count;
+    const int n = in ? ns[k] : 0;
+    cd *A = s_mat + row * PERM_ROW_LD;
+    if (in) {
+        const cd *M = reinterpret_cast<const cd *>(mats) + offs[k];
+        for (int e = lane; e < n * n; e += 16) A[e] = M[e];
+    }
+    __syncthreads();
+    const cd v = dispatch_row<PERM_THREAD_MAX + 1>(n, A, lane);
+    if (in && lane == 0) out[idx[k]] = v;
 }
 
 // Sum each wave-path matrix's partials in slot order, scale by 2^{-(n-1)},
@@ -298,12 +386,15 @@ __global__ void perm_finalize_kernel(const int64_t *__restrict__ idx, const int3
 struct PermPlanImpl {
     int64_t count = 0;
     int64_t nitems = 0, nwave_mats = 0, nsmall = 0;
+    int64_t nthread = 0;       // small matrices of a thread each, first in their list
+    int64_t ngroups = 0, nbig_groups = 0;   // the queue's parts, below d_groups
     int64_t nbig = 0;          // items of orders 29..32, after the nitems others in the queue
     int grid_big = 0;
     int single_n = 0;          // order shared by every wave item, or 0 if mixed
     int variant = 0;           // 0, 1, 3: low rows by order; 2, 4 (single-order plans): one low row
     int grid = 0;
     PermItem *d_items = nullptr;
+    uint32_t *d_groups = nullptr;   // first item of each group and the end: the queue of orders <= 28, then 29..32
     unsigned long long *d_cursor = nullptr;   // [0]: the queue of orders <= 28, [1]: orders 29..32
     cd *d_partials = nullptr;
     int64_t *d_wave_idx = nullptr;
@@ -324,11 +415,11 @@ static int pick_chunk_log2(int n, int max_c)
 }
 
 template <int NLO, int NHI, bool ONE>
-static int launch_wave(const PermPlanImpl *p, const double *mats, hipStream_t st, const PermItem *items,
-                       int64_t nitems, unsigned long long *cursor, int grid)
+static int launch_wave(const PermPlanImpl *p, const double *mats, hipStream_t st, const uint32_t *groups,
+                       int64_t ngroups, unsigned long long *cursor, int grid)
 {
-    hipLaunchKernelGGL((perm_wave_kernel<NLO, NHI, ONE>), dim3(grid), dim3(64), 0, st, mats, items, nitems, cursor,
-                       p->d_partials);
+    hipLaunchKernelGGL((perm_wave_kernel<NLO, NHI, ONE>), dim3(grid), dim3(64), 0, st, mats, p->d_items, groups,
+                       ngroups, cursor, p->d_partials);
     PCVL_HIP_CHECK(hipGetLastError());
     return OK;
 }
@@ -336,7 +427,7 @@ static int launch_wave(const PermPlanImpl *p, const double *mats, hipStream_t st
 template <int NLO, int NHI, bool ONE>
 static int launch_wave(const PermPlanImpl *p, const double *mats, hipStream_t st)
 {
-    return launch_wave<NLO, NHI, ONE>(p, mats, st, p->d_items, p->nitems, p->d_cursor, p->grid);
+    return launch_wave<NLO, NHI, ONE>(p, mats, st, p->d_groups, p->ngroups, p->d_cursor, p->grid);
 }
 
 static bool perm_one_low_row(int variant) { return variant == 2 || variant == 4; }
@@ -401,8 +492,45 @@ static constexpr int64_t PERM_MAX_ITEMS = int64_t(1) << 27;
 // arrays | small arrays, at these byte offsets.
 struct PermLayout {
     size_t o_items = 0, o_cursor = 0, o_part = 0, o_widx = 0, o_ws0 = 0, o_wns = 0, o_wn = 0, o_sidx = 0,
-           o_soff = 0, o_sn = 0, total = 0;
+           o_soff = 0, o_sn = 0, o_groups = 0, total = 0;
 };
+
+// Cuts items [i0, i1) of the sorted queue into the groups that a wave takes at
+// once; appends their starts and the end.  One pull from the cursor is an
+// atomic on one address for the whole chip, 12..20 ns each however many waves
+// wait, so small items cannot each have one: 20,000 of order 11 395 -> 112 us,
+// of order 14 599 -> 398, 4,000 of order 16 469 -> 327.  Where the pulls would take
+// more than a quarter of the work's time (estimated from the instructions of an
+// item), the first groups, one a wave and not pulled, hold 70% of the work (a
+// slow CU takes 1.3 times the average), and the rest is cut into as many groups
+// as pulls fit into the work's time.  Otherwise every item is a group.
+static int64_t perm_groups(const std::vector<PermItem> &items, int64_t i0, int64_t i1, int resident,
+                           std::vector<uint32_t> &starts)
+{
+    constexpr double PULL = 15e-9, ISSUE = 4.0 / 2.1e9, SIMDS = 1024.0;
+    auto cost = [&](int64_t i) {   // seconds of one SIMD: blocks, and the sums and constants before them
+        const double n = items[(size_t)i].n;
+        return ISSUE * (4.3 * n * std::ldexp(1.0, items[(size_t)i].c) + 2.0 * n * n + 40.0 * n);
+    };
+    const int64_t count = i1 - i0, first = (int64_t)starts.size();
+    double total = 0.0;
+    for (int64_t i = i0; i < i1; i++) total += cost(i);
+    const bool single = count <= resident || (double)count * PULL * 4.0 * SIMDS <= total;
+    const double pulls = std::max(total / SIMDS / PULL, 1.0);
+    const double own = 0.7 * total / std::max(resident, 1), pulled = 0.3 * total / pulls;
+    double sum = 0.0;
+    for (int64_t i = i0; i < i1; i++) {
+        const double want = (int64_t)starts.size() - first <= resident ? own : pulled;
+        if (single || i == i0 || sum + 0.5 * cost(i) >= want) {
+            starts.push_back((uint32_t)i);
+            sum = 0.0;
+        }
+        sum += cost(i);
+    }
+    const int64_t groups = (int64_t)starts.size() - first;
+    starts.push_back((uint32_t)i1);
+    return groups;
+}
 
 // Builds a plan on the host: the scheduling fields of p, the layout of its
 // device block and the block's contents (cursor zero).  No device call but
@@ -428,8 +556,6 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
         PCVL_ARG_CHECK(h_offsets[b] >= 0, "negative matrix offset");
         if (n <= PERM_SMALL_MAX) {
             small_idx.push_back(b);
-            small_off.push_back(h_offsets[b]);
-            small_n.push_back(n);
             continue;
         }
         wave_idx.push_back(b);
@@ -441,6 +567,13 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
         }
         nmin = std::min(nmin, n);
         nmax = std::max(nmax, n);
+    }
+    // the small ones by order, a thread each first
+    std::stable_sort(small_idx.begin(), small_idx.end(), [&](int64_t a, int64_t b) { return h_n[a] < h_n[b]; });
+    for (int64_t b : small_idx) {
+        small_off.push_back(h_offsets[b]);
+        small_n.push_back(h_n[b]);
+        if (h_n[b] <= PERM_THREAD_MAX) p.nthread++;
     }
     // orders <= 28: one launch, specialised when they share one order
     const int single_n = (nmax >= 0 && nmin == nmax) ? nmax : 0;
@@ -472,7 +605,9 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
         for (size_t r = order.size(); r-- > 0 && tail < resident;) {
             const size_t i = order[r];
             tail += (int64_t)((1ull << (wave_n[i] - 1 - wave_c[i])) / 64);
-            wave_c[i] = std::max(2, wave_c[i] - 2);
+            // not where an item would then be mostly sums and constants (1,000 of
+            // order 11 46 us with it, 22 without; 89 before the groups below)
+            if (wave_c[i] >= 4 && 4.3 * (1 << (wave_c[i] - 2)) >= 2.0 * wave_n[i] + 40.0) wave_c[i] -= 2;
         }
     }
     int64_t total_slots = 0;
@@ -507,15 +642,19 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
     const int64_t nregular = (int64_t)items.size();
     items.insert(items.end(), big_items.begin(), big_items.end());
 
+    std::vector<uint32_t> groups;
+    p.ngroups = perm_groups(items, 0, nregular, rw, groups);
+    p.nbig_groups = perm_groups(items, nregular, (int64_t)items.size(), rwb, groups);
+
     p.count = count;
     p.nitems = nregular;
     p.nbig = (int64_t)big_items.size();
-    p.grid_big = p.nbig > 0 ? (int)std::min<int64_t>(p.nbig, (int64_t)rwb) : 0;
+    p.grid_big = p.nbig > 0 ? (int)std::min<int64_t>(p.nbig_groups, (int64_t)rwb) : 0;
     p.nwave_mats = (int64_t)wave_idx.size();
     p.nsmall = (int64_t)small_idx.size();
     p.single_n = single_n;
     p.variant = kvariant;
-    p.grid = p.nitems > 0 ? (int)std::min<int64_t>(p.nitems, (int64_t)rw) : 0;
+    p.grid = p.nitems > 0 ? (int)std::min<int64_t>(p.ngroups, (int64_t)rw) : 0;
 
     auto align = [](size_t x) { return (x + 255) & ~size_t(255); };
     L.o_items = 0;
@@ -528,7 +667,8 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
     L.o_sidx = align(L.o_wn + sizeof(int32_t) * wave_idx.size());
     L.o_soff = align(L.o_sidx + sizeof(int64_t) * small_idx.size());
     L.o_sn = align(L.o_soff + sizeof(int64_t) * small_idx.size());
-    L.total = align(L.o_sn + sizeof(int32_t) * small_idx.size());
+    L.o_groups = align(L.o_sn + sizeof(int32_t) * small_idx.size());
+    L.total = align(L.o_groups + sizeof(uint32_t) * groups.size());
 
     host.assign(L.total, 0);
     auto put = [&](size_t off, const void *src, size_t bytes) { if (bytes) std::memcpy(host.data() + off, src, bytes); };
@@ -540,6 +680,7 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
     put(L.o_sidx, small_idx.data(), sizeof(int64_t) * small_idx.size());
     put(L.o_soff, small_off.data(), sizeof(int64_t) * small_idx.size());
     put(L.o_sn, small_n.data(), sizeof(int32_t) * small_idx.size());
+    put(L.o_groups, groups.data(), sizeof(uint32_t) * groups.size());
     return OK;
 }
 
@@ -557,6 +698,7 @@ static void perm_plan_bind(PermPlanImpl &p, const PermLayout &L, void *block)
     p.d_small_idx = reinterpret_cast<int64_t *>(base + L.o_sidx);
     p.d_small_off = reinterpret_cast<int64_t *>(base + L.o_soff);
     p.d_small_n = reinterpret_cast<int32_t *>(base + L.o_sn);
+    p.d_groups = reinterpret_cast<uint32_t *>(base + L.o_groups);
 }
 
 static int perm_plan_create_impl(const int32_t *h_n, const int64_t *h_offsets, int64_t count,
@@ -617,16 +759,17 @@ extern "C" int pcvl_perm_plan_execute(pcvl_perm_plan plan, const double *d_mats,
     PCVL_ARG_CHECK(d_mats && d_out, "null device buffer");
     cd *out = reinterpret_cast<cd *>(d_out);
     if (p.nsmall > 0) {
-        int blocks = (int)((p.nsmall + 255) / 256);
-        hipLaunchKernelGGL(perm_small_kernel, dim3(blocks), dim3(256), 0, stream, d_mats, p.d_small_idx,
-                           p.d_small_off, p.d_small_n, p.nsmall, out);
+        const unsigned first = (unsigned)((p.nthread + 16 * PERM_ROWS - 1) / (16 * PERM_ROWS));
+        const unsigned rows = (unsigned)((p.nsmall - p.nthread + PERM_ROWS - 1) / PERM_ROWS);
+        hipLaunchKernelGGL(perm_small_kernel, dim3(first + rows), dim3(16 * PERM_ROWS), 0, stream, d_mats,
+                           p.d_small_idx, p.d_small_off, p.d_small_n, p.nsmall, p.nthread, first, out);
         PCVL_HIP_CHECK(hipGetLastError());
     }
     if (p.nwave_mats > 0) {
         int rc = OK;
         if (p.nbig > 0)   // orders 29..32 first: the longest items
-            rc = launch_wave<PERM_BIG_MIN, PERM_BIG_MAX, false>(&p, d_mats, stream, p.d_items + p.nitems, p.nbig,
-                                                            p.d_cursor + 1, p.grid_big);
+            rc = launch_wave<PERM_BIG_MIN, PERM_BIG_MAX, false>(&p, d_mats, stream, p.d_groups + p.ngroups + 1,
+                                                                p.nbig_groups, p.d_cursor + 1, p.grid_big);
         if (rc == OK && p.nitems > 0)
             rc = p.single_n ? launch_single<PERM_WAVE_MIN>(&p, d_mats, stream)
                             : launch_wave<PERM_WAVE_MIN, PERM_WAVE_MAX, false>(&p, d_mats, stream);

@@ -829,6 +829,11 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     std::vector<uint32_t> fwords;
     std::vector<double> fpf;
     front_choose(&lay);
+    {
+        size_t words = 0;
+        for (int k = 1; k <= lay.front; k++) words += (size_t)lay.front_slots[(size_t)k] * lay.counts[(size_t)k];
+        fwords.reserve(words);
+    }
     for (int k = 1; k <= lay.front; k++) {
         const uint32_t cnt = (uint32_t)lay.counts[(size_t)k];
         const bool last = k == lay.nlayers;

@@ -49,6 +49,26 @@ def test_small_orders_vs_brute(gpu):
         assert _rel(g, ref) < 1e-12, (M.shape, g, ref)
 
 
+@pytest.mark.parametrize("lo,hi,count", [(0, 11, 300), (4, 6, 33), (10, 12, 17), (11, 11, 3000), (11, 14, 2500)])
+def test_small_and_grouped_items_vs_oracle(gpu, lo, hi, count):
+    """Orders around the lines between a thread (to 5), 16 lanes (to 10) and a
+    wave per matrix, in one batch, with counts off the 16 matrices of a
+    workgroup; and queues of so many small items that waves take them in groups,
+    executed twice (the cursor goes back to zero)."""
+    import torch
+    from perceval_amd.permanent import PermanentPlan, pack
+    rng = np.random.RandomState(lo + 100 * hi)
+    mats = [rng.randn(n, n) + 1j * rng.randn(n, n) for n in rng.randint(lo, hi + 1, count)]
+    orders, flat = pack(mats)
+    plan = PermanentPlan(orders)
+    d = torch.from_numpy(flat).cuda()
+    got = [plan(d).cpu().numpy() for _ in range(2)]
+    assert np.array_equal(got[0], got[1])
+    ref = oracle.perm_batch(mats, precise=True)
+    for g, r, M in zip(got[0], ref, mats):
+        assert _rel(g, r) < REL_TOL, (M.shape, g, r)
+
+
 @pytest.mark.parametrize("n", list(range(9, 25)))
 def test_wave_orders_vs_oracle(gpu, n):
     U = haar_unitary(64, seed=100 + n)
