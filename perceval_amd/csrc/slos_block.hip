@@ -846,18 +846,22 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
                 const uint32_t S = (uint32_t)nstates(w, r);
                 const int ns = std::min(r, w);
                 for_blocks(sub.kf - r, r, [&](uint32_t Bk, uint32_t PEh, const BlkOcc &occ, double pf) {
-                    for (uint32_t b = 0; b < S; b++) {
-                        const uint32_t loc = Bk + b, c = sub.out_base + loc;
-                        size_t at = off0 + c;
-                        auto put = [&](uint32_t rank, uint32_t mode) { fwords[at] = (rank << 8) | mode; at += cnt; };
-                        for (const auto &e : sub.her) put(e.second + loc, (uint32_t)m + e.first);
-                        for (const auto &e : occ) put(sub.par_base + loc - e.second, e.first);
-                        for (int d = 0; d < ns; d++) {
-                            const uint32_t word = sslot[(size_t)tslot[(size_t)r] + (size_t)d * S + b];
-                            if (word != 0xffffffffu) put(sub.par_base + Bk - PEh + (word >> 5), (uint32_t)h + (word & 31u));
-                        }
-                        if (last) fpf[c] = pf * spf[(size_t)tpf[(size_t)r] + b] * sub.hfact;
+                    uint32_t *at = fwords.data() + off0 + sub.out_base + Bk;   // the block's children, slot by slot
+                    auto run = [&](uint32_t rank, uint32_t mode) {             // parents at consecutive ranks
+                        for (uint32_t b = 0; b < S; b++) at[b] = ((rank + b) << 8) | mode;
+                        at += cnt;
+                    };
+                    for (const auto &e : sub.her) run(e.second + Bk, (uint32_t)m + e.first);
+                    for (const auto &e : occ) run(sub.par_base + Bk - e.second, e.first);
+                    const uint32_t add = ((sub.par_base + Bk - PEh) << 8) + (uint32_t)h;
+                    for (int d = 0; d < ns; d++, at += cnt) {
+                        const uint32_t *slot = sslot.data() + tslot[(size_t)r] + (size_t)d * S;
+                        for (uint32_t b = 0; b < S; b++)
+                            at[b] = slot[b] == 0xffffffffu ? slot[b] : ((slot[b] >> 5) << 8 | (slot[b] & 31u)) + add;
                     }
+                    if (last)
+                        for (uint32_t b = 0; b < S; b++)
+                            fpf[sub.out_base + Bk + b] = pf * spf[(size_t)tpf[(size_t)r] + b] * sub.hfact;
                 });
             }
         if (k < lay.front && k == lay.front_staged_layers + 1 && fwords.size() <= FRONT_STAGED) {
