@@ -1148,6 +1148,8 @@ struct SlosTreeImpl {
     std::vector<TreeNode> nodes;
     std::vector<int> level_ops;         // by depth: first entry of depth k in d_ops (nmax + 2 entries); empty: depth first
     BlkBatchOp *d_ops = nullptr;
+    int front = 0;                      // depths 1..front run in one launch (0: each its own)
+    const int32_t *d_paths = nullptr;   // input modes from the root of the nodes of depth front, behind d_ops
     uint64_t *d_T = nullptr, *d_E = nullptr;
     int grid_cap = 0;
     BlkLayout blk;                      // block layout of the layers, when they allow it
@@ -1239,9 +1241,26 @@ static int tree_levels(SlosTreeImpl &t, const std::vector<double> &inv_pin)
     }
     first.push_back((int)ops.size());
     if (ops.empty()) return OK;
-    hipError_t e = hipMalloc(&t.d_ops, sizeof(BlkBatchOp) * ops.size());
+    // the first depths in one launch, up to the one before the first outputs
+    int front = t.blk.front;
+    for (const TreeNode &nd : t.nodes)
+        if (!nd.inputs.empty()) front = std::min(front, nd.k - 1);
+    std::vector<int32_t> paths;
+    if (front >= 2)
+        for (size_t i = 0; i < t.nodes.size(); i++) {   // in the order of the ops
+            if (t.nodes[i].k != front) continue;
+            paths.resize(paths.size() + (size_t)front);
+            int at_node = (int)i;
+            for (int k = front; k >= 1; k--, at_node = t.nodes[(size_t)at_node].parent)
+                paths[paths.size() - (size_t)(front - k) - 1] = t.nodes[(size_t)at_node].mk;
+        }
+    const size_t b_ops = sizeof(BlkBatchOp) * ops.size();
+    hipError_t e = hipMalloc(&t.d_ops, b_ops + sizeof(int32_t) * paths.size());
     if (e != hipSuccess) { t.d_ops = nullptr; set_error(std::string("hipMalloc(slos tree ops): ") + hipGetErrorString(e)); return ERR_ALLOC; }
-    e = hipMemcpy(t.d_ops, ops.data(), sizeof(BlkBatchOp) * ops.size(), hipMemcpyHostToDevice);
+    e = hipMemcpy(t.d_ops, ops.data(), b_ops, hipMemcpyHostToDevice);
+    if (e == hipSuccess && !paths.empty())
+        e = hipMemcpy(reinterpret_cast<char *>(t.d_ops) + b_ops, paths.data(), sizeof(int32_t) * paths.size(),
+                      hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(t.d_ops);
         t.d_ops = nullptr;
@@ -1249,6 +1268,10 @@ static int tree_levels(SlosTreeImpl &t, const std::vector<double> &inv_pin)
         return ERR_HIP;
     }
     t.level_ops = std::move(first);
+    if (!paths.empty()) {
+        t.front = front;
+        t.d_paths = reinterpret_cast<const int32_t *>(reinterpret_cast<char *>(t.d_ops) + b_ops);
+    }
     t.work_bytes = off;
     return OK;
 }
@@ -1368,7 +1391,7 @@ extern "C" int pcvl_slos_tree_execute(pcvl_slos_tree plan, const double *d_U, in
     char *work = static_cast<char *>(d_work);
     const size_t esz = mode == PCVL_SLOS_PROBS ? sizeof(double) : sizeof(cd);
     const size_t lds = 2 * sizeof(uint64_t) * (size_t)t.m * t.w;
-    if (t.nmax > 0) {   // depth-0 buffer holds the vacuum coefficient
+    if (t.nmax > 0 && t.front == 0) {   // depth-0 buffer holds the vacuum coefficient
         hipLaunchKernelGGL(slos_vacuum_kernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<double *>(work + t.level_off[0]), 0);
         PCVL_HIP_CHECK(hipGetLastError());
     }
@@ -1410,10 +1433,12 @@ extern "C" int pcvl_slos_tree_execute(pcvl_slos_tree plan, const double *d_U, in
         PCVL_HIP_CHECK(hipGetLastError());
     }
     if (!t.level_ops.empty())
-        for (int k = 1; k <= t.nmax; k++) {
+        for (int k = std::max(t.front, 1); k <= t.nmax; k++) {
             const int a = t.level_ops[(size_t)k], n = t.level_ops[(size_t)k + 1] - a;
             if (n == 0) continue;
-            const int rc = blk_batch_launch(t.blk, t.d_ops + a, n, work, static_cast<char *>(d_out),
+            const int rc = k == t.front
+                ? blk_front_batch_launch(t.blk, k, t.d_ops + a, t.d_paths, n, work, U, t.m, stream)
+                : blk_batch_launch(t.blk, t.d_ops + a, n, work, static_cast<char *>(d_out),
                                             mode == PCVL_SLOS_PROBS, U, t.m, k, stream);
             if (rc != OK) return rc;
         }

@@ -188,4 +188,10 @@ struct BlkBatchOp {
 int blk_batch_launch(const BlkLayout &lay, const BlkBatchOp *d_ops, int nops, char *work, char *out, bool probs,
                      const cd *U, int m, int k, hipStream_t stream);
 
+// The nodes of a tree at depth front (<= lay.front) from the vacuum, in one
+// launch: node i into its layer buffer d_ops[i].lvl_off, along the input modes
+// d_paths[i * front ...].  Unmasked layouts.
+int blk_front_batch_launch(const BlkLayout &lay, int front, const BlkBatchOp *d_ops, const int32_t *d_paths, int nops,
+                           char *work, const cd *U, int m, hipStream_t stream);
+
 } // namespace pcvl

@@ -512,12 +512,16 @@ __device__ __forceinline__ cd front_child(const uint32_t *words, uint32_t count,
     return acc;
 }
 
+// MODE 2: the nodes of an input tree at depth `front`, blockIdx.y, each from
+// its own path of input modes (paths[y * front + k - 1]) into its layer buffer.
 template <int MODE>
 __global__ void __launch_bounds__(FRONT_THREADS) slos_front_kernel(
     const cd *__restrict__ U, int m, int mloc, const int32_t *__restrict__ rowmap, const uint32_t *__restrict__ words,
     const double *__restrict__ pf, FrontLayers f, int front, int staged_layers, uint32_t staged, uint32_t cap0,
-    uint32_t cap1, uint32_t share, void *__restrict__ out, double inv_prod_in, int sentinel)
+    uint32_t cap1, uint32_t share, void *__restrict__ out, double inv_prod_in, int sentinel,
+    const BlkBatchOp *__restrict__ ops, const int32_t *__restrict__ paths)
 {
+    if (MODE == 2) out = static_cast<char *>(out) + ops[blockIdx.y].lvl_off;
     extern __shared__ cd s_front[];
     cd *even = s_front, *odd = even + cap0, *su = odd + cap1;            // layers by parity; U column of each layer
     uint32_t *sw = reinterpret_cast<uint32_t *>(su + (size_t)front * mloc);
@@ -525,7 +529,8 @@ __global__ void __launch_bounds__(FRONT_THREADS) slos_front_kernel(
     for (uint32_t e = tid; e < staged; e += FRONT_THREADS) sw[e] = words[e];
     for (int e = tid; e < front * mloc; e += FRONT_THREADS) {
         const int k = e / mloc, i = e - k * mloc;
-        su[e] = U[(size_t)(rowmap ? rowmap[i] : i) * m + f.mk[k + 1]];
+        const int mk = MODE == 2 ? paths[blockIdx.y * front + k] : f.mk[k + 1];
+        su[e] = U[(size_t)(rowmap ? rowmap[i] : i) * m + mk];
     }
     if (tid == 0) even[0] = cd{1.0, 0.0};
     if (sentinel && blockIdx.x == 0 && tid == 0) reinterpret_cast<cd *>(out)[f.count[front]] = cd{0.0, 0.0};
@@ -548,7 +553,7 @@ __global__ void __launch_bounds__(FRONT_THREADS) slos_front_kernel(
     for (uint32_t c = lo + tid; c < hi; c += FRONT_THREADS) {
         const cd acc = front_child(words + f.off[front], count, c, f.slots[front], (front & 1) ? even : odd,
                                    su + (front - 1) * mloc);
-        blk_emit<MODE>(BlkDest{out, nullptr, MODE == 1}, c, acc, MODE == 1 ? pf[c] : 0.0, inv_prod_in);
+        blk_emit<MODE == 1>(BlkDest{out, nullptr, MODE == 1}, c, acc, MODE == 1 ? pf[c] : 0.0, inv_prod_in);
     }
 }
 
@@ -1252,14 +1257,10 @@ int blk_layer_launch(const BlkLayout &lay, const cd *parent, void *out, const cd
     return OK;
 }
 
-int blk_front_launch(const BlkLayout &lay, void *out, const cd *U, int m, const std::vector<int32_t> &mk, bool probs,
-                     double inv_prod_in, bool sentinel, hipStream_t stream)
+static int front_launch(const BlkLayout &lay, int front, void *out, const cd *U, int m, const int32_t *mk, bool probs,
+                        double inv_prod_in, bool sentinel, const BlkBatchOp *ops, const int32_t *paths, int nodes,
+                        hipStream_t stream)
 {
-    const int front = lay.front;
-    if (front < 1 || (int)mk.size() < front || !lay.d_mem || (probs && front != lay.nlayers)) {
-        set_error("block SLOS: first layers outside the layout");
-        return ERR_ARG;
-    }
     const uint32_t count = (uint32_t)lay.counts[(size_t)front];
     if (count == 0) return OK;
     FrontLayers f = {};
@@ -1268,20 +1269,47 @@ int blk_front_launch(const BlkLayout &lay, void *out, const cd *U, int m, const 
         if (k == 0) continue;
         f.off[k] = lay.front_off[(size_t)k];
         f.slots[k] = lay.front_slots[(size_t)k];
-        f.mk[k] = mk[(size_t)k - 1];
+        f.mk[k] = mk ? mk[k - 1] : 0;
     }
+    const int staged_layers = std::min(lay.front_staged_layers, front - 1);
+    const uint32_t staged = staged_layers < lay.front ? lay.front_off[(size_t)staged_layers + 1] : lay.front_staged;
     // 256 children a workgroup; at most one workgroup per CU (256)
     const uint32_t groups = std::min<uint32_t>(256, (count + 255) / 256);
     const uint32_t share = (count + groups - 1) / groups;
     const char *base = lay.d_mem;
-    auto kp = probs ? slos_front_kernel<1> : slos_front_kernel<0>;
-    hipLaunchKernelGGL(kp, dim3((count + share - 1) / share), dim3(FRONT_THREADS),
-                       front_lds(lay, front, lay.front_staged), stream, U, m, lay.mloc,
+    auto kp = ops ? slos_front_kernel<2> : probs ? slos_front_kernel<1> : slos_front_kernel<0>;
+    hipLaunchKernelGGL(kp, dim3((count + share - 1) / share, nodes), dim3(FRONT_THREADS), front_lds(lay, front, staged),
+                       stream, U, m, lay.mloc,
                        lay.row_identity ? nullptr : reinterpret_cast<const int32_t *>(base + lay.off_row),
                        reinterpret_cast<const uint32_t *>(base + lay.off_front),
-                       reinterpret_cast<const double *>(base + lay.off_front_pf), f, front, lay.front_staged_layers,
-                       lay.front_staged, lay.front_cap[0], lay.front_cap[1], share, out, inv_prod_in, sentinel ? 1 : 0);
+                       reinterpret_cast<const double *>(base + lay.off_front_pf), f, front, staged_layers, staged,
+                       lay.front_cap[0], lay.front_cap[1], share, out, inv_prod_in, sentinel ? 1 : 0, ops, paths);
     PCVL_HIP_CHECK(hipGetLastError());
+    return OK;
+}
+
+int blk_front_launch(const BlkLayout &lay, void *out, const cd *U, int m, const std::vector<int32_t> &mk, bool probs,
+                     double inv_prod_in, bool sentinel, hipStream_t stream)
+{
+    if (lay.front < 1 || (int)mk.size() < lay.front || !lay.d_mem || (probs && lay.front != lay.nlayers)) {
+        set_error("block SLOS: first layers outside the layout");
+        return ERR_ARG;
+    }
+    return front_launch(lay, lay.front, out, U, m, mk.data(), probs, inv_prod_in, sentinel, nullptr, nullptr, 1, stream);
+}
+
+int blk_front_batch_launch(const BlkLayout &lay, int front, const BlkBatchOp *d_ops, const int32_t *d_paths, int nops,
+                           char *work, const cd *U, int m, hipStream_t stream)
+{
+    if (front < 1 || front > lay.front || !lay.d_mem || !lay.row_identity) {
+        set_error("block SLOS: first layers outside the layout");
+        return ERR_ARG;
+    }
+    for (int o = 0; o < nops; o += 32768) {
+        const int rc = front_launch(lay, front, work, U, m, nullptr, false, 1.0, false, d_ops + o,
+                                    d_paths + (size_t)o * front, std::min(nops - o, 32768), stream);
+        if (rc != OK) return rc;
+    }
     return OK;
 }
 
@@ -1303,9 +1331,12 @@ int blk_batch_launch(const BlkLayout &lay, const BlkBatchOp *d_ops, int nops, ch
     auto kp = lay.nmax <= 12 ? slos_block_batch_kernel<true> : slos_block_batch_kernel<false>;
     for (int o = 0; o < nops; o += 32768) {
         const int ny = std::min(nops - o, 32768);
-        // about one resident round of workgroups over all nodes, each node at
-        // least 16 (a workgroup's tables cost it a few microseconds of loads)
-        const uint64_t cap = std::max<uint64_t>(16, ((uint64_t)lay.grid_cap / (uint64_t)ny + 7) / 8 * 8);
+        // one resident round of workgroups over all nodes (a workgroup's
+        // tables cost it a few microseconds of loads), each node at least 16;
+        // rounded down: 28 nodes of 177,100 states took 73 us with 1,344
+        // workgroups for 1,280 places, a second round for 64 of them, and the
+        // whole tree 209 us against 193
+        const uint64_t cap = std::max<uint64_t>(16, (uint64_t)lay.grid_cap / (uint64_t)ny / 8 * 8);
         const uint32_t grid = (uint32_t)((std::min<uint64_t>(want, cap) + 7) / 8 * 8);
         hipLaunchKernelGGL(kp, dim3(grid, (unsigned)ny), dim3(BLK_THREADS), lds, stream, work, out, probs ? 1 : 0,
                            d_ops + o, U, m, k, (uint32_t)lay.counts[(size_t)k], lay.h, lay.w, lay.m, lay.mloc, groups,
