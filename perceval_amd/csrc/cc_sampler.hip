@@ -813,23 +813,23 @@ __global__ void __launch_bounds__(64, K <= 20 ? 3 : 2) cc_slice_kernel(const cd 
 {
     __shared__ CCShared<K> sh;
     const int lane = threadIdx.x;
-    const int64_t total = slice0[nchunk];
-    // a wave takes at most `total` slices, so the loop is bounded whatever the cursor holds
-    for (int64_t iter = 0; iter < total; iter++) {
-        unsigned long long gk = 0;
-        if (lane == 0) gk = atomicAdd(cursor, 1ull);
-        gk = __shfl(gk, 0, 64);
-        const int64_t g = (int64_t)gk;
-        if (g >= total) break;
+    __shared__ SliceQueue::State squeue;
+    SliceQueue queue(squeue, slice0[nchunk]);
+    int64_t last = -1;   // sample in LDS
+    CCPlan pl = {};
+    for (int64_t g; (g = queue.next(cursor)) >= 0;) {
         int64_t t;
         int slice;
         slice_owner(owner[g], t, slice);
-        const int64_t s = s0 + t;
-        if (lane < K) sh.pc[lane] = pc_all[s * n + lane];
-        if (lane < K - 1) sh.r[lane] = r_all[s * n + lane];
-        __syncthreads();
-        const CCPlan pl = cc_plan<K>(sh, lane);
-        load_rows<K>(sh, pl, U, m, lane);
+        if (t != last) {
+            last = t;
+            const int64_t s = s0 + t;
+            if (lane < K) sh.pc[lane] = pc_all[s * n + lane];
+            if (lane < K - 1) sh.r[lane] = r_all[s * n + lane];
+            __syncthreads();
+            pl = cc_plan<K>(sh, lane);
+            load_rows<K>(sh, pl, U, m, lane);
+        }
         const uint32_t per = (pl.units + (uint32_t)pl.slices - 1) / (uint32_t)pl.slices;
         const uint32_t u0 = (uint32_t)slice * per;
         const uint32_t u1 = u0 + per < pl.units ? u0 + per : pl.units;

@@ -440,30 +440,33 @@ __global__ void __launch_bounds__(64, 2) mis_slice_kernel(const cd *__restrict__
     constexpr int LOW = MispShared<N>::LOW, P = MispShared<N>::P;
     __shared__ int32_t srec[MISP_REC];
     const int lane = threadIdx.x;
-    const int64_t total = slice0[B];
-    // a wave takes at most `total` slices, so the loop is bounded whatever the cursor holds
-    for (int64_t iter = 0; iter < total; iter++) {
-        unsigned long long gk = 0;
-        if (lane == 0) gk = atomicAdd(cursor, 1ull);
-        gk = __shfl(gk, 0, 64);
-        const int64_t g = (int64_t)gk;
-        if (g >= total) break;
+    __shared__ SliceQueue::State squeue;
+    SliceQueue queue(squeue, slice0[B]);
+    __shared__ int64_t last;   // proposal in LDS
+    if (lane == 0) last = -1;
+    __syncthreads();
+    for (int64_t g; (g = queue.next(cursor)) >= 0;) {
         // proposal and slice of global slice g
         int64_t pidx;
         int s;
         slice_owner(owner[g], pidx, s);
-        for (int e = lane; e < MISP_REC; e += 64) srec[e] = rec[pidx * MISP_REC + e];
+        const bool fresh = pidx != last;
+        if (fresh) {
+            for (int e = lane; e < MISP_REC; e += 64) srec[e] = rec[pidx * MISP_REC + e];
+        }
         __syncthreads();
+        if (lane == 0) last = pidx;
         // wave-uniform: loop bounds and row addresses in SGPRs
         const int nu = __builtin_amdgcn_readfirstlane(srec[0]), ng = __builtin_amdgcn_readfirstlane(srec[1]);
         const int c = __builtin_amdgcn_readfirstlane(srec[2]), slices = __builtin_amdgcn_readfirstlane(srec[3]);
         const int nrow = __builtin_amdgcn_readfirstlane(srec[6]);
         const uint64_t units = (uint64_t)(uint32_t)srec[4] | ((uint64_t)(uint32_t)srec[5] << 32);
-        for (int e = lane; e < nrow * N; e += 64) {
-            const int r = e / N, cc = e % N;
-            sh.A[e] = Uc[(size_t)srec[8 + r] * N + cc];
-        }
-        if (lane < ng) {
+        if (fresh)
+            for (int e = lane; e < nrow * N; e += 64) {
+                const int r = e / N, cc = e % N;
+                sh.A[e] = Uc[(size_t)srec[8 + r] * N + cc];
+            }
+        if (fresh && lane < ng) {
             const int k = srec[8 + MISP_MAX_N + lane];
             int w0 = 0;
             for (int gg = 0; gg < lane; gg++) w0 += srec[8 + MISP_MAX_N + gg] + 1;
@@ -479,7 +482,7 @@ __global__ void __launch_bounds__(64, 2) mis_slice_kernel(const cd *__restrict__
         // proposals with at least LOW Gray-coded rows per unit run in blocks
         const bool pairs = N >= MISP_PAIR_MIN && c >= LOW;
         if constexpr (N >= MISP_PAIR_MIN) {
-            if (pairs) {
+            if (pairs && fresh) {
                 auto pair_const = [&](int q, int r, int p) {
                     cd h = cmul(sh.A[q * N + 2 * p], sh.A[r * N + 2 * p + 1]);
                     cfma_acc(h, sh.A[q * N + 2 * p + 1], sh.A[r * N + 2 * p]);

@@ -110,6 +110,18 @@ def test_split_steps_do_not_depend_on_the_call(gpu, n, count):
     assert np.array_equal(together, apart)
 
 
+def test_many_short_slices_do_not_depend_on_the_call(gpu):
+    """So many slices that waves take several at a time and keep a sample's rows
+    between them: the samples of calls that take them one by one."""
+    from perceval_amd.sampling import cc_samples
+    m, n, count = 24, 16, 60000
+    U = haar_unitary(m, seed=8)
+    inp = [1] * n + [0] * (m - n)
+    together = cc_samples(U, inp, count, seed=3)
+    for first in (0, 31234, count - 500):
+        assert np.array_equal(cc_samples(U, inp, 500, seed=3, first_sample=first), together[first:first + 500])
+
+
 @pytest.mark.parametrize("inp", [[1, 1, 0, 1, 0], [2, 1, 0, 0]])
 def test_distribution_chi_square(gpu, inp):
     from perceval_amd.sampling import cc_samples

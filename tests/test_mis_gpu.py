@@ -408,3 +408,21 @@ def test_learned_proposal_beats_untrained_m20_n6(gpu):
         if trained:
             assert tv["tvd1_mean"] < 0.02
     assert accs[True] > accs[False]
+
+
+def test_multiset_permanents_many_short_slices(gpu):
+    """So many short slices that waves take several at a time: bunched proposals
+    of 16 photons in 12 modes, against the plain permanents of the submatrices."""
+    import torch
+    from perceval_amd.mis import LearnedMIS, ProposalNet
+    m, n, B = 12, 16, 60000
+    U = haar_unitary(m, seed=6)
+    inp = [2] * 4 + [1] * 8
+    rng = np.random.RandomState(4)
+    seqs = torch.from_numpy(np.sort(rng.randint(0, m, size=(B, n)), axis=1).astype(np.int32)).cuda()
+    net = ProposalNet(m, n, hidden=8)
+    a = LearnedMIS(U, inp, net, chunk=B).permanents(seqs).cpu().numpy()
+    b = LearnedMIS(U, inp, net, chunk=B, multiset=False).permanents(seqs).cpu().numpy()
+    # both sum 2^15 terms of products of 16 column sums in double: 1e-12 of the
+    # largest permanent of the batch
+    assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b))
