@@ -330,7 +330,7 @@ def bench_perm(args, res):
     res["perm"]["fp64_fma_probe_tflops"] = probe
     res["perm"]["frac_of_probe"] = achieved / probe
     log(f"[bench] FP64 FMA probe: {probe:.2f} TFLOP/s attainable; permanent kernel at {100 * achieved / probe:.1f}% "
-        f"of it (instruction ceiling of Glynn at n={n}: {100 * (8 * n - 4) / (2 * (6 * n - 4)):.1f}%)")
+        f"of it (a kernel of one update and product per column and term could reach {100 * (8 * n - 4) / (2 * (6 * n - 4)):.1f}%)")
     mix = fp64_mix_probe()
     res["perm"]["fp64_matrix_core_probe"] = mix
     log(f"[bench] FP64 matrix cores: alone {mix['mfma']['mfma_tflops']:.1f} TFLOP/s; vector FMA alone "

@@ -204,7 +204,8 @@ int pcvl_slos_plan_create_masks(int m, const int32_t *h_in_occ, int nrows, const
  * holds count rows of m occupations.  Outputs are concatenated in input
  * order: input i occupies elements [h_out_offsets[i], h_out_offsets[i+1]) of
  * d_out (complex for COEFS, double for PROBS, FSArray order each).  The
- * workspace holds one layer per depth below the largest photon number. */
+ * workspace holds the layer of every node with children where these fit 1 GiB
+ * together, else one layer per depth below the largest photon number. */
 typedef struct pcvl_slos_tree_s *pcvl_slos_tree;
 int pcvl_slos_tree_create(int m, const int32_t *h_inputs, int count, pcvl_slos_tree *out);
 /* h_out_offsets receives count + 1 entries; any output pointer may be NULL. */
@@ -281,8 +282,8 @@ int pcvl_cc_samples_multi(const double *d_U, int m, const int32_t *h_inputs, con
  *   h_kind[p] = 1: fixed 2x2 unitary on modes (h_mode[p], h_mode[p]+1),
  *                  h_const[8p..8p+7] row-major interleaved complex.
  * h_targets: ntargets rows of m int32.  m <= 32, 1..8 photons, <= 512 targets
- * (run in blocks of 64 whose cofactors sit in LDS); -4 when the program,
- * index tables and target norms would take more than 160 KiB of LDS (a
+ * (a thread each, in whole passes); -4 when the program, index tables, target
+ * norms and cofactors of 64 targets would take more than 160 KiB of LDS (a
  * caller then splits the targets over several plans and adds the results).
  * Synchronises `stream`.
  * ------------------------------------------------------------------------- */

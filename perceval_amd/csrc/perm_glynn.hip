@@ -832,7 +832,9 @@ extern "C" int pcvl_perm_batch(const double *d_mats, const int32_t *h_n, const i
 // or streams) race.  Each call rewrites the whole block it uses, the queue
 // cursor included (zero), before its kernels read it.
 constexpr size_t PERM_SCRATCH_BYTES = size_t(16) << 20;
-static __device__ __align__(256) char scratch[PERM_SCRATCH_BYTES];
+// The groups of the queue come on top of the 16 MiB (at most 4 bytes per item of
+// 40), so that the limit does not depend on them.
+static __device__ __align__(256) char scratch[PERM_SCRATCH_BYTES + PERM_SCRATCH_BYTES / 8];
 
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[64] = {};
@@ -865,8 +867,8 @@ static int perm_batch_noalloc_impl(const double *d_mats, const int32_t *h_n, con
     std::vector<char> host;
     int rc = perm_plan_build(h_n, h_offsets, count, 0, 0, p, L, host);
     if (rc != OK) return rc;
-    if (L.total > PERM_SCRATCH_BYTES) {
-        set_error("permanent batch needs " + std::to_string(L.total) + " bytes of plan scratch, above the " +
+    if (L.o_groups > PERM_SCRATCH_BYTES) {
+        set_error("permanent batch needs " + std::to_string(L.o_groups) + " bytes of plan scratch, above the " +
                   std::to_string(PERM_SCRATCH_BYTES) + " of pcvl_perm_batch_noalloc (split the batch or use "
                   "pcvl_perm_batch)");
         return ERR_RANGE;

@@ -163,7 +163,7 @@ def mesh_adjoint(program: MeshProgram, phases, in_occ, targets, want_probs: bool
     Returns (loss (B,), grad (B, P)[, probs (B, T)]) as CUDA tensors, with
     loss = sum_s w_s P(s) over the targets (weights None: all w_s = 1), e.g.
     the expectation of a diagonal observable over every output state.  A
-    plan takes up to 512 targets (run in blocks of 64 inside the kernel);
+    plan takes up to 512 targets (a thread each inside the kernel);
     more, or a set whose tables do not fit the kernel's LDS (-4), are split
     over several plans, whose losses and gradients add (the gradient is
     linear in the targets).  The program keeps one MeshPlan per (input

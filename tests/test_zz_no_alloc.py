@@ -66,3 +66,28 @@ def test_noalloc_refuses_a_batch_beyond_its_scratch(gpu):
     from perceval_amd import _native
     assert b"scratch" in lib.pcvl_last_error()
     del _native
+
+
+def test_noalloc_limit_leaves_room_for_the_groups(gpu):
+    """Matrices of order 11 that fill the scratch array to 99.5% with items and
+    partial sums; the groups that waves take them in come on top."""
+    import torch
+    from perceval_amd import _native
+    lib = _lib()
+    n = 11
+    per = 24 + 16 + 8 + 3 * 4   # item, partial sum, index, slot and order
+    limit = lib.pcvl_perm_noalloc_max_bytes()
+    count = int(0.995 * limit) // per
+    g = torch.Generator(device="cuda").manual_seed(5)
+    d = torch.randn(count * n * n, 2, dtype=torch.float64, device="cuda", generator=g)
+    orders = np.full(count, n, dtype=np.int32)
+    offsets = np.arange(count, dtype=np.int64) * n * n
+    got = []
+    for name in ("pcvl_perm_batch", "pcvl_perm_batch_noalloc"):
+        out = torch.full((count,), complex(np.nan, np.nan), dtype=torch.complex128, device="cuda")
+        rc = getattr(lib, name)(_native.ptr(d), orders.ctypes.data_as(P(ctypes.c_int32)),
+                                offsets.ctypes.data_as(P(ctypes.c_int64)), count, _native.ptr(out),
+                                _native.stream_handle())
+        assert rc == 0, name
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.isfinite(torch.view_as_real(got[0])).all()
