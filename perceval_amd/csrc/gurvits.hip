@@ -255,20 +255,20 @@ __global__ void __launch_bounds__(64 * GURVITS_WAVES, NP <= 32 ? 3 : 1) gurvits_
 //
 // The signs are whole numbers, so y = A x can be formed exactly from the digits
 // of a fixed-point A on the int8 matrix cores, 64 times the rate of the FP64
-// ones.  Row i is scaled by a power of two to components below 1 and rounded to
-// 63 bits, a 2^63 = sum_s d_s 2^(13 s) with five balanced digits d_s, and
-// d_s = lo + 64 hi splits a digit into two int8: one v_mfma_i32_16x16x64_i8
-// per digit takes the lo parts against x = +-1 in its first 32 products and the
-// hi parts against +-64 in the other 32.  |sum d_s x| <= 2^17, so two digits
-// share an int32 and three conversions and FMAs make a component of y.  The
-// rounding of a row is 2^-64 of its largest component, a thousandth of what
-// the FP64 sum of the row rounds; components down to 2^-10 of it are exact.
-// Error of the means against long double sums over the same draws (16 Haar
-// submatrices, 10^5 draws): 4.2e-16, 4.8e-16, 9.2e-16 at orders 30, 21, 12,
-// where the FP64 products give 1.4e-15, 9.1e-16, 1.6e-15.
-// Matrices where it would show (a component below 2^-40 of its row's largest,
-// or one that is not finite) keep the FP64 products.
-//
+// ones.  Row i is scaled by a power of two to components below 1, and every
+// component is exactly a 2^77 = sum_s d_s 2^(13 s) with six balanced digits
+// d_s; d_s = lo + 64 hi splits a digit into two int8: one
+// v_mfma_i32_16x16x64_i8 per digit takes the lo parts against x = +-1 in its
+// first 32 products and the hi parts against +-64 in the other 32.  |sum d_s x|
+// <= 2^17, so two digits share an int32, and three conversions and FMAs make a
+// component of y: its last bit or two is all that is rounded, also where large
+// entries of a row cancel.  Matrices with a component below 2^-24 of its row's
+// largest (its 53 bits would not fit 2^-77 of it), or one that is not finite,
+// keep the FP64 products.
+// Error of the means against long double sums over the same draws (8 Haar
+// submatrices, 65,536 draws, relative to the mean size of a draw's product):
+// 9.8e-18, 9.4e-18, 1.5e-17 at orders 30, 21, 12, where the FP64 products give
+// 3.1e-17, 1.8e-17, 1.8e-17.
 // Operand slots: lane l and byte j of its 16 hold row (A) or sample (B) l % 16
 // and slot 16 (l / 16) + j; A and B pair equal slots, whatever k the
 // instruction gives them.  Slot t is column t % 32, lo part for t < 32, hi
@@ -276,7 +276,8 @@ __global__ void __launch_bounds__(64 * GURVITS_WAVES, NP <= 32 ? 3 : 1) gurvits_
 // block and sample l % 16.  A padding row (i >= n) is 1 in column n, whose sign
 // is always +1, so that it multiplies by y = 1.
 typedef int gv_i4 __attribute__((ext_vector_type(4)));
-constexpr int GURVITS_DIGITS = 5;
+constexpr int GURVITS_DIGITS = 6;   // of 13 bits: 2^77 a, |a| < 1
+constexpr int GURVITS_SPAN = 24;    // 2^-77 is the last bit of components down to 2^-24 of the row's largest
 // Rounds of waves that a call is cut into: each part is dispatched as its own
 // workgroup (64 matrices of order 30, 10^6 samples: 2.03 ms; 2.21 ms with four
 // rounds on resident waves, whose compute units do not run at one speed).
@@ -330,7 +331,7 @@ __global__ void __launch_bounds__(256) gurvits_digits_kernel(const cd *__restric
                 mn = fmin(mn, __shfl_xor(mn, o, 64));
                 bad |= __shfl_xor((int)bad, o, 64) != 0;
             }
-            bad |= mn < ldexp(mx, -40);
+            bad |= mn < ldexp(mx, -GURVITS_SPAN);
             if ((tid & 7) == 0) {
                 sexp[i] = bad || mx == 0.0 ? 0 : ilogb(mx) + 1;   // |components| 2^-e < 1
                 if (bad) sbad = 1;
@@ -354,10 +355,13 @@ __global__ void __launch_bounds__(256) gurvits_digits_kernel(const cd *__restric
                     int d = 0;
                     if (col < NP) {
                         const cd a = sA[row * NP + col];
-                        // below 2^63 in magnitude, as the component is below 1
-                        int64_t v = __double2ll_rn(ldexp(comp ? a.i : a.r, 63 - e));
+                        // a 2^(77 - e) = f 2^53 2^(ex + 24 - e), f's 53 bits shifted by 0..24 places
+                        int ex;
+                        const double f = frexp(comp ? a.i : a.r, &ex);
+                        const int64_t mant = (int64_t)ldexp(f, 53);
+                        __int128 v = mant == 0 ? (__int128)0 : (__int128)mant << (ex + GURVITS_SPAN - e);
                         for (int k = 0; k <= ds; k++) {   // balanced digits from the low end
-                            d = k < GURVITS_DIGITS - 1 ? (int)(((v & 8191) ^ 4096) - 4096) : (int)v;
+                            d = k < GURVITS_DIGITS - 1 ? (int)(((int64_t)v & 8191) ^ 4096) - 4096 : (int)v;
                             v = (v - d) >> 13;
                         }
                     }
@@ -374,7 +378,7 @@ __global__ void __launch_bounds__(256) gurvits_digits_kernel(const cd *__restric
 // One wave per (matrix, part), 64 samples' signs at a time, 16 samples per
 // product.  A's fragments stay in VGPRs.  Bound by the vector ALU (busy 88%;
 // the matrix cores 30%): the conversions and FMAs of each y component and the
-// product over rows.  64 matrices of order 30, 10^6 samples each, take 2.03 ms
+// product over rows.  64 matrices of order 30, 10^6 samples each, take 2.13 ms
 // (4.79 ms on the FP64 matrix cores).
 template <int NP>
 __global__ void __launch_bounds__(64, NP <= 16 ? 4 : 3) gurvits_int8_kernel(const gv_i4 *__restrict__ frags,
@@ -427,23 +431,27 @@ __global__ void __launch_bounds__(64, NP <= 16 ? 4 : 3) gurvits_int8_kernel(cons
                     asm("" : "+v"(up));   // or the byte mask becomes a quarter-rate multiplication by 255
                     x[w] = (int)(((up - one) & xflip) ^ xbase);
                 }
-                // y comes out as 2^11 times the scaled row's sum; the sign is
-                // prod_j x_j, in one of the sample's four lanes
-                const double start = RB == 2 ? 0x1p-88 : 0x1p-44;
+                // y comes out as 2^25 times the scaled row's sum, four or eight
+                // rows to a lane; the sign is prod_j x_j, in one of the
+                // sample's four lanes
+                const double start = RB == 2 ? 0x1p-200 : 0x1p-100;
                 cd p = {quad == 0 && (__builtin_popcount(bits) & 1) ? -start : start, 0.0};
 #pragma unroll
                 for (int rb = 0; rb < RB; rb++) {
                     double y[2][4];
 #pragma unroll
                     for (int c = 0; c < 2; c++) {
-                        gv_i4 d[ND];
+                        // a pair of digits at a time, the high one first
 #pragma unroll
-                        for (int s = 0; s < ND; s++)
-                            d[s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[rb][c][s], x, gv_i4{0, 0, 0, 0}, 0, 0, 0);
+                        for (int s = ND - 2; s >= 0; s -= 2) {
+                            const gv_i4 lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[rb][c][s], x, gv_i4{0, 0, 0, 0}, 0, 0, 0);
+                            const gv_i4 hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[rb][c][s + 1], x, gv_i4{0, 0, 0, 0}, 0, 0, 0);
+                            const double unit = s == 4 ? 1.0 : s == 2 ? 0x1p-26 : 0x1p-52;
 #pragma unroll
-                        for (int v = 0; v < 4; v++) {
-                            const int lo = (d[1][v] << 13) + d[0][v], mid = (d[3][v] << 13) + d[2][v];
-                            y[c][v] = fma((double)lo, 0x1p-52, fma((double)mid, 0x1p-26, (double)d[4][v]));
+                            for (int v = 0; v < 4; v++) {
+                                const double t = (double)((hi[v] << 13) + lo[v]);
+                                y[c][v] = s == ND - 2 ? t : fma(t, unit, y[c][v]);
+                            }
                         }
                     }
 #pragma unroll

@@ -117,3 +117,58 @@ def test_naive_approx_backend(gpu):
     assert len(probs) == 330 and abs(probs.sum() - 1.0) < 0.05
     assert approx.name == "NaiveApprox"
     _ = BS  # noqa: F841
+
+
+def _draws(seed, stream, iters):
+    """Signs' bits of the samples 0..iters-1 of a stream (the counter-based
+    generator of the kernels)."""
+    def mix(x):
+        x = x + np.uint64(0x9E3779B97F4A7C15)
+        x = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        x = (x ^ (x >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        return x ^ (x >> np.uint64(31))
+    with np.errstate(over="ignore"):
+        key = mix(np.uint64(seed) ^ mix(np.uint64(stream)))
+        return mix(key + np.arange(iters, dtype=np.uint64) * np.uint64(0x9E3779B97F4A7C15))
+
+
+@pytest.mark.parametrize("n", [10, 16, 21, 32])
+def test_gurvits_cancelling_rows_are_exact(gpu, n):
+    """Rows whose large entries cancel before weak couplings are added: two rows
+    (a, a, w...) and (a, -a, w...) leave the sum of the weak ones in every draw.
+    Every operand is held in full, so the mean is within 4 n roundings of the
+    terms (a row sum's last bits and a complex product each) and the 100 of the
+    longest chain of additions of terms from the long double
+    mean over the same draws, whether a matrix takes the integer products
+    (couplings down to 2^-24 of the pair) or the FP64 ones (below)."""
+    from perceval_amd.permanent import gurvits
+    rng = np.random.RandomState(n)
+    powers = (12, 20, 23, 27, 36)
+    mats = []
+    for k in powers:
+        M = (rng.randn(n, n) + 1j * rng.randn(n, n)) / np.sqrt(n)
+        phase = np.exp(2j * np.pi * rng.rand(2, n)) * (1.0 + rng.rand(2, n))
+        M[:2] = phase * 2.0 ** -k
+        M[0, :2] = rng.randn() + 1j * rng.randn()
+        M[1, :2] = M[0, 0], -M[0, 0]
+        mats.append(M)
+    iters, seed = (1 << 16) + 5, 3
+    est, _ = gurvits(mats + [mats[0]] * 59, iters, seed=seed)   # long enough for the integer products
+    for b, (k, M) in enumerate(zip(powers, mats)):
+        bits = _draws(seed, b, iters)
+        tot, size = np.clongdouble(0), np.longdouble(0)
+        A = M.astype(np.clongdouble)
+        for s0 in range(0, iters, 1 << 16):
+            part = bits[s0:s0 + (1 << 16)]
+            x = 1 - 2 * ((part[:, None] >> np.arange(n, dtype=np.uint64)) & np.uint64(1)).astype(np.longdouble)
+            term = x.prod(axis=1).astype(np.clongdouble)
+            for i in range(n):
+                y = np.zeros(len(part), dtype=np.clongdouble)
+                for j in range(n):
+                    y += x[:, j] * A[i, j]
+                term *= y
+            tot += term.sum()
+            size += np.abs(term).sum()
+        rel = abs(est[b] - tot / iters) / (size / iters)
+        _say(f"order {n}, couplings 2^-{k}: {float(rel):.2e}")
+        assert rel <= (4 * n + 100) * 2.0 ** -53, (n, k, rel)
