@@ -282,10 +282,21 @@ constexpr int GURVITS_SPAN = 24;    // 2^-77 is the last bit of components down 
 // workgroup (64 matrices of order 30, 10^6 samples: 2.03 ms; 2.21 ms with four
 // rounds on resident waves, whose compute units do not run at one speed).
 constexpr int GURVITS_ROUNDS = 8;
-// Samples of a call from which the integer products pay for their two more
-// launches (about 20 us): at orders 17..32 2.1M samples take 276 against 344
-// us, at orders 9..16 4.2M samples save 35 us.
-constexpr int64_t gurvits_int8_min(int nmax) { return nmax <= 16 ? int64_t(1) << 22 : int64_t(1) << 21; }
+// Fragments kept at a time (10,922 matrices of orders up to 16, 5,461 above): a
+// call's workspace does not grow with its matrices beyond this.
+constexpr size_t GURVITS_CHUNK_BYTES = size_t(128) << 20;
+// The integer products pay for their two more launches (about 30 us) and for a
+// matrix's digits and fragments from so many samples of a call and of a matrix
+// on.  FP64 -> integer products, us, at orders 17..32: 64 matrices, 2^20 samples
+// in all 126 -> 105, 2^21 201 -> 133; 20,000 matrices of 209 samples 532 -> 614,
+// of 419 825 -> 770, of 838 1,442 -> 1,081.  At orders 9..16: 64 matrices, 2^21
+// samples 104 -> 106, 2^22 164 -> 148; 20,000 matrices of 419 samples 351 -> 390,
+// of 838 566 -> 558; 2,000 of 2,097 174 -> 171.
+constexpr bool gurvits_int8_pays(int nmax, int64_t count, int64_t iters)
+{
+    return nmax <= 16 ? iters >= 1024 && (double)count * (double)iters >= 0x1p22
+                      : iters >= 512 && (double)count * (double)iters >= 0x1p21;
+}
 
 // Fragments of one matrix: [row block][component][digit][lane].
 constexpr int gurvits_frags(int np) { return np / 16 * 2 * GURVITS_DIGITS * 64; }
@@ -293,17 +304,17 @@ constexpr int gurvits_frags(int np) { return np / 16 * 2 * GURVITS_DIGITS * 64; 
 template <int NP>
 __global__ void __launch_bounds__(256) gurvits_digits_kernel(const cd *__restrict__ mats,
                                                              const GurvitsItem *__restrict__ items, int64_t count,
-                                                             gv_i4 *__restrict__ frags, int32_t *__restrict__ scale)
+                                                             int split, gv_i4 *__restrict__ frags,
+                                                             int32_t *__restrict__ scale)
 {
     __shared__ cd sA[NP * NP];
     __shared__ int sexp[NP];
     __shared__ int sbad;
     const int tid = threadIdx.x;
-    // one block per (matrix, row block, component)
-    constexpr int RC = NP / 16 * 2, PER = gurvits_frags(NP) / RC;
-    for (int64_t w = blockIdx.x; w < count * RC; w += gridDim.x) {
-        const int64_t b = w / RC;
-        const int rc = (int)(w % RC);
+    constexpr int RC = NP / 16 * 2, PER = gurvits_frags(NP) / RC;   // row blocks x components
+    for (int64_t w = blockIdx.x; w < count * split; w += gridDim.x) {
+        const int64_t b = w / split;
+        const int rc0 = (int)(w % split);
         const int n = items[b].n;
         const int64_t off = items[b].off;
         if (tid == 0) sbad = 0;
@@ -338,37 +349,39 @@ __global__ void __launch_bounds__(256) gurvits_digits_kernel(const cd *__restric
             }
         }
         __syncthreads();
-        if (tid == 0 && rc == 0) {
+        if (tid == 0 && rc0 == 0) {
             int E = 0;
             for (int i = 0; i < n; i++) E += sexp[i];
             for (int i = n; i < NP; i++) E += sexp[i];   // padding rows: 2^-1 each against an exponent of 1
             scale[b] = sbad ? GURVITS_FP64 : E;
         }
         if (!sbad) {
-            for (int f = tid; f < PER; f += 256) {
-                const int lane = f & 63, ds = f >> 6;
-                const int comp = rc & 1, row = 16 * (rc >> 1) + (lane & 15), g = lane >> 4;
-                const int e = sexp[row];
-                union { gv_i4 v; int8_t b[16]; } u;
-                for (int j = 0; j < 16; j++) {
-                    const int col = (16 * g + j) & 31;
-                    int d = 0;
-                    if (col < NP) {
-                        const cd a = sA[row * NP + col];
-                        // a 2^(77 - e) = f 2^53 2^(ex + 24 - e), f's 53 bits shifted by 0..24 places
-                        int ex;
-                        const double f = frexp(comp ? a.i : a.r, &ex);
-                        const int64_t mant = (int64_t)ldexp(f, 53);
-                        __int128 v = mant == 0 ? (__int128)0 : (__int128)mant << (ex + GURVITS_SPAN - e);
-                        for (int k = 0; k <= ds; k++) {   // balanced digits from the low end
-                            d = k < GURVITS_DIGITS - 1 ? (int)(((int64_t)v & 8191) ^ 4096) - 4096 : (int)v;
-                            v = (v - d) >> 13;
-                        }
+            // thread: dword d4 of lane f's 16 bytes, every digit of its four columns
+            const int f = tid >> 2, d4 = tid & 3, g = f >> 4;
+            for (int rc = rc0; rc < RC; rc += split) {
+                const int comp = rc & 1, row = 16 * (rc >> 1) + (f & 15), e = sexp[row];
+                uint32_t word[GURVITS_DIGITS] = {};
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int col = (16 * g + 4 * d4 + j) & 31;
+                    if (col >= NP) continue;
+                    const cd a = sA[row * NP + col];
+                    // a 2^(77 - e) = f 2^53 2^(ex + 24 - e), f's 53 bits shifted by 0..24 places
+                    int ex;
+                    const double fr = frexp(comp ? a.i : a.r, &ex);
+                    const int64_t mant = (int64_t)ldexp(fr, 53);
+                    __int128 v = mant == 0 ? (__int128)0 : (__int128)mant << (ex + GURVITS_SPAN - e);
+#pragma unroll
+                    for (int k = 0; k < GURVITS_DIGITS; k++) {   // balanced digits from the low end
+                        const int d = k < GURVITS_DIGITS - 1 ? (int)(((int64_t)v & 8191) ^ 4096) - 4096 : (int)v;
+                        v = (v - d) >> 13;
+                        const int hi = (d + 32) >> 6;
+                        word[k] |= (uint32_t)(uint8_t)(g >= 2 ? hi : d - 64 * hi) << (8 * j);
                     }
-                    const int hi = (d + 32) >> 6;
-                    u.b[j] = (int8_t)(g >= 2 ? hi : d - 64 * hi);
                 }
-                frags[w * PER + f] = u.v;
+                uint32_t *dst = reinterpret_cast<uint32_t *>(frags + (b * RC + rc) * PER);
+#pragma unroll
+                for (int k = 0; k < GURVITS_DIGITS; k++) dst[(k * 64 + f) * 4 + d4] = word[k];
             }
         }
         __syncthreads();
@@ -486,22 +499,24 @@ __global__ void __launch_bounds__(64, NP <= 16 ? 4 : 3) gurvits_int8_kernel(cons
 
 // scale: powers of two of the matrices' rows that the sums leave out (NULL or
 // GURVITS_FP64: none).
-__global__ void gurvits_finalize_kernel(const double *__restrict__ partial, int64_t count, int parts, int64_t iters,
+// lanes: 64 a matrix, or one where it has few parts (200,000 matrices of order 12
+// and one part: 1,021 -> 956 us a call).
+__global__ void gurvits_finalize_kernel(const double *__restrict__ partial, int64_t count, int parts, int lanes,
+                                        int64_t iters,
                                         const int32_t *__restrict__ scale, cd *__restrict__ est,
                                         double *__restrict__ err)
 {
-    const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // one wave per matrix
-    const int lane = threadIdx.x & 63;
+    const int64_t b = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / lanes;
+    const int lane = threadIdx.x & (lanes - 1);
     if (b >= count) return;
     double sr = 0.0, si = 0.0, sq = 0.0;
-    for (int q = lane; q < parts; q += 64) {
+    for (int q = lane; q < parts; q += lanes) {
         const double *pp = partial + 3 * (b * parts + q);
         sr += pp[0];
         si += pp[1];
         sq += pp[2];
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
+    for (int o = lanes >> 1; o >= 1; o >>= 1) {
         sr += __shfl_xor(sr, o, 64);
         si += __shfl_xor(si, o, 64);
         sq += __shfl_xor(sq, o, 64);
@@ -541,21 +556,38 @@ static int launch_gurvits(const cd *mats, const GurvitsItem *items, int64_t coun
     return OK;
 }
 
-// Integer products: digits of every matrix, the int8 kernel, and the FP64
-// kernel for the matrices that keep it (usually none: its waves leave at once).
+// Integer products of a chunk of matrices: their digits, the int8 kernel, and
+// the FP64 kernel for those that keep it (usually none: its waves leave at
+// once).
 template <int NP>
 static int launch_gurvits_int8(const cd *mats, const GurvitsItem *items, int64_t count, int parts, int64_t iters,
                                int64_t per, uint64_t seed, uint64_t stream0, double *partial, gv_i4 *frags,
                                int32_t *scale, int cus, hipStream_t st)
 {
-    hipLaunchKernelGGL((gurvits_digits_kernel<NP>), dim3((unsigned)std::min<int64_t>(count * (NP / 8), (int64_t)cus * 8)),
-                       dim3(256), 0, st, mats, items, count, frags, scale);
+    // a workgroup per row block and component while matrices alone are few
+    const int split = count < 4 * (int64_t)cus ? NP / 8 : 1;
+    hipLaunchKernelGGL((gurvits_digits_kernel<NP>), dim3((unsigned)std::min<int64_t>(count * split, (int64_t)cus * 8)),
+                       dim3(256), 0, st, mats, items, count, split, frags, scale);
     PCVL_HIP_CHECK(hipGetLastError());
-    const unsigned grid = (unsigned)std::min<int64_t>(count * parts, int64_t(1) << 30);
-    hipLaunchKernelGGL((gurvits_int8_kernel<NP>), dim3(grid), dim3(64), 0, st, frags, items, count, parts, iters, per,
-                       seed, stream0, partial, scale);
+    hipLaunchKernelGGL((gurvits_int8_kernel<NP>), dim3((unsigned)(count * parts)), dim3(64), 0, st, frags, items, count,
+                       parts, iters, per, seed, stream0, partial, scale);
     PCVL_HIP_CHECK(hipGetLastError());
     return launch_gurvits<NP>(mats, items, count, parts, iters, per, seed, stream0, partial, scale, st);
+}
+
+// The same for a call's matrices, GURVITS_CHUNK_BYTES of fragments at a time.
+template <int NP>
+static int launch_gurvits_chunks(const cd *mats, const GurvitsItem *items, int64_t count, int parts, int64_t iters,
+                                 int64_t per, uint64_t seed, uint64_t stream0, double *partial, gv_i4 *frags,
+                                 int32_t *scale, int64_t chunk, int cus, hipStream_t st)
+{
+    for (int64_t c0 = 0; c0 < count; c0 += chunk) {
+        const int rc = launch_gurvits_int8<NP>(mats, items + c0, std::min(chunk, count - c0), parts, iters, per, seed,
+                                               stream0 + (uint64_t)c0, partial + 3 * c0 * parts, frags, scale + c0, cus,
+                                               st);
+        if (rc != OK) return rc;
+    }
+    return OK;
 }
 
 // Parts of a matrix for the integer kernel: equal rounds of the resident
@@ -594,14 +626,15 @@ extern "C" int pcvl_gurvits_batch(const double *d_mats, const int32_t *h_n, cons
     PCVL_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     // Integer products for orders 9..32 (orders up to 8 take the vector kernel,
     // above 32 a digit's two halves do not fit the 64 products of an instruction)
-    const bool int8 = nmax > 8 && nmax <= 32 && count <= INT32_MAX &&
-                      (double)count * (double)iters >= (double)gurvits_int8_min(nmax);
+    const bool int8 = nmax > 8 && nmax <= 32 && count <= INT32_MAX && gurvits_int8_pays(nmax, count, iters);
     // samples of a matrix are split into parts of at least 64 * 16 samples so
     // that the batch fills the device (4 waves per SIMD of 256 CUs)
     int parts = (int)std::max<int64_t>(1, std::min<int64_t>((4096 + count - 1) / count, iters / 1024));
+    const size_t frag = sizeof(gv_i4) * (size_t)gurvits_frags(nmax <= 16 ? 16 : 32);
+    const int64_t chunk = std::min<int64_t>(count, (int64_t)(GURVITS_CHUNK_BYTES / frag));
     if (int8) {
-        int rc = nmax <= 16 ? gurvits_int8_parts<16>(count, iters, cus, &parts)
-                            : gurvits_int8_parts<32>(count, iters, cus, &parts);
+        int rc = nmax <= 16 ? gurvits_int8_parts<16>(chunk, iters, cus, &parts)
+                            : gurvits_int8_parts<32>(chunk, iters, cus, &parts);
         if (rc != OK) return rc;
     }
     const int64_t per = (iters + parts - 1) / parts;
@@ -610,7 +643,7 @@ extern "C" int pcvl_gurvits_batch(const double *d_mats, const int32_t *h_n, cons
     const size_t b_items = al(sizeof(GurvitsItem) * items.size());
     const size_t b_part = al(sizeof(double) * 3 * (size_t)count * parts);
     const size_t b_scale = int8 ? al(sizeof(int32_t) * (size_t)count) : 0;
-    const size_t b_frag = int8 ? sizeof(gv_i4) * (size_t)gurvits_frags(nmax <= 16 ? 16 : 32) * (size_t)count : 0;
+    const size_t b_frag = int8 ? frag * (size_t)chunk : 0;
     char *blk = nullptr;
     PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk), b_items + b_part + b_scale + b_frag, stream));
     GurvitsItem *d_items = reinterpret_cast<GurvitsItem *>(blk);
@@ -626,9 +659,9 @@ extern "C" int pcvl_gurvits_batch(const double *d_mats, const int32_t *h_n, cons
     } else {
         const cd *mats = reinterpret_cast<const cd *>(d_mats);
         if (int8 && nmax <= 16)
-            rc = launch_gurvits_int8<16>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, d_frag, d_scale, cus, stream);
+            rc = launch_gurvits_chunks<16>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, d_frag, d_scale, chunk, cus, stream);
         else if (int8)
-            rc = launch_gurvits_int8<32>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, d_frag, d_scale, cus, stream);
+            rc = launch_gurvits_chunks<32>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, d_frag, d_scale, chunk, cus, stream);
         else if (nmax <= 8)
             rc = launch_gurvits<8>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, nullptr, stream);
         else if (nmax <= 16)
@@ -638,8 +671,9 @@ extern "C" int pcvl_gurvits_batch(const double *d_mats, const int32_t *h_n, cons
         else
             rc = launch_gurvits<48>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, nullptr, stream);
         if (rc == OK) {
-            hipLaunchKernelGGL(gurvits_finalize_kernel, dim3((unsigned)((count + 3) / 4)), dim3(256), 0, stream,
-                               d_part, count, parts, iters, d_scale, reinterpret_cast<cd *>(d_est), d_err);
+            const int lanes = parts < 16 ? 1 : 64;
+            hipLaunchKernelGGL(gurvits_finalize_kernel, dim3((unsigned)((count * lanes + 255) / 256)), dim3(256), 0, stream,
+                               d_part, count, parts, lanes, iters, d_scale, reinterpret_cast<cd *>(d_est), d_err);
             e = hipGetLastError();
             if (e != hipSuccess) { set_error(std::string("gurvits finalize: ") + hipGetErrorString(e)); rc = ERR_HIP; }
         }

@@ -172,3 +172,26 @@ def test_gurvits_cancelling_rows_are_exact(gpu, n):
         rel = abs(est[b] - tot / iters) / (size / iters)
         _say(f"order {n}, couplings 2^-{k}: {float(rel):.2e}")
         assert rel <= (4 * n + 100) * 2.0 ** -53, (n, k, rel)
+
+
+def test_gurvits_many_matrices_in_chunks(gpu):
+    """More matrices than the fragments of one chunk: the ones around its end and
+    one that keeps the FP64 products in the second chunk, against the oracle as
+    in test_gurvits_batch_vs_oracle; and a call of few draws per matrix, which
+    takes the FP64 products throughout, draws the same samples."""
+    from perceval_amd.permanent import gurvits
+    rng = np.random.RandomState(2)
+    n, count, iters = 17, 5600, 700
+    base = (rng.randn(40, n, n) + 1j * rng.randn(40, n, n)) / np.sqrt(n)
+    mats = [base[b % 40] for b in range(count)]
+    mats[5500] = mats[5500].copy()
+    mats[5500][2, 3] = 2.0 ** -50
+    check = [0, 1, 5459, 5460, 5461, 5462, 5500, count - 1]
+    est, err = gurvits(mats, iters, seed=4, stream0=9)
+    few, _ = gurvits([mats[b] for b in check[:2]], iters, seed=4, stream0=9)
+    assert np.max(np.abs(few - est[:2]) / np.abs(est[:2])) < 1e-11
+    for b in check:
+        ref_est, ref_err = oracle.gurvits(mats[b], iters, seed=4, stream=9 + b)
+        scale = max(ref_err * np.sqrt(iters) / 2.5758293035489004, abs(ref_est))
+        assert abs(est[b] - ref_est) <= 1e-11 * scale, (b, est[b], ref_est)
+        assert abs(err[b] - ref_err) <= 1e-6 * ref_err, (b, err[b], ref_err)
