@@ -41,7 +41,7 @@ struct MeshOp {
     int32_t kind;    // 0: phase shifter on mode q; 1: fixed 2x2 block on (q, q+1)
     int32_t q;
     int32_t param;   // phase index (kind 0), -1 for a constant phase
-    int32_t grad;    // whether this op writes its phase's gradient
+    int32_t grad;    // 0: no phase of its own; 1: the only op of its phase; 2: one of several
     double c[8];     // kind 0: c[0] = constant phase; kind 1: 2x2 block row-major (re, im)
 };
 
@@ -160,6 +160,7 @@ struct AdjIdx {
     int nparts; // partial sums of G: threads (part, j, i)
     int pass;   // targets per pass (a multiple of sub, or all of them)
     int block;  // targets whose cofactors are in LDS at once (a multiple of sub)
+    int nshared; // phases that several ops use
 };
 
 // Dynamic LDS of the kernel, in order (byte offsets rounded to 16): the mesh
@@ -219,17 +220,19 @@ __device__ __forceinline__ void adj_cell_matrix(const MeshOp *ops, const int32_t
 }
 
 // Gradients of cell c's phases from W's block B (rows and columns of the
-// cell's modes) after the cell: through the ops in reverse, a phase's is
-// -2 Im B_aa on its mode a, and B <- L^H B L.
+// cell's modes) after the cell: through the ops in reverse, a phase shifter's is
+// -2 Im B_aa on its mode a (to sink, with its op), and B <- L^H B L.  A phase's
+// gradient is the sum over its shifters.
+template <class Sink>
 __device__ __forceinline__ void adj_cell_grads(const MeshOp *ops, const int32_t *cell, const cd *zph, int c, cd (&B)[4],
-                                               double *grad)
+                                               Sink sink)
 {
     const int e0 = cell[c] >> 6, e1 = cell[c + 1] >> 6, q = cell[c] & 31;
     for (int e = e1 - 1; e >= e0; e--) {
         const MeshOp &op = ops[e];
         if (op.kind == 0) {
             const bool first = op.q == q;
-            if (op.grad) grad[op.param] = -2.0 * (first ? B[0].i : B[3].i);
+            if (op.grad) sink(op, -2.0 * (first ? B[0].i : B[3].i));
             const cd z = op.param >= 0 ? zph[op.param] : cexpi(op.c[0]);
             if (first) { B[1] = cmul(cconj(z), B[1]); B[2] = cmul(B[2], z); }
             else { B[1] = cmul(B[1], z); B[2] = cmul(cconj(z), B[2]); }
@@ -336,8 +339,8 @@ __device__ __forceinline__ void adj_targets(const AdjIdx &X, int m, int ntargets
 template <int N, bool STAGE, bool KEEP>
 __global__ void __launch_bounds__(ADJ_THREADS) mesh_adjoint_kernel(
     const MeshOp *__restrict__ ops_g, int nops, int m, const double *__restrict__ phases, int nparams, int nsets,
-    const int32_t *__restrict__ idx_g, AdjIdx X, const double *__restrict__ tn_g, const double *__restrict__ tw_g,
-    int ntargets, int grouped, double *__restrict__ loss_out, double *__restrict__ grad_out,
+    const int32_t *__restrict__ idx_g, AdjIdx X, const int32_t *__restrict__ shared_g,
+    const double *__restrict__ tn_g, const double *__restrict__ tw_g, int ntargets, int grouped, double *__restrict__ loss_out, double *__restrict__ grad_out,
     double *__restrict__ probs_out)
 {
     extern __shared__ uint64_t s_adj[];
@@ -470,7 +473,24 @@ __global__ void __launch_bounds__(ADJ_THREADS) mesh_adjoint_kernel(
                                         B[2] = W[(q + 1) * ld + q];
                                         B[3] = W[(q + 1) * ld + q + 1];
                                     }
-                                    adj_cell_grads(ops(), cell, zph, c, B, grad);
+                                    adj_cell_grads(ops(), cell, zph, c, B, [&](const MeshOp &op, double v) {
+                                        if (op.grad == 1) grad[op.param] = v;
+                                    });
+                                }
+                                // phases of several shifters: one cell after another
+                                for (int s = 0; X.nshared && s < slots; s++) {
+                                    if (slot == s && col == 0) {
+                                        cd B[4] = {W[q * ld + q], {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
+                                        if (two) {
+                                            B[1] = W[q * ld + q + 1];
+                                            B[2] = W[(q + 1) * ld + q];
+                                            B[3] = W[(q + 1) * ld + q + 1];
+                                        }
+                                        adj_cell_grads(ops(), cell, zph, c, B, [&](const MeshOp &op, double v) {
+                                            if (op.grad == 2) grad[op.param] += v;
+                                        });
+                                    }
+                                    __threadfence_block();
                                 }
                             }
                             cd b0 = {0.0, 0.0}, b1 = {0.0, 0.0};
@@ -505,7 +525,25 @@ __global__ void __launch_bounds__(ADJ_THREADS) mesh_adjoint_kernel(
                 cd B[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) B[k] = cells[4 * (X.ncells + c) + k];
-                adj_cell_grads(ops(), cell, zph, c, B, grad);
+                adj_cell_grads(ops(), cell, zph, c, B, [&](const MeshOp &op, double v) {
+                    if (op.grad == 1) grad[op.param] = v;
+                });
+            }
+            // phases of several shifters, a thread each over the cells that hold
+            // them: start[nshared + 1] | phase[nshared] | cells
+            for (int s = tid; s < X.nshared; s += ADJ_THREADS) {
+                const int32_t prm = shared_g[X.nshared + 1 + s];
+                double sum = 0.0;
+                for (int u = shared_g[s]; u < shared_g[s + 1]; u++) {
+                    const int c = shared_g[u];
+                    cd B[4];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) B[k] = cells[4 * (X.ncells + c) + k];
+                    adj_cell_grads(ops(), cell, zph, c, B, [&](const MeshOp &op, double v) {
+                        if (op.param == prm) sum += v;
+                    });
+                }
+                grad[prm] = sum;
             }
         }
         __syncthreads();   // U, W, zph and the cells are rewritten by the next set
@@ -521,9 +559,10 @@ struct pcvl_mesh_plan_s {
     AdjIdx X{};
     bool stage_ops = false, keep_cells = false, grouped = false;
     size_t lds = 0;
-    char *d_blk = nullptr;            // program, index tables, target norms
+    char *d_blk = nullptr;            // program, index tables, target norms and weights, shared phases
     const MeshOp *d_ops = nullptr;
     const int32_t *d_idx = nullptr;
+    const int32_t *d_shared = nullptr;   // phases of several shifters
     const double *d_tn = nullptr;
     double *d_tw = nullptr;           // per-target weights of the loss (ones unless set)
     int grid_cap = 0;
@@ -575,24 +614,19 @@ extern "C" int pcvl_mesh_plan_create(const int32_t *h_kind, const int32_t *h_mod
         PCVL_ARG_CHECK(ns == n, "target photon number differs from the input's");
         tnorm[s] = 1.0 / sqrt(ps * pin);
     }
-    // The gradient of a phase that several ops share is the share of the first
-    // of them in level order, an op's level being one above the last op on any
-    // of its modes (the last one listed where they tie).
-    int oplev = 0;   // levels of single ops
+    std::vector<int> uses((size_t)nparams, 0);   // shifters of each phase
+    for (const MeshOp &o : ops)
+        if (o.kind == 0 && o.param >= 0) uses[(size_t)o.param]++;
+    for (MeshOp &o : ops)
+        if (o.kind == 0 && o.param >= 0) o.grad = uses[(size_t)o.param] == 1 ? 1 : 2;
+    int oplev = 0;   // levels of single ops: one above the last op on any of its modes
     {
-        std::vector<int> on((size_t)m, 0), best((size_t)nparams, -1), at((size_t)nparams, 0);
-        for (int p = 0; p < nops; p++) {
-            const int q = ops[p].q, q2 = ops[p].kind == 1 ? q + 1 : q;
-            const int lv = std::max(on[(size_t)q], on[(size_t)q2]);
-            on[(size_t)q] = on[(size_t)q2] = lv + 1;
-            oplev = std::max(oplev, lv + 1);
-            const int prm = ops[p].kind == 0 ? ops[p].param : -1;
-            if (prm >= 0 && (best[(size_t)prm] < 0 || lv <= at[(size_t)prm])) {
-                if (best[(size_t)prm] >= 0) ops[(size_t)best[(size_t)prm]].grad = 0;
-                best[(size_t)prm] = p;
-                at[(size_t)prm] = lv;
-                ops[p].grad = 1;
-            }
+        std::vector<int> on((size_t)m, 0);
+        for (const MeshOp &o : ops) {
+            const int q2 = o.kind == 1 ? o.q + 1 : o.q;
+            const int lv = std::max(on[(size_t)o.q], on[(size_t)q2]) + 1;
+            on[(size_t)o.q] = on[(size_t)q2] = lv;
+            oplev = std::max(oplev, lv);
         }
     }
     // The size that a plan may have: U and Z, every phase, 64 targets'
@@ -648,7 +682,7 @@ extern "C" int pcvl_mesh_plan_create(const int32_t *h_kind, const int32_t *h_mod
     X.glog = 0;
     while ((1 << X.glog) < m) X.glog++;
     std::vector<int32_t> idx;
-    X.cell = (int)idx.size();
+    X.cell = (int)idx.size();   // 0
     std::vector<MeshOp> sorted;   // the program cell by cell
     sorted.reserve(ops.size());
     std::vector<int32_t> lstart((size_t)nlev + 1, 0);
@@ -659,6 +693,32 @@ extern "C" int pcvl_mesh_plan_create(const int32_t *h_kind, const int32_t *h_mod
     }
     idx.push_back((int32_t)sorted.size() << 6);
     ops.swap(sorted);
+    // phases of several shifters and the cells that hold them, in order
+    std::vector<int32_t> shared;
+    {
+        std::vector<int32_t> prms, at((size_t)nparams, -1);
+        for (int prm = 0; prm < nparams; prm++)
+            if (uses[(size_t)prm] > 1) {
+                at[(size_t)prm] = (int32_t)prms.size();
+                prms.push_back(prm);
+            }
+        std::vector<std::vector<int32_t>> held(prms.size());
+        for (int c = 0; c < X.ncells; c++)
+            for (int e = idx[(size_t)c] >> 6; e < idx[(size_t)c + 1] >> 6; e++) {
+                if (ops[(size_t)e].grad != 2) continue;
+                std::vector<int32_t> &h = held[(size_t)at[(size_t)ops[(size_t)e].param]];
+                if (h.empty() || h.back() != c) h.push_back(c);
+            }
+        X.nshared = (int)prms.size();
+        int32_t first = 2 * X.nshared + 1;
+        for (const auto &h : held) {
+            shared.push_back(first);
+            first += (int32_t)h.size();
+        }
+        shared.push_back(first);
+        shared.insert(shared.end(), prms.begin(), prms.end());
+        for (const auto &h : held) shared.insert(shared.end(), h.begin(), h.end());
+    }
     for (int lv = 0; lv < nlev; lv++) lstart[(size_t)lv + 1] += lstart[(size_t)lv];
     X.lstart = (int)idx.size();
     idx.insert(idx.end(), lstart.begin(), lstart.end());
@@ -755,7 +815,8 @@ extern "C" int pcvl_mesh_plan_create(const int32_t *h_kind, const int32_t *h_mod
     // one device block: program, index tables, norms
     const size_t b_ops = adj_al16(sizeof(MeshOp) * std::max(1, nops));
     const size_t b_idx = adj_al16(sizeof(int32_t) * idx.size()), b_n = adj_al16(sizeof(double) * ntargets);
-    hipError_t e = hipMalloc((void **)&plan->d_blk, b_ops + b_idx + 2 * b_n);
+    const size_t b_shared = X.nshared ? adj_al16(sizeof(int32_t) * shared.size()) : 0;
+    hipError_t e = hipMalloc((void **)&plan->d_blk, b_ops + b_idx + 2 * b_n + b_shared);
     if (e != hipSuccess) {
         delete plan;
         set_error(std::string("hipMalloc(mesh plan): ") + hipGetErrorString(e));
@@ -765,12 +826,16 @@ extern "C" int pcvl_mesh_plan_create(const int32_t *h_kind, const int32_t *h_mod
     plan->d_idx = reinterpret_cast<const int32_t *>(plan->d_blk + b_ops);
     plan->d_tn = reinterpret_cast<const double *>(plan->d_blk + b_ops + b_idx);
     plan->d_tw = reinterpret_cast<double *>(plan->d_blk + b_ops + b_idx + b_n);
+    plan->d_shared = reinterpret_cast<const int32_t *>(plan->d_blk + b_ops + b_idx + 2 * b_n);
     const std::vector<double> ones((size_t)ntargets, 1.0);
     if (nops) e = hipMemcpy(plan->d_blk, ops.data(), sizeof(MeshOp) * nops, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(plan->d_blk + b_ops, idx.data(), sizeof(int32_t) * idx.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(plan->d_blk + b_ops + b_idx, tnorm.data(), sizeof(double) * ntargets,
                                        hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(plan->d_tw, ones.data(), sizeof(double) * ntargets, hipMemcpyHostToDevice);
+    if (e == hipSuccess && b_shared)
+        e = hipMemcpy(plan->d_blk + b_ops + b_idx + 2 * b_n, shared.data(), sizeof(int32_t) * shared.size(),
+                      hipMemcpyHostToDevice);
     int dev = 0, cus = 0;
     if (e == hipSuccess) e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -797,7 +862,7 @@ static int launch_mesh(const pcvl_mesh_plan_s &P, const double *d_phases, int ns
         auto kp = P.stage_ops ? (P.keep_cells ? mesh_adjoint_kernel<N, true, true> : mesh_adjoint_kernel<N, true, false>)
                               : (P.keep_cells ? mesh_adjoint_kernel<N, false, true> : mesh_adjoint_kernel<N, false, false>);
         hipLaunchKernelGGL(kp, dim3(std::min(nsets, P.grid_cap)), dim3(ADJ_THREADS), P.lds, stream, P.d_ops, P.nops,
-                           P.m, d_phases, P.nparams, nsets, P.d_idx, P.X, P.d_tn, P.d_tw, P.ntargets,
+                           P.m, d_phases, P.nparams, nsets, P.d_idx, P.X, P.d_shared, P.d_tn, P.d_tw, P.ntargets,
                            P.grouped ? 1 : 0, d_loss, d_grad, d_probs);
         PCVL_HIP_CHECK(hipGetLastError());
         return OK;

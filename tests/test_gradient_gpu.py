@@ -307,3 +307,35 @@ def test_cells_passes_and_blocks_vs_torch(gpu, kind, m, n, T):
     tol = 1e4 * 2.0 ** -53 * max(1.0, np.abs(weights).sum())
     assert np.max(np.abs(loss.cpu().numpy() - ref_l)) < tol
     assert np.max(np.abs(grad.cpu().numpy() - ref_g)) < tol * max(1.0, np.abs(ref_g).max())
+
+
+@pytest.mark.parametrize("cells", [6, 1500])
+def test_phase_of_several_shifters_vs_torch(gpu, cells):
+    """A phase's gradient is the sum over its shifters: twice in one cell, in
+    cells of one level and of several, on a mode that no splitter touches, and in
+    a program of so many cells that their gradients are formed in the sweep.
+    The bar is the one of test_cells_passes_and_blocks_vs_torch."""
+    from perceval_amd.components import BS, PS, Circuit, Parameter
+    from perceval_amd.gradient import MeshProgram, mesh_adjoint
+    rng = np.random.RandomState(cells)
+    m, n = 6, 3
+    shared = [Parameter(f"s{i}") for i in range(3)]
+    circuit = Circuit(m)
+    circuit.add(5, PS(shared[0])).add(0, PS(shared[0])).add(1, PS("one"))
+    for k in range(cells):
+        q = (2 * k + k // 2) % 4
+        circuit.add(q, BS(theta=float(rng.uniform(0.3, 2.5)), phi_tr=0.4))
+        circuit.add(q + k % 2, PS(shared[k % 3]) if k % 97 < 6 else PS(0.1 * (k % 7)))
+        if k % 97 == 2:
+            circuit.add(q, PS(shared[0])).add(q, PS(f"p{k}")).add(q + 1, PS(shared[0]))
+    prog = MeshProgram(circuit)
+    assert max(np.bincount(prog.param[prog.param >= 0])) > 3
+    inp = [1, 1, 1, 0, 0, 0]
+    targets = np.array(oracle.fock_enumerate(m, n))[::3]
+    weights = rng.uniform(-2, 2, size=len(targets))
+    phases = rng.uniform(0, 2 * math.pi, size=(3, prog.nparams))
+    loss, grad = mesh_adjoint(prog, phases, inp, targets, weights=weights)
+    ref_l, ref_g = _torch_reference(prog, phases, inp, targets, weights)
+    tol = 1e4 * 2.0 ** -53 * max(1.0, np.abs(weights).sum())
+    assert np.max(np.abs(loss.cpu().numpy() - ref_l)) < tol
+    assert np.max(np.abs(grad.cpu().numpy() - ref_g)) < tol * max(1.0, np.abs(ref_g).max())
