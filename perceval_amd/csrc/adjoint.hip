@@ -414,6 +414,7 @@ __global__ void __launch_bounds__(ADJ_THREADS) mesh_adjoint_kernel(
                         if (two) u[ld] = cadd(cmul(M[2], x), cmul(M[3], y));
                     }
                 }
+                adj_wave_order();   // the next level's cells may read them from other slots
             }
         }
         __syncthreads();

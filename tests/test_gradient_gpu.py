@@ -339,3 +339,24 @@ def test_phase_of_several_shifters_vs_torch(gpu, cells):
     tol = 1e4 * 2.0 ** -53 * max(1.0, np.abs(weights).sum())
     assert np.max(np.abs(loss.cpu().numpy() - ref_l)) < tol
     assert np.max(np.abs(grad.cpu().numpy() - ref_g)) < tol * max(1.0, np.abs(ref_g).max())
+
+
+@pytest.mark.parametrize("m", [8, 17, 32])
+def test_levels_of_more_cells_than_slots_vs_torch(gpu, m):
+    """Cells of one level in several rounds of the wave's slots (8, 2 and 2 of
+    them), whose rows other slots read at the next level.  The bar is the one of
+    test_cells_passes_and_blocks_vs_torch."""
+    from perceval_amd.gradient import MeshProgram, mesh_adjoint
+    rng = np.random.RandomState(m)
+    n = 2
+    prog = MeshProgram(clements_mesh(m))
+    inp = [1, 1] + [0] * (m - 2)
+    states = oracle.fock_enumerate(m, n)
+    targets = np.array(states)[np.sort(rng.choice(len(states), 12, replace=False))]
+    weights = rng.uniform(-2, 2, size=12)
+    phases = rng.uniform(0, 2 * math.pi, size=(2, prog.nparams))
+    loss, grad = mesh_adjoint(prog, phases, inp, targets, weights=weights)
+    ref_l, ref_g = _torch_reference(prog, phases, inp, targets, weights)
+    tol = 1e4 * 2.0 ** -53 * max(1.0, np.abs(weights).sum())
+    assert np.max(np.abs(loss.cpu().numpy() - ref_l)) < tol
+    assert np.max(np.abs(grad.cpu().numpy() - ref_g)) < tol * max(1.0, np.abs(ref_g).max())
