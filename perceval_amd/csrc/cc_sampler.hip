@@ -51,6 +51,7 @@ struct CCShared {
     int r[K];
     // multiset steps: distinct output modes in the order fixed, unique, groups
     int mode[K], kg[K], w0[K];           // kg, w0: copies and first weight of each group
+    uint32_t inv[K];                     // ceil(2^32 / (k_g + 1)), see subperm_units
     double w[2 * K];                     // (-1)^t C(k_g, t), t = 0..k_g
 };
 
@@ -158,11 +159,22 @@ __device__ __forceinline__ void subperm_pair(const cd *__restrict__ B, int lane,
 // The O 2^nu terms are cut into units of 2^c Gray steps, one unit per lane
 // pair at a time.
 constexpr int CC_MULTI = 10;     // below, the terms are one or two passes of the 32 pairs
+// Above so many modes, steps 10..13 sum every row by itself: they repeat too
+// rarely to pay for the plan of the terms (100 modes, 100 samples of 12 photons
+// 139 us, 146 with multiplicities; 5,000 of 13 361 and 358).
+constexpr int CC_MULTI_MODES = 64;
 // From step 14 on, a sample's units are cut into slices (20,000 samples at
 // m = 60: step 15 takes 0.86 ms against 0.98 with one wave per sample, step 13
 // would lose the four extra launches).
 constexpr int CC_SLICED = 14;
 constexpr int CC_MAX_C = 8;
+// Up to step 15 and so many samples, one wave runs a sample's (two) slices one
+// after another and draws: one launch a step instead of five.  100 modes, 100
+// samples of 14 and 15 photons 230 -> 218 us and 328 -> 309, 5,000 of 15 856 ->
+// 769 us; 20,000 of 15 in 60 modes would take 2,234 us instead of 2,116, and one
+// of 16 with its step in it 262 us instead of 244.
+constexpr int CC_ONE_WAVE = 15;
+constexpr int64_t CC_ONE_WAVE_COUNT = 8192;
 
 // Most slices of a sample at step k: at most 2^13 terms each up to step 27
 // (0.2 ms of one wave: the tail when the last slices drain), 4,096 slices
@@ -205,16 +217,16 @@ __device__ __forceinline__ CCPlan cc_plan(CCShared<K> &sh, int lane)
         sh.mode[1 + p.nu + g] = r;
         sh.kg[g] = k;
     }
-    uint32_t O = (uint32_t)k + 1;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) O *= (uint32_t)__shfl_xor((int)O, off, 64);
-    O = __builtin_amdgcn_readfirstlane(O);
+    uint32_t O = 1;   // outer terms: the product of k_g + 1, at most 2^(K-2)
+    for (uint64_t left = gm; left != 0; left &= left - 1)
+        O *= (uint32_t)__builtin_amdgcn_readlane(k, __builtin_ctzll(left)) + 1;
     __syncthreads();
     if (lane < p.ng) {
         int w0 = 0;
         for (int g = 0; g < lane; g++) w0 += sh.kg[g] + 1;
         sh.w0[lane] = w0;
         const int kk = sh.kg[lane];
+        sh.inv[lane] = (uint32_t)((0x100000000ull + (uint32_t)kk) / (uint32_t)(kk + 1));
         double w = 1.0;   // every quotient is a whole number
         for (int t = 0; t <= kk; t++) {
             sh.w[w0 + t] = w;
@@ -227,18 +239,14 @@ __device__ __forceinline__ CCPlan cc_plan(CCShared<K> &sh, int lane)
     // own cost (rows into LDS, reduction of K sums).
     const int cmax = p.nu < CC_MAX_C ? p.nu : CC_MAX_C;
     const uint32_t setup = (uint32_t)((K + 1) * (2 + p.nu + p.ng) + 24 * p.ng + 40);
+    constexpr uint32_t cap = (uint32_t)cc_slice_cap(K);   // a power of two
     uint32_t best = 0xffffffffu;
-    p.c = cmax;
-    p.slices = 1;
-    p.units = O << (p.nu - cmax);
     for (int c = cmax; c >= 0 && c >= cmax - 4; c--) {
         const uint32_t units = O << (p.nu - c);
         const uint32_t want = (units + 31) / 32;
-        const uint32_t sl = want < (uint32_t)cc_slice_cap(K) ? want : (uint32_t)cc_slice_cap(K);
-        const uint32_t per = (units + sl - 1) / sl;
-        const uint32_t full = units / per, rest = units - full * per;
-        const uint32_t passes = full * ((per + 31) / 32) + (rest + 31) / 32;
-        const float est = (float)passes * (float)((7 * K + 24) * (1 << c) + (int)setup) + 4000.0f * (float)sl;
+        const uint32_t sl = want < cap ? want : cap;
+        const uint32_t passes = want < cap ? want : ((units + cap - 1) / cap + 31) / 32 * cap;
+        const float est = __builtin_fmaf((float)passes, (float)((7 * K + 24) * (1 << c) + (int)setup), 4000.0f * (float)sl);
         const uint32_t e = __float_as_uint(est);   // positive floats order as their bits
         if (e < best) {
             best = e;
@@ -308,7 +316,9 @@ __device__ __forceinline__ void subperm_units(const CCShared<K> &sh, const CCPla
 #pragma unroll 1
         for (int g = 0; g < pl.ng; g++) {
             const int k = sh.kg[g];
-            const uint32_t quot = o / (uint32_t)(k + 1);
+            // o / (k + 1): exact while o (k + 1) < 2^32, and o < 2^(K-2) where k < 16,
+            // below (k + 1) 2^(K-2-k) else
+            const uint32_t quot = __umulhi(o, sh.inv[g]);
             const int t = (int)(o - quot * (uint32_t)(k + 1));
             o = quot;
             W *= sh.w[sh.w0[g] + t];
@@ -539,7 +549,8 @@ __device__ __forceinline__ void cc_draw(const CCShared<K> &sh, const cd *__restr
 
 // Step k (= K) of every sample: one wavefront per sample, persistent.
 // r[s*n + i] holds the output mode of photon i (i < k-1 already drawn).
-template <int K>
+// MULTI: repeated rows by multiplicity.
+template <int K, bool MULTI>
 __global__ void __launch_bounds__(64) cc_step_kernel(const cd *__restrict__ U, int m, int n, int64_t count,
                                                      uint64_t seed, uint64_t first, const int32_t *__restrict__ pc_all,
                                                      int32_t *__restrict__ r_all, const int64_t *__restrict__ gidx)
@@ -554,7 +565,23 @@ __global__ void __launch_bounds__(64) cc_step_kernel(const cd *__restrict__ U, i
         if constexpr (K == 1) {
             if (lane == 0) sh.sub[0] = {1.0, 0.0};
         } else {
-            if constexpr (K >= CC_MULTI) {
+            static_assert(MULTI || K < CC_SLICED, "slices are of multiset terms");
+            if constexpr (K >= CC_SLICED) {
+                // the slices of the sample one after another, summed in order
+                // as by cc_slice_draw_kernel: the same bits
+                __shared__ cd s_part[K];
+                const CCPlan pl = cc_plan<K>(sh, lane);
+                load_rows<K>(sh, pl, U, m, lane);
+                const uint32_t per = (pl.units + (uint32_t)pl.slices - 1) / (uint32_t)pl.slices;
+                cd v = {0.0, 0.0};
+                for (uint32_t u0 = 0; u0 < pl.units; u0 += per) {
+                    subperms_units<K>(sh, pl, u0, u0 + per < pl.units ? u0 + per : pl.units, lane, s_part);
+                    __syncthreads();
+                    if (lane < K) v = cadd(v, s_part[lane]);
+                    __syncthreads();
+                }
+                if (lane < K) sh.sub[lane] = v;
+            } else if constexpr (MULTI) {
                 const CCPlan pl = cc_plan<K>(sh, lane);
                 load_rows<K>(sh, pl, U, m, lane);
                 subperms_units<K>(sh, pl, 0, pl.units, lane, sh.sub);
@@ -926,16 +953,19 @@ static int launch_step(int k, const cd *U, int m, int n, int64_t count, uint64_t
         return ERR_ARG;
     } else {
         if (k != K) return launch_step<K + 1>(k, U, m, n, count, seed, first, pc, r, work, cus, st, gidx);
-        if constexpr (K < CC_SLICED) {
+        if (K < CC_SLICED || (K <= CC_ONE_WAVE && count <= CC_ONE_WAVE_COUNT)) {
+            constexpr int KS = K <= CC_ONE_WAVE ? K : 1;   // the others have no such kernel
+            auto kp = cc_step_kernel<KS, (KS >= CC_MULTI)>;
+            if constexpr (KS >= CC_MULTI && KS < CC_SLICED) {
+                if (m > CC_MULTI_MODES) kp = cc_step_kernel<KS, false>;
+            }
             int per_cu = 0;
-            PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, reinterpret_cast<const void *>(&cc_step_kernel<K>), 64, 0));
+            PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(kp), 64, 0));
             if (per_cu < 1) per_cu = 1;
             const int grid = (int)std::min<int64_t>(count, (int64_t)cus * per_cu);
-            hipLaunchKernelGGL((cc_step_kernel<K>), dim3(grid), dim3(64), 0, st, U, m, n, count, seed, first, pc, r,
-                               gidx);
+            hipLaunchKernelGGL(kp, dim3(grid), dim3(64), 0, st, U, m, n, count, seed, first, pc, r, gidx);
             PCVL_HIP_CHECK(hipGetLastError());
-        } else {
+        } else if constexpr (K >= CC_SLICED) {
             int per_cu_s = 0, per_cu_d = 0;
             PCVL_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
                 &per_cu_s, reinterpret_cast<const void *>(&cc_slice_kernel<K>), 64, 0));

@@ -209,3 +209,26 @@ def test_backend_samples_for_inputs(gpu):
         assert all(o.n == s.n and o.m == 6 for o in got[s])
     with pytest.raises(AssertionError):
         b.samples_for_inputs({BasicState([1, 1, 0]): 2})
+
+
+@pytest.mark.parametrize("m,n", [(20, 14), (24, 15), (66, 15)])
+def test_one_wave_per_sample_and_slices_agree(gpu, m, n):
+    """Steps 14 and 15 run in one wave per sample up to 8,192 samples and in
+    slices above: the same samples, and the oracle's seed for seed."""
+    from perceval_amd.sampling import cc_samples
+    U = haar_unitary(m, seed=m + n)
+    inp = [1] * n + [0] * (m - n)
+    count = 8200
+    sliced = cc_samples(U, inp, count, seed=6)
+    assert np.array_equal(cc_samples(U, inp, 8192, seed=6), sliced[:8192])
+    assert np.array_equal(cc_samples(U, inp, 8, seed=6, first_sample=8192), sliced[8192:])
+    assert np.array_equal(oracle.cc_samples(U, inp, 40, seed=6), sliced[:40])
+
+
+@pytest.mark.parametrize("m,n", [(64, 13), (65, 10), (65, 13), (80, 14), (256, 11)])
+def test_same_seed_same_samples_row_by_row(gpu, m, n):
+    """Above 64 modes, steps 10..13 sum every row by itself, repeated ones too."""
+    from perceval_amd.sampling import cc_samples
+    U = haar_unitary(m, seed=m * n)
+    inp = [2, 1] + [1] * (n - 3) + [0] * (m - n + 1)
+    assert np.array_equal(cc_samples(U, inp, 150, seed=2), oracle.cc_samples(U, inp, 150, seed=2))
