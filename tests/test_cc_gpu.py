@@ -225,7 +225,7 @@ def test_one_wave_per_sample_and_slices_agree(gpu, m, n):
     assert np.array_equal(oracle.cc_samples(U, inp, 40, seed=6), sliced[:40])
 
 
-@pytest.mark.parametrize("m,n", [(64, 13), (65, 10), (65, 13), (80, 14), (256, 11)])
+@pytest.mark.parametrize("m,n", [(64, 13), (65, 10), (65, 13), (80, 14), (128, 11)])
 def test_same_seed_same_samples_row_by_row(gpu, m, n):
     """Above 64 modes, steps 10..13 sum every row by itself, repeated ones too."""
     from perceval_amd.sampling import cc_samples
