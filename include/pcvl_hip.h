@@ -248,8 +248,12 @@ int pcvl_slos_plan_block_width(pcvl_slos_plan plan);
  * counts.  At most 30 photons and 256 modes.
  * ------------------------------------------------------------------------- */
 
-/* Device workspace needed by pcvl_cc_samples for n photons and count samples. */
+/* Device workspace of pcvl_cc_samples for n photons and count samples: from 14
+ * photons on it holds the partial sums of up to 256 MiB of samples at a time.
+ * Any size from the least on is taken (fewer samples at a time, the same
+ * samples). */
 int pcvl_cc_workspace_bytes(int n, int64_t count, size_t *bytes);
+int pcvl_cc_workspace_least_bytes(int n, int64_t count, size_t *bytes);
 
 /* Enqueued on `stream`, which is synchronised before returning. */
 int pcvl_cc_samples(const double *d_U, int m, const int32_t *h_in_occ, int64_t count, uint64_t seed,

@@ -66,6 +66,7 @@ SIGNATURES = {
     "pcvl_slos_tree_execute": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
     "pcvl_slos_tree_destroy": (c_int, [c_void_p]),
     "pcvl_cc_workspace_bytes": (c_int, [c_int, c_i64, P(c_size_t)]),
+    "pcvl_cc_workspace_least_bytes": (c_int, [c_int, c_i64, P(c_size_t)]),
     "pcvl_mlp_gemm": (c_int, [c_void_p, c_i64, c_i64, c_void_p, c_int, c_i64, c_i64, c_void_p, c_i64, c_int, c_int,
                               c_int, c_void_p, c_int, c_int, c_void_p]),
     "pcvl_mlp_relu_bwd": (c_int, [c_void_p, c_void_p, c_i64, c_void_p]),
@@ -156,6 +157,19 @@ def stream_handle(stream=None) -> int:
     import torch
     s = stream if stream is not None else torch.cuda.current_stream()
     return int(s.cuda_stream)
+
+
+def workspace(nbytes: int, least: int, device):
+    """A workspace of nbytes, or of less where the device is nearly full, down to
+    the least size that the call takes."""
+    import torch
+    while True:
+        try:
+            return torch.empty(max(16, nbytes), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            if nbytes <= least:
+                raise
+            nbytes = max(least, nbytes // 4)
 
 
 def ptr(t) -> int:

@@ -926,15 +926,14 @@ struct CCSliceWork {
     size_t o_s0 = 0, o_cur = 0, o_own = 0, o_part = 0, total = 0;
 };
 
-static CCSliceWork cc_slice_work(int n, int64_t count)
+static CCSliceWork cc_slice_layout(int n, int64_t chunk)
 {
     CCSliceWork w;
-    if (n < CC_SLICED || count <= 0) return w;
+    if (n < CC_SLICED || chunk <= 0) return w;
     const size_t cap = (size_t)cc_slice_cap(n);
-    const size_t per_sample = cap * ((size_t)n * sizeof(cd) + sizeof(uint64_t));
-    w.chunk = std::min(count, std::max<int64_t>(1, (int64_t)(CC_PART_BYTES / per_sample)));
+    w.chunk = chunk;
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
-    const size_t c = (size_t)w.chunk;
+    const size_t c = (size_t)chunk;
     w.o_s0 = al(sizeof(int32_t) * c);
     w.o_cur = w.o_s0 + al(sizeof(int64_t) * (c + 1));
     w.o_own = w.o_cur + 256;
@@ -943,16 +942,33 @@ static CCSliceWork cc_slice_work(int n, int64_t count)
     return w;
 }
 
+// The chunks that `room` bytes hold, CC_PART_BYTES of slices at most and one
+// sample at least.
+static CCSliceWork cc_slice_work(int n, int64_t count, size_t room = SIZE_MAX)
+{
+    if (n <= CC_ONE_WAVE && count <= CC_ONE_WAVE_COUNT) return {};   // every step in one wave per sample
+    const size_t per_sample = (size_t)cc_slice_cap(n) * ((size_t)n * sizeof(cd) + sizeof(uint64_t));
+    int64_t lo = std::min<int64_t>(count, 1);
+    int64_t hi = std::min(count, std::max<int64_t>(1, (int64_t)(CC_PART_BYTES / std::max<size_t>(per_sample, 1))));
+    if (cc_slice_layout(n, hi).total <= room) lo = hi;
+    while (lo + 1 < hi) {
+        const int64_t mid = lo + (hi - lo) / 2;
+        if (cc_slice_layout(n, mid).total <= room) lo = mid;
+        else hi = mid;
+    }
+    return cc_slice_layout(n, lo);
+}
+
 template <int K>
 static int launch_step(int k, const cd *U, int m, int n, int64_t count, uint64_t seed, uint64_t first,
-                       const int32_t *pc, int32_t *r, char *work, int cus, hipStream_t st,
+                       const int32_t *pc, int32_t *r, const CCSliceWork &w, char *work, int cus, hipStream_t st,
                        const int64_t *gidx = nullptr)
 {
     if constexpr (K > CC_MAX_N) {
         set_error("internal: photon step out of range");
         return ERR_ARG;
     } else {
-        if (k != K) return launch_step<K + 1>(k, U, m, n, count, seed, first, pc, r, work, cus, st, gidx);
+        if (k != K) return launch_step<K + 1>(k, U, m, n, count, seed, first, pc, r, w, work, cus, st, gidx);
         if (K < CC_SLICED || (K <= CC_ONE_WAVE && count <= CC_ONE_WAVE_COUNT)) {
             constexpr int KS = K <= CC_ONE_WAVE ? K : 1;   // the others have no such kernel
             auto kp = cc_step_kernel<KS, (KS >= CC_MULTI)>;
@@ -973,7 +989,6 @@ static int launch_step(int k, const cd *U, int m, int n, int64_t count, uint64_t
                 &per_cu_d, reinterpret_cast<const void *>(&cc_slice_draw_kernel<K>), 64, 0));
             per_cu_s = std::max(per_cu_s, 1);
             per_cu_d = std::max(per_cu_d, 1);
-            const CCSliceWork w = cc_slice_work(n, count);
             int32_t *ns = reinterpret_cast<int32_t *>(work);
             int64_t *slice0 = reinterpret_cast<int64_t *>(work + w.o_s0);
             unsigned long long *cursor = reinterpret_cast<unsigned long long *>(work + w.o_cur);
@@ -1003,7 +1018,7 @@ static int launch_step(int k, const cd *U, int m, int n, int64_t count, uint64_t
 // Every photon of `count` samples whose columns are in pc, and their output
 // rows (row gidx[s], or s): the first steps, the steps after them, the rows.
 static int cc_run(const cd *U, int m, int n, int64_t count, uint64_t seed, uint64_t first, const int32_t *pc,
-                  int32_t *r, char *work, const int64_t *gidx, int32_t *out, int cus, hipStream_t st)
+                  int32_t *r, const CCSliceWork &w, char *work, const int64_t *gidx, int32_t *out, int cus, hipStream_t st)
 {
     int k = 1;
     if (m <= CC_FIRST_MODES) {
@@ -1013,7 +1028,7 @@ static int cc_run(const cd *U, int m, int n, int64_t count, uint64_t seed, uint6
         k = kmax + 1;
     }
     for (; k <= n; k++) {
-        const int rc = launch_step<1>(k, U, m, n, count, seed, first, pc, r, work, cus, st, gidx);
+        const int rc = launch_step<1>(k, U, m, n, count, seed, first, pc, r, w, work, cus, st, gidx);
         if (rc != OK) return rc;
     }
     const int64_t tot = count * m;
@@ -1030,15 +1045,33 @@ static int cc_run(const cd *U, int m, int n, int64_t count, uint64_t seed, uint6
 
 using namespace pcvl;
 
+// pc (count*n) | r (count*n) | cols (CC_MAX_N)
+static size_t cc_head_bytes(int n, int64_t count)
+{
+    return sizeof(int32_t) * ((size_t)2 * (size_t)count * (size_t)std::max(n, 1) + (size_t)CC_MAX_N);
+}
+
+// The head, then from a 256-byte boundary the slices of the sliced steps (14
+// photons and more).
+static size_t cc_work_bytes(int n, int64_t count, size_t slices)
+{
+    const size_t head = cc_head_bytes(n, count);
+    return slices ? ((head + 255) & ~size_t(255)) + slices : head;
+}
+
 extern "C" int pcvl_cc_workspace_bytes(int n, int64_t count, size_t *bytes)
 {
     PCVL_ARG_CHECK(bytes != nullptr, "bytes is null");
     PCVL_ARG_CHECK(n >= 0 && n <= CC_MAX_N && count >= 0, "n outside [0, 30] or count < 0");
-    // pc (count*n) | r (count*n) | cols (CC_MAX_N), then from a 256-byte
-    // boundary the slices of the sliced steps (14 photons and more)
-    const size_t head = sizeof(int32_t) * ((size_t)2 * (size_t)count * (size_t)std::max(n, 1) + (size_t)CC_MAX_N);
-    const size_t part = cc_slice_work(n, count).total;
-    *bytes = part ? ((head + 255) & ~size_t(255)) + part : head;
+    *bytes = cc_work_bytes(n, count, cc_slice_work(n, count).total);
+    return OK;
+}
+
+extern "C" int pcvl_cc_workspace_least_bytes(int n, int64_t count, size_t *bytes)
+{
+    PCVL_ARG_CHECK(bytes != nullptr, "bytes is null");
+    PCVL_ARG_CHECK(n >= 0 && n <= CC_MAX_N && count >= 0, "n outside [0, 30] or count < 0");
+    *bytes = cc_work_bytes(n, count, cc_slice_work(n, count, 0).total);
     return OK;
 }
 
@@ -1059,8 +1092,8 @@ extern "C" int pcvl_cc_samples(const double *d_U, int m, const int32_t *h_in_occ
     PCVL_ARG_CHECK(d_U && d_out, "null device buffer");
     const int n = (int)cols.size();
     size_t need = 0;
-    pcvl_cc_workspace_bytes(n, count, &need);
-    PCVL_ARG_CHECK(d_work != nullptr && work_bytes >= need, "workspace missing or smaller than pcvl_cc_workspace_bytes");
+    pcvl_cc_workspace_least_bytes(n, count, &need);
+    PCVL_ARG_CHECK(d_work != nullptr && work_bytes >= need, "workspace missing or smaller than pcvl_cc_workspace_least_bytes");
     if (n == 0) {
         const int64_t tot = count * m;
         hipLaunchKernelGGL(cc_finish_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, stream,
@@ -1072,8 +1105,9 @@ extern "C" int pcvl_cc_samples(const double *d_U, int m, const int32_t *h_in_occ
     int32_t *pc = static_cast<int32_t *>(d_work);
     int32_t *r = pc + (size_t)count * n;
     int32_t *d_cols = r + (size_t)count * n;
-    const size_t head = sizeof(int32_t) * ((size_t)2 * (size_t)count * (size_t)n + (size_t)CC_MAX_N);
-    char *slices = static_cast<char *>(d_work) + ((head + 255) & ~size_t(255));
+    const size_t head = (cc_head_bytes(n, count) + 255) & ~size_t(255);
+    char *slices = static_cast<char *>(d_work) + head;
+    const CCSliceWork work = cc_slice_work(n, count, work_bytes > head ? work_bytes - head : 0);
     PCVL_HIP_CHECK(hipMemcpyAsync(d_cols, cols.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, stream));
     const cd *U = reinterpret_cast<const cd *>(d_U);
     int dev = 0, cus = 0;
@@ -1082,7 +1116,7 @@ extern "C" int pcvl_cc_samples(const double *d_U, int m, const int32_t *h_in_occ
     hipLaunchKernelGGL(cc_init_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, d_cols, n, count,
                        seed, first_sample, pc);
     PCVL_HIP_CHECK(hipGetLastError());
-    const int rc = cc_run(U, m, n, count, seed, first_sample, pc, r, slices, nullptr, d_out, cus, stream);
+    const int rc = cc_run(U, m, n, count, seed, first_sample, pc, r, work, slices, nullptr, d_out, cus, stream);
     if (rc != OK) return rc;
     // the host column list copied above must outlive the copy
     PCVL_HIP_CHECK(hipStreamSynchronize(stream));
@@ -1148,12 +1182,23 @@ extern "C" int pcvl_cc_samples_multi(const double *d_U, int m, const int32_t *h_
         gmax = std::max(gmax, g.count);
         nmax = std::max(nmax, g.n);
     }
-    for (const Group &g : groups) b_part = std::max(b_part, cc_slice_work(g.n, gmax).total);
+    size_t least = 0;   // where the device is nearly full
+    for (const Group &g : groups) {
+        b_part = std::max(b_part, cc_slice_work(g.n, g.count).total);
+        least = std::max(least, cc_slice_work(g.n, g.count, 0).total);
+    }
     // device block: pc | r (gmax * nmax each) | gidx (gmax) | tables | slices
     const size_t b_pr = al(sizeof(int32_t) * (size_t)gmax * nmax);
     const size_t b_gidx = al(sizeof(int64_t) * (size_t)gmax);
+    const size_t b_head = 2 * b_pr + b_gidx + al(tab.size());
     char *blk = nullptr;
-    PCVL_HIP_CHECK(ws_alloc(reinterpret_cast<void **>(&blk), 2 * b_pr + b_gidx + al(tab.size()) + al(b_part), stream));
+    hipError_t e = ws_alloc(reinterpret_cast<void **>(&blk), b_head + al(b_part), stream);
+    while (e == hipErrorOutOfMemory && least < b_part) {
+        (void)hipGetLastError();
+        b_part = std::max(least, b_part / 4);
+        e = ws_alloc(reinterpret_cast<void **>(&blk), b_head + al(b_part), stream);
+    }
+    PCVL_HIP_CHECK(e);
     int32_t *pc = reinterpret_cast<int32_t *>(blk);
     int32_t *r = reinterpret_cast<int32_t *>(blk + b_pr);
     int64_t *d_gidx = reinterpret_cast<int64_t *>(blk + 2 * b_pr);
@@ -1162,7 +1207,7 @@ extern "C" int pcvl_cc_samples_multi(const double *d_U, int m, const int32_t *h_
     const cd *U = reinterpret_cast<const cd *>(d_U);
     int dev = 0, cus = 0;
     int rc = OK;
-    hipError_t e = hipGetDevice(&dev);
+    e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess) e = hipMemcpyAsync(d_tab, tab.data(), tab.size(), hipMemcpyHostToDevice, stream);
     if (e != hipSuccess) { set_error(std::string("cc multi tables: ") + hipGetErrorString(e)); rc = ERR_HIP; }
@@ -1177,7 +1222,8 @@ extern "C" int pcvl_cc_samples_multi(const double *d_U, int m, const int32_t *h_
         e = hipGetLastError();
         if (e != hipSuccess) { set_error(std::string("cc_init_multi: ") + hipGetErrorString(e)); rc = ERR_HIP; break; }
         if (g.n > 0) {
-            rc = cc_run(U, m, g.n, g.count, seed, first_sample, pc, r, slices, d_gidx, d_out, cus, stream);
+            rc = cc_run(U, m, g.n, g.count, seed, first_sample, pc, r, cc_slice_work(g.n, g.count, b_part), slices, d_gidx,
+                        d_out, cus, stream);
         } else {
             hipLaunchKernelGGL(cc_finish_multi_kernel, dim3((unsigned)((g.count * m + 255) / 256)), dim3(256), 0,
                                stream, r, d_gidx, m, 0, g.count, d_out);

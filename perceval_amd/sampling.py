@@ -29,9 +29,10 @@ def cc_samples_device(U, in_occ, count: int, seed: int, first_sample: int = 0, o
         raise ValueError(f"unitary must be {m} x {m}")
     if out is None:
         out = torch.empty((count, m), dtype=torch.int32, device=dU.device)
-    need = ctypes.c_size_t()
+    need, least = ctypes.c_size_t(), ctypes.c_size_t()
     _native.check(lib.pcvl_cc_workspace_bytes(n, count, ctypes.byref(need)), "pcvl_cc_workspace_bytes")
-    work = torch.empty(max(16, need.value), dtype=torch.uint8, device=dU.device)
+    _native.check(lib.pcvl_cc_workspace_least_bytes(n, count, ctypes.byref(least)), "pcvl_cc_workspace_least_bytes")
+    work = _native.workspace(need.value, least.value, dU.device)
     _native.check(lib.pcvl_cc_samples(_native.ptr(dU), m, in_occ.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)),
                                       int(count), int(seed) & (2 ** 64 - 1), int(first_sample), _native.ptr(out),
                                       _native.ptr(work), work.numel(), _native.stream_handle(stream)),

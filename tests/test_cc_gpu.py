@@ -232,3 +232,51 @@ def test_same_seed_same_samples_row_by_row(gpu, m, n):
     U = haar_unitary(m, seed=m * n)
     inp = [2, 1] + [1] * (n - 3) + [0] * (m - n + 1)
     assert np.array_equal(cc_samples(U, inp, 150, seed=2), oracle.cc_samples(U, inp, 150, seed=2))
+
+
+@pytest.mark.parametrize("n,count", [(14, 8300), (17, 300), (21, 40)])
+def test_smaller_workspaces_give_the_same_samples(gpu, n, count):
+    """Any workspace from the least size on is taken, with fewer samples of the
+    sliced steps at a time; one byte less than the least is refused."""
+    import ctypes
+    import torch
+    from perceval_amd import _native
+    from perceval_amd.sampling import cc_samples
+    lib = _native.load()
+    m = 24
+    U = haar_unitary(m, seed=n)
+    inp = np.array([1] * n + [0] * (m - n), dtype=np.int32)
+    ref = cc_samples(U, inp, count, seed=4)
+    full, least = ctypes.c_size_t(), ctypes.c_size_t()
+    _native.check(lib.pcvl_cc_workspace_bytes(n, count, ctypes.byref(full)), "bytes")
+    _native.check(lib.pcvl_cc_workspace_least_bytes(n, count, ctypes.byref(least)), "least")
+    assert least.value < full.value
+    dU = torch.from_numpy(U).cuda()
+    work = torch.empty(full.value, dtype=torch.uint8, device="cuda")
+    for size in (least.value, (least.value + full.value) // 2, full.value):
+        out = torch.empty((count, m), dtype=torch.int32, device="cuda")
+        rc = lib.pcvl_cc_samples(_native.ptr(dU), m, inp.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), count, 4, 0,
+                                 _native.ptr(out), _native.ptr(work), size, _native.stream_handle())
+        assert rc == 0 and np.array_equal(out.cpu().numpy(), ref), size
+    assert lib.pcvl_cc_samples(_native.ptr(dU), m, inp.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), count, 4, 0,
+                               _native.ptr(out), _native.ptr(work), least.value - 1, _native.stream_handle()) != 0
+
+
+def test_sampling_on_a_nearly_full_device(gpu):
+    """Where the whole workspace (44 MB here) does not fit, a smaller one is taken."""
+    import torch
+    from perceval_amd.sampling import cc_samples_device
+    m, n, count = 24, 21, 2000
+    dU = torch.from_numpy(haar_unitary(m, seed=n)).cuda()
+    inp = [1] * n + [0] * (m - n)
+    ref = cc_samples_device(dU, inp, count, seed=4).cpu().numpy()
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved() + (24 << 20)
+    try:
+        torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(0).total_memory)
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(40 << 20, dtype=torch.uint8, device="cuda")
+        got = cc_samples_device(dU, inp, count, seed=4)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert np.array_equal(got.cpu().numpy(), ref)
