@@ -205,12 +205,17 @@ int pcvl_slos_plan_create_masks(int m, const int32_t *h_in_occ, int nrows, const
  * order: input i occupies elements [h_out_offsets[i], h_out_offsets[i+1]) of
  * d_out (complex for COEFS, double for PROBS, FSArray order each).  The
  * workspace holds the layer of every node with children where these fit 1 GiB
- * together, else one layer per depth below the largest photon number. */
+ * together, and the nodes of a depth then run in one launch; else, and in a
+ * workspace of the least size or more, one layer per depth below the largest
+ * photon number, a launch for every layer and output of a node (layer_launches
+ * of them). */
 typedef struct pcvl_slos_tree_s *pcvl_slos_tree;
 int pcvl_slos_tree_create(int m, const int32_t *h_inputs, int count, pcvl_slos_tree *out);
 /* h_out_offsets receives count + 1 entries; any output pointer may be NULL. */
 int pcvl_slos_tree_info(pcvl_slos_tree plan, int *nmax, int64_t *h_out_offsets, size_t *work_bytes,
                         int64_t *layer_launches);
+/* Smallest workspace that execute takes. */
+int pcvl_slos_tree_least_bytes(pcvl_slos_tree plan, size_t *bytes);
 int pcvl_slos_tree_execute(pcvl_slos_tree plan, const double *d_U, int mode, void *d_out, void *d_work,
                            size_t work_bytes, hipStream_t stream);
 int pcvl_slos_tree_destroy(pcvl_slos_tree plan);

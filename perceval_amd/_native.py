@@ -63,6 +63,7 @@ SIGNATURES = {
     "pcvl_slos_plan_block_width": (c_int, [c_void_p]),
     "pcvl_slos_tree_create": (c_int, [c_int, P(c_i32), c_int, ctypes.POINTER(c_void_p)]),
     "pcvl_slos_tree_info": (c_int, [c_void_p, P(c_int), P(c_i64), P(ctypes.c_size_t), P(c_i64)]),
+    "pcvl_slos_tree_least_bytes": (c_int, [c_void_p, P(ctypes.c_size_t)]),
     "pcvl_slos_tree_execute": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, ctypes.c_size_t, c_void_p]),
     "pcvl_slos_tree_destroy": (c_int, [c_void_p]),
     "pcvl_cc_workspace_bytes": (c_int, [c_int, c_i64, P(c_size_t)]),

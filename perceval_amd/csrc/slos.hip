@@ -1115,8 +1115,8 @@ extern "C" int pcvl_slos_plan_destroy(pcvl_slos_plan plan)
 // node's layer fits TREE_LEVEL_BYTES of workspace together, the nodes of one
 // depth run in one launch (20 modes, 37 inputs of 6..8 photons: 101 launches
 // and 875 us one node at a time, see the batch kernel).  Larger trees, whose
-// layers fill the device by themselves, and those without a block layout run
-// depth first: node layers live in one buffer per depth, so a node's parent
+// layers fill the device by themselves, those without a block layout and calls
+// with a smaller workspace run depth first: node layers live in one buffer per depth, so a node's parent
 // layer is still in place when the node is computed.
 
 struct TreeOp {
@@ -1144,6 +1144,7 @@ struct SlosTreeImpl {
     std::vector<int> in_n;              // photons of each input
     std::vector<size_t> level_off;      // byte offset of depth buffer k in the workspace
     size_t work_bytes = 0;
+    size_t least_bytes = 0;             // depth first: one layer per depth
     std::vector<TreeOp> ops;            // depth-first launch list
     std::vector<TreeNode> nodes;
     std::vector<int> level_ops;         // by depth: first entry of depth k in d_ops (nmax + 2 entries); empty: depth first
@@ -1272,7 +1273,7 @@ static int tree_levels(SlosTreeImpl &t, const std::vector<double> &inv_pin)
         t.front = front;
         t.d_paths = reinterpret_cast<const int32_t *>(reinterpret_cast<char *>(t.d_ops) + b_ops);
     }
-    t.work_bytes = off;
+    t.work_bytes = std::max(off, t.least_bytes);
     return OK;
 }
 
@@ -1331,7 +1332,7 @@ extern "C" int pcvl_slos_tree_create(int m, const int32_t *h_inputs, int count, 
         t.level_off.push_back(off);
         off += ((sizeof(cd) * (size_t)t.counts[(size_t)k]) + 255) & ~size_t(255);
     }
-    t.work_bytes = off;
+    t.work_bytes = t.least_bytes = off;
     tree_decompose(t, 0, -1, std::move(targets), std::move(ids), inv_pin);
 
     std::vector<uint64_t> T, E;
@@ -1379,6 +1380,13 @@ extern "C" int pcvl_slos_tree_info(pcvl_slos_tree plan, int *nmax, int64_t *h_ou
     return OK;
 }
 
+extern "C" int pcvl_slos_tree_least_bytes(pcvl_slos_tree plan, size_t *bytes)
+{
+    PCVL_ARG_CHECK(plan != nullptr && bytes != nullptr, "null plan or output pointer");
+    *bytes = plan->impl.least_bytes;
+    return OK;
+}
+
 extern "C" int pcvl_slos_tree_execute(pcvl_slos_tree plan, const double *d_U, int mode, void *d_out, void *d_work,
                                       size_t work_bytes, hipStream_t stream)
 {
@@ -1386,17 +1394,18 @@ extern "C" int pcvl_slos_tree_execute(pcvl_slos_tree plan, const double *d_U, in
     PCVL_ARG_CHECK(mode == PCVL_SLOS_COEFS || mode == PCVL_SLOS_PROBS, "mode must be COEFS or PROBS");
     PCVL_ARG_CHECK(d_U && d_out, "null device buffer");
     const SlosTreeImpl &t = plan->impl;
-    PCVL_ARG_CHECK(work_bytes >= t.work_bytes && (t.work_bytes == 0 || d_work), "workspace too small");
+    PCVL_ARG_CHECK(work_bytes >= t.least_bytes && (t.least_bytes == 0 || d_work), "workspace too small");
+    const bool by_depth = !t.level_ops.empty() && work_bytes >= t.work_bytes;
     const cd *U = reinterpret_cast<const cd *>(d_U);
     char *work = static_cast<char *>(d_work);
     const size_t esz = mode == PCVL_SLOS_PROBS ? sizeof(double) : sizeof(cd);
     const size_t lds = 2 * sizeof(uint64_t) * (size_t)t.m * t.w;
-    if (t.nmax > 0 && t.front == 0) {   // depth-0 buffer holds the vacuum coefficient
+    if (t.nmax > 0 && !(by_depth && t.front > 0)) {   // depth-0 buffer holds the vacuum coefficient
         hipLaunchKernelGGL(slos_vacuum_kernel, dim3(1), dim3(64), 0, stream, reinterpret_cast<double *>(work + t.level_off[0]), 0);
         PCVL_HIP_CHECK(hipGetLastError());
     }
     for (const TreeOp &op : t.ops) {
-        if (op.k != 0 && !t.level_ops.empty()) continue;   // run by depth below
+        if (op.k != 0 && by_depth) continue;   // run by depth below
         if (op.k == 0) {   // input with no photon: vacuum output
             hipLaunchKernelGGL(slos_vacuum_kernel, dim3(1), dim3(64), 0, stream,
                                reinterpret_cast<double *>(static_cast<char *>(d_out) + esz * (size_t)t.out_off[(size_t)op.input]),
@@ -1432,7 +1441,7 @@ extern "C" int pcvl_slos_tree_execute(pcvl_slos_tree plan, const double *d_U, in
                                op.inv_prod_in);
         PCVL_HIP_CHECK(hipGetLastError());
     }
-    if (!t.level_ops.empty())
+    if (by_depth)
         for (int k = std::max(t.front, 1); k <= t.nmax; k++) {
             const int a = t.level_ops[(size_t)k], n = t.level_ops[(size_t)k + 1] - a;
             if (n == 0) continue;

@@ -157,8 +157,11 @@ class SlosTree:
                                               ctypes.byref(work), ctypes.byref(launches)), "pcvl_slos_tree_info")
         self.nmax = nmax.value
         self.offsets = offs
+        least = ctypes.c_size_t()
+        _native.check(lib.pcvl_slos_tree_least_bytes(self._plan, ctypes.byref(least)), "pcvl_slos_tree_least_bytes")
         self.work_bytes = work.value
-        self.layer_launches = launches.value
+        self.least_bytes = least.value
+        self.layer_launches = launches.value   # launches of a depth-first run; fewer when depths run together
         self._work = None
 
     def run(self, U, mode: int = PROBS, out=None, stream=None):
@@ -176,7 +179,7 @@ class SlosTree:
         elif out.dtype != dtype or out.numel() < total or not out.is_contiguous():
             raise ValueError("out has the wrong dtype, size or layout")
         if self._work is None or self._work.device != dU.device:
-            self._work = torch.empty(max(16, self.work_bytes), dtype=torch.uint8, device=dU.device)
+            self._work = _native.workspace(self.work_bytes, self.least_bytes, dU.device)
         _native.check(self._lib.pcvl_slos_tree_execute(self._plan, _native.ptr(dU), mode, _native.ptr(out),
                                                        _native.ptr(self._work), self._work.numel(),
                                                        _native.stream_handle(stream)), "pcvl_slos_tree_execute")

@@ -424,6 +424,56 @@ def test_slos_tree_depth_first_vs_single_plans(gpu):
     small.close()
 
 
+@pytest.mark.parametrize("m,inputs", [
+    (24, [[1] * 9 + [0] * 15, [0] * 15 + [1] * 9, [2] * 4 + [1] + [0] * 19, [1] * 7 + [0] * 17, [1] * 9 + [0] * 15]),
+    (12, [[1] * 5 + [0] * 7, [1] * 4 + [0] * 8, [0] * 12, [1] * 5 + [0] * 7, [0] * 7 + [1] * 5]),
+])
+def test_slos_tree_in_its_least_workspace(gpu, m, inputs):
+    """In a workspace smaller than all its layers a tree runs depth first, one
+    layer per depth: the amplitudes of a run by depth (the same sums in the same
+    order, so the same bits), a repeated input, one that ends inside another's
+    path and one without photons among them; and one byte less is refused."""
+    import ctypes
+    import torch
+    from perceval_amd import _native
+    from perceval_amd.slos import COEFS, PROBS, SlosTree
+    lib = _native.load()
+    tree = SlosTree(inputs)
+    nmax = max(sum(s) for s in inputs)
+    assert tree.least_bytes == sum((16 * math.comb(m + k - 1, k) + 255) // 256 * 256 for k in range(nmax))
+    assert tree.least_bytes < tree.work_bytes
+    dU = torch.from_numpy(haar_unitary(m, seed=m)).cuda()
+    work = torch.empty(tree.work_bytes, dtype=torch.uint8, device="cuda")
+    for mode in (PROBS, COEFS):
+        ref = torch.cat(tree.run(dU, mode))
+        for size in (tree.least_bytes, tree.work_bytes - 1):
+            out = torch.full_like(ref, float("nan"))
+            assert lib.pcvl_slos_tree_execute(tree._plan, _native.ptr(dU), mode, _native.ptr(out), _native.ptr(work),
+                                              size, _native.stream_handle()) == 0
+            assert torch.equal(out, ref), (mode, size)
+    assert lib.pcvl_slos_tree_execute(tree._plan, _native.ptr(dU), PROBS, _native.ptr(out), _native.ptr(work),
+                                      tree.least_bytes - 1, _native.stream_handle()) != 0
+    tree.close()
+
+
+def test_slos_tree_above_the_depth_limit(gpu):
+    """Layers of more than 1 GiB together: the plan asks for one layer per depth
+    and runs depth first (seven inputs of 9 photons with disjoint last layers)."""
+    from perceval_amd.slos import PROBS, SlosPlan, SlosTree
+    m = 24
+    inputs = [[0] * a + [1] * 9 + [0] * (15 - a) for a in (0, 15)] + \
+             [[3 if j in t else 0 for j in range(m)] for t in ((0, 12, 20), (3, 14, 21), (5, 9, 17), (1, 10, 18), (2, 11, 23))] + \
+             [[9] + [0] * 23, [0] * 23 + [9]]
+    tree = SlosTree(inputs)
+    assert tree.work_bytes == tree.least_bytes == 168293888
+    U = haar_unitary(m, seed=5)
+    for s, got in zip(inputs, tree.run(U, PROBS)):
+        plan = SlosPlan(s)
+        assert (got - plan.run(U, PROBS)).abs().max().item() < 1e-13, s
+        plan.close()
+    tree.close()
+
+
 def test_slos_backend_preprocess_shares_a_tree(gpu):
     from perceval_amd.backends import SLOSBackend
     from perceval_amd.components import Unitary
