@@ -1151,7 +1151,7 @@ struct SlosTreeImpl {
     BlkBatchOp *d_ops = nullptr;
     int front = 0;                      // depths 1..front run in one launch (0: each its own)
     const int32_t *d_paths = nullptr;   // input modes from the root of the nodes of depth front, behind d_ops
-    uint64_t *d_T = nullptr, *d_E = nullptr;
+    uint64_t *d_T = nullptr, *d_E = nullptr;   // without a block layout
     int grid_cap = 0;
     BlkLayout blk;                      // block layout of the layers, when they allow it
 };
@@ -1256,12 +1256,12 @@ static int tree_levels(SlosTreeImpl &t, const std::vector<double> &inv_pin)
                 paths[paths.size() - (size_t)(front - k) - 1] = t.nodes[(size_t)at_node].mk;
         }
     const size_t b_ops = sizeof(BlkBatchOp) * ops.size();
-    hipError_t e = hipMalloc(&t.d_ops, b_ops + sizeof(int32_t) * paths.size());
+    std::vector<char> image(b_ops + sizeof(int32_t) * paths.size());
+    std::memcpy(image.data(), ops.data(), b_ops);
+    if (!paths.empty()) std::memcpy(image.data() + b_ops, paths.data(), sizeof(int32_t) * paths.size());
+    hipError_t e = hipMalloc(&t.d_ops, image.size());
     if (e != hipSuccess) { t.d_ops = nullptr; set_error(std::string("hipMalloc(slos tree ops): ") + hipGetErrorString(e)); return ERR_ALLOC; }
-    e = hipMemcpy(t.d_ops, ops.data(), b_ops, hipMemcpyHostToDevice);
-    if (e == hipSuccess && !paths.empty())
-        e = hipMemcpy(reinterpret_cast<char *>(t.d_ops) + b_ops, paths.data(), sizeof(int32_t) * paths.size(),
-                      hipMemcpyHostToDevice);
+    e = hipMemcpy(t.d_ops, image.data(), image.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(t.d_ops);
         t.d_ops = nullptr;
@@ -1274,6 +1274,21 @@ static int tree_levels(SlosTreeImpl &t, const std::vector<double> &inv_pin)
         t.d_paths = reinterpret_cast<const int32_t *>(reinterpret_cast<char *>(t.d_ops) + b_ops);
     }
     t.work_bytes = std::max(off, t.least_bytes);
+    return OK;
+}
+
+// Rank tables of the per-state kernel.
+static int tree_tables(SlosTreeImpl &t)
+{
+    std::vector<uint64_t> T, E;
+    build_tables(t.m, t.nmax, T, E);
+    const size_t bytes = sizeof(uint64_t) * T.size();
+    hipError_t e = hipMalloc(&t.d_T, 2 * bytes);
+    if (e != hipSuccess) { t.d_T = nullptr; set_error(std::string("hipMalloc(slos tables): ") + hipGetErrorString(e)); return ERR_ALLOC; }
+    t.d_E = t.d_T + T.size();
+    e = hipMemcpy(t.d_T, T.data(), bytes, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(t.d_E, E.data(), bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) { set_error(std::string("hipMemcpy(slos tables): ") + hipGetErrorString(e)); return ERR_HIP; }
     return OK;
 }
 
@@ -1335,31 +1350,21 @@ extern "C" int pcvl_slos_tree_create(int m, const int32_t *h_inputs, int count, 
     t.work_bytes = t.least_bytes = off;
     tree_decompose(t, 0, -1, std::move(targets), std::move(ids), inv_pin);
 
-    std::vector<uint64_t> T, E;
-    build_tables(m, t.nmax, T, E);
-    const size_t bytes = sizeof(uint64_t) * T.size();
-    hipError_t e = hipMalloc(&t.d_T, 2 * bytes);
-    if (e != hipSuccess) { delete plan; set_error(std::string("hipMalloc(slos tables): ") + hipGetErrorString(e)); return ERR_ALLOC; }
-    t.d_E = t.d_T + T.size();
-    e = hipMemcpy(t.d_T, T.data(), bytes, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(t.d_E, E.data(), bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(t.d_T);
-        delete plan;
-        set_error(std::string("hipMemcpy(slos tables): ") + hipGetErrorString(e));
-        return ERR_HIP;
-    }
     int rc = device_grid_cap(&t.grid_cap);
     if (rc == OK && blk_layout_ok(m, t.nmax)) {
         rc = blk_layout_create(m, t.nmax, blk_default_width(m, t.nmax), &t.blk);
         if (rc == ERR_RANGE) rc = OK;   // the tree's per-state kernel then runs every layer
     }
-    if (rc == OK && !t.blk.d_mem && 2 * sizeof(uint64_t) * (size_t)m * (size_t)t.w > 160 * 1024) {
-        set_error("SLOS tree: modes and photons too many for the per-state kernel's tables");
-        rc = ERR_RANGE;
+    if (rc == OK && !t.blk.d_mem) {
+        if (2 * sizeof(uint64_t) * (size_t)m * (size_t)t.w > 160 * 1024) {
+            set_error("SLOS tree: modes and photons too many for the per-state kernel's tables");
+            rc = ERR_RANGE;
+        } else {
+            rc = tree_tables(t);
+        }
     }
     if (rc == OK && t.blk.d_mem) rc = tree_levels(t, inv_pin);
-    if (rc != OK) { blk_layout_destroy(&t.blk); (void)hipFree(t.d_T); delete plan; return rc; }
+    if (rc != OK) { blk_layout_destroy(&t.blk); if (t.d_T) (void)hipFree(t.d_T); delete plan; return rc; }
     *out = plan;
     return OK;
 }

@@ -599,6 +599,79 @@ static uint64_t local_rank(const std::vector<int> &beta)
 
 static size_t blk_lds_bytes(const BlkLayout &lay, int k);
 
+// Sums over modes of a table t[q][x], x the photons after mode q plus an
+// offset: cum(x, q) = t[0][x] + ... + t[q - 1][x], modulo 2^32 like every rank.
+struct BlkCum {
+    int modes;
+    std::vector<uint32_t> c;
+    template <class T>
+    BlkCum(int modes_, int xs, T t) : modes(modes_), c((size_t)xs * (modes_ + 1))
+    {
+        for (int x = 0; x < xs; x++)
+            for (int q = 0; q < modes; q++)
+                c[(size_t)x * (modes + 1) + q + 1] = c[(size_t)x * (modes + 1) + q] + (uint32_t)t(q, x);
+    }
+    const uint32_t *row(int x) const { return c.data() + (size_t)x * (modes + 1); }
+};
+
+// An occupied mode of a state: the photons after it, the sums over the modes
+// before it (of two tables) and the factorials of the modes up to it.
+struct BlkOcc {
+    int q, n, after;
+    uint32_t e, t;
+    double pf;
+};
+
+// Every state of `photons` photons in e.modes modes, descending lexicographic
+// order: f(occupied modes, their count, sum of e, sum of t, prod n!), sums at
+// x = off + photons after.  A step rewrites the last occupied modes only, and a
+// single last photon walks to the end in one loop.
+template <class F>
+static void blk_states(int photons, int off, const BlkCum &e, const BlkCum &t, F f)
+{
+    const int M = e.modes;
+    const uint32_t *e0 = e.row(off), *t0 = t.row(off);
+    if (photons == 0) {
+        f((const BlkOcc *)nullptr, 0, e0[M], t0[M], 1.0);
+        return;
+    }
+    BlkOcc occ[32];
+    int n = 0;
+    auto push = [&](int q, int v) {
+        BlkOcc o{0, 0, photons, 0, 0, 1.0};
+        if (n) o = occ[n - 1];
+        const uint32_t *er = e.row(off + o.after), *tr = t.row(off + o.after);
+        o.e += er[q] - er[o.q];
+        o.t += tr[q] - tr[o.q];
+        for (int u = 2; u <= v; u++) o.pf *= u;
+        o.q = q;
+        o.n = v;
+        o.after -= v;
+        occ[n++] = o;
+    };
+    push(0, photons);
+    while (true) {
+        BlkOcc &last = occ[n - 1];
+        auto emit = [&]() { f((const BlkOcc *)occ, n, last.e + e0[M] - e0[last.q], last.t + t0[M] - t0[last.q], last.pf); };
+        emit();
+        if (last.n == 1 && last.q < M - 1) {
+            const uint32_t *e1 = e.row(off + 1), *t1 = t.row(off + 1);
+            do {
+                last.e += e1[last.q + 1] - e1[last.q];
+                last.t += t1[last.q + 1] - t1[last.q];
+                last.q++;
+                emit();
+            } while (last.q < M - 1);
+        }
+        const int tail = last.q == M - 1 ? last.n : 0;
+        if (tail) n--;
+        if (n == 0) return;
+        const BlkOcc o = occ[--n];
+        if (o.n > 1) push(o.q, o.n - 1);
+        push(o.q + 1, tail + 1);
+    }
+}
+
 // LDS of the launch of layers 1..front.
 static size_t front_lds(const BlkLayout &lay, int front, uint32_t staged)
 {
@@ -678,6 +751,7 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     std::vector<double> spf;
     std::vector<uint32_t> sslot;
     std::vector<uint32_t> tpf((size_t)nmax + 1), tslot((size_t)nmax + 1);
+    const BlkCum drop(w, nmax + 1, [&](int q, int x) { return q + 2 <= w ? blk_binom((int64_t)x + w - q - 3, w - q - 2) : 0; });
     for (int r = 0; r <= nmax; r++) {
         const uint64_t S = nstates(w, r);
         const int ns = std::min(r, w);
@@ -686,84 +760,35 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
         const size_t p0 = spf.size(), s0 = sslot.size();
         spf.resize(p0 + S);
         sslot.resize(s0 + S * (size_t)ns, 0xffffffffu);
-        std::vector<int> beta((size_t)w, 0), after((size_t)w + 1, 0);
-        beta[0] = r;
-        for (uint64_t i = 0; i < S; i++) {
-            double pf = 1.0;
-            int d = 0;
-            // beta has rank i; taking a photon from mode j lowers the photons
-            // after each mode q < j by one, which lowers the rank by
-            // sum_{q<j} C(after_q + w - q - 3, w - q - 2) (Pascal's rule on
-            // each term of the rank sum)
-            for (int q = w - 1; q >= 0; q--) after[(size_t)q] = after[(size_t)q + 1] + beta[(size_t)q];
-            uint64_t drop = 0;
-            for (int j = 0; j < w; j++) {
-                for (int v = 2; v <= beta[(size_t)j]; v++) pf *= v;
-                if (beta[(size_t)j] > 0) {
-                    const uint64_t lp = i - drop;
-                    sslot[s0 + (size_t)d * S + i] = (uint32_t)(lp << 5) | (uint32_t)j;
-                    d++;
-                }
-                if (j + 2 <= w) drop += blk_binom((int64_t)after[(size_t)j + 1] + w - j - 3, w - j - 2);
-            }
+        // beta has rank i; taking a photon from mode j lowers the photons after
+        // each mode q < j by one, which lowers the rank by
+        // sum_{q<j} C(after_q + w - q - 3, w - q - 2) (Pascal's rule on each
+        // term of the rank sum)
+        uint64_t i = 0;
+        blk_states(r, 0, drop, drop, [&](const BlkOcc *occ, int n, uint32_t, uint32_t, double pf) {
+            for (int d = 0; d < n; d++)
+                sslot[s0 + (size_t)d * S + i] = (((uint32_t)i - occ[d].e) << 5) | (uint32_t)occ[d].q;
             spf[p0 + i] = pf;
-            // next state in descending lexicographic order
-            if (i + 1 < S) {
-                const int tail = beta[(size_t)w - 1];
-                beta[(size_t)w - 1] = 0;
-                int t = w - 2;
-                while (beta[(size_t)t] == 0) t--;
-                beta[(size_t)t]--;
-                beta[(size_t)t + 1] = tail + 1;
-            }
-        }
+            i++;
+        });
     }
     // groups per layer: each sub-layer, suffix photons r = 0..kf; the blocks
     // of whole-wave groups get their walk precomputed (records)
     lay.cmax = std::max(1, std::min(h, nmax));
     std::vector<BlkRec> recs;
-    // every block (K, r) in order: f(B_k, PE_h, (mode, PE_j) of its occupied prefix modes, prod alpha!)
-    auto for_blocks = [&](int K, int r, auto &&f) {
-        std::vector<int> alpha((size_t)h, 0);
-        alpha[0] = K;
-        const uint64_t nb = nstates(h, K);
-        std::vector<int> after((size_t)h + 1, 0);
-        std::vector<std::pair<uint32_t, uint32_t>> occ;
-        for (uint64_t i = 0; i < nb; i++) {
-            uint64_t Bk = 0, PE = 0;
-            double pf = 1.0;
-            for (int q = h - 1; q >= 0; q--) after[(size_t)q] = after[(size_t)q + 1] + alpha[(size_t)q];
-            occ.clear();
-            for (int q = 0; q < h; q++) {
-                const uint64_t tev = te[(size_t)q * wt + r + after[(size_t)q + 1]];
-                Bk += tev & 0xffffffffull;
-                if (alpha[(size_t)q] > 0) {
-                    occ.push_back({(uint32_t)q, (uint32_t)PE});
-                    for (int v = 2; v <= alpha[(size_t)q]; v++) pf *= v;
-                }
-                PE += tev >> 32;
-            }
-            f((uint32_t)Bk, (uint32_t)PE, occ, pf);
-            if (i + 1 < nb) {   // next alpha in descending lexicographic order
-                const int tail = alpha[(size_t)h - 1];
-                alpha[(size_t)h - 1] = 0;
-                int t = h - 2;
-                while (alpha[(size_t)t] == 0) t--;
-                alpha[(size_t)t]--;
-                alpha[(size_t)t + 1] = tail + 1;
-            }
-        }
-    };
-    using BlkOcc = std::vector<std::pair<uint32_t, uint32_t>>;
+    // every block (K, r) in order: f(its occupied prefix modes (e: PE_j), their
+    // count, PE_h, B_k, prod alpha!)
+    const BlkCum ce(h, wt, [&](int q, int x) { return te[(size_t)q * wt + x] >> 32; });
+    const BlkCum ct(h, wt, [&](int q, int x) { return te[(size_t)q * wt + x] & 0xffffffffull; });
     auto add_records = [&](int K, int r) {
-        for_blocks(K, r, [&](uint32_t Bk, uint32_t PEh, const BlkOcc &occ, double pf) {
+        blk_states(K, r, ce, ct, [&](const BlkOcc *occ, int n, uint32_t PEh, uint32_t Bk, double pf) {
             BlkRec rec{};
             rec.w[0] = Bk;
             rec.w[1] = PEh;
-            rec.w[2] = (uint32_t)occ.size();
-            for (size_t c = 0; c < occ.size(); c++) {
-                rec.w[4 + c / 4] |= occ[c].first << (8 * (c % 4));
-                rec.w[10 + c] = occ[c].second;
+            rec.w[2] = (uint32_t)n;
+            for (int c = 0; c < n; c++) {
+                rec.w[4 + c / 4] |= (uint32_t)occ[c].q << (8 * (c % 4));
+                rec.w[10 + c] = occ[c].e;
             }
             std::memcpy(&rec.w[8], &pf, sizeof(double));
             recs.push_back(rec);
@@ -830,50 +855,18 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
         }
         lay.items[(size_t)k] = items;
     }
-    // the first layers in one launch: how many, and their parent words
-    std::vector<uint32_t> fwords;
-    std::vector<double> fpf;
+    // the first layers in one launch: how many, and where their parent words go
     front_choose(&lay);
-    {
-        size_t words = 0;
-        for (int k = 1; k <= lay.front; k++) words += (size_t)lay.front_slots[(size_t)k] * lay.counts[(size_t)k];
-        fwords.reserve(words);
-    }
+    size_t nwords = 0;
     for (int k = 1; k <= lay.front; k++) {
-        const uint32_t cnt = (uint32_t)lay.counts[(size_t)k];
-        const bool last = k == lay.nlayers;
-        const size_t off0 = fwords.size();
-        lay.front_off[(size_t)k] = (uint32_t)off0;
-        fwords.resize(off0 + (size_t)lay.front_slots[(size_t)k] * cnt, 0xffffffffu);
-        if (last) fpf.assign(cnt, 1.0);
-        for (const BlkSub &sub : subs[(size_t)k])
-            for (int r = 0; r <= sub.kf; r++) {
-                const uint32_t S = (uint32_t)nstates(w, r);
-                const int ns = std::min(r, w);
-                for_blocks(sub.kf - r, r, [&](uint32_t Bk, uint32_t PEh, const BlkOcc &occ, double pf) {
-                    uint32_t *at = fwords.data() + off0 + sub.out_base + Bk;   // the block's children, slot by slot
-                    auto run = [&](uint32_t rank, uint32_t mode) {             // parents at consecutive ranks
-                        for (uint32_t b = 0; b < S; b++) at[b] = ((rank + b) << 8) | mode;
-                        at += cnt;
-                    };
-                    for (const auto &e : sub.her) run(e.second + Bk, (uint32_t)m + e.first);
-                    for (const auto &e : occ) run(sub.par_base + Bk - e.second, e.first);
-                    const uint32_t add = ((sub.par_base + Bk - PEh) << 8) + (uint32_t)h;
-                    for (int d = 0; d < ns; d++, at += cnt) {
-                        const uint32_t *slot = sslot.data() + tslot[(size_t)r] + (size_t)d * S;
-                        for (uint32_t b = 0; b < S; b++)
-                            at[b] = slot[b] == 0xffffffffu ? slot[b] : ((slot[b] >> 5) << 8 | (slot[b] & 31u)) + add;
-                    }
-                    if (last)
-                        for (uint32_t b = 0; b < S; b++)
-                            fpf[sub.out_base + Bk + b] = pf * spf[(size_t)tpf[(size_t)r] + b] * sub.hfact;
-                });
-            }
-        if (k < lay.front && k == lay.front_staged_layers + 1 && fwords.size() <= FRONT_STAGED) {
+        lay.front_off[(size_t)k] = (uint32_t)nwords;
+        nwords += (size_t)lay.front_slots[(size_t)k] * lay.counts[(size_t)k];
+        if (k < lay.front && k == lay.front_staged_layers + 1 && nwords <= FRONT_STAGED) {
             lay.front_staged_layers = k;
-            lay.front_staged = (uint32_t)fwords.size();
+            lay.front_staged = (uint32_t)nwords;
         }
     }
+    const size_t npf = lay.front && lay.front == lay.nlayers ? (size_t)lay.counts[(size_t)lay.front] : 0;
     // one device allocation
     auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
     size_t off = 0;
@@ -893,8 +886,8 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     lay.off_slot = off; off += al(sizeof(uint32_t) * std::max<size_t>(sslot.size(), 1));
     lay.nrec = recs.size();
     lay.off_rec = off; off += al(sizeof(BlkRec) * std::max<size_t>(recs.size(), 1));
-    lay.off_front = off; off += al(sizeof(uint32_t) * std::max<size_t>(fwords.size(), 1));
-    lay.off_front_pf = off; off += al(sizeof(double) * std::max<size_t>(fpf.size(), 1));
+    lay.off_front = off; off += al(sizeof(uint32_t) * std::max<size_t>(nwords, 1));
+    lay.off_front_pf = off; off += al(sizeof(double) * std::max<size_t>(npf, 1));
     lay.bytes = off;
     if (blk_lds_bytes(lay, lay.nlayers) > 160 * 1024) {
         set_error("block SLOS layout: the walk tables and lists outgrow the LDS (too many modes and photons)");
@@ -915,8 +908,37 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     std::memcpy(host.data() + lay.off_pf, spf.data(), sizeof(double) * spf.size());
     if (!sslot.empty()) std::memcpy(host.data() + lay.off_slot, sslot.data(), sizeof(uint32_t) * sslot.size());
     if (!recs.empty()) std::memcpy(host.data() + lay.off_rec, recs.data(), sizeof(BlkRec) * recs.size());
-    if (!fwords.empty()) std::memcpy(host.data() + lay.off_front, fwords.data(), sizeof(uint32_t) * fwords.size());
-    if (!fpf.empty()) std::memcpy(host.data() + lay.off_front_pf, fpf.data(), sizeof(double) * fpf.size());
+    // parent words of the first layers, all ones past a child's last parent
+    uint32_t *fwords = reinterpret_cast<uint32_t *>(host.data() + lay.off_front);
+    double *fpf = reinterpret_cast<double *>(host.data() + lay.off_front_pf);
+    if (nwords) std::memset(fwords, 0xff, sizeof(uint32_t) * nwords);
+    for (int k = 1; k <= lay.front; k++) {
+        const uint32_t cnt = (uint32_t)lay.counts[(size_t)k];
+        const bool last = k == lay.nlayers;
+        for (const BlkSub &sub : subs[(size_t)k])
+            for (int r = 0; r <= sub.kf; r++) {
+                const uint32_t S = (uint32_t)nstates(w, r);
+                const int ns = std::min(r, w);
+                blk_states(sub.kf - r, r, ce, ct, [&](const BlkOcc *occ, int n, uint32_t PEh, uint32_t Bk, double pf) {
+                    uint32_t *at = fwords + lay.front_off[(size_t)k] + sub.out_base + Bk;   // the block's children, slot by slot
+                    auto run = [&](uint32_t rank, uint32_t mode) {                         // parents at consecutive ranks
+                        for (uint32_t b = 0; b < S; b++) at[b] = ((rank + b) << 8) | mode;
+                        at += cnt;
+                    };
+                    for (const auto &e : sub.her) run(e.second + Bk, (uint32_t)m + e.first);
+                    for (int c = 0; c < n; c++) run(sub.par_base + Bk - occ[c].e, (uint32_t)occ[c].q);
+                    const uint32_t add = ((sub.par_base + Bk - PEh) << 8) + (uint32_t)h;
+                    for (int d = 0; d < ns; d++, at += cnt) {
+                        const uint32_t *slot = sslot.data() + tslot[(size_t)r] + (size_t)d * S;
+                        for (uint32_t b = 0; b < S; b++)
+                            at[b] = slot[b] == 0xffffffffu ? slot[b] : ((slot[b] >> 5) << 8 | (slot[b] & 31u)) + add;
+                    }
+                    if (last)
+                        for (uint32_t b = 0; b < S; b++)
+                            fpf[sub.out_base + Bk + b] = pf * spf[(size_t)tpf[(size_t)r] + b] * sub.hfact;
+                });
+            }
+    }
     *out = std::move(lay);
     return OK;
 }

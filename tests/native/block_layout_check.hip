@@ -10,7 +10,10 @@
 //   * each child's parent list, in the order it is summed, equals brute force
 //     (rank of c - e_j for the occupied modes j, increasing);
 //   * the factorial product of each child equals prod s!;
-//   * each precomputed block record equals the block's walk.
+//   * each precomputed block record equals the block's walk;
+//   * the parent words of the first layers (slos_front_kernel) are every
+//     child's parents in the order of summation, then all ones, and its last
+//     layer's factorials are prod s!.
 // The replay restates the kernel's index arithmetic line for line; it must be
 // kept in step with the kernel.  Exit status 0 when every check holds.
 #include "../../perceval_amd/csrc/slos_block.hip"
@@ -19,6 +22,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <set>
 
@@ -58,6 +62,61 @@ static uint64_t rank_of(const std::vector<int> &s)
 
 static int fails = 0;
 #define CHECK(c, ...) do { if (!(c)) { if (fails++ < 20) { printf("FAIL %s:%d ", __FILE__, __LINE__); printf(__VA_ARGS__); printf("\n"); } } } while (0)
+
+// The parent words of layers 1..front and the factorials of a front that ends
+// with the last layer; arguments as replay's.
+static void replay_front(const BlkLayout &lay, const std::vector<char> &img,
+                         const std::vector<std::vector<std::vector<int>>> &layers, const std::vector<int32_t> &perm,
+                         const char *what)
+{
+    const uint32_t *words = (const uint32_t *)(img.data() + lay.off_front);
+    const double *pf = (const double *)(img.data() + lay.off_front_pf);
+    const size_t n_words = (lay.off_front_pf - lay.off_front) / 4, n_pf = (lay.bytes - lay.off_front_pf) / 8;
+    const int32_t *rowmap = (const int32_t *)(img.data() + lay.off_row);
+    CHECK(lay.front <= lay.nlayers && lay.front_staged_layers <= lay.front, "%s: front %d", what, lay.front);
+    size_t next = 0;
+    for (int k = 1; k <= lay.front; k++) {
+        const auto &children = layers[(size_t)k], &parents = layers[(size_t)k - 1];
+        const size_t count = children.size(), slots = (size_t)lay.front_slots[(size_t)k];
+        CHECK(lay.front_off[(size_t)k] == next, "%s: first word of layer %d", what, k);
+        next += slots * count;
+        CHECK(next <= n_words, "%s: words of layer %d", what, k);
+        if (next > n_words) return;
+        if (k < lay.front) CHECK(count <= lay.front_cap[k & 1], "%s: LDS of layer %d", what, k);
+        if (k == lay.front_staged_layers) CHECK(lay.front_staged == next, "%s: staged words", what);
+        std::map<std::vector<int>, uint64_t> pidx;
+        for (size_t i = 0; i < parents.size(); i++) pidx[parents[i]] = i;
+        for (size_t c = 0; c < count; c++) {
+            std::vector<std::pair<uint64_t, int>> exp, got;
+            double pfe = 1;
+            auto parent = [&](int e) {
+                const int j = perm[(size_t)e];
+                if (children[c][(size_t)j] == 0) return;
+                auto s = children[c];
+                s[(size_t)j]--;
+                exp.push_back({pidx.at(s), j});
+            };
+            for (int e = lay.m; e < lay.mloc; e++) parent(e);
+            for (int e = 0; e < lay.m; e++) parent(e);
+            for (int v : children[c])
+                for (int u = 2; u <= v; u++) pfe *= u;
+            for (size_t d = 0; d < slots; d++) {
+                const uint32_t w = words[lay.front_off[(size_t)k] + d * count + c];
+                if (w == 0xffffffffu) {
+                    CHECK(d >= exp.size(), "%s: k=%d child %zu: word %zu missing", what, k, c, d);
+                    continue;
+                }
+                CHECK((w & 255u) < (uint32_t)lay.mloc, "%s: k=%d child %zu: mode", what, k, c);
+                got.push_back({w >> 8, rowmap[std::min<uint32_t>(w & 255u, (uint32_t)lay.mloc - 1)]});
+            }
+            CHECK(got == exp, "%s: k=%d child %zu: parent words differ", what, k, c);
+            if (k == lay.nlayers) {
+                CHECK(c < n_pf, "%s: factorial index", what);
+                if (c < n_pf) CHECK(std::abs(pf[c] - pfe) <= 1e-14 * pfe, "%s: child %zu: pf %g vs %g", what, c, pf[c], pfe);
+            }
+        }
+    }
+}
 
 // Replays every layer of a layout.  `layers[k]` lists the states of layer k in
 // the layout's order as occupation vectors over the ORIGINAL modes; `perm`
@@ -239,6 +298,7 @@ static void replay(const BlkLayout &lay, const std::vector<char> &img, const std
         for (uint64_t i = 0; i < nchild; i++)
             CHECK(written[i] == 1, "%s: layer %d child %lu written %d times", what, k, (unsigned long)i, written[i]);
     }
+    replay_front(lay, img, layers, perm, what);
 }
 
 static void emulate(int m, int nmax, int w, size_t max_records = BLK_MAX_RECORDS)
