@@ -24,6 +24,7 @@
 #include "../../include/pcvl_hip.h"
 
 #include <algorithm>
+#include <numeric>
 #include <cstring>
 #include <new>
 #include <mutex>
@@ -488,11 +489,13 @@ struct pcvl_perm_plan_s {
 // device); partial-sum slots are int32 on the device.
 static constexpr int64_t PERM_MAX_ITEMS = int64_t(1) << 27;
 
-// Device image of a plan: one block holding items | cursor | partials | wave
-// arrays | small arrays, at these byte offsets.
+// Device block of a plan: items | cursor | wave arrays | small arrays | groups |
+// partials, at these byte offsets.
 struct PermLayout {
     size_t o_items = 0, o_cursor = 0, o_part = 0, o_widx = 0, o_ws0 = 0, o_wns = 0, o_wn = 0, o_sidx = 0,
            o_soff = 0, o_sn = 0, o_groups = 0, total = 0;
+    size_t image = 0;     // bytes that are uploaded: all but the partials, which the waves write
+    size_t scratch = 0;   // bytes that count against the scratch of pcvl_perm_batch_noalloc: all but the groups
 };
 
 // Cuts items [i0, i1) of the sorted queue into the groups that a wave takes at
@@ -504,28 +507,40 @@ struct PermLayout {
 // item), the first groups, one a wave and not pulled, hold 70% of the work (a
 // slow CU takes 1.3 times the average), and the rest is cut into as many groups
 // as pulls fit into the work's time.  Otherwise every item is a group.
-static int64_t perm_groups(const std::vector<PermItem> &items, int64_t i0, int64_t i1, int resident,
+//
+// perm_cost: an item's seconds of one SIMD: blocks, and the sums and constants
+// before them; total: of all items.
+static double perm_cost(int n, int c)
+{
+    constexpr double ISSUE = 4.0 / 2.1e9;
+    return ISSUE * (4.3 * n * std::ldexp(1.0, c) + 2.0 * n * n + 40.0 * n);
+}
+
+static int64_t perm_groups(const std::vector<PermItem> &items, int64_t i0, int64_t i1, int resident, double total,
                            std::vector<uint32_t> &starts)
 {
-    constexpr double PULL = 15e-9, ISSUE = 4.0 / 2.1e9, SIMDS = 1024.0;
-    auto cost = [&](int64_t i) {   // seconds of one SIMD: blocks, and the sums and constants before them
-        const double n = items[(size_t)i].n;
-        return ISSUE * (4.3 * n * std::ldexp(1.0, items[(size_t)i].c) + 2.0 * n * n + 40.0 * n);
-    };
+    constexpr double PULL = 15e-9, SIMDS = 1024.0;
     const int64_t count = i1 - i0, first = (int64_t)starts.size();
-    double total = 0.0;
-    for (int64_t i = i0; i < i1; i++) total += cost(i);
-    const bool single = count <= resident || (double)count * PULL * 4.0 * SIMDS <= total;
+    auto each_item = [&]() {
+        starts.resize((size_t)(first + count + 1));
+        std::iota(starts.begin() + first, starts.end(), (uint32_t)i0);
+        return count;
+    };
+    if (count <= resident || (double)count * PULL * 4.0 * SIMDS <= total) return each_item();
     const double pulls = std::max(total / SIMDS / PULL, 1.0);
     const double own = 0.7 * total / std::max(resident, 1), pulled = 0.3 * total / pulls;
     double sum = 0.0;
+    int n = -1, c = -1;
+    double cost = 0.0;
     for (int64_t i = i0; i < i1; i++) {
+        const PermItem &it = items[(size_t)i];
+        if (it.n != n || it.c != c) cost = perm_cost(n = it.n, c = it.c);
         const double want = (int64_t)starts.size() - first <= resident ? own : pulled;
-        if (single || i == i0 || sum + 0.5 * cost(i) >= want) {
+        if (i == i0 || sum + 0.5 * cost >= want) {
             starts.push_back((uint32_t)i);
             sum = 0.0;
         }
-        sum += cost(i);
+        sum += cost;
     }
     const int64_t groups = (int64_t)starts.size() - first;
     starts.push_back((uint32_t)i1);
@@ -545,8 +560,9 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
     PCVL_ARG_CHECK(max_chunk_log2 >= 2 && max_chunk_log2 <= 24, "max_chunk_log2 outside [2, 24]");
 
     std::vector<PermItem> items;
-    std::vector<int64_t> wave_idx, small_idx, small_off;
-    std::vector<int32_t> wave_slot0, wave_nslot, wave_n, small_n;
+    std::vector<int64_t> wave_idx;
+    std::vector<int32_t> wave_slot0, wave_nslot, wave_n;
+    int64_t small_at[PERM_SMALL_MAX + 2] = {};   // small matrices of each order, then the first of each
     std::vector<int> wave_c;
     int nmin = 1 << 30, nmax = -1;
     bool any_big = false;
@@ -555,7 +571,7 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
         PCVL_ARG_CHECK(n >= 0 && n <= PERM_BIG_MAX, "matrix order outside [0, 32]");
         PCVL_ARG_CHECK(h_offsets[b] >= 0, "negative matrix offset");
         if (n <= PERM_SMALL_MAX) {
-            small_idx.push_back(b);
+            small_at[n + 1]++;
             continue;
         }
         wave_idx.push_back(b);
@@ -569,12 +585,9 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
         nmax = std::max(nmax, n);
     }
     // the small ones by order, a thread each first
-    std::stable_sort(small_idx.begin(), small_idx.end(), [&](int64_t a, int64_t b) { return h_n[a] < h_n[b]; });
-    for (int64_t b : small_idx) {
-        small_off.push_back(h_offsets[b]);
-        small_n.push_back(h_n[b]);
-        if (h_n[b] <= PERM_THREAD_MAX) p.nthread++;
-    }
+    for (int n = 0; n <= PERM_SMALL_MAX; n++) small_at[n + 1] += small_at[n];
+    const size_t nsmall = (size_t)small_at[PERM_SMALL_MAX + 1];
+    p.nthread = small_at[PERM_THREAD_MAX + 1];
     // orders <= 28: one launch, specialised when they share one order
     const int single_n = (nmax >= 0 && nmin == nmax) ? nmax : 0;
     const int kvariant = single_n ? variant : 0;
@@ -620,12 +633,14 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
     }
     items.reserve((size_t)total_slots);
     std::vector<PermItem> big_items;
+    double work[2] = {0.0, 0.0};   // of the queue's two parts
     int32_t slots = 0;
     for (size_t i = 0; i < wave_idx.size(); i++) {
         const int n = wave_n[i], c = wave_c[i];
         const int64_t waves = (int64_t)((1ull << (n - 1 - c)) / 64);
         wave_slot0.push_back(slots);
         wave_nslot.push_back((int32_t)waves);
+        work[n >= PERM_BIG_MIN] += (double)waves * perm_cost(n, c);
         std::vector<PermItem> &dst = n >= PERM_BIG_MIN ? big_items : items;
         for (int64_t w = 0; w < waves; w++)
             dst.push_back(PermItem{h_offsets[wave_idx[i]], (uint32_t)(w * 64), slots + (int32_t)w, n, c});
@@ -643,15 +658,15 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
     items.insert(items.end(), big_items.begin(), big_items.end());
 
     std::vector<uint32_t> groups;
-    p.ngroups = perm_groups(items, 0, nregular, rw, groups);
-    p.nbig_groups = perm_groups(items, nregular, (int64_t)items.size(), rwb, groups);
+    p.ngroups = perm_groups(items, 0, nregular, rw, work[0], groups);
+    p.nbig_groups = perm_groups(items, nregular, (int64_t)items.size(), rwb, work[1], groups);
 
     p.count = count;
     p.nitems = nregular;
     p.nbig = (int64_t)big_items.size();
     p.grid_big = p.nbig > 0 ? (int)std::min<int64_t>(p.nbig_groups, (int64_t)rwb) : 0;
     p.nwave_mats = (int64_t)wave_idx.size();
-    p.nsmall = (int64_t)small_idx.size();
+    p.nsmall = (int64_t)nsmall;
     p.single_n = single_n;
     p.variant = kvariant;
     p.grid = p.nitems > 0 ? (int)std::min<int64_t>(p.ngroups, (int64_t)rw) : 0;
@@ -659,27 +674,37 @@ static int perm_plan_build(const int32_t *h_n, const int64_t *h_offsets, int64_t
     auto align = [](size_t x) { return (x + 255) & ~size_t(255); };
     L.o_items = 0;
     L.o_cursor = align(L.o_items + sizeof(PermItem) * items.size());
-    L.o_part = align(L.o_cursor + 2 * sizeof(unsigned long long));
-    L.o_widx = align(L.o_part + sizeof(cd) * (size_t)slots);
+    L.o_widx = align(L.o_cursor + 2 * sizeof(unsigned long long));
     L.o_ws0 = align(L.o_widx + sizeof(int64_t) * wave_idx.size());
     L.o_wns = align(L.o_ws0 + sizeof(int32_t) * wave_idx.size());
     L.o_wn = align(L.o_wns + sizeof(int32_t) * wave_idx.size());
     L.o_sidx = align(L.o_wn + sizeof(int32_t) * wave_idx.size());
-    L.o_soff = align(L.o_sidx + sizeof(int64_t) * small_idx.size());
-    L.o_sn = align(L.o_soff + sizeof(int64_t) * small_idx.size());
-    L.o_groups = align(L.o_sn + sizeof(int32_t) * small_idx.size());
-    L.total = align(L.o_groups + sizeof(uint32_t) * groups.size());
+    L.o_soff = align(L.o_sidx + sizeof(int64_t) * nsmall);
+    L.o_sn = align(L.o_soff + sizeof(int64_t) * nsmall);
+    L.o_groups = align(L.o_sn + sizeof(int32_t) * nsmall);
+    L.o_part = align(L.o_groups + sizeof(uint32_t) * groups.size());
+    L.total = align(L.o_part + sizeof(cd) * (size_t)slots);
+    L.image = L.o_part;
+    L.scratch = L.total - (L.o_part - L.o_groups);
 
-    host.assign(L.total, 0);
+    host.assign(L.image, 0);
     auto put = [&](size_t off, const void *src, size_t bytes) { if (bytes) std::memcpy(host.data() + off, src, bytes); };
     put(L.o_items, items.data(), sizeof(PermItem) * items.size());
     put(L.o_widx, wave_idx.data(), sizeof(int64_t) * wave_idx.size());
     put(L.o_ws0, wave_slot0.data(), sizeof(int32_t) * wave_idx.size());
     put(L.o_wns, wave_nslot.data(), sizeof(int32_t) * wave_idx.size());
     put(L.o_wn, wave_n.data(), sizeof(int32_t) * wave_idx.size());
-    put(L.o_sidx, small_idx.data(), sizeof(int64_t) * small_idx.size());
-    put(L.o_soff, small_off.data(), sizeof(int64_t) * small_idx.size());
-    put(L.o_sn, small_n.data(), sizeof(int32_t) * small_idx.size());
+    int64_t *small_idx = reinterpret_cast<int64_t *>(host.data() + L.o_sidx);
+    int64_t *small_off = reinterpret_cast<int64_t *>(host.data() + L.o_soff);
+    int32_t *small_n = reinterpret_cast<int32_t *>(host.data() + L.o_sn);
+    for (int64_t b = 0; nsmall && b < count; b++) {
+        const int n = h_n[b];
+        if (n > PERM_SMALL_MAX) continue;
+        const int64_t at = small_at[n]++;
+        small_idx[at] = b;
+        small_off[at] = h_offsets[b];
+        small_n[at] = n;
+    }
     put(L.o_groups, groups.data(), sizeof(uint32_t) * groups.size());
     return OK;
 }
@@ -720,7 +745,7 @@ static int perm_plan_create_impl(const int32_t *h_n, const int64_t *h_offsets, i
         return ERR_ALLOC;
     }
     perm_plan_bind(p, L, p.d_block);
-    e = hipMemcpy(p.d_block, host.data(), L.total, hipMemcpyHostToDevice);
+    e = hipMemcpy(p.d_block, host.data(), L.image, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         set_error(std::string("hipMemcpy(perm plan): ") + hipGetErrorString(e));
         (void)hipFree(p.d_block);
@@ -867,8 +892,8 @@ static int perm_batch_noalloc_impl(const double *d_mats, const int32_t *h_n, con
     std::vector<char> host;
     int rc = perm_plan_build(h_n, h_offsets, count, 0, 0, p, L, host);
     if (rc != OK) return rc;
-    if (L.o_groups > PERM_SCRATCH_BYTES) {
-        set_error("permanent batch needs " + std::to_string(L.o_groups) + " bytes of plan scratch, above the " +
+    if (L.scratch > PERM_SCRATCH_BYTES) {
+        set_error("permanent batch needs " + std::to_string(L.scratch) + " bytes of plan scratch, above the " +
                   std::to_string(PERM_SCRATCH_BYTES) + " of pcvl_perm_batch_noalloc (split the batch or use "
                   "pcvl_perm_batch)");
         return ERR_RANGE;
@@ -879,7 +904,7 @@ static int perm_batch_noalloc_impl(const double *d_mats, const int32_t *h_n, con
     rc = scratch_ptr(&base);
     if (rc != OK) return rc;
     perm_plan_bind(p, L, base);
-    PCVL_HIP_CHECK(hipMemcpyAsync(base, host.data(), L.total, hipMemcpyHostToDevice, stream));
+    PCVL_HIP_CHECK(hipMemcpyAsync(base, host.data(), L.image, hipMemcpyHostToDevice, stream));
     rc = pcvl_perm_plan_execute(&plan, d_mats, d_out, stream);
     // the host image must outlive its copy, and results are ready on return
     hipError_t e = hipStreamSynchronize(stream);
