@@ -6,7 +6,7 @@
 // Step t of the binary-reflected Gray code flips row 1 + ctz(t); the sign of
 // term t is (-1)^t.
 //
-// Work decomposition (orders 9..28): the 2^{n-1} terms of a matrix are cut
+// Work decomposition (orders 11..28): the 2^{n-1} terms of a matrix are cut
 // into lane chunks of 2^c terms; one wavefront takes 64 consecutive chunks.
 // The lowest one or two rows after row 0 are the low rows: a block of 2 or 4
 // terms takes every low sign pattern, and the Gray code runs over the high
@@ -17,8 +17,8 @@
 // each chunk start, which bounds their drift to 2^(c-2) or 2^(c-1) updates.
 // One persistent launch drains a cost-sorted queue of wave items of mixed
 // order (largest first), then a second kernel sums each matrix's wave partials
-// in a fixed order (bit-reproducible).  Orders 0..8 take 16 lanes per
-// matrix.
+// in a fixed order (bit-reproducible).  Orders 0..5 take a thread per matrix,
+// 6..10 16 lanes.
 #include "common.h"
 #include "glynn_blocks.h"
 #include "../../include/pcvl_hip.h"
@@ -73,7 +73,7 @@ constexpr int perm_low_rows(int n, bool one) { return (n <= PERM_LOW2_MAX && !on
 template <int N, int LOW>
 __device__ __forceinline__ cd glynn_wave_item(const double *__restrict__ mats, const PermItem &it, cd *sA)
 {
-    static_assert(N >= 9 && (LOW == 1 || LOW == 2), "unsupported order or low rows");
+    static_assert(N >= PERM_WAVE_MIN && (LOW == 1 || LOW == 2), "unsupported order or low rows");
     constexpr int P = N / 2;
     constexpr bool ODD = (N & 1) != 0;
     const int lane = threadIdx.x & 63;
@@ -340,11 +340,12 @@ __device__ __forceinline__ cd dispatch_row(int n, const cd *A, int lane)
 // lanes, of order 6 65 and 23.  PERM_SMALL_MAX: 20,000 of order 11 are 112 us in
 // the queue, and 16 lanes would do 64 terms each, ten times order 8's work.
 constexpr int PERM_ROWS = 16;
+constexpr int64_t PERM_ROW_LAUNCH = int64_t(1) << 22;   // matrices of one launch, milliseconds of work
 constexpr int PERM_ROW_LD = PERM_SMALL_MAX * PERM_SMALL_MAX + 1;   // the four matrices of a wave on different banks
 
 __global__ void __launch_bounds__(16 * PERM_ROWS, 4) perm_small_kernel(
     const double *__restrict__ mats, const int64_t *__restrict__ idx, const int64_t *__restrict__ offs,
-    const int32_t *__restrict__ ns, int64_t count, int64_t nthread, unsigned first, cd *__restrict__ out)
+    const int32_t *__restrict__ ns, int64_t count, int64_t nthread, int64_t row0, unsigned first, cd *__restrict__ out)
 {
     __shared__ cd s_mat[PERM_ROWS * PERM_ROW_LD];
     if (blockIdx.x < first) {
@@ -353,7 +354,7 @@ __global__ void __launch_bounds__(16 * PERM_ROWS, 4) perm_small_kernel(
         return;
     }
     const int lane = threadIdx.x & 15, row = threadIdx.x >> 4;
-    const int64_t k = nthread + (int64_t)(blockIdx.x - first) * PERM_ROWS + row;
+    const int64_t k = row0 + (int64_t)(blockIdx.x - first) * PERM_ROWS + row;
     const bool in = k < count;
     const int n = in ? ns[k] : 0;
     cd *A = s_mat + row * PERM_ROW_LD;
@@ -784,11 +785,17 @@ extern "C" int pcvl_perm_plan_execute(pcvl_perm_plan plan, const double *d_mats,
     PCVL_ARG_CHECK(d_mats && d_out, "null device buffer");
     cd *out = reinterpret_cast<cd *>(d_out);
     if (p.nsmall > 0) {
-        const unsigned first = (unsigned)((p.nthread + 16 * PERM_ROWS - 1) / (16 * PERM_ROWS));
-        const unsigned rows = (unsigned)((p.nsmall - p.nthread + PERM_ROWS - 1) / PERM_ROWS);
-        hipLaunchKernelGGL(perm_small_kernel, dim3(first + rows), dim3(16 * PERM_ROWS), 0, stream, d_mats,
-                           p.d_small_idx, p.d_small_off, p.d_small_n, p.nsmall, p.nthread, first, out);
-        PCVL_HIP_CHECK(hipGetLastError());
+        unsigned first = (unsigned)((p.nthread + 16 * PERM_ROWS - 1) / (16 * PERM_ROWS));
+        int64_t row0 = p.nthread;
+        do {   // PERM_ROW_LAUNCH at a time: a grid holds fewer than 2^32 threads, 2^28 such matrices
+            const int64_t end = std::min(p.nsmall, row0 + PERM_ROW_LAUNCH);
+            const unsigned rows = (unsigned)((end - row0 + PERM_ROWS - 1) / PERM_ROWS);
+            hipLaunchKernelGGL(perm_small_kernel, dim3(first + rows), dim3(16 * PERM_ROWS), 0, stream, d_mats,
+                               p.d_small_idx, p.d_small_off, p.d_small_n, end, p.nthread, row0, first, out);
+            PCVL_HIP_CHECK(hipGetLastError());
+            first = 0;
+            row0 = end;
+        } while (row0 < p.nsmall);
     }
     if (p.nwave_mats > 0) {
         int rc = OK;

@@ -4,6 +4,7 @@ Bar (north star): relative error <= 1e-10 against a complex128 CPU oracle; the
 oracle here is the long-double Glynn of oracle/pcvl_oracle.c, itself pinned in
 tests/test_oracle.py.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -205,3 +206,48 @@ def test_plan_refuses_more_work_items_than_it_can_index(gpu):
     with pytest.raises(NativeError, match="work items"):
         PermanentPlan([28] * 4096, max_chunk_log2=2)
     PermanentPlan([28] * 4, max_chunk_log2=11).close()
+
+
+@pytest.mark.parametrize("n", [11, 12])
+@pytest.mark.parametrize("variant", [0, 2])
+def test_smallest_orders_of_the_wave_path(gpu, n, variant):
+    """The smallest orders that take waves: one block per lane (its sign is the
+    lane's), two, and as many as fit, with two low rows and with one."""
+    import torch
+    from perceval_amd.permanent import PermanentPlan, pack
+    rng = np.random.RandomState(n)
+    mats = [(rng.randn(n, n) + 1j * rng.randn(n, n)) * 10.0 ** rng.uniform(-3, 3, size=n) for _ in range(5)]
+    orders, flat = pack(mats)
+    ref = _oracle(mats)
+    for chunk in (2, 3, 11):
+        plan = PermanentPlan(orders, max_chunk_log2=chunk, variant=variant)
+        got = plan(torch.from_numpy(flat).cuda()).cpu().numpy()
+        plan.close()
+        for g, r in zip(got, ref):
+            assert _rel(g, r) < REL_TOL, (n, chunk, variant, g, r)
+
+
+def test_small_matrices_in_several_launches(gpu):
+    """More matrices of 16 lanes each than one launch takes (2^22), behind some
+    of a thread each: all of them share a few matrices."""
+    import torch
+    from perceval_amd import _native
+    from perceval_amd.permanent import pack
+    lib = _native.load()
+    rng = np.random.RandomState(3)
+    mats = [rng.randn(n, n) + 1j * rng.randn(n, n) for n in (3, 6, 7)]
+    orders, flat = pack(mats)
+    offs = np.concatenate([[0], np.cumsum(orders.astype(np.int64) ** 2)[:-1]])
+    which = np.arange((1 << 22) + 5000) % 2 + 1
+    which[::1000] = 0
+    ns = np.ascontiguousarray(orders[which], dtype=np.int32)
+    of = np.ascontiguousarray(offs[which], dtype=np.int64)
+    out = torch.full((len(which),), complex(np.nan, np.nan), dtype=torch.complex128, device="cuda")
+    d = torch.from_numpy(flat).cuda()
+    assert lib.pcvl_perm_batch(_native.ptr(d), ns.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)),
+                               of.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)), len(ns), _native.ptr(out),
+                               _native.stream_handle()) == 0
+    ref = oracle.perm_batch(mats, precise=True)
+    got = out.cpu().numpy()
+    for k, r in enumerate(ref):
+        assert np.max(np.abs(got[which == k] - r)) < REL_TOL * abs(r), k
