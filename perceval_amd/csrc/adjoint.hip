@@ -646,53 +646,65 @@ extern "C" int pcvl_mesh_plan_create(const int32_t *h_kind, const int32_t *h_mod
         }
     }
     // cells: an op joins the cell that last touched its modes; a phase on a
-    // mode that no cell has touched waits for the first one that does
-    struct Cell { int q; bool single; int level; std::vector<int> ops; };
+    // mode that no cell has touched joins the first one that does, or has the
+    // mode to itself
+    struct Cell { int32_t q, level, ops; bool single; };
     std::vector<Cell> cells;
-    std::vector<int> last((size_t)m, -1);
-    std::vector<std::vector<int>> waiting((size_t)m);
+    std::vector<int32_t> last((size_t)m, -1), first((size_t)m, -1), cell_of((size_t)nops, -1);
     int nlev = 0;
     for (int p = 0; p < nops; p++) {
         const int q = ops[p].q;
-        if (ops[p].kind == 0) {
-            if (last[q] >= 0) cells[(size_t)last[q]].ops.push_back(p);
-            else waiting[q].push_back(p);
-            continue;
+        int32_t c = last[q];
+        if (ops[p].kind == 1 && (c < 0 || c != last[q + 1])) {   // only a cell of this pair touches both
+            Cell cell{q, 0, 0, false};
+            c = (int32_t)cells.size();
+            for (int x : {q, q + 1}) {
+                if (last[x] >= 0) cell.level = std::max(cell.level, cells[(size_t)last[x]].level + 1);
+                else first[x] = c;
+                last[x] = c;
+            }
+            cells.push_back(cell);
         }
-        if (last[q] >= 0 && last[q] == last[q + 1]) {   // only a cell of this pair touches both
-            cells[(size_t)last[q]].ops.push_back(p);
-            continue;
-        }
-        Cell c{q, false, 0, {}};
-        for (int x : {q, q + 1}) {
-            if (last[x] >= 0) c.level = std::max(c.level, cells[(size_t)last[x]].level + 1);
-            c.ops.insert(c.ops.end(), waiting[x].begin(), waiting[x].end());
-            waiting[x].clear();
-        }
-        c.ops.push_back(p);
-        last[q] = last[q + 1] = (int)cells.size();
-        cells.push_back(std::move(c));
+        cell_of[(size_t)p] = c;
     }
-    for (int q = 0; q < m; q++)
-        if (!waiting[q].empty()) cells.push_back(Cell{q, true, 0, waiting[q]});
-    std::stable_sort(cells.begin(), cells.end(), [](const Cell &a, const Cell &b) { return a.level < b.level; });
+    for (int p = 0; p < nops; p++) {
+        int32_t &c = cell_of[(size_t)p];
+        if (c < 0) {
+            const int q = ops[p].q;
+            if (first[q] < 0) {
+                first[q] = (int32_t)cells.size();
+                cells.push_back(Cell{q, 0, 0, true});
+            }
+            c = first[q];
+        }
+        cells[(size_t)c].ops++;
+    }
     for (const Cell &c : cells) nlev = std::max(nlev, c.level + 1);
     AdjIdx X;
     X.nlev = nlev;
     X.ncells = (int)cells.size();
     X.glog = 0;
     while ((1 << X.glog) < m) X.glog++;
-    std::vector<int32_t> idx;
-    X.cell = (int)idx.size();   // 0
-    std::vector<MeshOp> sorted;   // the program cell by cell
-    sorted.reserve(ops.size());
-    std::vector<int32_t> lstart((size_t)nlev + 1, 0);
-    for (const Cell &c : cells) {
-        idx.push_back(((int32_t)sorted.size() << 6) | (c.single ? 32 : 0) | c.q);
-        for (int p : c.ops) sorted.push_back(ops[p]);
-        lstart[(size_t)c.level + 1]++;
+    // in level order, and the program cell by cell
+    std::vector<int32_t> lstart((size_t)nlev + 1, 0), at((size_t)X.ncells), order((size_t)X.ncells);
+    for (const Cell &c : cells) lstart[(size_t)c.level + 1]++;
+    for (int lv = 0; lv < nlev; lv++) lstart[(size_t)lv + 1] += lstart[(size_t)lv];
+    {
+        std::vector<int32_t> next(lstart);
+        for (int c = 0; c < X.ncells; c++) order[(size_t)next[(size_t)cells[(size_t)c].level]++] = c;
     }
-    idx.push_back((int32_t)sorted.size() << 6);
+    std::vector<int32_t> idx;
+    idx.reserve((size_t)X.ncells + 1);
+    X.cell = (int)idx.size();   // 0
+    int32_t nsorted = 0;
+    for (int32_t c : order) {
+        at[(size_t)c] = nsorted;
+        idx.push_back((nsorted << 6) | (cells[(size_t)c].single ? 32 : 0) | cells[(size_t)c].q);
+        nsorted += cells[(size_t)c].ops;
+    }
+    idx.push_back(nsorted << 6);
+    std::vector<MeshOp> sorted(ops.size());
+    for (int p = 0; p < nops; p++) sorted[(size_t)at[(size_t)cell_of[(size_t)p]]++] = ops[(size_t)p];
     ops.swap(sorted);
     // phases of several shifters and the cells that hold them, in order
     std::vector<int32_t> shared;
@@ -720,7 +732,6 @@ extern "C" int pcvl_mesh_plan_create(const int32_t *h_kind, const int32_t *h_mod
         shared.insert(shared.end(), prms.begin(), prms.end());
         for (const auto &h : held) shared.insert(shared.end(), h.begin(), h.end());
     }
-    for (int lv = 0; lv < nlev; lv++) lstart[(size_t)lv + 1] += lstart[(size_t)lv];
     X.lstart = (int)idx.size();
     idx.insert(idx.end(), lstart.begin(), lstart.end());
     const int common = (int)idx.size();
@@ -775,15 +786,15 @@ extern "C" int pcvl_mesh_plan_create(const int32_t *h_kind, const int32_t *h_mod
     // per sub-block and mode i the (s, r) whose target row is i (rstart[b * (m + 1) + i])
     X.rstart = (int)idx.size();
     const int nsub = (ntargets + sub - 1) / sub;
-    std::vector<int32_t> rstart((size_t)nsub * (m + 1), 0), rlist;
+    std::vector<int32_t> rstart((size_t)nsub * (m + 1), 0), rlist((size_t)ntargets * n), next((size_t)m);
     for (int b = 0; b < nsub; b++) {
         const int e0 = b * sub * n, e1 = std::min(ntargets, (b + 1) * sub) * n;
-        for (int i = 0; i < m; i++) {
-            rstart[(size_t)b * (m + 1) + i] = (int32_t)rlist.size();
-            for (int e = e0; e < e1; e++)
-                if (tmodes[(size_t)e] == i) rlist.push_back(e);
-        }
-        rstart[(size_t)b * (m + 1) + m] = (int32_t)rlist.size();
+        int32_t *rs = rstart.data() + (size_t)b * (m + 1);
+        rs[0] = e0;
+        for (int e = e0; e < e1; e++) rs[tmodes[(size_t)e] + 1]++;
+        for (int i = 0; i < m; i++) rs[i + 1] += rs[i];
+        std::copy(rs, rs + m, next.begin());
+        for (int e = e0; e < e1; e++) rlist[(size_t)next[(size_t)tmodes[(size_t)e]]++] = e;
     }
     idx.insert(idx.end(), rstart.begin(), rstart.end());
     X.rlist = (int)idx.size();
