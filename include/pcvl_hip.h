@@ -374,7 +374,7 @@ int pcvl_mlp_adam_multi(int tensors, float *const *d_w, const float *const *d_g,
  * photons over m modes with H hidden units, for R rows x (R x (m + n)) with
  * targets and mask bounds, in one pass (deterministic).  Networks up to 64
  * modes, 96 inputs (m + n) and 256 hidden units; the workspace call returns 0
- * floats for larger ones, which the products above compute.  d_work is aligned
+ * floats for larger and empty ones, which the products above compute.  d_work is aligned
  * to 16 bytes. */
 int pcvl_mis_grads_workspace(int R, int m, int n, int H, int64_t *floats);
 int pcvl_mis_grads(const float *d_x, int R, int m, int n, int H, const uint16_t *d_W1, const float *d_b1,

@@ -939,9 +939,9 @@ extern "C" int pcvl_mlp_ce(const float *d_logits, int M, int m, const int32_t *d
 extern "C" int pcvl_mis_grads_workspace(int R, int m, int n, int H, int64_t *floats)
 {
     PCVL_ARG_CHECK(floats != nullptr, "null output pointer");
-    PCVL_ARG_CHECK(R >= 0 && m >= 1 && n >= 1 && H >= 1, "negative or empty size");
+    PCVL_ARG_CHECK(R >= 0 && m >= 0 && n >= 0 && H >= 0, "negative size");
     *floats = 0;
-    if (m > TG_M || H > TG_H || m + n > 16 * TG_DT) return OK;
+    if (m < 1 || n < 1 || H < 1 || m > TG_M || H > TG_H || m + n > 16 * TG_DT) return OK;
     const int64_t tiles = ((int64_t)R + TG_ROWS - 1) / TG_ROWS;
     *floats = std::max<int64_t>(1, std::min<int64_t>(tiles, TG_BLOCKS)) *
               4 * tg_part((m + n + 15) / 16);
@@ -974,7 +974,7 @@ extern "C" int pcvl_mis_grads(const float *d_x, int R, int m, int n, int H, cons
     int64_t need = 0;
     const int rc = pcvl_mis_grads_workspace(R, m, n, H, &need);
     if (rc != OK) return rc;
-    PCVL_ARG_CHECK(need > 0, "network larger than 64 modes, 96 inputs or 256 hidden units");
+    PCVL_ARG_CHECK(need > 0, "network empty or larger than 64 modes, 96 inputs or 256 hidden units");
     PCVL_ARG_CHECK(d_W1 && d_b1 && d_W2 && d_b2 && d_dW1 && d_db1 && d_dW2 && d_db2, "null device buffer");
     PCVL_ARG_CHECK(R == 0 || (d_x && d_target && d_lo && d_loss), "null device buffer");
     PCVL_ARG_CHECK(d_work && work_floats >= need, "workspace too small");
@@ -1004,6 +1004,7 @@ extern "C" int pcvl_mlp_adam_multi(int tensors, float *const *d_w, const float *
     AdamTensors T = {};
     int64_t most = 0;
     for (int k = 0; k < tensors; k++) {
+        PCVL_ARG_CHECK(counts[k] <= 0 || (d_w[k] && d_g[k] && d_m1[k] && d_m2[k]), "null device buffer");
         T.w[k] = d_w[k];
         T.g[k] = d_g[k];
         T.m1[k] = d_m1[k];

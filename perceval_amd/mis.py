@@ -132,12 +132,12 @@ class ProposalNet:
         n = len(pairs)
 
         def table(tensors):
-            return (ctypes.c_void_p * n)(*(None if t is None else _p(t) for t in tensors))
+            return (ctypes.c_void_p * n)(*(_p(t) for t in tensors))
         counts = (ctypes.c_int64 * n)(*(p.numel() for p, _ in pairs))
+        bf16 = (ctypes.c_void_p * n)(*(_p(self.W1b), None, _p(self.W2b), None)[:n])
         _native.check(_lib().pcvl_mlp_adam_multi(n, table(p for p, _ in pairs), table(g for _, g in pairs),
                                                  table(self._m1[:n]), table(self._m2[:n]),
-                                                 table((self.W1b, None, self.W2b, None)[:n]), counts, lr, beta1,
-                                                 beta2, eps, self._step, _s()), "adam")
+                                                 bf16, counts, lr, beta1, beta2, eps, self._step, _s()), "adam")
 
     # ------------------------------------------------------------------ data
     def teacher_forcing(self, seqs):

@@ -234,6 +234,32 @@ def test_entry_points_reject_bad_arguments_before_touching_the_device():
     assert rc == -4 and "LDS" in lib.pcvl_last_error().decode() and not plan.value
 
 
+def test_training_entry_points_refuse_null_tensors_and_pass_on_empty_networks():
+    """A tensor without gradient (or weights, or moments) is refused on the host;
+    empty networks are left to the general products, like large ones."""
+    import ctypes
+    from perceval_amd import _native
+    lib = _native.load(require_gpu=False)
+    some = ctypes.c_void_p(4096)   # never read: the null is found first
+    counts = (ctypes.c_int64 * 2)(5, 3)
+
+    def table(*p):
+        return (ctypes.c_void_p * 2)(*p)
+    full, wb = table(some, some), table(None, None)
+    for k in range(4):
+        args = [table(some, None) if i == k else full for i in range(4)]
+        assert lib.pcvl_mlp_adam_multi(2, *args, wb, counts, 1e-3, 0.9, 0.999, 1e-8, 1, None) != 0
+        assert "null device buffer" in lib.pcvl_last_error().decode()
+    assert lib.pcvl_mlp_adam(some, None, some, some, None, 5, 1e-3, 0.9, 0.999, 1e-8, 1, None) != 0
+    assert lib.pcvl_mlp_adam_multi(2, wb, wb, wb, wb, wb, (ctypes.c_int64 * 2)(0, 0), 1e-3, 0.9, 0.999, 1e-8, 1, None) == 0
+    f = ctypes.c_int64()
+    for m, n, H in ((5, 0, 16), (0, 3, 16), (5, 3, 0), (65, 3, 16)):
+        f.value = -1
+        assert lib.pcvl_mis_grads_workspace(10, m, n, H, ctypes.byref(f)) == 0 and f.value == 0
+    assert lib.pcvl_mis_grads_workspace(10, 5, 3, 16, ctypes.byref(f)) == 0 and f.value > 0
+    assert lib.pcvl_mis_grads_workspace(-1, 5, 3, 16, ctypes.byref(f)) != 0
+
+
 def test_output_submatrices_match_the_per_state_construction():
     """The batched gather of the Naive submatrices (rows: output photons'
     modes, columns: input photons' modes, ascending with repetition,

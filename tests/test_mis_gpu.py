@@ -426,3 +426,23 @@ def test_multiset_permanents_many_short_slices(gpu):
     # both sum 2^15 terms of products of 16 column sums in double: 1e-12 of the
     # largest permanent of the batch
     assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b))
+
+
+def test_training_step_without_a_gradient_or_photons(gpu):
+    """A missing gradient is refused before a kernel reads it; a network of no
+    photons takes the general products."""
+    import torch
+    from perceval_amd.mis import ProposalNet
+    net = ProposalNet(6, 3, hidden=16)
+    before = [p.clone() for p in net.params]
+    grads = [torch.ones_like(p) for p in net.params]
+    with pytest.raises(AttributeError):
+        net.adam_step(grads[:1] + [None] + grads[2:])
+    assert all(torch.equal(a, b) for a, b in zip(before, net.params))
+    net.adam_step(grads[:2])
+    assert not torch.equal(before[1], net.params[1]) and torch.equal(before[2], net.params[2])
+    empty = ProposalNet(4, 0, hidden=8)
+    x = torch.zeros((3, 4), dtype=torch.float32, device="cuda")
+    lo = torch.zeros(3, dtype=torch.int32, device="cuda")
+    loss, grads = empty.loss_and_grads(x, lo, lo, 1.0)
+    assert torch.allclose(loss, torch.full_like(loss, np.log(4.0)), atol=1e-6) and grads[0].shape == (8, 4)
