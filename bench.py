@@ -531,7 +531,7 @@ def bench_slos_tree(args, res):
     for p in plans:
         p.close()
     res["slos_tree_m20_37inputs"] = {"ms": tree_ms, "ms_separate_plans": sep_ms, "speedup": sep_ms / tree_ms,
-                                     "inputs": len(inputs), "layer_launches": tree.layer_launches,
+                                     "inputs": len(inputs), "depth_first_launches": tree.layer_launches,
                                      "outputs": int(tree.offsets[-1]),
                                      "max_abs_sum_err": max(abs(v - 1.0) for v in sums)}
     tree.close()
@@ -635,7 +635,7 @@ def bench_gradient(args, res):
             mesh_adjoint(prog6, ph6, [1] * 6, t6, weights=lam)
     ms6 = t.ms / reps
     res["gradient_qml_m6_n6"] = {"ms_per_batch": ms6, "sets_per_s": 256 / (ms6 * 1e-3), "targets": len(t6),
-                                 "plans": (len(t6) + 63) // 64}
+                                 "plans": len(prog6._plans)}
     log(f"[bench] gradient of sum_s lambda_s P(s) over all {len(t6)} outputs, m=n=6: {ms6:.3f} ms per 256 sets")
     if not args.no_cpu:
         import oracle
