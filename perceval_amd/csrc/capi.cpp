@@ -3,6 +3,7 @@
 #include "common.h"
 #include "../../include/pcvl_hip.h"
 
+#include <cstring>
 #include <mutex>
 
 namespace pcvl {
@@ -10,6 +11,29 @@ namespace pcvl {
 static thread_local std::string g_last_error;
 
 void set_error(const std::string &msg) { g_last_error = msg; }
+
+hipError_t upload(void *dst, const void *src, size_t bytes)
+{
+    constexpr size_t STAGE = size_t(256) << 10;   // one buffer for the process, of any device
+    static std::mutex mu;
+    static void *stage = nullptr;
+    if (bytes > 8192 && bytes <= STAGE) {
+        std::unique_lock<std::mutex> lock(mu, std::try_to_lock);   // taken: a plain copy
+        if (lock.owns_lock()) {
+            if (!stage && hipHostMalloc(&stage, STAGE, hipHostMallocPortable) != hipSuccess) {
+                (void)hipGetLastError();
+                stage = nullptr;
+            }
+            if (stage) {
+                std::memcpy(stage, src, bytes);
+                hipError_t e = hipMemcpy(dst, stage, bytes, hipMemcpyHostToDevice);
+                if (e == hipSuccess) e = hipStreamSynchronize(nullptr);   // the buffer is free again
+                return e;
+            }
+        }
+    }
+    return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+}
 
 // One stream-ordered pool per device, created on first use.  Up to its
 // release threshold (512 MiB), memory freed into it stays mapped for the next

@@ -748,52 +748,20 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     for (int a = 2; a <= 12; a++) f32[(size_t)a] = f32[(size_t)a - 1] * (uint32_t)a;
     for (int a = 2; a <= nmax; a++) fd[(size_t)a] = fd[(size_t)a - 1] * (double)a;
     // suffix tables: per r, pf[beta] and slot[d][beta]
-    std::vector<double> spf;
-    std::vector<uint32_t> sslot;
     std::vector<uint32_t> tpf((size_t)nmax + 1), tslot((size_t)nmax + 1);
-    const BlkCum drop(w, nmax + 1, [&](int q, int x) { return q + 2 <= w ? blk_binom((int64_t)x + w - q - 3, w - q - 2) : 0; });
+    size_t nspf = 0, nslot = 0;
     for (int r = 0; r <= nmax; r++) {
-        const uint64_t S = nstates(w, r);
-        const int ns = std::min(r, w);
-        tpf[(size_t)r] = (uint32_t)spf.size();
-        tslot[(size_t)r] = (uint32_t)sslot.size();
-        const size_t p0 = spf.size(), s0 = sslot.size();
-        spf.resize(p0 + S);
-        sslot.resize(s0 + S * (size_t)ns, 0xffffffffu);
-        // beta has rank i; taking a photon from mode j lowers the photons after
-        // each mode q < j by one, which lowers the rank by
-        // sum_{q<j} C(after_q + w - q - 3, w - q - 2) (Pascal's rule on each
-        // term of the rank sum)
-        uint64_t i = 0;
-        blk_states(r, 0, drop, drop, [&](const BlkOcc *occ, int n, uint32_t, uint32_t, double pf) {
-            for (int d = 0; d < n; d++)
-                sslot[s0 + (size_t)d * S + i] = (((uint32_t)i - occ[d].e) << 5) | (uint32_t)occ[d].q;
-            spf[p0 + i] = pf;
-            i++;
-        });
+        tpf[(size_t)r] = (uint32_t)nspf;
+        tslot[(size_t)r] = (uint32_t)nslot;
+        nspf += nstates(w, r);
+        nslot += nstates(w, r) * (size_t)std::min(r, w);
     }
     // groups per layer: each sub-layer, suffix photons r = 0..kf; the blocks
     // of whole-wave groups get their walk precomputed (records)
     lay.cmax = std::max(1, std::min(h, nmax));
-    std::vector<BlkRec> recs;
-    // every block (K, r) in order: f(its occupied prefix modes (e: PE_j), their
-    // count, PE_h, B_k, prod alpha!)
-    const BlkCum ce(h, wt, [&](int q, int x) { return te[(size_t)q * wt + x] >> 32; });
-    const BlkCum ct(h, wt, [&](int q, int x) { return te[(size_t)q * wt + x] & 0xffffffffull; });
-    auto add_records = [&](int K, int r) {
-        blk_states(K, r, ce, ct, [&](const BlkOcc *occ, int n, uint32_t PEh, uint32_t Bk, double pf) {
-            BlkRec rec{};
-            rec.w[0] = Bk;
-            rec.w[1] = PEh;
-            rec.w[2] = (uint32_t)n;
-            for (int c = 0; c < n; c++) {
-                rec.w[4 + c / 4] |= (uint32_t)occ[c].q << (8 * (c % 4));
-                rec.w[10 + c] = occ[c].e;
-            }
-            std::memcpy(&rec.w[8], &pf, sizeof(double));
-            recs.push_back(rec);
-        });
-    };
+    struct Recs { int K, r; size_t first; };
+    std::vector<Recs> recs;
+    size_t nrec = 0;
     // records hold at most 16 occupied prefix modes and mode indices below 256
     const bool use_records = lay.cmax <= BLK_REC_MAX && h <= 256;
     std::vector<uint32_t> hert;   // (herald index, parent sub-layer offset) pairs
@@ -825,9 +793,10 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
                 if (g.S >= BLK_A_MIN && use_records) {
                     const auto key = std::make_pair(sub.kf - r, r);
                     auto rit = rec_of.find(key);
-                    if (rit == rec_of.end() && recs.size() + g.nb <= max_records) {
-                        rit = rec_of.emplace(key, (uint32_t)recs.size()).first;
-                        add_records(sub.kf - r, r);
+                    if (rit == rec_of.end() && nrec + g.nb <= max_records) {
+                        rit = rec_of.emplace(key, (uint32_t)nrec).first;
+                        recs.push_back({sub.kf - r, r, nrec});
+                        nrec += g.nb;
                     }
                     if (rit != rec_of.end()) {
                         rec = true;
@@ -882,10 +851,10 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
         lay.group_off[(size_t)k] = off;
         off += al(sizeof(BlkGroup) * lay.groups[(size_t)k].size());
     }
-    lay.off_pf = off; off += al(sizeof(double) * spf.size());
-    lay.off_slot = off; off += al(sizeof(uint32_t) * std::max<size_t>(sslot.size(), 1));
-    lay.nrec = recs.size();
-    lay.off_rec = off; off += al(sizeof(BlkRec) * std::max<size_t>(recs.size(), 1));
+    lay.off_pf = off; off += al(sizeof(double) * nspf);
+    lay.off_slot = off; off += al(sizeof(uint32_t) * std::max<size_t>(nslot, 1));
+    lay.nrec = nrec;
+    lay.off_rec = off; off += al(sizeof(BlkRec) * std::max<size_t>(nrec, 1));
     lay.off_front = off; off += al(sizeof(uint32_t) * std::max<size_t>(nwords, 1));
     lay.off_front_pf = off; off += al(sizeof(double) * std::max<size_t>(npf, 1));
     lay.bytes = off;
@@ -905,9 +874,43 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
     for (int k = 1; k <= lay.nlayers; k++)
         std::memcpy(host.data() + lay.group_off[(size_t)k], lay.groups[(size_t)k].data(),
                     sizeof(BlkGroup) * lay.groups[(size_t)k].size());
-    std::memcpy(host.data() + lay.off_pf, spf.data(), sizeof(double) * spf.size());
-    if (!sslot.empty()) std::memcpy(host.data() + lay.off_slot, sslot.data(), sizeof(uint32_t) * sslot.size());
-    if (!recs.empty()) std::memcpy(host.data() + lay.off_rec, recs.data(), sizeof(BlkRec) * recs.size());
+    // the large tables are written where they are sent from
+    double *spf = reinterpret_cast<double *>(host.data() + lay.off_pf);
+    uint32_t *sslot = reinterpret_cast<uint32_t *>(host.data() + lay.off_slot);
+    if (nslot) std::memset(sslot, 0xff, sizeof(uint32_t) * nslot);
+    const BlkCum drop(w, nmax + 1, [&](int q, int x) { return q + 2 <= w ? blk_binom((int64_t)x + w - q - 3, w - q - 2) : 0; });
+    for (int r = 0; r <= nmax; r++) {
+        const size_t S = nstates(w, r);
+        uint32_t *slot = sslot + tslot[(size_t)r];
+        double *pfs = spf + tpf[(size_t)r];
+        // beta has rank i; taking a photon from mode j lowers the photons after
+        // each mode q < j by one, which lowers the rank by
+        // sum_{q<j} C(after_q + w - q - 3, w - q - 2) (Pascal's rule on each
+        // term of the rank sum)
+        uint32_t i = 0;
+        blk_states(r, 0, drop, drop, [&](const BlkOcc *occ, int n, uint32_t, uint32_t, double pf) {
+            for (int d = 0; d < n; d++) slot[(size_t)d * S + i] = ((i - occ[d].e) << 5) | (uint32_t)occ[d].q;
+            pfs[i++] = pf;
+        });
+    }
+    // every block (K, r) in order, with its occupied prefix modes (e: PE_j),
+    // PE_h, B_k and prod alpha!
+    const BlkCum ce(h, wt, [&](int q, int x) { return te[(size_t)q * wt + x] >> 32; });
+    const BlkCum ct(h, wt, [&](int q, int x) { return te[(size_t)q * wt + x] & 0xffffffffull; });
+    for (const Recs &rs : recs) {
+        BlkRec *rec = reinterpret_cast<BlkRec *>(host.data() + lay.off_rec) + rs.first;
+        blk_states(rs.K, rs.r, ce, ct, [&](const BlkOcc *occ, int n, uint32_t PEh, uint32_t Bk, double pf) {
+            rec->w[0] = Bk;
+            rec->w[1] = PEh;
+            rec->w[2] = (uint32_t)n;
+            for (int c = 0; c < n; c++) {
+                rec->w[4 + c / 4] |= (uint32_t)occ[c].q << (8 * (c % 4));
+                rec->w[10 + c] = occ[c].e;
+            }
+            std::memcpy(&rec->w[8], &pf, sizeof(double));
+            rec++;
+        });
+    }
     // parent words of the first layers, all ones past a child's last parent
     uint32_t *fwords = reinterpret_cast<uint32_t *>(host.data() + lay.off_front);
     double *fpf = reinterpret_cast<double *>(host.data() + lay.off_front_pf);
@@ -929,7 +932,7 @@ int blk_layout_build_host_ex(int m, int nmax, int w, const std::vector<std::vect
                     for (int c = 0; c < n; c++) run(sub.par_base + Bk - occ[c].e, (uint32_t)occ[c].q);
                     const uint32_t add = ((sub.par_base + Bk - PEh) << 8) + (uint32_t)h;
                     for (int d = 0; d < ns; d++, at += cnt) {
-                        const uint32_t *slot = sslot.data() + tslot[(size_t)r] + (size_t)d * S;
+                        const uint32_t *slot = sslot + tslot[(size_t)r] + (size_t)d * S;
                         for (uint32_t b = 0; b < S; b++)
                             at[b] = slot[b] == 0xffffffffu ? slot[b] : ((slot[b] >> 5) << 8 | (slot[b] & 31u)) + add;
                     }
@@ -1222,7 +1225,7 @@ int blk_layout_upload(BlkLayout *lay, const std::vector<char> &image)
         set_error(std::string("hipMalloc(block SLOS tables): ") + hipGetErrorString(e));
         return ERR_ALLOC;
     }
-    e = hipMemcpy(lay->d_mem, image.data(), lay->bytes, hipMemcpyHostToDevice);
+    e = upload(lay->d_mem, image.data(), lay->bytes);
     if (e != hipSuccess) {
         (void)hipFree(lay->d_mem);
         lay->d_mem = nullptr;
