@@ -47,8 +47,9 @@ int pcvl_abi_version(void);
  *
  * Batch layout: matrix b has order h_n[b] (0..32) and occupies h_n[b]^2
  * complex elements, row-major, starting at complex element h_offsets[b] of
- * d_mats.  d_out receives one complex permanent per matrix.  Orders 9..28
- * share one persistent launch; orders 29..32 take a launch of their own.
+ * d_mats.  d_out receives one complex permanent per matrix.  Orders
+ * 0..10 share one launch, 11..28 one persistent launch; orders 29..32 take a
+ * launch of their own.
  * ------------------------------------------------------------------------- */
 typedef struct pcvl_perm_plan_s *pcvl_perm_plan;
 

@@ -12,13 +12,15 @@
 // shared and prod_{l' != l} c_l' is the product of a prefix and a suffix.
 //
 // Mapping: one launch for steps 1..9 of up to 64 modes (16 lanes a sample), then
-// one launch per photon step k, specialised on k so that each step
-// gets its own register allocation; within such a launch one wavefront owns one
-// sample (persistent over samples), or one slice of a sample's terms from step
-// 14 on.  The terms (2^{k-2}; from step 10 on fewer, repeated rows being summed
-// by multiplicity) are split over the 32 lane pairs; partial sums of the k
-// sub-permanents are reduced across the wave, then lane i computes the weight
-// of candidate row i and a wave prefix sum draws r_k.  Per-sample state (permuted columns, drawn modes)
+// one launch per photon step k, specialised on k so that each step gets its own
+// register allocation.  A wavefront owns one sample (persistent over samples) up
+// to step 13 and, for up to CC_ONE_WAVE_COUNT samples, up to CC_ONE_WAVE; above,
+// one slice of a sample's terms.  The terms (2^{k-2}; fewer from step 10 on, or
+// from 14 on above CC_MULTI_MODES modes, where repeated rows are summed by
+// multiplicity) are split over the 32 lane pairs; partial sums of the k
+// sub-permanents are reduced across the wave, then lane i computes the weight of
+// candidate row i and a wave prefix sum draws r_k.  Per-sample state (permuted
+// columns, drawn modes)
 // lives in a caller-provided workspace.  Random numbers
 // are the counter-based uniforms of common.h: stream = sample index, counters
 // 0..n-2 for the column permutation (Fisher-Yates, i = n-1 down to 1) and

@@ -279,8 +279,9 @@ typedef int gv_i4 __attribute__((ext_vector_type(4)));
 constexpr int GURVITS_DIGITS = 6;   // of 13 bits: 2^77 a, |a| < 1
 constexpr int GURVITS_SPAN = 24;    // 2^-77 is the last bit of components down to 2^-24 of the row's largest
 // Rounds of waves that a call is cut into: each part is dispatched as its own
-// workgroup (64 matrices of order 30, 10^6 samples: 2.03 ms; 2.21 ms with four
-// rounds on resident waves, whose compute units do not run at one speed).
+// workgroup (64 matrices of order 30, 10^6 samples, at five digits: 2.03 ms; 2.21
+// ms with four rounds on resident waves, whose compute units do not run at one
+// speed).
 constexpr int GURVITS_ROUNDS = 8;
 // Fragments kept at a time (10,922 matrices of orders up to 16, 5,461 above): a
 // call's workspace does not grow with its matrices beyond this.

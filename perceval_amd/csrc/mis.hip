@@ -252,8 +252,11 @@ __global__ void mis_gather_kernel(const int32_t *__restrict__ prop, const int64_
 // One wavefront per proposal; lanes take (o, inner chunk) units.
 constexpr int MISP_MAX_N = 28;
 
-// Low rows of the block loop (glynn_blocks.h): two up to order 24, one above,
-// as in the permanent kernel; below order 6 there is no block loop.
+// Low rows of the block loop (glynn_blocks.h): two up to order 24, one above;
+// below order 6 there is no block loop.  Two -> one at m = 60: 4,000 proposals of
+// order 21 6.09 -> 6.63 ms, 2,000 of 22 5.86 -> 6.22, 512 of 24 6.21 -> 6.28 (21..24
+// spill 56..88 bytes with two); 256 of order 25 6.48 -> 6.37, 128 of 26 7.72 ->
+// 7.01, 32 of 28 17.6 -> 9.0.
 constexpr int MISP_PAIR_MIN = 6;
 constexpr int misp_low_rows(int n) { return n <= 24 ? 2 : 1; }
 

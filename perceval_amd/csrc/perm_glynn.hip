@@ -53,8 +53,10 @@ struct PermItem {
 
 // Low rows of an order: two up to order 24, one above.  A pair's state is 16
 // VGPRs with two (T, T', E_1, E_2) and 12 with one, and two waves per SIMD
-// leave 256: 256 order-24 matrices take 6.80 ms with two (8.83 before), orders
-// 25 and up would spill inside the block loop.
+// leave 256: 22..24 spill 12..56 bytes and gain all the same, above the spills
+// are inside the block loop.  Two -> one: 1,024 of order 21 3.40 -> 3.80 ms, 256 of
+// 23 3.62 -> 3.94, 128 of 24 3.69 -> 3.99, 64 of 25 4.22 -> 4.19, 32 of 26 5.83 ->
+// 4.38, 8 of 28 9.40 -> 5.09.
 constexpr int PERM_LOW2_MAX = 24;
 constexpr int perm_low_rows(int n, bool one) { return (n <= PERM_LOW2_MAX && !one) ? 2 : 1; }
 

@@ -2,10 +2,10 @@
 
 Replaces ``xq.permanent_cx`` (perceval/backends/_naive.py:70-71).  A batch is a
 packed complex128 device tensor holding row-major matrices back to back; the
-orders may differ from matrix to matrix (0..32); orders 9..28 are handled in
-one persistent launch, orders 29..32 in a second one.  ``PermanentPlan`` keeps the launch plan for a batch shape so
-repeated batches (sampler acceptance, Naive all_prob over a fixed Fock space)
-pay the host-side scheduling once.
+orders may differ from matrix to matrix (0..32); orders 0..10 are handled in
+one launch, 11..28 in a persistent one and 29..32 in another.  ``PermanentPlan``
+keeps the launch plan for a batch shape so repeated batches (sampler acceptance,
+Naive all_prob over a fixed Fock space) pay the host-side scheduling once.
 """
 from __future__ import annotations
 
