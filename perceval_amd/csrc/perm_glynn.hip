@@ -345,9 +345,11 @@ constexpr int PERM_ROWS = 16;
 constexpr int64_t PERM_ROW_LAUNCH = int64_t(1) << 22;   // matrices of one launch, milliseconds of work
 constexpr int PERM_ROW_LD = PERM_SMALL_MAX * PERM_SMALL_MAX + 1;   // the four matrices of a wave on different banks
 
+// nthread: the first matrix of 16 lanes in this launch; the ones before take a
+// thread each in the first launch (first > 0).
 __global__ void __launch_bounds__(16 * PERM_ROWS, 4) perm_small_kernel(
     const double *__restrict__ mats, const int64_t *__restrict__ idx, const int64_t *__restrict__ offs,
-    const int32_t *__restrict__ ns, int64_t count, int64_t nthread, int64_t row0, unsigned first, cd *__restrict__ out)
+    const int32_t *__restrict__ ns, int64_t count, int64_t nthread, unsigned first, cd *__restrict__ out)
 {
     __shared__ cd s_mat[PERM_ROWS * PERM_ROW_LD];
     if (blockIdx.x < first) {
@@ -356,7 +358,7 @@ __global__ void __launch_bounds__(16 * PERM_ROWS, 4) perm_small_kernel(
         return;
     }
     const int lane = threadIdx.x & 15, row = threadIdx.x >> 4;
-    const int64_t k = row0 + (int64_t)(blockIdx.x - first) * PERM_ROWS + row;
+    const int64_t k = nthread + (int64_t)(blockIdx.x - first) * PERM_ROWS + row;
     const bool in = k < count;
     const int n = in ? ns[k] : 0;
     cd *A = s_mat + row * PERM_ROW_LD;
@@ -793,7 +795,7 @@ extern "C" int pcvl_perm_plan_execute(pcvl_perm_plan plan, const double *d_mats,
             const int64_t end = std::min(p.nsmall, row0 + PERM_ROW_LAUNCH);
             const unsigned rows = (unsigned)((end - row0 + PERM_ROWS - 1) / PERM_ROWS);
             hipLaunchKernelGGL(perm_small_kernel, dim3(first + rows), dim3(16 * PERM_ROWS), 0, stream, d_mats,
-                               p.d_small_idx, p.d_small_off, p.d_small_n, end, p.nthread, row0, first, out);
+                               p.d_small_idx, p.d_small_off, p.d_small_n, end, row0, first, out);
             PCVL_HIP_CHECK(hipGetLastError());
             first = 0;
             row0 = end;
