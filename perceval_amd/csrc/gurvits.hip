@@ -500,24 +500,25 @@ __global__ void __launch_bounds__(64, NP <= 16 ? 4 : 3) gurvits_int8_kernel(cons
 
 // scale: powers of two of the matrices' rows that the sums leave out (NULL or
 // GURVITS_FP64: none).
-// lanes: 64 a matrix, or one where it has few parts (200,000 matrices of order 12
+// LANES: 64 a matrix, or one where it has few parts (200,000 matrices of order 12
 // and one part: 1,021 -> 956 us a call).
-__global__ void gurvits_finalize_kernel(const double *__restrict__ partial, int64_t count, int parts, int lanes,
-                                        int64_t iters,
+template <int LANES>
+__global__ void gurvits_finalize_kernel(const double *__restrict__ partial, int64_t count, int parts, int64_t iters,
                                         const int32_t *__restrict__ scale, cd *__restrict__ est,
                                         double *__restrict__ err)
 {
-    const int64_t b = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / lanes;
-    const int lane = threadIdx.x & (lanes - 1);
+    const int64_t b = (int64_t)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const int lane = threadIdx.x % LANES;
     if (b >= count) return;
     double sr = 0.0, si = 0.0, sq = 0.0;
-    for (int q = lane; q < parts; q += lanes) {
+    for (int q = lane; q < parts; q += LANES) {
         const double *pp = partial + 3 * (b * parts + q);
         sr += pp[0];
         si += pp[1];
         sq += pp[2];
     }
-    for (int o = lanes >> 1; o >= 1; o >>= 1) {
+#pragma unroll
+    for (int o = LANES / 2; o >= 1; o >>= 1) {
         sr += __shfl_xor(sr, o, 64);
         si += __shfl_xor(si, o, 64);
         sq += __shfl_xor(sq, o, 64);
@@ -673,8 +674,9 @@ extern "C" int pcvl_gurvits_batch(const double *d_mats, const int32_t *h_n, cons
             rc = launch_gurvits<48>(mats, d_items, count, parts, iters, per, seed, stream0, d_part, nullptr, stream);
         if (rc == OK) {
             const int lanes = parts < 16 ? 1 : 64;
-            hipLaunchKernelGGL(gurvits_finalize_kernel, dim3((unsigned)((count * lanes + 255) / 256)), dim3(256), 0, stream,
-                               d_part, count, parts, lanes, iters, d_scale, reinterpret_cast<cd *>(d_est), d_err);
+            hipLaunchKernelGGL(lanes == 1 ? gurvits_finalize_kernel<1> : gurvits_finalize_kernel<64>,
+                               dim3((unsigned)((count * lanes + 255) / 256)), dim3(256), 0, stream, d_part, count, parts,
+                               iters, d_scale, reinterpret_cast<cd *>(d_est), d_err);
             e = hipGetLastError();
             if (e != hipSuccess) { set_error(std::string("gurvits finalize: ") + hipGetErrorString(e)); rc = ERR_HIP; }
         }
