@@ -14,8 +14,8 @@
 // Mapping: one launch for steps 1..9 of up to 64 modes (16 lanes a sample), then
 // one launch per photon step k, specialised on k so that each step gets its own
 // register allocation.  A wavefront owns one sample (persistent over samples) up
-// to step 13 and, for up to CC_ONE_WAVE_COUNT samples, up to CC_ONE_WAVE; above,
-// one slice of a sample's terms.  The terms (2^{k-2}; fewer from step 10 on, or
+// to step 13 and, by the rule of cc_one_wave, in steps 14 and 15; above, one slice
+// of a sample's terms.  The terms (2^{k-2}; fewer from step 10 on, or
 // from 14 on above CC_MULTI_MODES modes, where repeated rows are summed by
 // multiplicity) are split over the 32 lane pairs; partial sums of the k
 // sub-permanents are reduced across the wave, then lane i computes the weight of
@@ -170,13 +170,25 @@ constexpr int CC_MULTI_MODES = 64;
 // would lose the four extra launches).
 constexpr int CC_SLICED = 14;
 constexpr int CC_MAX_C = 8;
-// Up to step 15 and so many samples, one wave runs a sample's (two) slices one
-// after another and draws: one launch a step instead of five.  100 modes, 100
-// samples of 14 and 15 photons 230 -> 218 us and 328 -> 309, 5,000 of 15 856 ->
-// 769 us; 20,000 of 15 in 60 modes would take 2,234 us instead of 2,116, and one
-// of 16 with its step in it 262 us instead of 244.
+// Steps of two slices at most that one wave may run one after another, drawing at
+// their end: one launch a step instead of five.  Step 14 gains up to 8,192 samples
+// (100 modes, 100 samples 230 -> 218 us; 48 modes, one sample 178 -> 164).  Step 15
+// gains where many samples fill the waves and few of them repeat rows (60 modes,
+// 1,000 samples 314 -> 287 us, 2,000 410 -> 366; 100 modes, 5,000 856 -> 769); with
+// few samples the second slice is waited for (30 modes, one sample 204 -> 219 us,
+// 64 243 -> 270, 500 282 -> 306; 38 modes, 256 280 -> 303; 100 modes, one 254 ->
+// 282, but 16 305 -> 301), with many up to 64 modes slices balance better (38
+// modes, 8,000 874 -> 900).  Of 16 photons, step 16 in it would take 262 us instead
+// of 244.
 constexpr int CC_ONE_WAVE = 15;
 constexpr int64_t CC_ONE_WAVE_COUNT = 8192;
+constexpr bool cc_one_wave(int k, int m, int64_t count)
+{
+    if (k < CC_SLICED) return true;
+    if (k > CC_ONE_WAVE || count > CC_ONE_WAVE_COUNT) return false;
+    if (k < CC_ONE_WAVE) return true;
+    return m > CC_MULTI_MODES ? count >= 4 : m > 32 && count >= 512 && count <= CC_ONE_WAVE_COUNT / 2;
+}
 
 // Most slices of a sample at step k: at most 2^13 terms each up to step 27
 // (0.2 ms of one wave: the tail when the last slices drain), 4,096 slices
@@ -948,7 +960,7 @@ static CCSliceWork cc_slice_layout(int n, int64_t chunk)
 // sample at least.
 static CCSliceWork cc_slice_work(int n, int64_t count, size_t room = SIZE_MAX)
 {
-    if (n <= CC_ONE_WAVE && count <= CC_ONE_WAVE_COUNT) return {};   // every step in one wave per sample
+    if (n < CC_ONE_WAVE && count <= CC_ONE_WAVE_COUNT) return {};   // every step in one wave per sample
     const size_t per_sample = (size_t)cc_slice_cap(n) * ((size_t)n * sizeof(cd) + sizeof(uint64_t));
     int64_t lo = std::min<int64_t>(count, 1);
     int64_t hi = std::min(count, std::max<int64_t>(1, (int64_t)(CC_PART_BYTES / std::max<size_t>(per_sample, 1))));
@@ -971,7 +983,7 @@ static int launch_step(int k, const cd *U, int m, int n, int64_t count, uint64_t
         return ERR_ARG;
     } else {
         if (k != K) return launch_step<K + 1>(k, U, m, n, count, seed, first, pc, r, w, work, cus, st, gidx);
-        if (K < CC_SLICED || (K <= CC_ONE_WAVE && count <= CC_ONE_WAVE_COUNT)) {
+        if (cc_one_wave(K, m, count)) {
             constexpr int KS = K <= CC_ONE_WAVE ? K : 1;   // the others have no such kernel
             auto kp = cc_step_kernel<KS, (KS >= CC_MULTI)>;
             if constexpr (KS >= CC_MULTI && KS < CC_SLICED) {

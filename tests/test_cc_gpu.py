@@ -213,8 +213,8 @@ def test_backend_samples_for_inputs(gpu):
 
 @pytest.mark.parametrize("m,n", [(20, 14), (24, 15), (66, 15)])
 def test_one_wave_per_sample_and_slices_agree(gpu, m, n):
-    """Steps 14 and 15 run in one wave per sample up to 8,192 samples and in
-    slices above: the same samples, and the oracle's seed for seed."""
+    """Steps 14 and 15 run in one wave per sample or in slices by the number of
+    samples: the same samples, and the oracle's seed for seed."""
     from perceval_amd.sampling import cc_samples
     U = haar_unitary(m, seed=m + n)
     inp = [1] * n + [0] * (m - n)
@@ -223,6 +223,20 @@ def test_one_wave_per_sample_and_slices_agree(gpu, m, n):
     assert np.array_equal(cc_samples(U, inp, 8192, seed=6), sliced[:8192])
     assert np.array_equal(cc_samples(U, inp, 8, seed=6, first_sample=8192), sliced[8192:])
     assert np.array_equal(oracle.cc_samples(U, inp, 40, seed=6), sliced[:40])
+
+
+@pytest.mark.parametrize("m,n,counts", [(32, 15, (511, 512)), (33, 16, (511, 512, 4096, 4097)), (65, 15, (3, 4))])
+def test_step_15_in_one_wave_or_in_slices(gpu, m, n, counts):
+    """The sample counts between which step 15 changes its kernel, above 32 and
+    above 64 modes: the same samples on both sides, in a workspace of the size
+    that the library names."""
+    from perceval_amd.sampling import cc_samples
+    U = haar_unitary(m, seed=m + n)
+    inp = [1] * n + [0] * (m - n)
+    ref = cc_samples(U, inp, max(counts), seed=8)
+    assert np.array_equal(oracle.cc_samples(U, inp, 3, seed=8), ref[:3])
+    for count in counts:
+        assert np.array_equal(cc_samples(U, inp, count, seed=8), ref[:count])
 
 
 @pytest.mark.parametrize("m,n", [(64, 13), (65, 10), (65, 13), (80, 14), (128, 11)])
