@@ -162,8 +162,13 @@ def _target_rows(targets) -> np.ndarray:
     other type goes through lists."""
     if type(targets) is np.ndarray and targets.ndim == 2 and targets.dtype.kind in "iu":
         rows = np.ascontiguousarray(targets, dtype=np.int32)
-        if rows.dtype != targets.dtype and not np.array_equal(rows, targets):
-            raise OverflowError("target occupation out of bounds for int32")
+        if rows.dtype != targets.dtype:
+            # signed numbers as bytes: 3 us less of a call than a comparison of
+            # the arrays, which unsigned ones need (their wrapped bytes are the same)
+            same = (rows.astype(targets.dtype).tobytes() == targets.tobytes() if targets.dtype.kind == "i"
+                    else np.array_equal(rows, targets))
+            if not same:
+                raise OverflowError("target occupation out of bounds for int32")
         return rows
     return np.ascontiguousarray(np.asarray([list(t) for t in targets], dtype=np.int32))
 
@@ -182,7 +187,7 @@ def mesh_adjoint(program: MeshProgram, phases, in_occ, targets, want_probs: bool
     linear in the targets).  The program keeps one MeshPlan per (input
     state, targets)."""
     import torch
-    in_occ = tuple(int(v) for v in in_occ)
+    in_occ = tuple(map(int, in_occ))
     targets = _target_rows(targets)
     w = None if weights is None else np.asarray(weights, dtype=np.float64).reshape(-1)
     if w is not None and w.size != len(targets):
@@ -207,7 +212,7 @@ def mesh_adjoint(program: MeshProgram, phases, in_occ, targets, want_probs: bool
         wp = None if w is None else w[t0:t0 + size]
         t0 += size
         if not (wp is None and plan.weights is None) and not (wp is not None and plan.weights is not None
-                                                              and np.array_equal(wp, plan.weights)):
+                                                              and wp.tobytes() == plan.weights.tobytes()):
             plan.set_weights(wp)
         res = plan(phases, want_probs)
         loss = res[0] if loss is None else loss + res[0]
