@@ -124,7 +124,7 @@ class MeshPlan:
             raise ValueError(f"expected {self.ntargets} target weights, got {w.size}")
         _native.check(self._lib.pcvl_mesh_plan_set_weights(self._plan, w.ctypes.data_as(ctypes.POINTER(ctypes.c_double))),
                       "pcvl_mesh_plan_set_weights")
-        self.weights = w
+        self.weights = w.copy()   # the caller's array may change
 
     def __call__(self, phases, want_probs: bool = False, stream=None):
         import torch

@@ -360,3 +360,16 @@ def test_levels_of_more_cells_than_slots_vs_torch(gpu, m):
     tol = 1e4 * 2.0 ** -53 * max(1.0, np.abs(weights).sum())
     assert np.max(np.abs(loss.cpu().numpy() - ref_l)) < tol
     assert np.max(np.abs(grad.cpu().numpy() - ref_g)) < tol * max(1.0, np.abs(ref_g).max())
+
+
+def test_weights_changed_in_place_are_used(gpu):
+    """A call uses the weights as they are then, also where the caller changed the
+    array of the call before: twice the weights give exactly twice the results."""
+    from perceval_amd.gradient import mesh_adjoint
+    _, prog, phases, targets = _setup(batch=3)
+    w = np.linspace(-1.0, 2.0, len(targets))
+    loss, grad = mesh_adjoint(prog, phases, IN, targets, weights=w)
+    w *= 2.0
+    loss2, grad2 = mesh_adjoint(prog, phases, IN, targets, weights=w)
+    assert np.array_equal(2.0 * loss.cpu().numpy(), loss2.cpu().numpy())
+    assert np.array_equal(2.0 * grad.cpu().numpy(), grad2.cpu().numpy())
